@@ -1,0 +1,72 @@
+"""The many-days kernel (the graph-free path of step_days) against the eager path,
+one launch per day and part, which the parity tests pin to the oracle: every state
+field, the day's outputs and the daily station series, bit for bit.
+
+The sizes are where it can go wrong: grids below, at and above one wavefront, call
+lengths that take different wavefront tables (levels per wavefront) and that make the
+ring of transported volumes wrap, members, and cells with lakes, reservoirs, inland
+sinks and no land."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def run(wg, w, f, members, calls, profiled):
+    m = wg.WaterBalanceModel(w, n_members=members)
+    rng = np.random.default_rng(3)
+    if members > 1:
+        m.set_member_params(gamma=rng.uniform(0.2, 4.0, (members, w.n)), cfa=rng.uniform(0.7, 1.3, (members, w.n)))
+        m.set_forcing_perturbation(np.arange(5, 5 + members, dtype=np.uint64))
+    m.set_stations(np.unique(np.concatenate([w.basin_outlet, [0, w.n // 2]])).astype(np.int32))
+    m.load_forcing(f)
+    day, daily = 0, []
+    for k in calls:
+        m.step_days(day, day % 365 + 1, k, profiled=profiled)
+        daily.append(m.station_discharge(max_days=k)[1])
+        day += k
+    states = [m.get_state(q) for q in range(members)]
+    outs = [m.day_outputs(q) for q in range(members)]
+    total = m.station_discharge()[0]
+    m.close()
+    return states, outs, total, np.concatenate(daily, axis=1)
+
+
+@pytest.mark.parametrize("rows, cols, members, calls", [
+    (1, 1, 1, [8, 9]), (7, 9, 1, [9, 1]), (8, 8, 2, [8]), (5, 13, 1, [10]),
+    (40, 50, 1, [8] * 9), (40, 50, 3, [40, 33, 2, 70]), (30, 41, 1, [120])])
+def test_many_days_equals_eager(wg, rows, cols, members, calls):
+    print("case: many days", rows, cols, members, calls[:3], flush=True)
+    w = wg.World(wg.regional_spec(seed=rows * 100 + cols, nrows=rows, ncols=cols, edge_cases=rows * cols > 60,
+                                  glolake_every=9, res_every=14))
+    if w.n > 100:
+        w.contfreq[::37] = 0.0  # cells without land keep a zero volume
+    f = w.forcing(seed=2, day0=0, n_days=sum(calls))
+    a = run(wg, w, f, members, calls, False)
+    b = run(wg, w, f, members, calls, True)
+    for q in range(members):
+        for k in b[0][q]:
+            assert np.array_equal(np.asarray(a[0][q][k]), np.asarray(b[0][q][k]), equal_nan=True), (q, k)
+        for k in b[1][q]:
+            assert np.array_equal(a[1][q][k], b[1][q][k], equal_nan=True), (q, k)
+    assert np.array_equal(a[2], b[2], equal_nan=True)
+    assert np.array_equal(a[3], b[3], equal_nan=True)
+
+
+def test_autotune_on_the_many_days_path(wg):
+    """The tuner's saved state leaves the tables and the ring alone that its own first
+    call of the many-days kernel makes."""
+    print("case: many days, autotune of 12 days", flush=True)
+    w = wg.World(wg.regional_spec(seed=4, nrows=20, ncols=21))
+    f = w.forcing(seed=3, day0=0, n_days=30)
+    out = []
+    for tune in (True, False):
+        m = wg.WaterBalanceModel(w)
+        m.load_forcing(f)
+        if tune:
+            m.autotune(n_days=12)
+        m.step_days(0, 1, 30)
+        out.append(m.get_state())
+        m.close()
+    for k in out[0]:
+        assert np.array_equal(np.asarray(out[0][k]), np.asarray(out[1][k])), k

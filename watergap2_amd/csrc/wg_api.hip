@@ -34,6 +34,14 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+// A division of the grid's cells over the wavefronts of the many-days kernel.
+struct WgDayTable {
+  int32_t n_waves = 0;
+  WgDayWave *waves = nullptr;
+  WgDaySlot *slots = nullptr;
+  uint8_t *ranks = nullptr;
+};
+
 // One partition of the routing groups.  With two partitions the deepest groups
 // form the first; each partition's days run as a graph of its own on a stream of
 // its own, so that the long walk of the deep groups overlaps the other groups'
@@ -70,6 +78,17 @@ struct wg_handle {
   // d_wave_items[i][d_wave_item_off[i][W g + w] .. [W g + w + 1])
   int32_t *d_wave_wide = nullptr, *d_wave_item_off[2] = {nullptr, nullptr};
   WgWaveItem *d_wave_items[2] = {nullptr, nullptr};
+  // many-days kernel: the cells of each level, its wavefront tables (keyed by levels
+  // per wavefront), the wavefronts that fit on the chip at once, and the ring of
+  // transported volumes of the last ring_slots days (allocated by the first call
+  // that needs it; ring_day days written since it was cleared)
+  std::vector<int32_t> day_level_cells;
+  std::map<int32_t, WgDayTable> day_tables;
+  int64_t day_capacity = 0;
+  unsigned long long *d_ring = nullptr;
+  int32_t ring_slots = 0;
+  int64_t ring_day = 0;
+  int32_t *host_flow_error = nullptr;  // pinned, written by the many-days kernel at its spin limit
   // host copies needed at the boundary
   std::vector<double> snow_ch0;   // [M][N] channel 0 of G_SnowInElevation (never read by calcNewDay)
   WgStatic S{};
@@ -581,6 +600,137 @@ void wave_tables(const wg_handle *H, int nw, std::vector<int32_t> &item_off, std
   if (items.empty()) items.push_back(WgWaveItem{0, 0, 0, 0});
 }
 
+// Wavefronts of the many-days kernel: the cells of the whole grid in (level, device)
+// order, up to 64 at a time spanning at most `span` levels, so that a wavefront only
+// needs cells of its own and of earlier wavefronts.  The number of wavefronts and
+// the most levels in one follow from the cells per level alone.
+struct DayPlan {
+  int32_t span, n_waves, max_levels;
+};
+
+DayPlan day_plan(const std::vector<int32_t> &level_cells, int32_t span) {
+  DayPlan d{span, 0, 1};
+  int32_t l = 0, used = 0;  // next cell: number `used` of level l
+  const int32_t L = int32_t(level_cells.size());
+  while (l < L) {
+    const int32_t l0 = l;
+    int32_t last = l;
+    for (int32_t room = 64; room > 0 && l < L && l < l0 + span;) {
+      const int32_t take = std::min(room, level_cells[l] - used);
+      room -= take;
+      used += take;
+      last = l;
+      if (used == level_cells[l]) {
+        l++;
+        used = 0;
+      }
+    }
+    d.n_waves++;
+    d.max_levels = std::max(d.max_levels, last - l0 + 1);
+  }
+  return d;
+}
+
+void free_day_table(WgDayTable &t) {
+  void *bufs[] = {t.waves, t.slots, t.ranks};
+  for (void *b : bufs)
+    if (b) (void)hipFree(b);
+  t = WgDayTable{};
+}
+
+// The wavefronts of a plan; a cell's rank is its number of upstream cells in a row
+// within its wavefront.
+int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
+  const int32_t n = H->n;
+  std::vector<int32_t> at(H->day_level_cells.size() + 1, 0), order(n), gstart(n), lane(n, -1);
+  for (size_t l = 0; l + 1 < at.size(); l++) at[l + 1] = at[l] + H->day_level_cells[l];
+  for (int32_t p = 0; p < n; p++) order[at[H->clink[p].level]++] = p;
+  for (int32_t gg = 0; gg < H->n_groups; gg++) {
+    const int32_t gs = H->level_off[H->group_first_level[gg]], ge = H->level_off[H->group_first_level[gg + 1]];
+    for (int32_t p = gs; p < ge; p++) gstart[p] = gs;
+  }
+  std::vector<WgDayWave> waves;
+  std::vector<WgDaySlot> slots(size_t(plan.n_waves) * 64, WgDaySlot{-1, 0, 0xffffffffu, 0xffffffffu});
+  std::vector<uint8_t> ranks(size_t(plan.n_waves) * 64, 0);
+  for (int32_t i = 0; i < n;) {  // `lane` holds the lanes of the wavefront being built
+    WgDayWave w{1, 0};
+    const size_t base = waves.size() * 64;
+    const int32_t l0 = H->clink[order[i]].level;
+    int32_t j = i;
+    for (; j < n && j - i < 64 && H->clink[order[j]].level < l0 + plan.span; j++) lane[order[j]] = j - i;
+    if (int32_t(waves.size()) >= plan.n_waves) return fail(H, WG_E_STATE, "many-days plan and wavefronts differ");
+    for (int32_t k = i; k < j; k++) {
+      const int32_t p = order[k];
+      const WgChainLink &lk = H->clink[p];
+      uint64_t near = ~uint64_t(0);
+      int r = 0;
+      for (int u = 0; u < lk.nu; u++) {
+        const int32_t q = lane[gstart[p] + lk.up[u]];
+        if (q < 0) continue;
+        near = (near & ~(uint64_t(0xff) << (8 * u))) | (uint64_t(q) << (8 * u));
+        r = std::max(r, int(ranks[base + q]) + 1);
+      }
+      slots[base + (k - i)] = WgDaySlot{p, gstart[p], uint32_t(near), uint32_t(near >> 32)};
+      ranks[base + (k - i)] = uint8_t(r);
+      w.passes = std::max<int16_t>(w.passes, int16_t(r + 1));
+      w.nu = std::max(w.nu, lk.nu);
+    }
+    for (int32_t k = i; k < j; k++) lane[order[k]] = -1;
+    waves.push_back(w);
+    i = j;
+  }
+  t.n_waves = int32_t(waves.size());
+  // not among h->bufs: those are the state that wg_autotune saves and restores
+  auto put = [](auto **dst, const auto &v) {
+    const size_t bytes = v.size() * sizeof(v[0]);
+    return hipMalloc(reinterpret_cast<void **>(dst), bytes) == hipSuccess &&
+           hipMemcpy(*dst, v.data(), bytes, hipMemcpyHostToDevice) == hipSuccess;
+  };
+  if (put(&t.waves, waves) && put(&t.slots, slots) && put(&t.ranks, ranks)) return WG_OK;
+  (void)hipGetLastError();
+  free_day_table(t);
+  return WG_E_NOMEM;
+}
+
+// Chooses the wavefronts of a launch of `days` days: more levels per wavefront cost
+// each day a pass per level in the deepest-packed wavefront, fewer cost a hand over
+// between wavefronts per level once per launch.  Only plans whose wavefronts all
+// fit on the chip at once are taken: with more of them a day costs each its share
+// of the chip, and one launch per day and part, which keeps three wavefronts per
+// SIMD, was faster (64 members of the global grid: 1.99 ms a day against 2.6).
+// Calls of few days stay with it too: the hand overs along the deepest basin are
+// paid once per launch (one day of the global grid: 359 us a call against 502).
+// The chosen table is built by the first call that needs it and kept.  Returns NULL
+// when no plan fits or the memory for its tables is not there.
+constexpr int32_t kManyDaysMin = 8;
+const WgDayTable *day_table(wg_handle *h, int32_t days) {
+  constexpr double kHandOver = 2.5, kPass = 0.7;  // us
+  if (days < kManyDaysMin || h->day_capacity <= 0) return nullptr;
+  if (h->day_level_cells.empty()) {
+    h->day_level_cells.assign(size_t(h->max_depth), 0);
+    for (int32_t p = 0; p < h->n; p++) h->day_level_cells[h->clink[p].level]++;
+  }
+  DayPlan best{0, 0, 0};
+  double cost = 0.;
+  for (int32_t span : {1, 2, 4, 8, 16, 64}) {
+    const DayPlan d = day_plan(h->day_level_cells, span);
+    if (int64_t(d.n_waves) * h->m > h->day_capacity) continue;
+    const double c = kHandOver * h->max_depth / span + kPass * (double(days) * (d.max_levels - 1) + h->max_depth);
+    if (!best.span || c < cost) {
+      best = d;
+      cost = c;
+    }
+  }
+  if (!best.span) return nullptr;
+  auto it = h->day_tables.find(best.span);
+  if (it == h->day_tables.end()) {
+    WgDayTable t;
+    if (build_day_table(h, best, t)) return nullptr;
+    it = h->day_tables.emplace(best.span, t).first;
+  }
+  return &it->second;
+}
+
 int upload_tiles(wg_handle *h) {
   if (int32_t(h->tile_start.size()) > h->tile_capacity) return fail(h, WG_E_ARG, "tile table too large");
   HIP_CHECK(h, hipMemcpy(const_cast<int32_t *>(h->S.tile_start), h->tile_start.data(),
@@ -949,6 +1099,13 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
         if (r_) { *out = h.release(); return r_; }
       }
     }
+    {
+      int per_cu = 0, cus = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wg_days_kernel<false>, 64, kDaysLdsBytes) ==
+              hipSuccess &&
+          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, H->device) == hipSuccess)
+        H->day_capacity = int64_t(per_cu) * cus;
+    }
     // the largest upstream count of each level
     for (int32_t l = 0; l + 1 < int32_t(H->level_off.size()); l++) {
       int16_t mx = 0;
@@ -1023,6 +1180,10 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
   if (!rc) rc = dev_alloc(H, &H->d_clock, 1);
   if (!rc) rc = dev_alloc(H, &H->d_seeds, size_t(M));
   if (rc) { *out = h.release(); return rc; }
+  e = hipHostMalloc(reinterpret_cast<void **>(&H->host_flow_error), sizeof(int32_t), hipHostMallocDefault);
+  if (e != hipSuccess) { *out = h.release(); return WG_E_NOMEM; }
+  *H->host_flow_error = 0;
+  X.flow_error_host = H->host_flow_error;
   X.member_seed = H->d_seeds;
   X.perturb = 0;
   H->snow_ch0.assign(NM, 0.0);
@@ -1093,6 +1254,9 @@ extern "C" int wg_destroy(wg_handle *h) {
   for (auto &kv : h->graphs) (void)hipGraphExecDestroy(kv.second);
   for (auto &b : h->bufs) (void)hipFree(b.p);
   if (h->d_forcing) (void)hipFree(h->d_forcing);
+  if (h->d_ring) (void)hipFree(h->d_ring);
+  for (auto &kv : h->day_tables) free_day_table(kv.second);
+  if (h->host_flow_error) (void)hipHostFree(h->host_flow_error);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1325,7 +1489,8 @@ void launch_cell(wg_handle *h, const WgStatic &S, hipStream_t stream, dim3 grid,
   // the kernels without water use carry no use code
   auto *kern = h->snow_chunk == 10 ? (S.use_on ? wg_cell_kernel<10, true> : wg_cell_kernel<10, false>)
                                    : (S.use_on ? wg_cell_kernel<5, true> : wg_cell_kernel<5, false>);
-  hipLaunchKernelGGL(kern, grid, dim3(h->block_threads_cell), 0, stream, S, h->X, h->T, h->d_forcing,
+  hipLaunchKernelGGL(kern, grid, dim3(h->block_threads_cell),
+                     size_t(h->block_threads_cell / 64) * WG_EXP2_LDS_BYTES, stream, S, h->X, h->T, h->d_forcing,
                      h->n_forcing_days, h->d_clock, k, do_post, do_vertical, write_diag, slot);
 }
 
@@ -1440,9 +1605,61 @@ int check_step_args(wg_handle *h, int32_t forcing_day0, int32_t first_doy, int32
   return WG_OK;
 }
 
+// Ring of the many-days kernel for launches of up to `days` days (fewer when the
+// members' rows would take more than kRingBytes; at least kRingMinSlots).  Returns
+// false when the memory is not there.
+constexpr size_t kRingBytes = size_t(2) << 30;
+constexpr int32_t kRingMinSlots = 8;
+bool ensure_ring(wg_handle *h, int32_t days) {
+  const size_t row = size_t(h->m) * h->n * sizeof(double);
+  const int32_t cap = int32_t(std::max<size_t>(kRingMinSlots, std::min<size_t>(WG_DAILY_SLOTS, kRingBytes / row)));
+  const int32_t want = std::min(cap, std::max(days, 32));
+  if (h->ring_slots >= want) return true;
+  unsigned long long *fresh = nullptr;
+  if (hipMalloc(&fresh, row * want) != hipSuccess) {
+    (void)hipGetLastError();
+    return h->d_ring != nullptr;
+  }
+  if (hipMemsetAsync(fresh, 0, row * want, h->stream) != hipSuccess ||
+      hipStreamSynchronize(h->stream) != hipSuccess) {
+    (void)hipFree(fresh);
+    return h->d_ring != nullptr;
+  }
+  if (h->d_ring) (void)hipFree(h->d_ring);
+  h->d_ring = fresh;
+  h->ring_slots = want;
+  h->ring_day = 0;
+  return true;
+}
+
+// Launches `days` days of the many-days kernel, in launches of at most ring_slots.
+int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int days) {
+  for (int done = 0; done < days;) {
+    const int k = std::min(days - done, h->ring_slots);
+    auto *kern = h->S.use_on ? wg_days_kernel<true> : wg_days_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(t.n_waves, h->m), dim3(64), kDaysLdsBytes, h->stream, h->S, h->X, h->T,
+                       h->d_forcing, t.waves, t.slots, t.ranks, h->d_ring, h->ring_slots, h->ring_day, day + done,
+                       (doy - 1 + done) % 365 + 1, (h->started || done > 0) ? 1 : 0, k, done);
+    HIP_CHECK(h, hipGetLastError());
+    h->ring_day += k;
+    done += k;
+  }
+  return WG_OK;
+}
+
 // The dataflow chain kernel flags a walk that hit its spin limit (it cannot for a
 // valid schedule); the day's routing is then incomplete and the call fails.
 int check_flow_error(wg_handle *h) {
+  if (*static_cast<volatile int32_t *>(h->host_flow_error)) {
+    // the many-days kernel: its ring holds a partial day; start a fresh one
+    *h->host_flow_error = 0;
+    const int32_t zero = 0;
+    (void)hipFree(h->d_ring);
+    h->d_ring = nullptr;
+    h->ring_slots = 0;
+    HIP_CHECK(h, hipMemcpy(h->X.flow_error, &zero, sizeof(int32_t), hipMemcpyHostToDevice));
+    return fail(h, WG_E_STATE, "many-days routing exceeded its spin limit");
+  }
   if (h->chain_mode != 1) return WG_OK;
   int32_t flag = 0;
   HIP_CHECK(h, hipMemcpy(&flag, h->X.flow_error, sizeof(int32_t), hipMemcpyDeviceToHost));
@@ -1470,8 +1687,26 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   int remaining = n_days;
   int64_t launches = 0;
   const int n_parts = int(h->parts.size());
+  const WgDayTable *table = h->chain_mode == 3 ? day_table(h, std::min(block, n_days)) : nullptr;
+  if (table && !ensure_ring(h, std::min(block, n_days))) table = nullptr;
   while (remaining > 0) {
     const int k = std::min(block, remaining);
+    if (table) {
+      rc = launch_days(h, *table, day, doy, k);
+      if (rc) return rc;
+      if (h->n_stations > 0) {
+        const int nsm = h->n_stations * h->m;
+        hipLaunchKernelGGL(wg_station_reduce, dim3((nsm + 255) / 256), dim3(256), 0, h->stream, h->X,
+                           h->n_stations, h->m, 0, k);
+        HIP_CHECK(h, hipGetLastError());
+      }
+      h->started = true;
+      day += k;
+      doy = (doy - 1 + k) % 365 + 1;
+      remaining -= k;
+      launches++;
+      continue;
+    }
     hipLaunchKernelGGL(wg_clock_set, dim3(1), dim3(64), 0, h->stream, h->d_clock, day, doy, h->started ? 1 : 0);
     HIP_CHECK(h, hipGetLastError());
     if (n_parts < 2) {
@@ -1617,6 +1852,8 @@ extern "C" int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double
         if (md == 1 && h->max_depth > WG_MAX_GROUP_DEPTH) continue;
         // the wave walk runs 4 or 8 wavefronts (256 or 512 threads); the level walks up to 256 threads
         if (md == 3 ? (ch != 256 && ch != 512) : ch > 256) continue;
+        // mode 3 runs the many-days kernel, whose launch has no such choices: once
+        if (md == 3 && (c != 256 || ch != 256 || k != 5)) continue;
         rc = apply_config(h, c, ch, k, md);
         double ms = 0;
         // the first pass loads the kernels and captures the graphs of the path that
@@ -2097,7 +2334,7 @@ extern "C" int wg_libm_eval(int32_t fn, int32_t n, const double *x, const double
              hipMemcpy(dy, y ? y : x, b, hipMemcpyHostToDevice) != hipSuccess) {
     rc = WG_E_HIP;
   } else {
-    hipLaunchKernelGGL(wg_libm_kernel, dim3((n + 255) / 256), dim3(256), 0, 0, fn, n, dx, dy, dout);
+    hipLaunchKernelGGL(wg_libm_kernel, dim3((n + 255) / 256), dim3(256), 4 * WG_EXP2_LDS_BYTES, 0, fn, n, dx, dy, dout);
     if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
         hipMemcpy(out, dout, b, hipMemcpyDeviceToHost) != hipSuccess)
       rc = WG_E_HIP;

@@ -1,0 +1,418 @@
+// wg_days_kernel.h -- many days of the day loop in one launch: each wavefront keeps
+// 64 cells for all days of a block and passes transported volumes to the
+// wavefronts downstream through a ring in memory.
+//
+// Water moves only downstream, so day d of a cell needs day d of the cells above it
+// and its own day d - 1, nothing else: upstream wavefronts may run days ahead, and a
+// day costs a wavefront its own work instead of the slowest cell's day plus the
+// deepest group's walk (the bound of one launch per day and part).
+//
+// Ring: [slot][member][N] transported volumes of the last ring_slots days, slot =
+// (days since the ring was cleared) mod ring_slots.  A volume is never negative, so
+// its sign bit says which turn of the ring wrote it: a reader waits until the sign
+// is the turn's, and value and flag arrive in one 8-byte access at agent scope (the
+// XCDs' L2 caches are not coherent for plain accesses).  A launch covers at most
+// ring_slots days, so it never overwrites a volume that it has yet to read.
+//
+// Wavefronts take the cells in level order over the whole grid, so that one of them
+// spans few levels (often one): a level within a wavefront costs a pass of the
+// routing step each day, a level between wavefronts only delays the first day.
+//
+// Progress: a wavefront waits only for cells before its own in level order, never
+// for later ones, and workgroups start in index order; so the first unfinished
+// wavefront can always run.  A spin limit ends the launch with an error flag should
+// that ever fail.
+#ifndef WG_DAYS_KERNEL_H
+#define WG_DAYS_KERNEL_H
+
+namespace {
+
+// Per-cell statics kept in LDS, [field][64 lanes] doubles behind the exp/log/pow
+// table: read once per launch instead of once per day from memory.
+enum DayField : int {
+  DF_M_PREC, DF_ALPHA, DF_PET_MXDY, DF_M_NETRAD, DF_MCWH, DF_SNOWFZ, DF_SNOWMT, DF_GRADNT, DF_MELT, DF_ALBEDO,
+  DF_ALBEDO_SNOW, DF_EMIS, DF_LAI, DF_CLASS, DF_SMAX, DF_GWF, DF_GAMMA, DF_CFA, DF_PCRIT, DF_RGMAX, DF_AREA,
+  DF_AREA_M, DF_CF100, DF_FSWB, DF_E_GW, DF_INV_KGW, DF_OME_GW, DF_E_SW, DF_K_SW, DF_INV_KSW, DF_OME_SW,
+  DF_RED_EXP, DF_LL, DF_LL100, DF_LL_MAX, DF_LW, DF_LW100, DF_LW_MAX, DF_GW, DF_GW100, DF_GW_MAX, DF_LENGTH,
+  DF_BOTTOM, DF_VEL_C1, DF_VEL_C2, DF_RW_C0, DF_RW_C1, DF_RW_C2, DF_RW_C3, DF_RIVER_MAX, DF_MAX_RAF,
+  DF_COUNT,
+  DF_TV = DF_COUNT,  // the day's transported volumes of the wavefront's cells
+  DF_ROWS
+};
+constexpr int kDaysLdsBytes = WG_EXP2_LDS_BYTES + DF_ROWS * 64 * int(sizeof(double));
+
+// bits of DF_GWF's second word
+enum { DB_ARID = 1, DB_CUT = 2, DB_LDD = 4, DB_CONT = 8, DB_LAKE = 16, DB_RES = 32, DB_FULL_LAKE = 64 };
+
+struct WordPair {
+  int32_t a, b;
+};
+
+constexpr int kDaysSpinLimit = 1 << 22;
+
+}  // namespace
+
+template <bool kUse>
+__global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, WgTables T,
+                                                        const float *__restrict__ forcing,
+                                                        const WgDayWave *__restrict__ waves,
+                                                        const WgDaySlot *__restrict__ slots,
+                                                        const uint8_t *__restrict__ ranks,
+                                                        unsigned long long *ring, int32_t ring_slots,
+                                                        int64_t ring_day, int64_t fday0, int32_t doy0,
+                                                        int32_t started0, int32_t days, int32_t slot0) {
+  load_exp2_table();
+  const WgDayWave wv = waves[blockIdx.x];
+  const int lane = threadIdx.x;
+  const WgDaySlot slot = slots[blockIdx.x * 64 + lane];
+  const int p = slot.cell;
+  if (p < 0) return;
+  const int m = blockIdx.y;
+  const int n = S.n;
+  const int64_t mp = int64_t(m) * n + p;
+  double *F = wg_lds + WG_EXP2_LDS_BYTES / sizeof(double) + lane;
+  auto fld = [&](int f) -> double { return F[f * 64]; };
+
+  const WgChainLink link = load_link(S, p);
+  const int rank = ranks[blockIdx.x * 64 + lane];
+  auto near_lane = [&](int u) -> int { return int((u < 4 ? slot.near_lo : slot.near_hi) >> (8 * (u & 3)) & 0xffu); };
+  int bits = 0;
+  {
+    DayStatA a;
+    DayStatB b;
+    DayStatEnd e;
+    load_stat_a(S, T, p, a);
+    load_stat_b(S, X, mp, p, b);
+    load_stat_end(S, p, e);
+    const WgChainStatic cs = load_cstat(S, p);
+    bits = (b.arid ? DB_ARID : 0) | (b.recharge_cut ? DB_CUT : 0) | (b.ldd >= 0 ? DB_LDD : 0) |
+           (e.contcell ? DB_CONT : 0) | (e.lake_area > 0. ? DB_LAKE : 0) | (e.reservoir_area > 0. ? DB_RES : 0) |
+           (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0);
+    F[DF_M_PREC * 64] = a.m_prec;
+    F[DF_ALPHA * 64] = a.alpha;
+    F[DF_PET_MXDY * 64] = a.pet_mxdy;
+    F[DF_M_NETRAD * 64] = a.m_netrad;
+    F[DF_MCWH * 64] = a.mcwh;
+    F[DF_SNOWFZ * 64] = a.t_snowfz;
+    F[DF_SNOWMT * 64] = a.t_snowmt;
+    F[DF_GRADNT * 64] = a.t_gradnt;
+    F[DF_MELT * 64] = a.melt_factor;
+    F[DF_ALBEDO * 64] = a.albedo;
+    F[DF_ALBEDO_SNOW * 64] = a.albedo_snow;
+    F[DF_EMIS * 64] = a.emis;
+    F[DF_LAI * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, float(a.lmin)),
+                                                         __builtin_bit_cast(int32_t, float(a.lmax))});
+    F[DF_CLASS * 64] = __builtin_bit_cast(double, WordPair{a.initial_days, a.lct | (a.elev0 << 8)});
+    F[DF_SMAX * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.smax),
+                                                          __builtin_bit_cast(int32_t, b.built_up)});
+    F[DF_GWF * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.gw_factor), bits});
+    F[DF_GAMMA * 64] = b.gamma;
+    F[DF_CFA * 64] = b.cfa;
+    F[DF_PCRIT * 64] = b.pcritgwa;
+    F[DF_RGMAX * 64] = b.rgmax;
+    F[DF_AREA * 64] = b.area;
+    F[DF_AREA_M * 64] = b.area_m;
+    F[DF_CF100 * 64] = b.cf100;
+    F[DF_FSWB * 64] = b.fswb_catchment;
+    F[DF_E_GW * 64] = b.e_gw;
+    F[DF_INV_KGW * 64] = cs.inv_kgw;
+    F[DF_OME_GW * 64] = cs.ome_gw;
+    F[DF_E_SW * 64] = b.e_sw;
+    F[DF_K_SW * 64] = b.k_sw;
+    F[DF_INV_KSW * 64] = cs.inv_ksw;
+    F[DF_OME_SW * 64] = cs.ome_sw;
+    F[DF_RED_EXP * 64] = b.red_exp;
+    F[DF_LL * 64] = b.loc_lake;
+    F[DF_LL100 * 64] = b.ll100;
+    F[DF_LL_MAX * 64] = b.ll_max;
+    F[DF_LW * 64] = b.loc_wetland;
+    F[DF_LW100 * 64] = b.lw100;
+    F[DF_LW_MAX * 64] = b.lw_max;
+    F[DF_GW * 64] = b.glo_wetland;
+    F[DF_GW100 * 64] = b.gw100;
+    F[DF_GW_MAX * 64] = b.gw_max;
+    F[DF_LENGTH * 64] = b.river_length;
+    F[DF_BOTTOM * 64] = b.bottom;
+    F[DF_VEL_C1 * 64] = b.vel_c1;
+    F[DF_VEL_C2 * 64] = b.vel_c2;
+    F[DF_RW_C0 * 64] = e.rw_c0;
+    F[DF_RW_C1 * 64] = e.rw_c1;
+    F[DF_RW_C2 * 64] = e.rw_c2;
+    F[DF_RW_C3 * 64] = e.rw_c3;
+    F[DF_RIVER_MAX * 64] = e.river_stor_max;
+    F[DF_MAX_RAF * 64] = e.max_raf;
+    F[DF_TV * 64] = 0.;
+  }
+  const bool cont = (bits & DB_CONT) != 0;
+  // upstream cells: bit u of ext when upstream cell u belongs to an earlier wavefront
+  uint32_t ext = 0;
+  if (cont) {
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (u < link.nu && near_lane(u) == 0xff) ext |= 1u << u;
+  }
+
+  CellState s;
+  load_state_a(X, mp, s);
+  load_state_b(X, mp, s);
+  load_state_end(X, mp, s);
+  s.laf_prev = X.laf_prev[mp];
+  s.red_gl = X.red_gl[mp];
+  s.red_res = X.red_res[mp];
+  WgD2 *sp = X.snow2 + int64_t(m) * WG_DEV_NPAIR * n + p;
+  const int32_t *ep = S.elev_pairs + p;
+  const int64_t ring_stride = int64_t(S.n_members) * n;
+  const float *fd = forcing + fday0 * 4 * int64_t(n) + p;
+  float f0 = fd[0], f1 = fd[n], f2 = fd[2 * int64_t(n)], f3 = fd[3 * int64_t(n)];
+
+#pragma unroll 1
+  for (int k = 0; k < days; k++) {
+    const int64_t fday = fday0 + k;
+    const int doy = int((doy0 - 1 + k) % 365) + 1;
+    const DayInfo di = day_info(doy);
+    const int64_t gday = ring_day + k;
+    const int64_t turn = gday / ring_slots;
+    unsigned long long *rrow = ring + (gday - turn * ring_slots) * ring_stride + int64_t(m) * n;
+    const unsigned long long sign = (turn & 1) ? 0ull : 0x8000000000000000ull;
+    double *daily = X.st_daily + (int64_t(m) * WG_DAILY_SLOTS + slot0 + k) * S.n_stations;
+    double rem = 0.;
+    if (!cont) {
+      // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
+      // routing.cpp:1876); other cells keep a zero transported volume.
+      __hip_atomic_store(rrow + p, sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (link.station >= 0) daily[link.station] = 0.;
+    } else {
+      float tf = f0, pf = f1;
+      const float swf = f2, lwf = f3;
+      if (k + 1 < days) {
+        fd += 4 * int64_t(n);
+        f0 = fd[0];
+        f1 = fd[n];
+        f2 = fd[2 * int64_t(n)];
+        f3 = fd[3 * int64_t(n)];
+      }
+      if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
+      double use_desired = 0., use_nag = 0.;
+      int64_t use_t = 0;
+      if (kUse) use_t = day_use(S, X, mp, p, fday, di.month, use_desired, use_nag);
+      const double laf_prev = (started0 || k > 0) ? s.laf_prev : s.laf;  // daily.cpp:159-169
+      DayFlux v;
+      {
+        DayStatA a;
+        a.m_prec = fld(DF_M_PREC);
+        a.alpha = fld(DF_ALPHA);
+        a.pet_mxdy = 0.;
+        a.m_netrad = fld(DF_M_NETRAD);
+        a.mcwh = fld(DF_MCWH);
+        a.t_snowfz = fld(DF_SNOWFZ);
+        a.t_snowmt = fld(DF_SNOWMT);
+        a.t_gradnt = fld(DF_GRADNT);
+        a.melt_factor = fld(DF_MELT);
+        a.albedo = fld(DF_ALBEDO);
+        a.albedo_snow = fld(DF_ALBEDO_SNOW);
+        a.emis = fld(DF_EMIS);
+        const WordPair lai = __builtin_bit_cast(WordPair, fld(DF_LAI)), cl = __builtin_bit_cast(WordPair, fld(DF_CLASS));
+        a.lmin = __builtin_bit_cast(float, lai.a);
+        a.lmax = __builtin_bit_cast(float, lai.b);
+        a.initial_days = cl.a;
+        a.lct = cl.b & 0xff;
+        a.elev0 = cl.b >> 8;
+        a.arid = (bits & DB_ARID) != 0;
+        day_pet_canopy(a, s, v, tf, pf, swf, lwf, laf_prev);
+        day_snow<5>(a, s, v, laf_prev, sp, ep, n);
+      }
+      ChainRec c;
+      {
+        DayStatB b;
+        const WordPair sm = __builtin_bit_cast(WordPair, fld(DF_SMAX)), gf = __builtin_bit_cast(WordPair, fld(DF_GWF));
+        b.smax = __builtin_bit_cast(float, sm.a);
+        b.built_up = __builtin_bit_cast(float, sm.b);
+        b.gw_factor = __builtin_bit_cast(float, gf.a);
+        b.gamma = fld(DF_GAMMA);
+        b.cfa = fld(DF_CFA);
+        b.pet_mxdy = fld(DF_PET_MXDY);
+        b.t_snowfz = fld(DF_SNOWFZ);
+        b.pcritgwa = fld(DF_PCRIT);
+        b.rgmax = fld(DF_RGMAX);
+        b.recharge_cut = (bits & DB_CUT) != 0;
+        b.arid = (bits & DB_ARID) != 0;
+        b.ldd = (bits & DB_LDD) ? 0 : -1;
+        day_soil(b, s, v, laf_prev);
+        if (k == days - 1) {
+          X.d_surf[mp] = v.surf_runoff;
+          X.d_recharge[mp] = v.recharge;
+          X.d_ow_pet[mp] = v.ow_pet;
+          X.d_aet[mp] = v.aet;
+          X.d_prec[mp] = v.prec;
+        }
+        b.area = fld(DF_AREA);
+        b.area_m = fld(DF_AREA_M);
+        b.cf100 = fld(DF_CF100);
+        b.fswb_catchment = fld(DF_FSWB);
+        b.e_gw = fld(DF_E_GW);
+        b.inv_kgw = fld(DF_INV_KGW);
+        b.ome_gw = fld(DF_OME_GW);
+        b.e_sw = fld(DF_E_SW);
+        b.k_sw = fld(DF_K_SW);
+        b.red_exp = fld(DF_RED_EXP);
+        b.loc_lake = fld(DF_LL);
+        b.ll100 = fld(DF_LL100);
+        b.ll_max = fld(DF_LL_MAX);
+        b.loc_wetland = fld(DF_LW);
+        b.lw100 = fld(DF_LW100);
+        b.lw_max = fld(DF_LW_MAX);
+        b.glo_wetland = fld(DF_GW);
+        b.gw100 = fld(DF_GW100);
+        b.gw_max = fld(DF_GW_MAX);
+        b.river_length = fld(DF_LENGTH);
+        b.bottom = fld(DF_BOTTOM);
+        b.vel_b4 = -b.bottom / 4.0;
+        b.vel_b16 = b.bottom * b.bottom / 16.0;
+        b.vel_c1 = fld(DF_VEL_C1);
+        b.vel_c2 = fld(DF_VEL_C2);
+        // global lakes and reservoirs (one cell in a hundred) read their statics here
+        DayStatLake lake{0., 0., 0., 0., 0., 0.};
+        if ((bits & (DB_LAKE | DB_RES)) || (link.flags & (CFL_LAKE | CFL_RES))) {
+          load_stat_lake(S, p, lake);
+          if (kUse) lake.prov_rel = S.use_provrel[use_t];
+        }
+        c.inv_ksw = fld(DF_INV_KSW);
+        c.ome_sw = fld(DF_OME_SW);
+        c.inv_kgw = b.inv_kgw;
+        c.ome_gw = b.ome_gw;
+        c.area = b.area;
+        c.cf100 = b.cf100;
+        c.flags = link.flags;
+        PotTerms pot;
+        day_local_routing<kUse>(b, lake, s, v, use_desired, use_nag, c, pot);
+        if (X.pot_base) {
+          X.pot_base[mp] = pot.base;
+          X.pot_ow[mp] = pot.ow;
+        }
+      }
+      // transported volumes of upstream cells in earlier wavefronts: wait for the
+      // day's values (they are there already unless this wavefront has caught up)
+      unsigned long long t[8];
+      int spins = 0;
+      for (;;) {
+        bool ready = true;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (u < wv.nu && (ext >> u & 1)) {
+            t[u] = __hip_atomic_load(rrow + slot.group + uint16_t(link.up[u]), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            ready = ready && ((t[u] ^ sign) >> 63) == 0;
+          }
+        if (__builtin_amdgcn_ballot_w64(!ready) == 0) break;
+        if (++spins >= kDaysSpinLimit ||
+            ((spins & 1023) == 0 &&
+             __hip_atomic_load(X.flow_error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          __hip_atomic_store(X.flow_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(X.flow_error_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      const StepPre pre = step_pre<kUse>(c);
+      ChainOut o = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
+      for (int r = 0; r < wv.passes; r++) {
+        if (rank == r) {
+          // gather in routing order (the serial += of routing.cpp:3955-3958)
+          double up = 0.;
+#pragma unroll
+          for (int u = 0; u < 8; u++)
+            if (u < wv.nu) {
+              const double near =
+                  wg_lds[WG_EXP2_LDS_BYTES / sizeof(double) + DF_TV * 64 + (near_lane(u) & 63)];
+              const double far = __builtin_bit_cast(double, t[u] & 0x7fffffffffffffffull);
+              const double q = (ext >> u & 1) ? far : near;
+              up += (u < link.nu) ? q : 0.;
+            }
+          bool slow;
+          o = step_fast<kUse>(c, pre, up, slow);
+          if (slow) o = chain_step<kUse>(c, up, di);
+          const unsigned long long w = __builtin_bit_cast(unsigned long long, o.tv) & 0x7fffffffffffffffull;
+          __hip_atomic_store(rrow + p, w | sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          F[DF_TV * 64] = o.tv;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+      }
+      if (c.flags & CFL_LAKE) s.glo_lake = o.glo_lake;
+      if (c.flags & CFL_RES) {
+        s.res = o.res;
+        s.k_release = o.k_release;
+      }
+      if (c.flags & CFL_GWET) s.glo_wetl = o.glo_wetl;
+      if (c.flags & CFL_ARID) s.gw = o.gw;
+      if ((c.flags & CFL_ARID) && X.pot_lgw) X.pot_lgw[mp] = o.lgw;
+      s.river = o.river;
+      rem = o.rem;
+      if (link.station >= 0) daily[link.station] = (c.flags & CFL_LDD) ? o.tv : 0.;
+      if (k == days - 1) X.tv[mp] = o.tv;
+      if (X.pot_acc) add_pot_runoff(S, X, mp, p);
+    }
+    {
+      DayStatEnd e;
+      e.red_exp = fld(DF_RED_EXP);
+      e.area = fld(DF_AREA);
+      e.river_length = fld(DF_LENGTH);
+      e.rw_c0 = fld(DF_RW_C0);
+      e.rw_c1 = fld(DF_RW_C1);
+      e.rw_c2 = fld(DF_RW_C2);
+      e.rw_c3 = fld(DF_RW_C3);
+      e.river_stor_max = fld(DF_RIVER_MAX);
+      e.max_raf = fld(DF_MAX_RAF);
+      e.f_glo_lake = (bits & DB_FULL_LAKE) ? 1. : 0.;
+      e.loc_lake = fld(DF_LL);
+      e.loc_wetland = fld(DF_LW);
+      e.glo_wetland = fld(DF_GW);
+      e.gw_max = fld(DF_GW_MAX);
+      e.lake_area = 0.;
+      e.lake_max = 0.;
+      e.reservoir_area = 0.;
+      e.stor_cap = 0.;
+      if (bits & (DB_LAKE | DB_RES)) {
+        e.lake_area = S.lake_area[p];
+        e.lake_max = e.lake_area * S.lake_depth[p];
+        e.reservoir_area = S.reservoir_area[p];
+        e.stor_cap = S.stor_cap[p];
+      }
+      e.contcell = cont;
+      if (kUse && cont) {
+        const int fin_ym = int((fday - S.use_day0) / 365) * 12 + di.month;
+        day_end_use(S, X.use + mp, p, s, rem, e.loc_lake, fld(DF_LL_MAX), e.red_exp, fin_ym, doy == 365);
+      }
+      day_end(e, s);
+    }
+  }
+
+  X.canopy[mp] = s.canopy;
+  X.soil[mp] = s.soil;
+  X.snow[mp] = s.snow;
+  X.transfer[mp] = s.transfer;
+  X.lai_precsum[mp] = s.lai_precsum;
+  X.lai_days[mp] = s.lai_days;
+  X.lai_status[mp] = s.lai_status;
+  X.snow_any[mp] = s.snow_any ? 1 : 0;
+  X.gw[mp] = s.gw;
+  X.loc_lake[mp] = s.loc_lake;
+  X.loc_wetl[mp] = s.loc_wetl;
+  X.glo_lake[mp] = s.glo_lake;
+  X.glo_wetl[mp] = s.glo_wetl;
+  X.res[mp] = s.res;
+  X.river[mp] = s.river;
+  X.red_ll[mp] = s.red_ll;
+  X.red_lw[mp] = s.red_lw;
+  X.red_gl[mp] = s.red_gl;
+  X.red_gw[mp] = s.red_gw;
+  X.red_res[mp] = s.red_res;
+  X.red_river[mp] = s.red_river;
+  X.river_frac_next[mp] = s.river_frac_next;
+  X.river_frac_change[mp] = s.river_frac_change;
+  X.fswb_next[mp] = s.fswb_next;
+  X.laf[mp] = s.laf;
+  X.laf_prev[mp] = s.laf_prev;
+  X.k_release[mp] = s.k_release;
+}
+
+#endif  // WG_DAYS_KERNEL_H

@@ -36,6 +36,20 @@ struct alignas(16) WgWaveItem {
   int32_t start, end, level, lakeres;
 };
 
+// One wavefront of the many-days kernel; passes: 1 + the longest chain of upstream
+// cells within it; nu: the most upstream cells of one of its cells.
+struct WgDayWave {
+  int16_t passes, nu;
+};
+
+// One lane of such a wavefront: the cell (device order, -1: none), the first cell of
+// its routing group, and for each upstream cell a byte: the lane that holds it, or
+// 0xff when it belongs to an earlier wavefront.
+struct alignas(16) WgDaySlot {
+  int32_t cell, group;
+  uint32_t near_lo, near_hi;
+};
+
 // Outflow constants of the storages on the routing chain (global lake / wetland,
 // arid groundwater).
 struct alignas(16) WgChainStatic {
@@ -144,7 +158,8 @@ struct WgState {
   // stations
   double *st_sum;               // [M][n_stations]
   double *st_daily;             // [M][WG_DAILY_SLOTS][n_stations]
-  int32_t *flow_error;           // [1] set when the dataflow chain walk hits its spin limit
+  int32_t *flow_error;           // [1] set when the dataflow chain walk or the many-days kernel hits its spin limit
+  int32_t *flow_error_host;      // [1] pinned host copy, set by the many-days kernel
   // forcing perturbation
   const uint64_t *member_seed;
   double prec_sigma, temp_sigma;

@@ -23,22 +23,23 @@
 #include <hip/hip_runtime.h>
 
 #include "wg_device.h"
-// The exp/log/pow table lives in LDS, one copy per wavefront (up to 4 per
-// workgroup): a lane-varying index into a global table costs a vector-memory
-// round trip per lookup, two per pow.
-__shared__ double wg_exp2_lds[4][128];
-#define WG_EXP2_TAB_LDS (wg_exp2_lds[threadIdx.x >> 6])
+// The exp/log/pow table lives in LDS, one copy per wavefront at the front of the
+// workgroup's dynamic LDS (WG_EXP2_LDS_BYTES per wavefront): a lane-varying index
+// into a global table costs a vector-memory round trip per lookup, two per pow.
+extern __shared__ double wg_lds[];
+#define WG_EXP2_LDS_BYTES 1024
+#define WG_EXP2_TAB_LDS (wg_lds + 128 * (threadIdx.x >> 6))
 #include "wg_libm.h"
 
 namespace {
 // Copies the table into the wavefront's LDS copy with one direct global-to-LDS load
 // (16 bytes per lane, lane i to bytes 16i..16i+15).  The compiler waits for it
-// before the first LDS read; workgroups of at most 256 threads.
+// before the first LDS read.
 __device__ inline void load_exp2_table() {
   const int lane = threadIdx.x & 63;
   __builtin_amdgcn_global_load_lds((const void *)(wg_exp2_tab_d + 2 * lane),
-                                   (__attribute__((address_space(3))) void *)&wg_exp2_lds[threadIdx.x >> 6][0], 16,
-                                   0, 0);
+                                   (__attribute__((address_space(3))) void *)(wg_lds + 128 * (threadIdx.x >> 6)), 16, 0,
+                                   0);
 }
 }  // namespace
 
@@ -123,595 +124,217 @@ __device__ inline void store_chain(const WgState &X, int64_t mp, int flags, cons
   if (X.use_rem) X.use_rem[mp] = o.rem;
 }
 
-// updateNetAbstractionGW, routing.cpp:5503-5572: the day's net abstraction from
-// groundwater, with the return flows of irrigation from surface water reduced
-// when the last day's surface-water use went unsatisfied (G_dailyRemainingUse > 0)
-// or given back when a delayed use was satisfied (< 0).  U points at the cell's
-// first water-use field, us is the stride between fields.
-__device__ inline double update_net_abstraction_gw(double *U, int64_t us, double frgi, double nug) {
-  double &dru = U[WG_USE_DAILY_REMAINING * us], &ui = U[WG_USE_UNSAT_IRRIG * us];
-  double &uo = U[WG_USE_UNSAT_OTHER * us], &rrf = U[WG_USE_REDUCED_RETURN * us];
-  const double wu = U[WG_USE_WITHDRAWAL_IRRIG * us], cu = U[WG_USE_CONSUMPTIVE_IRRIG * us];
-  if (dru > 1.e-12) {
-    if (wu > 0.) {
-      const double eff = cu / wu;
-      const double factor = 1 - (1 - frgi) * (1 - eff);
-      double WUsiNew = 1 / factor * (wu * factor - dru);
-      if (WUsiNew < 0.) {
-        WUsiNew = 0.;
-        ui += wu * factor;
-        uo += dru - (wu * factor);
-      } else {
-        ui += dru;
-      }
-      const double returnflowChange = (frgi * (1 - eff) * (WUsiNew - wu));
-      rrf += returnflowChange;
-      dru = 0.;
-      return nug - returnflowChange;
-    }
-    uo += dru;
-    return nug;
-  }
-  if (dru < -1.e-12) {
-    double fromIrrig = dru + uo;
-    if (fromIrrig < 0.) {
-      uo = 0.;
-    } else {
-      uo += dru;
-      dru = 0.;
-      return nug;
-    }
-    if (ui == 0.) {
-      dru = 0.;
-      return nug;
-    }
-    double ratio = (fromIrrig / ui);
-    if (ratio < -1.) {
-      ratio = -1.;
-      fromIrrig = ui * -1.;
-    }
-    const double returnflowChange = (ratio * rrf);
-    ui += fromIrrig;
-    rrf += returnflowChange;
-    dru = 0.;
-    return nug - returnflowChange;
-  }
-  return nug;
-}
-
-// annualWaterUsePostProcessing, routing.cpp:5257-5296, for one cell
-__device__ inline void water_use_year_end(double *U, int64_t us) {
-  double &tu = U[WG_USE_TOTAL_UNSAT * us], &ui = U[WG_USE_UNSAT_IRRIG * us];
-  double &uo = U[WG_USE_UNSAT_OTHER * us], &rrf = U[WG_USE_REDUCED_RETURN * us];
-  double &tu_py = U[WG_USE_UNSAT_PREV_YEAR * us], &ui_py = U[WG_USE_UNSAT_IRRIG_PREV_YEAR * us];
-  double &uo_py = U[WG_USE_UNSAT_OTHER_PREV_YEAR * us], &rrf_py = U[WG_USE_REDUCED_RETURN_PREV_YEAR * us];
-  if (tu < tu_py) {
-    tu_py = tu;
-    ui_py = ui;
-    uo_py = uo;
-    rrf_py = rrf;
-    ui = 0.;
-    uo = 0.;
-    rrf = 0.;
-    tu = 0.;
-  } else {
-    tu -= tu_py;
-    ui -= ui_py;
-    uo -= uo_py;
-    rrf -= rrf_py;
-    if ((ui + uo) < 0) {
-      ui = 0;
-      uo = 0;
-      rrf = 0;
-    } else if (uo < 0) {
-      ui += uo;
-      uo = 0;
-    } else if (ui < 0) {
-      uo += ui;
-      ui = 0;
-      rrf = 0;
-    }
-    if (rrf > 0) {
-      rrf = 0;
-      ui = 0;
-    }
-  }
-}
-
-// routing.cpp:7309-7341 getNewRiverVelocity
-// c1 = 1. / (mult * rough) and c2 = pow(slope, 0.5) are per-cell constants computed
-// on the host with the same operations, so the product below is the reference's.
-__device__ inline double new_river_velocity(double c1, double c2, double bottom, double stor, double length) {
-  const double csa = (stor / length) * 1000000.;
-  const double depth = -bottom / 4.0 + sqrt(bottom * bottom / 16.0 + 0.5 * csa);
-  const double wp = bottom + 2.0 * depth * sqrt(5.0);
-  const double hr = csa / wp;
-  double v = c1 * wg_pow(hr, (2. / 3.)) * c2;
-  v = v * 86.4;
-  return (v < 0.00001) ? 0.00001 : v;
-}
-
-// LAI state machine, lai.cpp:179-293
-__device__ inline double lai_day(int &days, int init_days, int &status, int lct, bool arid, double lmin,
-                                 double lmax, double &precsum, double prec, bool growing) {
-  if (growing) {
-    if (status == 0) {
-      if (days >= init_days) {
-        days++;
-        precsum += prec;
-        if (precsum > 40.) {
-          if (days >= init_days + 30) {
-            days = init_days + 30;
-            status = 1;
-          }
-          return (lmin + (lmax - lmin) * (days - init_days) / 30.);
-        }
-        days = init_days;
-        return lmin;
-      }
-      days++;
-      precsum += prec;
-      return lmin;
-    }
-    if (days <= 30) {
-      days--;
-      if (lct <= 2) status = 0;
-      if (days <= 0) {
-        days = 0;
-        status = 0;
-        precsum = 0.;
-      }
-      return (lmax - (lmax - lmin) * (30 - days) / 30.);
-    }
-    if (arid && (prec < 0.5))
-      days--;
-    else
-      days = 30 + init_days;
-    return lmax;
-  }
-  if (status == 0) {
-    if (days > init_days) {
-      days++;
-      precsum += prec;
-      if (precsum > 40.) {
-        if (days >= init_days + 30) {
-          days = init_days + 30;
-          status = 1;
-        }
-        return (lmin + (lmax - lmin) * (days - init_days) / 30.);
-      }
-      days = init_days;
-      return lmin;
-    }
-    precsum += prec;
-    return lmin;
-  }
-  if (days <= 30) {
-    days--;
-    if (days <= 0) {
-      days = 0;
-      status = 0;
-      precsum = 0.;
-    }
-    return (lmax - (lmax - lmin) * (30 - days) / 30.);
-  }
-  days--;
-  return lmax;
-}
-
-// Finish the previous day for one cell: reduction factors of the global
-// storages, river width and area fraction (routing.cpp:2792-2802, 3071-3078,
-// 3286-3295, 3546-3586), then the surface-water and land area fractions
-// (routing.cpp:5046-5174) and updateLandAreaFrac (routing.cpp:5343-5352).
-struct PostDay {
-  double laf, laf_prev, red_ll, red_lw, red_gw, red_gl, red_res, river_frac_next;
-};
-
-// With water use, the finished day's end of the routing loop comes first
-// (routing.cpp:3590-3622, 3898-3919): the use the river left is taken from the
-// local lake, whose area reduction factor is recomputed, the unsatisfied use is
-// kept and the month's irrigation withdrawal and consumptive use are recorded
-// (fin_ym: model year x 12 + month of the finished day); after day 365 the
-// year-end processing follows (fin_year_end).
-template <bool kUse>
-__device__ void post_day(const WgStatic &S, const WgState &X, int64_t mp, int p, PostDay &out, int fin_ym,
-                         bool fin_year_end) {
-  // Every input is loaded before the first store, so that the loads are in flight
-  // together (the arrays cover all cells, so the loads of unused fields are in bounds).
-  const double evarexp = S.evarexp[p];
-  const double cellArea = S.cell_area[p];
-  const double lake_area = S.lake_area[p], lake_depth = S.lake_depth[p], glo_lake = X.glo_lake[mp];
-  const double reservoir_area = S.reservoir_area[p], stor_cap = S.stor_cap[p], res = X.res[mp];
-  const double glo_wetland = S.glo_wetland[p], wetl_depth = S.wetl_depth[p], glo_wetl = X.glo_wetl[mp];
-  const bool contcell = S.contcell[p] != 0;
-  const double L = S.river_length[p];
-  const double rw_c0 = S.rw_c0[p], rw_c1 = S.rw_c1[p], rw_c2 = S.rw_c2[p], rw_c3 = S.rw_c3[p];
-  const double st = X.river[mp], smax = S.river_stor_max[p];
-  const double loc_lake = S.loc_lake[p], loc_wetland = S.loc_wetland[p];
-  const double f_glo_lake = S.f_glo_lake[p], contfreq = S.contfreq[p];
-  double red_ll = X.red_ll[mp], red_lw = X.red_lw[mp], red_gw = X.red_gw[mp];
-  double river_frac_next = X.river_frac_next[mp];
-  double river_frac_change = X.river_frac_change[mp];
-  double red_river = X.red_river[mp];
-  const double fswb_old = X.fswb_next[mp];
-  const double laf = X.laf[mp];
-  if (kUse && contcell) {
-    const int64_t us = S.use_stride;
-    double *U = X.use + mp;
-    double rem = X.use_rem[mp];
-    if ((loc_lake > 0.) && (rem > 0.)) {
-      const double maxStorage = ((loc_lake) / 100.) * cellArea * lake_depth;
-      double ls = X.loc_lake[mp];
-      if (ls > (-1.) * maxStorage) {
-        if (rem < (maxStorage + ls)) {
-          ls -= rem;
-          rem = 0.;
-        } else {
-          rem -= (maxStorage + ls);
-          ls = (-1.) * maxStorage;
-        }
-      }
-      double r = 1. - wg_pow(fabs(ls - maxStorage) / (2. * maxStorage), (evarexp * kEvapoRedExp));
-      if (r < 0.) r = 0.;
-      if (r > 1.) r = 1.;
-      red_ll = r;
-      X.loc_lake[mp] = ls;
-    }
-    if (S.use_delayed == 1) {
-      const double tu = U[WG_USE_TOTAL_UNSAT * us];
-      U[WG_USE_PREV_TOTAL_UNSAT * us] = tu;
-      U[WG_USE_DAILY_REMAINING * us] = rem - tu;
-      U[WG_USE_TOTAL_UNSAT * us] = rem;
-    } else {
-      U[WG_USE_TOTAL_UNSAT * us] += rem;
-      U[WG_USE_DAILY_REMAINING * us] = rem;
-    }
-    const int64_t t = int64_t(fin_ym) * S.n + p;
-    U[WG_USE_WITHDRAWAL_IRRIG * us] = S.use_wu[t];
-    U[WG_USE_CONSUMPTIVE_IRRIG * us] = S.use_cu[t];
-    X.use_rem[mp] = 0.;
-    if (fin_year_end) water_use_year_end(U, us);
-  }
-
-  double red_gl = 0., red_res = 0.;
-  if (lake_area > 0.) {
-    const double maxStorage = lake_area * lake_depth;
-    double r = 1. - wg_pow(fabs(glo_lake - maxStorage) / (2. * maxStorage), (evarexp * kEvapoRedExp));
-    if (r < 0.) r = 0.;
-    if (r > 1.) r = 1.;
-    red_gl = r;
-  }
-  if (reservoir_area > 0.) {
-    const double maxStorage = stor_cap;
-    double r = 1. - wg_pow(fabs(res - maxStorage) / maxStorage, kEvapoRedExpRes);
-    if (r < 0.) r = 0.;
-    if (r > 1.) r = 1.;
-    red_res = r;
-  }
-  if (glo_wetland > 0) {
-    const double maxStorage = ((glo_wetland) / 100.) * cellArea * wetl_depth;
-    double r = 1. - wg_pow(fabs(glo_wetl - maxStorage) / maxStorage, (evarexp * kEvapoRedExp));
-    if (r < 0.) r = 0.;
-    if (r > 1.) r = 1.;
-    red_gw = r;
-  }
-  if (contcell) {
-    const double riverAreaFrac = river_frac_next;
-    const double csa = st / L;
-    // -B / (4. * 1000.), B / 1000. * B / (16. * 1000.), B / 1000. and width_bf / 1000.
-    // are per-cell constants computed on the host with these operations
-    const double depth = rw_c0 + sqrt(rw_c1 + 0.5 * csa);
-    double width = rw_c2 + 4. * depth;
-    if (width > rw_c3) width = rw_c3;
-    red_river = 1. - wg_pow(fabs(st - smax) / smax, (evarexp * kEvapoRedExp));
-    if (red_river < 0.) red_river = 0.;
-    if (red_river > 1.) red_river = 1.;
-    river_frac_next = red_river * L * width * 100. / cellArea;
-    river_frac_change = river_frac_next - riverAreaFrac;
-  }
-  // fractions for the next day
-  double fLocLake, fLocWet, fGloWet;
-  if ((loc_lake > 0.) && (red_ll > 0.))
-    fLocLake = (red_ll * loc_lake / 100.);
-  else
-    fLocLake = 0.;
-  if ((loc_wetland > 0.) && (red_lw > 0.))
-    fLocWet = (red_lw * loc_wetland / 100.);
-  else
-    fLocWet = 0.;
-  if ((glo_wetland > 0.) && (red_gw > 0.))
-    fGloWet = (red_gw * glo_wetland / 100.);
-  else
-    fGloWet = 0.;
-  double fswb_next = fLocLake + fLocWet + fGloWet;
-  const double max_raf = contfreq / 100. - f_glo_lake;
-  if (((lake_area > 0.) || (reservoir_area > 0.)) && (f_glo_lake == 1.)) {
-    river_frac_next = 0.;
-    river_frac_change = 0.;
-    red_river = 0.;
-  } else {
-    if (river_frac_next <= max_raf) {
-      if (fswb_next > (max_raf - river_frac_next)) {
-        const double corr = (max_raf - river_frac_next) / fswb_next;
-        red_ll *= corr;
-        red_lw *= corr;
-        red_gw *= corr;
-        if ((fLocLake > 0.) && (red_ll > 0.)) {
-          fLocLake = (red_ll * loc_lake / 100.);
-        } else {
-          red_ll = 0.;
-          fLocLake = 0.;
-        }
-        if ((fLocWet > 0.) && (red_lw > 0.)) {
-          fLocWet = (red_lw * loc_wetland / 100.);
-        } else {
-          red_lw = 0.;
-          fLocWet = 0.;
-        }
-        if ((fGloWet > 0.) && (red_gw > 0.)) {
-          fGloWet = (red_gw * glo_wetland / 100.);
-        } else {
-          red_gw = 0.;
-          fGloWet = 0.;
-        }
-      }
-    } else {
-      const double deficit = river_frac_next - max_raf;
-      river_frac_change -= deficit;
-      red_river *= max_raf / river_frac_next;
-      river_frac_next = max_raf;
-      fLocLake = 0.;
-      fLocWet = 0.;
-      fGloWet = 0.;
-    }
-  }
-  fswb_next = fLocLake + fLocWet + fGloWet;
-  const double change_pct = fswb_next * 100. - fswb_old * 100.;
-  double laf_next = laf - (change_pct + (river_frac_change * 100.));
-  if (laf_next < 0.) laf_next = 0.;
-  if (lake_area > 0.) X.red_gl[mp] = red_gl;
-  if (reservoir_area > 0.) X.red_res[mp] = red_res;
-  X.laf_prev[mp] = laf;
-  X.laf[mp] = laf_next;
-  X.fswb_next[mp] = fswb_next;
-  X.red_ll[mp] = red_ll;
-  X.red_lw[mp] = red_lw;
-  X.red_gw[mp] = red_gw;
-  X.red_river[mp] = red_river;
-  X.river_frac_next[mp] = river_frac_next;
-  X.river_frac_change[mp] = river_frac_change;
-  out.laf = laf_next;
-  out.laf_prev = laf;
-  out.red_ll = red_ll;
-  out.red_lw = red_lw;
-  out.red_gw = red_gw;
-  out.red_gl = red_gl;
-  out.red_res = red_res;
-  out.river_frac_next = river_frac_next;
-}
-
-
-// ---- one elevation sub-cell of the snow loop, daily.cpp:920-1044 ----
-
-struct SnowDay {
-  double tempC, gradnt, scale_num, laf, prec_to_soil, soil_pet, snowfz, snowmt, melt_factor;
-  double eff_bare;  // the effective precipitation of a sub-cell without snow above freezing
-  double inv_laf;   // 1 / laf, correctly rounded
-  int elev0;
-  bool melt_ok;     // melt_factor >= 0 (a NaN or negative factor takes the full step)
-};
-
-struct SnowAcc {
-  double snow_sum, eff, evapo, change, temp_max;
-  int thresh;
-};
-
-// Updates one sub-cell storage s and the cell's running sums in sub-cell order
-// (daily.cpp:920-1044); temp_elev is the sub-cell temperature T - (z_e - z0) gradnt
-// and melt_factor = M_DEGDAY_F * ddf_lct (daily.cpp:1013).  The reference's branches
-// are selects here: every operation is the reference's, on the same operands, and
-// a branch not taken adds +0 to a sum, which leaves it unchanged (the sums start at
-// +0 and never hold -0).  Without branches the two sub-cells of a pair are
-// independent chains that the compiler interleaves.
-__device__ inline double snow_subcell(double s, double temp_elev, int elev_e, bool first, const SnowDay &d,
-                                      SnowAcc &a) {
-  {
-    // s * scale_num / laf with the reused reciprocal: q0 = x (1/laf), one exact
-    // residual and one correction give the correctly rounded quotient (Markstein's
-    // theorem for a correctly rounded reciprocal; tests/test_division.py compares
-    // it with the division on random operands).  An infinite or NaN x is its own quotient by the
-    // finite positive laf.  (The quotient of a finite x overflows only for
-    // x > 1e292 mm, since a positive land area fraction is at least about 1e-16.)
-    const double x = s * d.scale_num;
-    const double q0 = x * d.inv_laf;
-    const double q = fma(fma(-q0, d.laf, x), d.inv_laf, q0);
-    s = (fabs(x) <= 1.7976931348623157e308) ? q : x;
-  }
-  s = (fabs(s) <= kMinStorVol) ? 0. : s;
-  const double init_s = s;
-  // threshold elevation above 1000 mm of storage (daily.cpp:958-976)
-  const bool big = s > 1000.;
-  const bool use_thresh = big && a.thresh > 0;
-  const double temp_thresh = d.tempC - ((a.thresh - d.elev0) * d.gradnt);
-  a.thresh = (big && a.thresh == 0) ? elev_e : a.thresh;
-  temp_elev = use_thresh ? temp_thresh : temp_elev;
-  // snowfall and sublimation below the freezing temperature, rain above it
-  const bool freeze = temp_elev <= d.snowfz;
-  const double s_fall = s + d.prec_to_soil;
-  const bool keeps = s_fall > d.soil_pet;
-  const double s_subl = s_fall - d.soil_pet;
-  a.evapo += freeze ? (keeps ? d.soil_pet : s_fall) : 0.;
-  s = freeze ? (keeps ? s_subl : 0.) : s;
-  const double eff_before = freeze ? 0. : d.prec_to_soil;
-  // degree-day melt
-  const bool melts = (temp_elev > d.snowmt) && !(s < 0.);
-  const double melt_pot = d.melt_factor * (temp_elev - d.snowmt);
-  const bool all = melt_pot > s;
-  const double s_left = s - melt_pot;
-  const double snowmelt_elev = melts ? (all ? s : melt_pot) : 0.;
-  s = melts ? (all ? 0. : s_left) : s;
-  const double eff_elev = eff_before + snowmelt_elev;
-  a.change += s - init_s;
-  if (first) a.temp_max = temp_elev;
-  a.snow_sum += s;
-  a.eff += eff_elev;
-  return s;
-}
+#include "wg_cell_day.h"
 
 }  // namespace
 
-// Per-cell inputs of the cell kernel: statics (s_), state (x_) and land-cover
-// table entries (t_).  The kernel loads them at two points, each before the first
-// store of the part that reads them, so that a part's loads are in flight together
-// (after a store the compiler must keep later loads behind it): load_cell_in before
-// post_day for PET, LAI, canopy and snow, load_cell_in_b after the snow loop for
-// soil and routing.  Every array covers all cells, so the loads of fields a cell
+namespace {
+
+// Loads of a cell's statics and state, grouped by the part of the day that reads
+// them.  A kernel issues a part's loads before the first store of that part, so
+// that they are in flight together (after a store the compiler must keep later
+// loads behind it).  Every array covers all cells, so the loads of fields a cell
 // does not use are in bounds.
-struct CellIn {
-  int16_t s_aindex;
-  double s_alpha;
-  double s_bottom_width;
-  float s_built_up;
-  double s_cell_area;
-  double s_contfreq;
-  double s_degday;
-  double s_e_gw;
-  double s_e_sw;
-  int16_t s_elev0;
-  double s_evarexp;
-  double s_fswb_init;
-  double s_glo_wetland;
-  float s_gw_factor;
-  double s_inv_kgw;
-  double s_k_sw;
-  float s_lai_max;
-  double s_lake_area;
-  double s_lake_depth;
-  int8_t s_land_cover;
-  int8_t s_ldd;
-  double s_loc_lake;
-  double s_loc_wetland;
-  double s_m_netrad;
-  double s_m_prec;
-  double s_mcwh;
-  double s_mean_outflow, s_prov_rel;
-  double s_ome_gw;
-  double s_pcritgwa;
-  double s_pet_mxdy;
-  double s_reservoir_area;
-  int16_t s_rgmax;
-  double s_river_length;
-  double s_vel_c1;
-  double s_vel_c2;
-  double s_stor_cap;
-  double s_t_gradnt;
-  double s_t_snowfz;
-  double s_t_snowmt;
-  int8_t s_texture;
-  double s_wetl_depth;
-  double x_canopy;
-  double x_cfa;
-  double x_gamma;
-  double x_glo_lake;
-  double x_glo_wetl;
-  double x_gw;
-  double x_k_release;
-  int32_t x_lai_days;
-  double x_lai_precsum;
-  int32_t x_lai_status;
-  double x_loc_lake;
-  double x_loc_wetl;
-  double x_res;
-  double x_river;
-  float x_smax;
-  double x_snow;
-  uint8_t x_snow_any;
-  double x_soil;
-  double x_transfer;
-  double t_albedo, t_albedo_snow, t_ddf, t_emissivity;
-  float t_lai_a, t_lai_b;
-  int32_t t_initial_days;
-  WgChainLink link;
-  WgChainStatic cstat;
-};
-
-__device__ inline void load_cell_in(const WgStatic &S, const WgState &X, const WgTables &T, int64_t mp, int p,
-                                    CellIn &ci) {
-  ci.s_aindex = S.aindex[p];
-  ci.s_alpha = S.alpha[p];
-  ci.s_degday = S.degday[p];
-  ci.s_elev0 = S.elev0[p];
-  ci.s_lai_max = S.lai_max[p];
-  ci.s_land_cover = S.land_cover[p];
-  ci.s_m_netrad = S.m_netrad[p];
-  ci.s_m_prec = S.m_prec[p];
-  ci.s_mcwh = S.mcwh[p];
-  ci.s_pet_mxdy = S.pet_mxdy[p];
-  ci.s_t_gradnt = S.t_gradnt[p];
-  ci.s_t_snowfz = S.t_snowfz[p];
-  ci.s_t_snowmt = S.t_snowmt[p];
-  ci.x_canopy = X.canopy[mp];
-  ci.x_lai_days = X.lai_days[mp];
-  ci.x_lai_precsum = X.lai_precsum[mp];
-  ci.x_lai_status = X.lai_status[mp];
-  ci.x_snow = X.snow[mp];
-  ci.x_snow_any = X.snow_any[mp];
-  ci.x_transfer = X.transfer[mp];
-  const int l = ci.s_land_cover - 1;
-  ci.t_albedo = T.albedo[l];
-  ci.t_albedo_snow = T.albedo_snow[l];
-  ci.t_ddf = T.ddf[l];
-  ci.t_emissivity = T.emissivity[l];
-  ci.t_initial_days = T.initial_days[l];
-  ci.t_lai_a = T.lai_a[l];
-  ci.t_lai_b = T.lai_b[l];
+__device__ __forceinline__ void load_stat_a(const WgStatic &S, const WgTables &T, int p, DayStatA &a) {
+  const int l = S.land_cover[p] - 1;
+  const float lmax_f = S.lai_max[p];
+  a.m_prec = S.m_prec[p];
+  a.alpha = S.alpha[p];
+  a.pet_mxdy = S.pet_mxdy[p];
+  a.m_netrad = S.m_netrad[p];
+  a.mcwh = S.mcwh[p];
+  a.t_snowfz = S.t_snowfz[p];
+  a.t_snowmt = S.t_snowmt[p];
+  a.t_gradnt = S.t_gradnt[p];
+  a.melt_factor = S.degday[p] * T.ddf[l];
+  a.albedo = T.albedo[l];
+  a.albedo_snow = T.albedo_snow[l];
+  a.emis = T.emissivity[l] * 0.000000004903;
+  a.lmin = T.lai_a[l] + T.lai_b[l] * lmax_f;
+  a.lmax = lmax_f;
+  a.initial_days = T.initial_days[l];
+  a.lct = l + 1;
+  a.elev0 = S.elev0[p];
+  a.arid = S.aindex[p] == 1;
 }
 
-__device__ inline void load_cell_in_b(const WgStatic &S, const WgState &X, int64_t mp, int p, CellIn &ci) {
-  ci.s_bottom_width = S.bottom_width[p];
-  ci.s_built_up = S.built_up[p];
-  ci.s_cell_area = S.cell_area[p];
-  ci.s_contfreq = S.contfreq[p];
-  ci.s_e_gw = S.e_gw[p];
-  ci.s_e_sw = S.e_sw[p];
-  ci.s_evarexp = S.evarexp[p];
-  ci.s_fswb_init = S.fswb_init[p];
-  ci.s_glo_wetland = S.glo_wetland[p];
-  ci.s_gw_factor = S.gw_factor[p];
-  ci.s_inv_kgw = S.inv_kgw[p];
-  ci.s_k_sw = S.k_sw[p];
-  ci.s_lake_area = S.lake_area[p];
-  ci.s_lake_depth = S.lake_depth[p];
-  ci.s_ldd = S.ldd[p];
-  ci.s_loc_lake = S.loc_lake[p];
-  ci.s_loc_wetland = S.loc_wetland[p];
-  ci.s_mean_outflow = S.mean_outflow[p];
-  ci.s_prov_rel = S.res_prov_rel[p];
-  ci.s_ome_gw = S.ome_gw[p];
-  ci.s_pcritgwa = S.pcritgwa[p];
-  ci.s_reservoir_area = S.reservoir_area[p];
-  ci.s_rgmax = S.rgmax[p];
-  ci.s_river_length = S.river_length[p];
-  ci.s_vel_c1 = S.vel_c1[p];
-  ci.s_vel_c2 = S.vel_c2[p];
-  ci.s_stor_cap = S.stor_cap[p];
-  ci.s_texture = S.texture[p];
-  ci.s_wetl_depth = S.wetl_depth[p];
-  ci.x_cfa = X.cfa[mp];
-  ci.x_gamma = X.gamma[mp];
-  ci.x_glo_lake = X.glo_lake[mp];
-  ci.x_glo_wetl = X.glo_wetl[mp];
-  ci.x_gw = X.gw[mp];
-  ci.x_k_release = X.k_release[mp];
-  ci.x_loc_lake = X.loc_lake[mp];
-  ci.x_loc_wetl = X.loc_wetl[mp];
-  ci.x_res = X.res[mp];
-  ci.x_river = X.river[mp];
-  ci.x_smax = X.smax[mp];
-  ci.x_soil = X.soil[mp];
-  ci.link = load_link(S, p);
-  ci.cstat = load_cstat(S, p);
+__device__ __forceinline__ void load_stat_b(const WgStatic &S, const WgState &X, int64_t mp, int p, DayStatB &b) {
+  b.built_up = S.built_up[p];
+  b.smax = X.smax[mp];
+  b.gw_factor = S.gw_factor[p];
+  b.gamma = X.gamma[mp];
+  b.cfa = X.cfa[mp];
+  b.pet_mxdy = S.pet_mxdy[p];
+  b.t_snowfz = S.t_snowfz[p];
+  b.pcritgwa = S.pcritgwa[p];
+  const int16_t rgmax = S.rgmax[p];
+  b.rgmax = rgmax / 100.;
+  b.arid = S.aindex[p] == 1;
+  b.ldd = S.ldd[p];
+  b.recharge_cut = (b.arid && (S.texture[p] < 21)) && (b.ldd >= 0);
+  b.area = S.cell_area[p];
+  b.area_m = b.area / 1000000.;
+  b.cf100 = S.contfreq[p] / 100.;
+  double f = S.fswb_init[p] * 20.;
+  if (f > 1.) f = 1.;
+  b.fswb_catchment = f;
+  b.e_gw = S.e_gw[p];
+  b.inv_kgw = S.inv_kgw[p];
+  b.ome_gw = S.ome_gw[p];
+  b.e_sw = S.e_sw[p];
+  b.k_sw = S.k_sw[p];
+  b.red_exp = S.evarexp[p] * kEvapoRedExp;
+  const double lake_depth = S.lake_depth[p], wetl_depth = S.wetl_depth[p];
+  b.loc_lake = S.loc_lake[p];
+  b.ll100 = b.loc_lake / 100.;
+  b.ll_max = b.ll100 * b.area * lake_depth;
+  b.loc_wetland = S.loc_wetland[p];
+  b.lw100 = b.loc_wetland / 100.;
+  b.lw_max = b.lw100 * b.area * wetl_depth;
+  b.glo_wetland = S.glo_wetland[p];
+  b.gw100 = b.glo_wetland / 100.;
+  b.gw_max = b.gw100 * b.area * wetl_depth;
+  b.river_length = S.river_length[p];
+  b.bottom = S.bottom_width[p];
+  b.vel_b4 = -b.bottom / 4.0;
+  b.vel_b16 = b.bottom * b.bottom / 16.0;
+  b.vel_c1 = S.vel_c1[p];
+  b.vel_c2 = S.vel_c2[p];
 }
+
+__device__ __forceinline__ void load_stat_lake(const WgStatic &S, int p, DayStatLake &k) {
+  k.lake_area = S.lake_area[p];
+  k.lake_depth = S.lake_depth[p];
+  k.reservoir_area = S.reservoir_area[p];
+  k.stor_cap = S.stor_cap[p];
+  k.mean_outflow = S.mean_outflow[p];
+  k.prov_rel = S.res_prov_rel[p];
+}
+
+__device__ __forceinline__ void load_stat_end(const WgStatic &S, int p, DayStatEnd &e) {
+  e.red_exp = S.evarexp[p] * kEvapoRedExp;
+  e.area = S.cell_area[p];
+  e.river_length = S.river_length[p];
+  e.rw_c0 = S.rw_c0[p];
+  e.rw_c1 = S.rw_c1[p];
+  e.rw_c2 = S.rw_c2[p];
+  e.rw_c3 = S.rw_c3[p];
+  e.river_stor_max = S.river_stor_max[p];
+  e.f_glo_lake = S.f_glo_lake[p];
+  e.max_raf = S.contfreq[p] / 100. - e.f_glo_lake;
+  e.loc_lake = S.loc_lake[p];
+  e.loc_wetland = S.loc_wetland[p];
+  e.glo_wetland = S.glo_wetland[p];
+  e.gw_max = e.glo_wetland / 100. * e.area * S.wetl_depth[p];
+  e.lake_area = S.lake_area[p];
+  e.lake_max = e.lake_area * S.lake_depth[p];
+  e.reservoir_area = S.reservoir_area[p];
+  e.stor_cap = S.stor_cap[p];
+  e.contcell = S.contcell[p] != 0;
+}
+
+// State read by PET, LAI, canopy and snow.
+__device__ __forceinline__ void load_state_a(const WgState &X, int64_t mp, CellState &s) {
+  s.canopy = X.canopy[mp];
+  s.lai_days = X.lai_days[mp];
+  s.lai_precsum = X.lai_precsum[mp];
+  s.lai_status = X.lai_status[mp];
+  s.snow = X.snow[mp];
+  s.snow_any = X.snow_any[mp] != 0;
+  s.transfer = X.transfer[mp];
+}
+
+// State read by soil and local routing.
+__device__ __forceinline__ void load_state_b(const WgState &X, int64_t mp, CellState &s) {
+  s.soil = X.soil[mp];
+  s.gw = X.gw[mp];
+  s.loc_lake = X.loc_lake[mp];
+  s.loc_wetl = X.loc_wetl[mp];
+  s.glo_lake = X.glo_lake[mp];
+  s.glo_wetl = X.glo_wetl[mp];
+  s.res = X.res[mp];
+  s.river = X.river[mp];
+  s.k_release = X.k_release[mp];
+}
+
+// State read by the day's end (with loc_lake for the water use).
+__device__ __forceinline__ void load_state_end(const WgState &X, int64_t mp, CellState &s) {
+  s.glo_lake = X.glo_lake[mp];
+  s.glo_wetl = X.glo_wetl[mp];
+  s.res = X.res[mp];
+  s.river = X.river[mp];
+  s.red_ll = X.red_ll[mp];
+  s.red_lw = X.red_lw[mp];
+  s.red_gl = 0.;
+  s.red_gw = X.red_gw[mp];
+  s.red_res = 0.;
+  s.red_river = X.red_river[mp];
+  s.river_frac_next = X.river_frac_next[mp];
+  s.river_frac_change = X.river_frac_change[mp];
+  s.fswb_next = X.fswb_next[mp];
+  s.laf = X.laf[mp];
+}
+
+// Writes what the day's end changed.
+__device__ __forceinline__ void store_state_end(const WgState &X, int64_t mp, const DayStatEnd &e,
+                                                const CellState &s) {
+  if (e.lake_area > 0.) X.red_gl[mp] = s.red_gl;
+  if (e.reservoir_area > 0.) X.red_res[mp] = s.red_res;
+  X.laf_prev[mp] = s.laf_prev;
+  X.laf[mp] = s.laf;
+  X.fswb_next[mp] = s.fswb_next;
+  X.red_ll[mp] = s.red_ll;
+  X.red_lw[mp] = s.red_lw;
+  X.red_gw[mp] = s.red_gw;
+  X.red_river[mp] = s.red_river;
+  X.river_frac_next[mp] = s.river_frac_next;
+  X.river_frac_change[mp] = s.river_frac_change;
+}
+
+// The day's perturbed temperature and precipitation of one (member, cell).
+__device__ __forceinline__ void perturb_forcing(const WgStatic &S, const WgState &X, int m, int p, int64_t fday,
+                                                float &tf, float &pf) {
+  const uint64_t seed = X.member_seed[m];
+  const uint32_t ref = uint32_t(S.ref_index[p]);
+  double zp, zt;
+  normal_pair(seed, ref, uint32_t(fday), zp, zt);
+  pf = float(double(pf) * wg_exp(X.prec_sigma * zp));
+  tf = float(double(tf) + X.temp_sigma * zt);
+}
+
+// Water use of the day: the desired surface-water use (routing.cpp:2193-2290) and
+// the net abstraction from groundwater (routing.cpp:7440-7441, adapted by
+// updateNetAbstractionGW in every groundwater branch when the last day left a
+// remaining use; the adaptation reads only the last day's state, so it is done
+// here for (semi-)arid cells too, whose groundwater step the chain runs).
+// Returns the index of the day's tables.
+__device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, int64_t mp, int p, int64_t fday,
+                                           int month, double &desired, double &nag) {
+  const int64_t t = (int64_t((fday - S.use_day0) / 365) * 12 + month) * S.n + p;
+  const int64_t us = S.use_stride;
+  double *U = X.use + mp;
+  nag = S.use_nug[t];
+  if (U[WG_USE_DAILY_REMAINING * us] != 0.) nag = update_net_abstraction_gw(U, us, S.use_frgi[p], nag);
+  desired = S.use_nus[t];
+  if (S.use_delayed == 1) desired += U[WG_USE_TOTAL_UNSAT * us];
+  return t;
+}
+
+// Adds the day's potential cell runoff of a continental cell to its running sum,
+// G_potCellRunoff[n] += potCellRunoff (routing.cpp:1970, 2053, 2187, 3379): the
+// local runoff terms, then the arid groundwater step's runoff where that step ran,
+// then the open-water balance, in the reference's order of addition.
+__device__ __forceinline__ void add_pot_runoff(const WgStatic &S, const WgState &X, int64_t mp, int p) {
+  const double base = X.pot_base[mp];
+  const double lake_balance = X.pot_ow[mp] * X.cfa[mp];  // (dailyPrec - dailyOpenWaterPET) * CFA
+  const double ow = (lake_balance / 1000000.0) *
+                    ((S.lake_area[p] + S.reservoir_area[p]) +
+                     ((S.cell_area[p] / 100.0) * ((S.loc_lake[p] + S.loc_wetland[p]) + S.glo_wetland[p])));
+  const double pot = (S.cflags[p] & CFL_ARID) ? (base + X.pot_lgw[mp]) + ow : base + ow;
+  X.pot_acc[mp] += pot;
+}
+
+}  // namespace
 
 struct WgClock {
   int64_t day0;   // forcing day (index into the loaded forcing) of launch offset 0
@@ -741,30 +364,38 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   const int n = S.n;
   const int64_t mp = int64_t(m) * n + p;
 
-  CellIn ci;
-  if (do_vertical) load_cell_in(S, X, T, mp, p, ci);
-  // the fractions post_day writes, which the rest of the kernel reads
-  PostDay pd;
+  DayStatA sa;
+  CellState s;
+  if (do_vertical) {
+    load_stat_a(S, T, p, sa);
+    load_state_a(X, mp, s);
+  }
   if (do_post) {
-    // the finished day is day k - 1 of the block (the closing pass runs with k = days)
-    int fin_ym = 0;
-    bool fin_year_end = false;
-    if (kUse) {
+    DayStatEnd e;
+    load_stat_end(S, p, e);
+    load_state_end(X, mp, s);
+    if (kUse && e.contcell) {
+      // the finished day is day k - 1 of the block (the closing pass runs with k = days)
       const int64_t fin = clock->day0 + k - 1;
       const int fin_doy = int((clock->doy0 - 1 + k - 1) % 365) + 1;
-      fin_ym = int((fin - S.use_day0) / 365) * 12 + day_info(fin_doy).month;
-      fin_year_end = fin_doy == 365;
+      const int fin_ym = int((fin - S.use_day0) / 365) * 12 + day_info(fin_doy).month;
+      s.loc_lake = X.loc_lake[mp];
+      day_end_use(S, X.use + mp, p, s, X.use_rem[mp], e.loc_lake,
+                  e.loc_lake / 100. * e.area * S.lake_depth[p], e.red_exp, fin_ym, fin_doy == 365);
+      X.loc_lake[mp] = s.loc_lake;
+      X.use_rem[mp] = 0.;
     }
-    post_day<kUse>(S, X, mp, p, pd, fin_ym, fin_year_end);
+    day_end(e, s);
+    store_state_end(X, mp, e, s);
   } else if (do_vertical) {
-    pd.laf = X.laf[mp];
-    pd.laf_prev = X.laf_prev[mp];
-    pd.red_ll = X.red_ll[mp];
-    pd.red_lw = X.red_lw[mp];
-    pd.red_gw = X.red_gw[mp];
-    pd.red_gl = X.red_gl[mp];
-    pd.red_res = X.red_res[mp];
-    pd.river_frac_next = X.river_frac_next[mp];
+    s.laf = X.laf[mp];
+    s.laf_prev = X.laf_prev[mp];
+    s.red_ll = X.red_ll[mp];
+    s.red_lw = X.red_lw[mp];
+    s.red_gw = X.red_gw[mp];
+    s.red_gl = X.red_gl[mp];
+    s.red_res = X.red_res[mp];
+    s.river_frac_next = X.river_frac_next[mp];
   }
   // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
   // routing.cpp:1876); other cells keep a zero transported volume.
@@ -782,627 +413,85 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   const float *f = forcing + fday * 4 * int64_t(n);
   float tf = f[p], pf = f[n + p];
   const float swf = f[2 * n + p], lwf = f[3 * n + p];
-  if (X.perturb) {
-    const uint64_t seed = X.member_seed[m];
-    const uint32_t ref = uint32_t(S.ref_index[p]);
-    double zp, zt;
-    normal_pair(seed, ref, uint32_t(fday), zp, zt);
-    pf = float(double(pf) * wg_exp(X.prec_sigma * zp));
-    tf = float(double(tf) + X.temp_sigma * zt);
-  }
-  // water use of the day: the desired surface-water use (routing.cpp:2193-2290)
-  // and the net abstraction from groundwater (routing.cpp:7440-7441, adapted by
-  // updateNetAbstractionGW in every groundwater branch when the last day left a
-  // remaining use; the adaptation reads only the last day's state, so it is done
-  // here for (semi-)arid cells too, whose groundwater step the chain runs)
+  if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
   double use_desired = 0., use_nag = 0.;
   int64_t use_t = 0;
-  if (kUse) {
-    use_t = (int64_t((fday - S.use_day0) / 365) * 12 + day_info(doy).month) * n + p;
-    const int64_t us = S.use_stride;
-    double *U = X.use + mp;
-    use_nag = S.use_nug[use_t];
-    if (U[WG_USE_DAILY_REMAINING * us] != 0.) use_nag = update_net_abstraction_gw(U, us, S.use_frgi[p], use_nag);
-    use_desired = S.use_nus[use_t];
-    if (S.use_delayed == 1) use_desired += U[WG_USE_TOTAL_UNSAT * us];
-  }
+  if (kUse) use_t = day_use(S, X, mp, p, fday, day_info(doy).month, use_desired, use_nag);
 
-  // ------------------------------------------------------------------
-  // calcNewDay, daily.cpp:94-1279
-  // ------------------------------------------------------------------
-  const int lct = ci.s_land_cover;
-  const bool arid_gw = (ci.s_aindex == 1);
-  const double landAreaFrac = pd.laf;
-  const double lafPrev = started ? pd.laf_prev : landAreaFrac;  // daily.cpp:159-169
-  double dailyTempC = tf, dailyPrec = pf;
-  const double dailyShortWave = swf, dailyLongWave = lwf;
-  dailyPrec = ci.s_m_prec * dailyPrec;  // daily.cpp:248
-  const double temp2 = dailyTempC + 237.3;
-  const double e_s = 0.6108 * wg_exp(17.27 * dailyTempC / temp2);
-  const double alpha = ci.s_alpha;
-  const double maxDailyPET = ci.s_pet_mxdy;
-
-  // lai.cpp:152-177
-  double dailyLai;
-  {
-    const float lmax_f = ci.s_lai_max;
-    const double lmax = double(lmax_f);
-    const double lmin = ci.t_lai_a + ci.t_lai_b * lmax_f;
-    int days = ci.x_lai_days, status = ci.x_lai_status;
-    double precsum = ci.x_lai_precsum;
-    dailyLai = lai_day(days, ci.t_initial_days, status, lct, arid_gw, lmin, lmax, precsum, dailyPrec,
-                       dailyTempC > 8.);
-    X.lai_days[mp] = days;
-    X.lai_status[mp] = status;
-    X.lai_precsum[mp] = precsum;
-  }
-  // daily.cpp:366-462 albedo, latent heat, radiation (cloud = 1)
-  const double albedo = (ci.x_snow > 3.) ? ci.t_albedo_snow : ci.t_albedo;
-  const double lat_heat = (dailyTempC > 0) ? (2.501 - 0.002361 * dailyTempC) : 2.835;
-  const double conv_Wm2_to_mmd = 0.0864 / lat_heat;
-  const double solar_rad = conv_Wm2_to_mmd * dailyShortWave;
-  const double long_wave_rad_in = conv_Wm2_to_mmd * dailyLongWave;
-  const double temp_K = dailyTempC + 273.2;
-  const double long_wave_rad_out = ci.t_emissivity * 0.000000004903 * wg_pow(temp_K, 4.) / lat_heat;
-  const double net_long_wave_rad = long_wave_rad_in - long_wave_rad_out;
-  const double net_short_wave_rad = solar_rad * (1. - albedo);
-  const double net_rad = ci.s_m_netrad * (net_short_wave_rad + net_long_wave_rad);
-  const double openWaterNetRad = solar_rad * (1. - kOpenWaterAlbedo) + net_long_wave_rad;
-  // daily.cpp:476-522 Priestley-Taylor
-  const double inc_svp = 4098. * e_s / (temp2 * temp2);
-  const double gamma = (0.0016286 * 101.3) / lat_heat;
-  const double dailyPET = (net_rad <= 0.) ? 0. : alpha * (inc_svp * net_rad) / (inc_svp + gamma);
-  const double dailyOpenWaterPET =
-      (openWaterNetRad <= 0.) ? 0. : alpha * (inc_svp * openWaterNetRad) / (inc_svp + gamma);
-
-  double landStorageChangeSum = 0., initialStorage = 0.;
-  double dailyCanopyEvapo = 0., daily_prec_to_soil = 0., dailySoilPET = 0.;
-  double dailySnowEvapo = 0., dailyEffPrec = 0., immediate_runoff = 0., dailyAET = 0.;
-  double daily_runoff = 0., total_daily_runoff = 0., daily_gw_recharge = 0., pot_gw_recharge = 0.;
-  double soil_water_overflow = 0., neg_land_aet = 0.;
-  double dailyCellLandAET_uncorr = 0.;
-  double transfer = ci.x_transfer;
-
-  // interception, daily.cpp:825-895
-  double canopy = ci.x_canopy;
-  if (landAreaFrac <= 0.) {
-    transfer = canopy;
-    canopy = 0.;
-  } else {
-    canopy *= lafPrev / landAreaFrac;
-    if (fabs(canopy) <= kMinStorVol) canopy = 0.;
-    initialStorage = canopy;
-    if (dailyLai > 0.00001) {
-      const double max_canopy_storage = ci.s_mcwh * dailyLai;
-      const double canopy_deficiency = max_canopy_storage - canopy;
-      if (dailyPrec < canopy_deficiency) {
-        canopy += dailyPrec;
-        daily_prec_to_soil = 0.;
-      } else {
-        canopy = max_canopy_storage;
-        daily_prec_to_soil = dailyPrec - canopy_deficiency;
-      }
-      const double canopy_water_content = canopy;
-      dailyCanopyEvapo = dailyPET * wg_pow((canopy_water_content / max_canopy_storage), kCanopyEvapoExp);
-      if (dailyCanopyEvapo > canopy_water_content) {
-        dailyCanopyEvapo = canopy_water_content;
-        dailySoilPET = dailyPET - canopy_water_content;
-        canopy = 0.0;
-      } else {
-        canopy -= dailyCanopyEvapo;
-        dailySoilPET = dailyPET - dailyCanopyEvapo;
-      }
-    } else {
-      daily_prec_to_soil = dailyPrec;
-      dailySoilPET = dailyPET;
-      dailyCanopyEvapo = 0.0;
-    }
-    landStorageChangeSum += canopy - initialStorage;
-  }
-  X.canopy[mp] = canopy;
-  if (dailySoilPET < 0.) dailySoilPET = 0.0;
-
-  // snow on the elevation sub-cells, daily.cpp:897-1062, serial in sub-cell order.
-  // Sub-cells are stored in pairs ([member][pair][cell] x 2 doubles, elevations as
-  // packed int16 pairs) and streamed in double-buffered chunks so that a
-  // wavefront keeps many 16-byte loads in flight.
-  const double T_SNOWFZ = ci.s_t_snowfz, T_SNOWMT = ci.s_t_snowmt;
-  const double T_GRADNT = ci.s_t_gradnt, DEGDAY_F = ci.s_degday;
-  const double ddf = ci.t_ddf;
-  SnowAcc acc;
-  acc.snow_sum = 0.;
-  acc.eff = 0.;
-  acc.evapo = 0.;
-  acc.change = 0.;
-  acc.temp_max = 0.;
-  acc.thresh = 0;
-  const int elev0 = ci.s_elev0;
-  WgD2 *sp = X.snow2 + int64_t(m) * WG_DEV_NPAIR * n + p;
-  const int32_t *ep = S.elev_pairs + p;
-  // A cell whose sub-cell storages are all exactly zero (snow_any == 0) starts the
-  // loop from zeros without reading them, and stores only storages that become
-  // non-zero: on warm days such a cell moves no snow bytes at all.
-  const bool snow_any = ci.x_snow_any != 0;
-  if (landAreaFrac <= 0.) {
-    for (int k = 0; k < WG_DEV_NPAIR; k++) {
-      const WgD2 v = snow_any ? sp[int64_t(k) * n] : WgD2{0., 0.};
-      transfer += v.x / 100.;
-      transfer += v.y / 100.;
-      if (snow_any) sp[int64_t(k) * n] = WgD2{0., 0.};
-    }
-    X.snow_any[mp] = 0;
-  } else {
-    SnowDay sd;
-    sd.tempC = dailyTempC;
-    sd.elev0 = elev0;
-    sd.gradnt = T_GRADNT;
-    sd.scale_num = lafPrev;
-    sd.laf = landAreaFrac;
-    sd.prec_to_soil = daily_prec_to_soil;
-    sd.soil_pet = dailySoilPET;
-    sd.snowfz = T_SNOWFZ;
-    sd.snowmt = T_SNOWMT;
-    sd.melt_factor = DEGDAY_F * ddf;
-    sd.eff_bare = daily_prec_to_soil + 0.;
-    sd.inv_laf = 1. / landAreaFrac;
-    sd.melt_ok = sd.melt_factor >= 0.;
-    bool any_after = false;
-    WgD2 sa[kSnowChunk], sb[kSnowChunk];
-    int32_t ea[kSnowChunk], eb[kSnowChunk];
-#pragma unroll
-    for (int j = 0; j < kSnowChunk; j++) {
-      sa[j] = snow_any ? sp[int64_t(j) * n] : WgD2{0., 0.};
-      ea[j] = ep[int64_t(j) * n];
-    }
-#pragma unroll 1
-    for (int c = 0; c < WG_DEV_NPAIR / kSnowChunk; c++) {
-      const bool more = c + 1 < WG_DEV_NPAIR / kSnowChunk;
-      if (more) {
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          sb[j] = snow_any ? sp[int64_t((c + 1) * kSnowChunk + j) * n] : WgD2{0., 0.};
-          eb[j] = ep[int64_t((c + 1) * kSnowChunk + j) * n];
-        }
-      }
-      // Sub-cells without snow above freezing keep a zero storage and add
-      // eff_bare = prec_to_soil + 0 to the effective precipitation, the full step's
-      // result for them.  The wavefront takes that path for the whole chunk when all
-      // its lanes may; otherwise every lane runs the full step, one straight-line
-      // block for the chunk, whose sub-cells the compiler interleaves.
-      double tx[kSnowChunk], ty[kSnowChunk];
-      int ex[kSnowChunk], ey[kSnowChunk];
-      bool bare = true;
-#pragma unroll
-      for (int j = 0; j < kSnowChunk; j++) {
-        const int32_t e2 = ea[j];
-        ex[j] = int(int16_t(e2 & 0xffff));
-        ey[j] = int(int16_t(e2 >> 16));
-        tx[j] = sd.tempC - ((ex[j] - sd.elev0) * sd.gradnt);
-        ty[j] = sd.tempC - ((ey[j] - sd.elev0) * sd.gradnt);
-        bare = bare && sa[j].x == 0. && sa[j].y == 0. && tx[j] > sd.snowfz && ty[j] > sd.snowfz;
-      }
-      bare = bare && sd.melt_ok;
-      if (__builtin_amdgcn_ballot_w64(!bare) == 0) {
-        if (c == 0) acc.temp_max = tx[0];
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          acc.eff += sd.eff_bare;
-          acc.eff += sd.eff_bare;
-          sa[j] = WgD2{0., 0.};
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          sa[j].x = snow_subcell(sa[j].x, tx[j], ex[j], c == 0 && j == 0, sd, acc);
-          sa[j].y = snow_subcell(sa[j].y, ty[j], ey[j], false, sd, acc);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kSnowChunk; j++) {
-        const WgD2 v = sa[j];
-        const bool nz = v.x != 0. || v.y != 0.;
-        any_after |= nz;
-        if (snow_any || nz) sp[int64_t(c * kSnowChunk + j) * n] = v;
-      }
-      if (more) {
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          sa[j] = sb[j];
-          ea[j] = eb[j];
-        }
-      }
-    }
-    X.snow_any[mp] = any_after ? 1 : 0;
-    dailySnowEvapo = acc.evapo;
-    acc.snow_sum /= 100.;
-    acc.eff /= 100.;
-    dailySnowEvapo /= 100.;
-    acc.change /= 100.;
-    landStorageChangeSum += acc.change;
-  }
-  load_cell_in_b(S, X, mp, p, ci);
-  const double snow_sum = acc.snow_sum;
-  const double TempElevMax = acc.temp_max;
-  dailyEffPrec = acc.eff;
-  X.snow[mp] = snow_sum;
-
-  // immediate runoff, daily.cpp:1066-1071
-  const float built_up = ci.s_built_up;
-  if (built_up > 0.) {
-    immediate_runoff = kRunoffFracBuiltUp * dailyEffPrec * built_up;
-    dailyEffPrec -= immediate_runoff;
-  }
-
-  // soil, runoff, AET, recharge, daily.cpp:1080-1239
-  const double cfa = ci.x_cfa;
-  const float smax = ci.x_smax;
-  double soil = ci.x_soil;
-  if (landAreaFrac <= 0.) {
-    transfer += soil;
-    transfer *= cfa;
-    soil = 0.;
-    daily_gw_recharge = 0.;
-    total_daily_runoff = 0.;
-  } else {
-    soil *= lafPrev / landAreaFrac;
-    initialStorage = soil;
-    soil_water_overflow = 0;
-    if (soil > smax) {
-      soil_water_overflow = soil - smax;
-      soil = smax;
-    }
-    if (TempElevMax > T_SNOWFZ) {
-      if (smax > 0.) {
-        const double soil_saturation = soil / smax;
-        daily_runoff = dailyEffPrec * wg_pow(soil_saturation, ci.x_gamma);
-        if (dailySoilPET > (maxDailyPET - dailyCanopyEvapo) * soil_saturation)
-          dailyAET = (maxDailyPET - dailyCanopyEvapo) * soil_saturation;
-        else
-          dailyAET = dailySoilPET;
-        soil += dailyEffPrec - dailyAET - daily_runoff;
-        if (fabs(soil) <= kMinStorVol) soil = 0.;
-        dailyEffPrec = 0.;
-        if (soil < 0.) {
-          dailyAET += soil;
-          soil = 0.;
-        }
-        daily_runoff *= cfa;
-        immediate_runoff *= cfa;
-        const double rgmax = ci.s_rgmax / 100.;
-        const float fg = ci.s_gw_factor;
-        if (rgmax < (fg * daily_runoff))
-          daily_gw_recharge = rgmax;
-        else
-          daily_gw_recharge = fg * daily_runoff;
-        pot_gw_recharge = 0.;
-        if (((arid_gw) && (ci.s_texture < 21)) && (ci.s_ldd >= 0)) {
-          if (dailyPrec <= ci.s_pcritgwa) {
-            pot_gw_recharge = daily_gw_recharge;
-            daily_gw_recharge = 0.;
-          }
-        }
-        daily_runoff -= pot_gw_recharge;
-        pot_gw_recharge /= cfa;
-        soil += pot_gw_recharge;
-        if (soil > smax) {
-          soil_water_overflow += soil - smax;
-          soil = smax;
-        }
-        soil_water_overflow *= cfa;
-        total_daily_runoff = daily_runoff + immediate_runoff + soil_water_overflow;
-      } else {
-        total_daily_runoff = 0.;
-        daily_gw_recharge = 0.;
-      }
-    } else {
-      soil_water_overflow *= cfa;
-      dailyEffPrec *= cfa;
-      total_daily_runoff += soil_water_overflow + dailyEffPrec;
-      daily_gw_recharge = 0.;
-      dailyAET = 0.;
-    }
-    landStorageChangeSum += soil - initialStorage;
-    double cell_aet = landStorageChangeSum * (cfa - 1.0) - dailyPrec * (cfa - 1.0) +
-                      (dailyAET + dailyCanopyEvapo + dailySnowEvapo) * cfa;
-    if (cell_aet < 0.) neg_land_aet = cell_aet;
-    dailyCellLandAET_uncorr = (dailyAET + dailyCanopyEvapo + dailySnowEvapo);
-  }
-  // G_dailyGwRecharge is handed to routing before the corrections below (daily.cpp:1214)
-  const double recharge_handoff = daily_gw_recharge;
-  // surface runoff, daily.cpp:1241-1257
-  if (neg_land_aet < 0.) total_daily_runoff = total_daily_runoff + neg_land_aet;
-  if (total_daily_runoff < 0.) total_daily_runoff = 0.;
-  if ((total_daily_runoff - daily_gw_recharge) < 0.) {
-    const double neg_runoff = total_daily_runoff - daily_gw_recharge;
-    daily_gw_recharge = total_daily_runoff;
-    soil += neg_runoff;
-  }
-  const double surf_runoff = total_daily_runoff - daily_gw_recharge;
-  X.soil[mp] = soil;
-  X.transfer[mp] = transfer;
+  const double laf_prev = started ? s.laf_prev : s.laf;  // daily.cpp:159-169
+  DayFlux v;
+  day_pet_canopy(sa, s, v, tf, pf, swf, lwf, laf_prev);
+  X.lai_days[mp] = s.lai_days;
+  X.lai_status[mp] = s.lai_status;
+  X.lai_precsum[mp] = s.lai_precsum;
+  X.canopy[mp] = s.canopy;
+  day_snow<kSnowChunk>(sa, s, v, laf_prev, X.snow2 + int64_t(m) * WG_DEV_NPAIR * n + p, S.elev_pairs + p, n);
+  X.snow_any[mp] = s.snow_any ? 1 : 0;
+  DayStatB sb;
+  DayStatLake lake;
+  load_stat_b(S, X, mp, p, sb);
+  load_stat_lake(S, p, lake);
+  load_state_b(X, mp, s);
+  const WgChainLink lk = load_link(S, p);
+  const WgChainStatic cs = load_cstat(S, p);
+  if (kUse) lake.prov_rel = S.use_provrel[use_t];
+  X.snow[mp] = s.snow;
+  day_soil(sb, s, v, laf_prev);
+  X.soil[mp] = s.soil;
+  X.transfer[mp] = s.transfer;
   if (write_diag) {
-    X.d_surf[mp] = surf_runoff;
-    X.d_recharge[mp] = recharge_handoff;
-    X.d_ow_pet[mp] = dailyOpenWaterPET;
-    X.d_aet[mp] = dailyCellLandAET_uncorr;
-    X.d_prec[mp] = dailyPrec;
+    X.d_surf[mp] = v.surf_runoff;
+    X.d_recharge[mp] = v.recharge;
+    X.d_ow_pet[mp] = v.ow_pet;
+    X.d_aet[mp] = v.aet;
+    X.d_prec[mp] = v.prec;
   }
-
-  // ------------------------------------------------------------------
-  // routing without upstream water, routing.cpp:1877-2617
-  // ------------------------------------------------------------------
-  const double cellArea = ci.s_cell_area;
-  const double cf = ci.s_contfreq;
-  const int ldd = ci.s_ldd;
-  const double laf = landAreaFrac;      // G_landAreaFrac of the day
-  const double laf_prev = pd.laf_prev;
-  const double ow_prec = dailyPrec, ow_pet = dailyOpenWaterPET;
-  double dailyLocalSurfaceRunoff, fswb_catchment = 0.;
-  double localRunoff = 0., lrir = 0., lgwrir = 0., recharge_km3 = 0.;
-  if (laf <= 0.)
-    dailyLocalSurfaceRunoff = transfer * cellArea / 1000000. * laf_prev / 100.;
-  else
-    dailyLocalSurfaceRunoff = surf_runoff * cellArea / 1000000. * laf / 100.;
-  if (ldd >= 0) {
-    fswb_catchment = ci.s_fswb_init * 20.;
-    if (fswb_catchment > 1.) fswb_catchment = 1.;
-    lrir = (1. - fswb_catchment) * dailyLocalSurfaceRunoff;
-  }
-  const bool arid = (ci.s_aindex == 1);
-  if (arid && (ldd >= 0)) {
-    localRunoff = fswb_catchment * dailyLocalSurfaceRunoff;
-    recharge_km3 = recharge_handoff * cellArea * (laf / 100.) / 1000000.;
-  } else {
-    // humid cells (routing.cpp:1968-2039) and inland sinks (2112-2159)
-    const double gw_prev = ci.x_gw;
-    double netGWin = recharge_handoff * cellArea * (laf / 100.) / 1000000.;
-    if (kUse) netGWin -= use_nag;  // routing.cpp:1990-1996, 2131-2137
-    double gw = gw_prev * ci.s_e_gw + ci.s_inv_kgw * netGWin * ci.s_ome_gw;
-    if (fabs(gw) <= kMinStorVol) gw = 0.;
-    double gw_runoff = gw_prev - gw + netGWin;
-    if (gw_runoff <= 0.) {
-      gw_runoff = 0.;
-      gw = gw_prev + netGWin;
-      if (fabs(gw) <= kMinStorVol) gw = 0.;
-    }
-    X.gw[mp] = gw;
-    if (ldd >= 0) {
-      lgwrir = (1. - fswb_catchment) * gw_runoff;
-      const double localGWRunoff = fswb_catchment * gw_runoff;
-      localRunoff = (fswb_catchment * dailyLocalSurfaceRunoff) + localGWRunoff;
-    } else {
-      if (laf == 0.)
-        dailyLocalSurfaceRunoff = transfer * cellArea / 1000000. * laf_prev / 100.;
-      else
-        dailyLocalSurfaceRunoff = surf_runoff * cellArea / 1000000. * laf / 100.;
-      localRunoff = dailyLocalSurfaceRunoff + gw_runoff;
-    }
-  }
-
-  if (X.pot_base) {
-    // terms of the potential cell runoff: the local runoff terms (routing.cpp:2045-2047
-    // humid, 2180 inland sinks; (semi-)arid cells add their groundwater runoff in the
-    // chain, 3372-3373) and the open-water precipitation minus evaporation of
-    // G_lakeBalance (daily.cpp:773), which wg_pot_runoff_kernel completes
-    X.pot_base[mp] = (ldd < 0) ? localRunoff : (arid ? localRunoff + lrir : (localRunoff + lrir) + lgwrir);
-    X.pot_ow[mp] = ow_prec - ow_pet;
-  }
-
-  double inflow = localRunoff, outflow = 0.;
-  const double k_sw = ci.s_k_sw;
-  const double evarexp = ci.s_evarexp;
-  const bool arid_swb = arid && (ldd >= 0);
-  double gwr_loclak = 0., gwr_locwet = 0.;
-  // local lake, routing.cpp:2316-2490
-  const double loc_lake = ci.s_loc_lake;
-  if (loc_lake > 0.) {
-    const double prev = ci.x_loc_lake, rf = pd.red_ll;
-    const double maxStorage = ((loc_lake) / 100.) * cellArea * ci.s_lake_depth;
-    double evap = ((1.0 - cfa) * ow_prec * rf) + (cfa * (ow_pet * rf));
-    if (evap < 0.) evap = 0.;
-    const double totalInflow = inflow + (ow_prec * rf) * (cellArea / 1000000.) * (loc_lake / 100.);
-    if (arid_swb) gwr_loclak = kKswbgw * rf * loc_lake / 100. / (cf / 100.);
-    const double PETgwr = evap * (cellArea / 1000000.) * (loc_lake / 100.) + gwr_loclak * cellArea * (cf / 100.) / 1000000.;
-    double PETgwrMax = prev + maxStorage + totalInflow;
-    if (PETgwrMax < 0.) PETgwrMax = 0.;
-    double st;
-    if (PETgwr > PETgwrMax) {
-      st = (-1.) * maxStorage;
-      gwr_loclak *= PETgwrMax / PETgwr;
-    } else {
-      st = prev + totalInflow - PETgwr;
-    }
-    if (prev > 0.) {
-      outflow = k_sw * prev * wg_pow((prev / maxStorage), kLakeOutflowExp);
-      if (st <= 0.) {
-        outflow = 0;
-      } else {
-        if (outflow > st) outflow = st;
-      }
-    } else {
-      outflow = 0.;
-    }
-    st -= outflow;
-    if (fabs(st) <= kMinStorVol) st = 0.;
-    if (st > maxStorage) {
-      outflow += (st - maxStorage);
-      st = maxStorage;
-    }
-    inflow = outflow;
-    double r = 1. - wg_pow(fabs(st - maxStorage) / (2. * maxStorage), (evarexp * kEvapoRedExp));
-    if (r < 0.) r = 0.;
-    if (r > 1.) r = 1.;
-    X.loc_lake[mp] = st;
-    X.red_ll[mp] = r;
-  }
-  // local wetland, routing.cpp:2495-2617
-  const double loc_wetland = ci.s_loc_wetland;
-  if (loc_wetland > 0.) {
-    const double prev = ci.x_loc_wetl, rf = pd.red_lw;
-    const double maxStorage = ((loc_wetland) / 100.) * cellArea * ci.s_wetl_depth;
-    double evap = ((1.0 - cfa) * ow_prec * rf) + (cfa * (ow_pet * rf));
-    if (evap < 0.) evap = 0.;
-    const double totalInflow = inflow + (ow_prec * rf * (cellArea / 1000000.) * (loc_wetland / 100.));
-    if (arid_swb) gwr_locwet = kKswbgw * rf * loc_wetland / 100. / (cf / 100.);
-    const double PETgwr = evap * (cellArea / 1000000.) * (loc_wetland / 100.) + gwr_locwet * cellArea * (cf / 100.) / 1000000.;
-    const double PETgwrMax = prev + totalInflow;
-    double st;
-    if (PETgwr > PETgwrMax) {
-      st = 0.;
-      gwr_locwet *= PETgwrMax / PETgwr;
-    } else {
-      st = prev + totalInflow - PETgwr;
-    }
-    if (fabs(st) <= kMinStorVol) st = 0.;
-    if (st > 0.) {
-      outflow = k_sw * st * wg_pow((st / maxStorage), kWetlOutflowExp);
-      if (outflow > st) outflow = st;
-    } else {
-      outflow = 0.;
-    }
-    st -= outflow;
-    if (st > maxStorage) {
-      outflow += (st - maxStorage);
-      st = maxStorage;
-    }
-    inflow = outflow;
-    double r = 1. - wg_pow(fabs(st - maxStorage) / (maxStorage), (evarexp * kEvapoRedExp));
-    if (r < 0.) r = 0.;
-    if (r > 1.) r = 1.;
-    X.loc_wetl[mp] = st;
-    X.red_lw[mp] = r;
-  }
-
-  // record of the routing terms that do not depend on the inflow from upstream
-  // (routing.cpp:2630-3514)
-  const WgChainLink lk = ci.link;
   ChainRec c;
-  double *v = c.v;
-  const double e_sw = ci.s_e_sw;
-  {
-    const WgChainStatic &cs = ci.cstat;
-    c.inv_ksw = cs.inv_ksw;
-    c.ome_sw = cs.ome_sw;
-    c.inv_kgw = cs.inv_kgw;
-    c.ome_gw = cs.ome_gw;
-    c.area = cs.area;
-    c.cf100 = cs.cf100;
-    c.flags = lk.flags;
+  double *w = c.v;
+  c.inv_ksw = cs.inv_ksw;
+  c.ome_sw = cs.ome_sw;
+  c.inv_kgw = cs.inv_kgw;
+  c.ome_gw = cs.ome_gw;
+  c.area = cs.area;
+  c.cf100 = cs.cf100;
+  c.flags = lk.flags;
+  PotTerms pot;
+  day_local_routing<kUse>(sb, lake, s, v, use_desired, use_nag, c, pot);
+  if (!(sb.arid && (sb.ldd >= 0))) X.gw[mp] = s.gw;
+  if (X.pot_base) {
+    X.pot_base[mp] = pot.base;  // wg_pot_runoff_kernel completes the terms
+    X.pot_ow[mp] = pot.ow;
   }
-  {
-    // river velocity and storage terms, routing.cpp:3424-3478
-    const double L = ci.s_river_length;
-    const double prev = ci.x_river;
-    const double velocity = new_river_velocity(ci.s_vel_c1, ci.s_vel_c2, ci.s_bottom_width, prev, L);
-    const double K = velocity / L;
-    const double eK = wg_exp(-1. * K);
-    const double riverAreaFrac = pd.river_frac_next;
-    v[CF_INFLOW] = inflow;
-    v[CF_LRIR] = lrir;
-    v[CF_LGWRIR] = lgwrir;
-    v[CF_RV_PREV] = prev;
-    v[CF_RV_S0E] = prev * eK;
-    v[CF_RV_INVK] = 1. / K;
-    v[CF_RV_OME] = 1. - eK;
-    v[CF_RV_TERM] = (K * prev * eK) / (1. - eK);
-    v[CF_RV_EVAP] = ((1.0 - cfa) * (ow_prec) + (cfa * ow_pet)) * riverAreaFrac / 100. * cellArea / 1000000.;
-    v[CF_RV_PREC] = ow_prec * riverAreaFrac / 100. * cellArea / 1000000.;
+  if (sb.loc_lake > 0.) {
+    X.loc_lake[mp] = s.loc_lake;
+    X.red_ll[mp] = s.red_ll;
   }
-  v[CF_OW_PREC] = ow_prec;
-  v[CF_OW_PET] = ow_pet;
-  {
-    // global lake, routing.cpp:2633-2676
-    const double lake_area = ci.s_lake_area;
-    v[CF_GL_LP] = 0.;
-    v[CF_GL_USE] = 0.;
-    v[CF_GL_MAX] = 0.;
-    v[CF_GL_PREV] = 0.;
-    v[CF_GL_S0E] = 0.;
-    v[CF_GL_GWR] = 0.;
-    if (lake_area > 0.) {
-      const double prev = ci.x_glo_lake, rf = pd.red_gl;
-      double evap = ((1.0 - cfa) * ow_prec) + (cfa * ow_pet * rf);
-      if (evap < 0.) evap = 0.;
-      const double gwr = arid_swb ? kKswbgw * rf * (lake_area / (cellArea * (cf / 100.))) : 0.;
-      v[CF_GL_MAX] = lake_area * ci.s_lake_depth;
-      v[CF_GL_LP] = (ow_prec * (lake_area / 1000000.));
-      v[CF_GL_GWR] = gwr;
-      // the lake's share of the use, half of it when the cell has a reservoir too
-      // (routing.cpp:2680-2695)
-      const double use_lake = (lk.flags & CFL_RES) ? 0.5 * use_desired : use_desired;
-      v[CF_GL_USE] = evap * (lake_area / 1000000.) + gwr * cellArea * (cf / 100.) / 1000000. +
-                     (kUse ? use_lake : 0.);
-      v[CF_GL_PREV] = prev;
-      v[CF_GL_S0E] = prev * e_sw;
-    }
+  if (sb.loc_wetland > 0.) {
+    X.loc_wetl[mp] = s.loc_wetl;
+    X.red_lw[mp] = s.red_lw;
   }
-  {
-    // global wetland, routing.cpp:3181-3222
-    const double glo_wetland = ci.s_glo_wetland;
-    v[CF_GW_WP] = 0.;
-    v[CF_GW_PET] = 0.;
-    v[CF_GW_MAX] = 0.;
-    v[CF_GW_PREV] = 0.;
-    v[CF_GW_S0E] = 0.;
-    v[CF_GW_GWR] = 0.;
-    if (glo_wetland > 0) {
-      const double prev = ci.x_glo_wetl, rf = pd.red_gw;
-      double evap = ((1.0 - cfa) * (ow_prec * rf)) + (cfa * (ow_pet * rf));
-      if (evap < 0.) evap = 0.;
-      const double gwr = arid_swb ? kKswbgw * rf * glo_wetland / 100. / (cf / 100.) : 0.;
-      v[CF_GW_MAX] = ((glo_wetland) / 100.) * cellArea * ci.s_wetl_depth;
-      v[CF_GW_WP] = (ow_prec * rf * (cellArea / 1000000.) * (glo_wetland / 100.));
-      v[CF_GW_GWR] = gwr;
-      v[CF_GW_PET] = evap * (cellArea / 1000000.) * ((glo_wetland) / 100.) + gwr * cellArea * (cf / 100.) / 1000000.;
-      v[CF_GW_PREV] = prev;
-      v[CF_GW_S0E] = prev * e_sw;
-    }
-  }
-  {
-    // groundwater of (semi-)arid cells, routing.cpp:3310-3330
-    v[CF_A_GWR_LL] = gwr_loclak;
-    v[CF_A_GWR_LW] = gwr_locwet;
-    v[CF_A_RECH] = recharge_km3;
-    const double gprev = arid_swb ? ci.x_gw : 0.;
-    v[CF_A_PREV] = gprev;
-    v[CF_A_S0E] = gprev * ci.s_e_gw;
-  }
-  {
-    // reservoir, routing.cpp:2807-2860 inputs
-    const bool res = (lk.flags & CFL_RES) != 0;
-    v[CF_RES_PREV] = res ? ci.x_res : 0.;
-    v[CF_RES_RED] = res ? pd.red_res : 0.;
-    v[CF_RES_CFA] = cfa;
-    v[CF_RES_KREL] = res ? ci.x_k_release : 0.;
-    v[CF_RES_CAP] = res ? ci.s_stor_cap : 0.;
-    v[CF_RES_QMEAN] = res ? ci.s_mean_outflow : 0.;
-    v[CF_RES_AREA] = res ? ci.s_reservoir_area : 0.;
-    v[CF_RES_PROVREL] = res ? (kUse ? S.use_provrel[use_t] : ci.s_prov_rel) : 0.;
-    v[CF_RES_PAD] = 0.;
-  }
-  v[CF_USE] = use_desired;
-  v[CF_A_NUG] = use_nag;
   if (lk.nu == 0) {
     // no upstream cell: G_riverInflow[n] is still 0 when the cell is routed
     const ChainOut o = chain_step<kUse>(c, 0.0, day_info(doy));
     store_chain(X, mp, c.flags, o);
     if (lk.station >= 0)
-      X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + lk.station] = (ldd >= 0) ? o.tv : 0.;
+      X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + lk.station] = (sb.ldd >= 0) ? o.tv : 0.;
   } else {
-    // the prefix for every routed cell, the suffix for cells with a global lake or reservoir
     // the pairs holding the prefix for every routed cell (the last of them also
     // holds the first suffix field), the rest for cells with a lake or reservoir
     WgD2 *dst = rec_at(X, n, m, p);
     constexpr int kPrefixPairs = (CF_PREFIX + 1) / 2;
 #pragma unroll
-    for (int k = 0; k < kPrefixPairs; k++) dst[int64_t(k) * n] = WgD2{v[2 * k], v[2 * k + 1]};
+    for (int k = 0; k < kPrefixPairs; k++) dst[int64_t(k) * n] = WgD2{w[2 * k], w[2 * k + 1]};
     if (lk.flags & (CFL_LAKE | CFL_RES)) {
 #pragma unroll
-      for (int k = kPrefixPairs; k < CF_USE / 2; k++) dst[int64_t(k) * n] = WgD2{v[2 * k], v[2 * k + 1]};
+      for (int k = kPrefixPairs; k < CF_USE / 2; k++) dst[int64_t(k) * n] = WgD2{w[2 * k], w[2 * k + 1]};
     }
-    if (kUse) dst[int64_t(CF_USE / 2) * n] = WgD2{v[CF_USE], v[CF_A_NUG]};
+    if (kUse) dst[int64_t(CF_USE / 2) * n] = WgD2{w[CF_USE], w[CF_A_NUG]};
   }
 }
+
+#include "wg_days_kernel.h"
 
 // Workgroup barrier that orders LDS only.  The level walk exchanges data between
 // threads through LDS alone (its global stores are read by later kernels), and a
@@ -2057,24 +1146,11 @@ __global__ void wg_station_reduce(WgState X, int32_t n_stations, int32_t n_membe
   X.st_sum[i] = s;
 }
 
-// Adds the day's potential cell runoff of every continental cell of [p0, p1)
-// (device order) to its running sum, G_potCellRunoff[n] += potCellRunoff
-// (routing.cpp:1970, 2053, 2187, 3379): the local runoff terms, then the arid
-// groundwater step's runoff where that step ran, then the open-water balance, in
-// the reference's order of addition.
 __global__ void wg_pot_runoff_kernel(WgStatic S, WgState X, int32_t p0, int32_t p1) {
   const int p = p0 + int(blockIdx.x * blockDim.x + threadIdx.x);
   if (p >= p1) return;
-  const int f = S.cflags[p];
-  if (!(f & CFL_CONT)) return;
-  const int64_t mp = int64_t(blockIdx.y) * S.n + p;
-  const double base = X.pot_base[mp];
-  const double lake_balance = X.pot_ow[mp] * X.cfa[mp];  // (dailyPrec - dailyOpenWaterPET) * CFA
-  const double ow = (lake_balance / 1000000.0) *
-                    ((S.lake_area[p] + S.reservoir_area[p]) +
-                     ((S.cell_area[p] / 100.0) * ((S.loc_lake[p] + S.loc_wetland[p]) + S.glo_wetland[p])));
-  const double pot = (f & CFL_ARID) ? (base + X.pot_lgw[mp]) + ow : base + ow;
-  X.pot_acc[mp] += pot;
+  if (!(S.cflags[p] & CFL_CONT)) return;
+  add_pot_runoff(S, X, int64_t(blockIdx.y) * S.n + p, p);
 }
 
 // Sets the day clock read by the kernels of a captured block of days; launched
