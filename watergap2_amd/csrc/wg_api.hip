@@ -985,12 +985,14 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
     UP(df, lai_max); S.lai_max = df;
     // elevation: channel 0 [N], sub-cells as packed int16 pairs [50][N]
     std::vector<int16_t> e0(n);
-    std::vector<int32_t> pairs(size_t(WG_DEV_NPAIR) * n);
+    std::vector<int32_t> pairs(size_t(WG_DEV_NPAIR) * n), range(n);
     for (int32_t p = 0; p < n; p++) {
       const int16_t *ev = st->elevation + size_t(H->perm[p]) * WG_NELEV;
       e0[p] = ev[0];
       for (int k = 0; k < WG_DEV_NPAIR; k++)
         pairs[size_t(k) * n + p] = int32_t(uint32_t(uint16_t(ev[1 + 2 * k])) | (uint32_t(uint16_t(ev[2 + 2 * k])) << 16));
+      const auto mm = std::minmax_element(ev + 1, ev + 1 + WG_DEV_NSUB);
+      range[p] = int32_t(uint32_t(uint16_t(*mm.first)) | (uint32_t(uint16_t(*mm.second)) << 16));
     }
     int16_t *de0;
     int r_ = upload(H, &de0, e0);
@@ -1000,6 +1002,9 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
     r_ = upload(H, &dpairs, pairs);
     if (r_) { *out = h.release(); return r_; }
     S.elev_pairs = dpairs;
+    r_ = upload(H, &dpairs, range);
+    if (r_) { *out = h.release(); return r_; }
+    S.elev_range = dpairs;
   }
   // upstream CSR in device indices, each list in routing order (the order of the
   // reference's serial += into the downstream cell's inflow)
@@ -1100,11 +1105,15 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
       }
     }
     {
-      int per_cu = 0, cus = 0;
+      int per_cu = 0, cus = 0, lds_cu = 0;
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wg_days_kernel<false>, 64, kDaysLdsBytes) ==
               hipSuccess &&
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, H->device) == hipSuccess)
-        H->day_capacity = int64_t(per_cu) * cus;
+          hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, H->device) ==
+              hipSuccess &&
+          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, H->device) == hipSuccess) {
+        constexpr int kGiven = (kDaysLdsBytes + kLdsStep - 1) / kLdsStep * kLdsStep;
+        H->day_capacity = int64_t(std::min(per_cu, lds_cu / kGiven)) * cus;
+      }
     }
     // the largest upstream count of each level
     for (int32_t l = 0; l + 1 < int32_t(H->level_off.size()); l++) {

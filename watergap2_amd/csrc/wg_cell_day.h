@@ -13,12 +13,12 @@
 // updateNetAbstractionGW, routing.cpp:5503-5572: the day's net abstraction from
 // groundwater, with the return flows of irrigation from surface water reduced
 // when the last day's surface-water use went unsatisfied (G_dailyRemainingUse > 0)
-// or given back when a delayed use was satisfied (< 0).  U points at the cell's
-// first water-use field, us is the stride between fields.
-__device__ inline double update_net_abstraction_gw(double *U, int64_t us, double frgi, double nug) {
-  double &dru = U[WG_USE_DAILY_REMAINING * us], &ui = U[WG_USE_UNSAT_IRRIG * us];
-  double &uo = U[WG_USE_UNSAT_OTHER * us], &rrf = U[WG_USE_REDUCED_RETURN * us];
-  const double wu = U[WG_USE_WITHDRAWAL_IRRIG * us], cu = U[WG_USE_CONSUMPTIVE_IRRIG * us];
+// or given back when a delayed use was satisfied (< 0).  U points at the
+// member's first water-use field, us is the stride between fields.
+__device__ inline double update_net_abstraction_gw(double *U, int64_t us, uint32_t p, double frgi, double nug) {
+  double &dru = at(U + WG_USE_DAILY_REMAINING * us, p), &ui = at(U + WG_USE_UNSAT_IRRIG * us, p);
+  double &uo = at(U + WG_USE_UNSAT_OTHER * us, p), &rrf = at(U + WG_USE_REDUCED_RETURN * us, p);
+  const double wu = at(U + WG_USE_WITHDRAWAL_IRRIG * us, p), cu = at(U + WG_USE_CONSUMPTIVE_IRRIG * us, p);
   if (dru > 1.e-12) {
     if (wu > 0.) {
       const double eff = cu / wu;
@@ -67,11 +67,11 @@ __device__ inline double update_net_abstraction_gw(double *U, int64_t us, double
 }
 
 // annualWaterUsePostProcessing, routing.cpp:5257-5296, for one cell
-__device__ inline void water_use_year_end(double *U, int64_t us) {
-  double &tu = U[WG_USE_TOTAL_UNSAT * us], &ui = U[WG_USE_UNSAT_IRRIG * us];
-  double &uo = U[WG_USE_UNSAT_OTHER * us], &rrf = U[WG_USE_REDUCED_RETURN * us];
-  double &tu_py = U[WG_USE_UNSAT_PREV_YEAR * us], &ui_py = U[WG_USE_UNSAT_IRRIG_PREV_YEAR * us];
-  double &uo_py = U[WG_USE_UNSAT_OTHER_PREV_YEAR * us], &rrf_py = U[WG_USE_REDUCED_RETURN_PREV_YEAR * us];
+__device__ inline void water_use_year_end(double *U, int64_t us, uint32_t p) {
+  double &tu = at(U + WG_USE_TOTAL_UNSAT * us, p), &ui = at(U + WG_USE_UNSAT_IRRIG * us, p);
+  double &uo = at(U + WG_USE_UNSAT_OTHER * us, p), &rrf = at(U + WG_USE_REDUCED_RETURN * us, p);
+  double &tu_py = at(U + WG_USE_UNSAT_PREV_YEAR * us, p), &ui_py = at(U + WG_USE_UNSAT_IRRIG_PREV_YEAR * us, p);
+  double &uo_py = at(U + WG_USE_UNSAT_OTHER_PREV_YEAR * us, p), &rrf_py = at(U + WG_USE_REDUCED_RETURN_PREV_YEAR * us, p);
   if (tu < tu_py) {
     tu_py = tu;
     ui_py = ui;
@@ -192,7 +192,6 @@ __device__ inline double lai_day(int &days, int init_days, int &status, int lct,
 
 struct SnowDay {
   double tempC, gradnt, scale_num, laf, prec_to_soil, soil_pet, snowfz, snowmt, melt_factor;
-  double eff_bare;  // the effective precipitation of a sub-cell without snow above freezing
   double inv_laf;   // 1 / laf, correctly rounded
   int elev0;
   bool melt_ok;     // melt_factor >= 0 (a NaN or negative factor takes the full step)
@@ -397,13 +396,61 @@ __device__ __forceinline__ void day_pet_canopy(const DayStatA &a, CellState &s, 
   v.land_change = change;
 }
 
-// Snow on the elevation sub-cells, daily.cpp:897-1062, serial in sub-cell order.
-// Sub-cells are stored in pairs ([member][pair][cell] x 2 doubles, elevations as
-// packed int16 pairs) and streamed in double-buffered chunks so that a wavefront
-// keeps many 16-byte loads in flight.  sp, ep: pair 0 of the cell; n: stride of pairs.
+// Elevation extremes of a cell's sub-cells and its first sub-cell, for the test
+// whether a whole day is bare.
+struct ElevRange {
+  int16_t lo, hi, first;
+};
+
+// One sub-cell of snow_subcell for finite storages 0 <= q (rescaled, before the
+// zeroing of tiny ones) and prec_to_soil not NaN, with minima and maxima in place of
+// most selects: precipitation pr and demand pe count only when freezing, so that
+// max((s + pr) - pe, 0) is the storage after sublimation (s itself when not
+// freezing) and min(pe, s + pr) the sublimation (0 then); the melt potential is
+// negative or zero exactly when the temperature is not above M_T_SNOWMT, so its
+// maximum with 0 is the melt demand and min(demand, s) the melt.  Each result is
+// the reference's branch's, in value and rounding; a zero's sign may differ where
+// it is only added to or subtracted from a sum that is not -0.
+// kThresh: storages above 1,000 mm may occur (daily.cpp:958-976).
+template <bool kThresh>
+__device__ __forceinline__ double snow_subcell_fast(double q, double temp_elev, int elev_e, bool first,
+                                                    const SnowDay &d, SnowAcc &a) {
+  double s = (q <= kMinStorVol) ? 0. : q;
+  const double init_s = s;
+  if (kThresh) {
+    const bool big = s > 1000.;
+    const bool use_thresh = big && a.thresh > 0;
+    const double temp_thresh = d.tempC - ((a.thresh - d.elev0) * d.gradnt);
+    a.thresh = (big && a.thresh == 0) ? elev_e : a.thresh;
+    temp_elev = use_thresh ? temp_thresh : temp_elev;
+  }
+  const bool freeze = temp_elev <= d.snowfz;
+  const double pr = freeze ? d.prec_to_soil : 0.;
+  const double pe = freeze ? d.soil_pet : 0.;
+  const double s_fall = s + pr;
+  a.evapo += fmin(pe, s_fall);
+  s = fmax(s_fall - pe, 0.);
+  const double demand = fmax(d.melt_factor * (temp_elev - d.snowmt), 0.);
+  const double melt = fmin(demand, s);
+  s = fmax(s - demand, 0.);
+  a.change += s - init_s;
+  if (first) a.temp_max = temp_elev;
+  a.snow_sum += s;
+  a.eff += (d.prec_to_soil - pr) + melt;
+  return s;
+}
+
+// Snow on the elevation sub-cells of a cell with land (s.laf > 0), daily.cpp:897-1062,
+// serial in sub-cell order.  Sub-cells are stored in pairs ([member][pair][cell] x 2 doubles, elevations as
+// packed int16 pairs) and streamed in chunks, the next one loaded while one is
+// stepped, so that a wavefront keeps many 16-byte loads in flight.  sub, elev: the member's pairs [k][n], cell p.
+// What bounds it is VALU issue: a sub-cell is 38 instructions (61 before the minima
+// and maxima of snow_subcell_fast), a bare one 2 additions' share.
 template <int kSnowChunk>
 __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlux &v, double laf_prev,
-                                         WgD2 *__restrict__ sp, const int32_t *__restrict__ ep, int n) {
+                                         const ElevRange &er, WgD2 *sub, const int32_t *elev, uint32_t p, int n) {
+  auto sp = [&](int k) -> WgD2 & { return at(sub + int64_t(k) * n, p); };
+  auto ep = [&](int k) -> int32_t { return at(elev + int64_t(k) * n, p); };
   SnowAcc acc;
   acc.snow_sum = 0.;
   acc.eff = 0.;
@@ -415,106 +462,137 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
   // loop from zeros without reading them, and stores only storages that become
   // non-zero: on warm days such a cell moves no snow bytes at all.
   const bool snow_any = s.snow_any;
-  if (s.laf <= 0.) {
-    for (int k = 0; k < WG_DEV_NPAIR; k++) {
-      const WgD2 w = snow_any ? sp[int64_t(k) * n] : WgD2{0., 0.};
-      s.transfer += w.x / 100.;
-      s.transfer += w.y / 100.;
-      if (snow_any) sp[int64_t(k) * n] = WgD2{0., 0.};
-    }
-    s.snow_any = false;
-    v.snow_evapo = 0.;
+  SnowDay sd;
+  sd.tempC = v.temp;
+  sd.elev0 = a.elev0;
+  sd.gradnt = a.t_gradnt;
+  sd.scale_num = laf_prev;
+  sd.laf = s.laf;
+  sd.prec_to_soil = v.prec_to_soil;
+  sd.soil_pet = v.soil_pet;
+  sd.snowfz = a.t_snowfz;
+  sd.snowmt = a.t_snowmt;
+  sd.melt_factor = a.melt_factor;
+  sd.inv_laf = 1. / s.laf;
+  sd.melt_ok = sd.melt_factor >= 0.;
+  bool any_after = false;
+  // The sub-cell temperature T - (z - z0) gradnt is monotonic in z, rounding
+  // included, so the lowest and the highest sub-cell tell whether every sub-cell is
+  // above freezing.  Without snow each of them then adds prec_to_soil + 0 to the
+  // effective precipitation and nothing else: a wavefront of such cells reads no
+  // sub-cell at all.
+  const double t_lo = sd.tempC - ((er.lo - sd.elev0) * sd.gradnt);
+  const double t_hi = sd.tempC - ((er.hi - sd.elev0) * sd.gradnt);
+  const bool bare_day = !snow_any && sd.melt_ok && t_lo > sd.snowfz && t_hi > sd.snowfz;
+  if (__builtin_amdgcn_ballot_w64(!bare_day) == 0) {
+    const double eff_bare = v.prec_to_soil + 0.;
+    acc.temp_max = sd.tempC - ((er.first - sd.elev0) * sd.gradnt);
+#pragma unroll 20
+    for (int j = 0; j < 2 * WG_DEV_NPAIR; j++) acc.eff += eff_bare;
   } else {
-    SnowDay sd;
-    sd.tempC = v.temp;
-    sd.elev0 = a.elev0;
-    sd.gradnt = a.t_gradnt;
-    sd.scale_num = laf_prev;
-    sd.laf = s.laf;
-    sd.prec_to_soil = v.prec_to_soil;
-    sd.soil_pet = v.soil_pet;
-    sd.snowfz = a.t_snowfz;
-    sd.snowmt = a.t_snowmt;
-    sd.melt_factor = a.melt_factor;
-    sd.eff_bare = v.prec_to_soil + 0.;
-    sd.inv_laf = 1. / s.laf;
-    sd.melt_ok = sd.melt_factor >= 0.;
-    bool any_after = false;
-    WgD2 sa[kSnowChunk], sb[kSnowChunk];
-    int32_t ea[kSnowChunk], eb[kSnowChunk];
+    // snow_subcell_fast needs a number for the precipitation and a melt factor >= 0
+    const bool usual = sd.melt_ok && sd.prec_to_soil == sd.prec_to_soil;
+    WgD2 in[kSnowChunk];
+    int32_t en[kSnowChunk];
 #pragma unroll
     for (int j = 0; j < kSnowChunk; j++) {
-      sa[j] = snow_any ? sp[int64_t(j) * n] : WgD2{0., 0.};
-      ea[j] = ep[int64_t(j) * n];
+      in[j] = snow_any ? sp(j) : WgD2{0., 0.};
+      en[j] = ep(j);
     }
 #pragma unroll 1
     for (int c = 0; c < WG_DEV_NPAIR / kSnowChunk; c++) {
-      const bool more = c + 1 < WG_DEV_NPAIR / kSnowChunk;
-      if (more) {
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          sb[j] = snow_any ? sp[int64_t((c + 1) * kSnowChunk + j) * n] : WgD2{0., 0.};
-          eb[j] = ep[int64_t((c + 1) * kSnowChunk + j) * n];
-        }
-      }
-      // Sub-cells without snow above freezing keep a zero storage and add
-      // eff_bare = prec_to_soil + 0 to the effective precipitation, the full step's
-      // result for them.  The wavefront takes that path for the whole chunk when all
-      // its lanes may; otherwise every lane runs the full step, one straight-line
-      // block for the chunk, whose sub-cells the compiler interleaves.
-      double tx[kSnowChunk], ty[kSnowChunk];
-      int ex[kSnowChunk], ey[kSnowChunk];
-      bool bare = true;
+      // The land-area rescaling s * scale_num / laf with the reused reciprocal:
+      // q0 = x (1/laf), one exact residual and one correction give the correctly
+      // rounded quotient (as in snow_subcell).  Storages in [0, 1000) mm, by the
+      // high word of q, are the usual case; larger finite ones take the step with
+      // the threshold elevation, anything else (negative, NaN, infinite, -0, or
+      // not `usual`) the general step.
+      WgD2 q[kSnowChunk];
+      int32_t e2[kSnowChunk];
+      uint32_t top = usual ? 0u : 0xffffffffu;
 #pragma unroll
       for (int j = 0; j < kSnowChunk; j++) {
-        const int32_t e2 = ea[j];
-        ex[j] = int(int16_t(e2 & 0xffff));
-        ey[j] = int(int16_t(e2 >> 16));
-        tx[j] = sd.tempC - ((ex[j] - sd.elev0) * sd.gradnt);
-        ty[j] = sd.tempC - ((ey[j] - sd.elev0) * sd.gradnt);
-        bare = bare && sa[j].x == 0. && sa[j].y == 0. && tx[j] > sd.snowfz && ty[j] > sd.snowfz;
+        const double x0 = in[j].x * sd.scale_num, y0 = in[j].y * sd.scale_num;
+        const double rx = x0 * sd.inv_laf, ry = y0 * sd.inv_laf;
+        q[j].x = fma(fma(-rx, sd.laf, x0), sd.inv_laf, rx);
+        q[j].y = fma(fma(-ry, sd.laf, y0), sd.inv_laf, ry);
+        top = max(top, max(uint32_t(__double2hiint(q[j].x)), uint32_t(__double2hiint(q[j].y))));
+        e2[j] = en[j];
       }
-      bare = bare && sd.melt_ok;
-      if (__builtin_amdgcn_ballot_w64(!bare) == 0) {
-        if (c == 0) acc.temp_max = tx[0];
+      // the next chunk's loads fly while this chunk is stepped
+      if (c + 1 < WG_DEV_NPAIR / kSnowChunk) {
 #pragma unroll
         for (int j = 0; j < kSnowChunk; j++) {
-          acc.eff += sd.eff_bare;
-          acc.eff += sd.eff_bare;
-          sa[j] = WgD2{0., 0.};
+          in[j] = snow_any ? sp((c + 1) * kSnowChunk + j) : WgD2{0., 0.};
+          en[j] = ep((c + 1) * kSnowChunk + j);
+        }
+      }
+      if (__builtin_amdgcn_ballot_w64(top >= 0x7ff00000u) != 0) {
+#pragma unroll 1
+        for (int j = 0; j < kSnowChunk; j++) {
+          const WgD2 w0 = snow_any ? sp(c * kSnowChunk + j) : WgD2{0., 0.};
+          const int32_t ee = ep(c * kSnowChunk + j);
+          const int e0 = int(int16_t(ee & 0xffff)), e1 = int(int16_t(ee >> 16));
+          WgD2 w;
+          w.x = snow_subcell(w0.x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0, sd, acc);
+          w.y = snow_subcell(w0.y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
+          const bool nz = w.x != 0. || w.y != 0.;
+          any_after |= nz;
+          if (snow_any || nz) sp(c * kSnowChunk + j) = w;
         }
       } else {
+        const bool thresh = __builtin_amdgcn_ballot_w64(top >= 0x408f4000u) != 0;
+        if (thresh) {
 #pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          sa[j].x = snow_subcell(sa[j].x, tx[j], ex[j], c == 0 && j == 0, sd, acc);
-          sa[j].y = snow_subcell(sa[j].y, ty[j], ey[j], false, sd, acc);
+          for (int j = 0; j < kSnowChunk; j++) {
+            const int e0 = int(int16_t(e2[j] & 0xffff)), e1 = int(int16_t(e2[j] >> 16));
+            q[j].x = snow_subcell_fast<true>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0,
+                                             sd, acc);
+            q[j].y = snow_subcell_fast<true>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < kSnowChunk; j++) {
+            const int e0 = int(int16_t(e2[j] & 0xffff)), e1 = int(int16_t(e2[j] >> 16));
+            q[j].x = snow_subcell_fast<false>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0,
+                                              sd, acc);
+            q[j].y = snow_subcell_fast<false>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
+          }
         }
-      }
-#pragma unroll
-      for (int j = 0; j < kSnowChunk; j++) {
-        const WgD2 w = sa[j];
-        const bool nz = w.x != 0. || w.y != 0.;
-        any_after |= nz;
-        if (snow_any || nz) sp[int64_t(c * kSnowChunk + j) * n] = w;
-      }
-      if (more) {
 #pragma unroll
         for (int j = 0; j < kSnowChunk; j++) {
-          sa[j] = sb[j];
-          ea[j] = eb[j];
+          const bool nz = q[j].x != 0. || q[j].y != 0.;
+          any_after |= nz;
+          if (snow_any || nz) sp(c * kSnowChunk + j) = q[j];
         }
       }
     }
-    s.snow_any = any_after;
-    acc.snow_sum /= 100.;
-    acc.eff /= 100.;
-    v.snow_evapo = acc.evapo / 100.;
-    acc.change /= 100.;
-    v.land_change += acc.change;
   }
+  s.snow_any = any_after;
+  v.snow_evapo = acc.evapo / 100.;
+  v.land_change += acc.change / 100.;
   v.temp_elev_max = acc.temp_max;
-  v.eff_prec = acc.eff;
-  s.snow = acc.snow_sum;
+  v.eff_prec = acc.eff / 100.;
+  s.snow = acc.snow_sum / 100.;
+}
+
+// The same for a cell without land: its snow leaves with the storage transfer.
+__device__ __forceinline__ void day_snow_no_land(CellState &s, DayFlux &v, WgD2 *sub, uint32_t p, int n) {
+  s.transfer += 0.;  // sub-cells without snow add 0
+  if (s.snow_any) {
+    for (int k = 0; k < WG_DEV_NPAIR; k++) {
+      WgD2 &sp = at(sub + int64_t(k) * n, p);
+      const WgD2 w = sp;
+      s.transfer += w.x / 100.;
+      s.transfer += w.y / 100.;
+      sp = WgD2{0., 0.};
+    }
+  }
+  s.snow_any = false;
+  s.snow = 0.;
+  v.snow_evapo = 0.;
+  v.temp_elev_max = 0.;
+  v.eff_prec = 0.;
 }
 
 // Immediate runoff, soil, runoff, AET and recharge, daily.cpp:1066-1257.
@@ -862,8 +940,8 @@ __device__ __forceinline__ void day_local_routing(const DayStatB &b, const DaySt
 // the unsatisfied use is kept and the month's irrigation withdrawal and
 // consumptive use are recorded (fin_ym: model year x 12 + month of the finished
 // day); after day 365 the year-end processing follows (fin_year_end).  U points at
-// the cell's first water-use field.
-__device__ __forceinline__ void day_end_use(const WgStatic &S, double *U, int p, CellState &s, double rem,
+// the member's first water-use field.
+__device__ __forceinline__ void day_end_use(const WgStatic &S, double *U, uint32_t p, CellState &s, double rem,
                                             double loc_lake, double ll_max, double red_exp, int fin_ym,
                                             bool fin_year_end) {
   const int64_t us = S.use_stride;
@@ -886,18 +964,18 @@ __device__ __forceinline__ void day_end_use(const WgStatic &S, double *U, int p,
     s.loc_lake = ls;
   }
   if (S.use_delayed == 1) {
-    const double tu = U[WG_USE_TOTAL_UNSAT * us];
-    U[WG_USE_PREV_TOTAL_UNSAT * us] = tu;
-    U[WG_USE_DAILY_REMAINING * us] = rem - tu;
-    U[WG_USE_TOTAL_UNSAT * us] = rem;
+    const double tu = at(U + WG_USE_TOTAL_UNSAT * us, p);
+    at(U + WG_USE_PREV_TOTAL_UNSAT * us, p) = tu;
+    at(U + WG_USE_DAILY_REMAINING * us, p) = rem - tu;
+    at(U + WG_USE_TOTAL_UNSAT * us, p) = rem;
   } else {
-    U[WG_USE_TOTAL_UNSAT * us] += rem;
-    U[WG_USE_DAILY_REMAINING * us] = rem;
+    at(U + WG_USE_TOTAL_UNSAT * us, p) += rem;
+    at(U + WG_USE_DAILY_REMAINING * us, p) = rem;
   }
-  const int64_t t = int64_t(fin_ym) * S.n + p;
-  U[WG_USE_WITHDRAWAL_IRRIG * us] = S.use_wu[t];
-  U[WG_USE_CONSUMPTIVE_IRRIG * us] = S.use_cu[t];
-  if (fin_year_end) water_use_year_end(U, us);
+  const int64_t t = int64_t(fin_ym) * S.n;
+  at(U + WG_USE_WITHDRAWAL_IRRIG * us, p) = at(S.use_wu + t, p);
+  at(U + WG_USE_CONSUMPTIVE_IRRIG * us, p) = at(S.use_cu + t, p);
+  if (fin_year_end) water_use_year_end(U, us, p);
 }
 
 // The end of a day: reduction factors of the global storages, river width and area

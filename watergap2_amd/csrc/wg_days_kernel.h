@@ -27,21 +27,32 @@
 
 namespace {
 
-// Per-cell statics kept in LDS, [field][64 lanes] doubles behind the exp/log/pow
-// table: read once per launch instead of once per day from memory.
+// Per-cell statics and some of the state, kept in LDS, [field][64 lanes] doubles
+// behind the exp/log/pow table: read once per launch instead of once per day from
+// memory, and out of registers.  Two wavefronts per SIMD hold 256 registers each; the
+// kernel is kept within them, because a spill costs a memory round trip a day and
+// because this compiler can place a spill's store before the point where a branch's
+// lanes rejoin.
 enum DayField : int {
   DF_M_PREC, DF_ALPHA, DF_PET_MXDY, DF_M_NETRAD, DF_MCWH, DF_SNOWFZ, DF_SNOWMT, DF_GRADNT, DF_MELT, DF_ALBEDO,
-  DF_ALBEDO_SNOW, DF_EMIS, DF_LAI, DF_CLASS, DF_SMAX, DF_GWF, DF_GAMMA, DF_CFA, DF_PCRIT, DF_RGMAX, DF_AREA,
+  DF_ALBEDO_SNOW, DF_EMIS, DF_LAI, DF_CLASS, DF_SMAX, DF_GWF, DF_GAMMA, DF_CFA, DF_PCRIT, DF_AREA,
   DF_AREA_M, DF_CF100, DF_FSWB, DF_E_GW, DF_INV_KGW, DF_OME_GW, DF_E_SW, DF_K_SW, DF_INV_KSW, DF_OME_SW,
-  DF_RED_EXP, DF_LL, DF_LL100, DF_LL_MAX, DF_LW, DF_LW100, DF_LW_MAX, DF_GW, DF_GW100, DF_GW_MAX, DF_LENGTH,
+  DF_RED_EXP, DF_LL, DF_LL100, DF_LL_MAX, DF_LW, DF_LW100, DF_LW_MAX, DF_GW, DF_GW_MAX, DF_LENGTH,
   DF_BOTTOM, DF_VEL_C1, DF_VEL_C2, DF_RW_C0, DF_RW_C1, DF_RW_C2, DF_RW_C3, DF_RIVER_MAX, DF_MAX_RAF,
-  DF_COUNT,
-  DF_TV = DF_COUNT,  // the day's transported volumes of the wavefront's cells
+  // state that a day reads once or few cells have
+  DF_LAI_PREC, DF_TRANSFER, DF_GLO_LAKE, DF_RES, DF_K_RELEASE, DF_RED_GL, DF_RED_RES, DF_RED_RIVER, DF_FRAC_CHANGE,
+  DF_NEAR,  // WgDaySlot's near_lo and near_hi
+  DF_TV,    // the day's transported volumes of the wavefront's cells
   DF_ROWS
 };
 constexpr int kDaysLdsBytes = WG_EXP2_LDS_BYTES + DF_ROWS * 64 * int(sizeof(double));
+// LDS is given out in steps of 1,280 bytes: 25 of them, so that a CU's 160 KB hold the
+// rows of five wavefronts (with 32,768 bytes only four started, whatever the occupancy
+// query says, and the rest of the grid waited for whole launches)
+constexpr int kLdsStep = 1280;
+static_assert(kDaysLdsBytes <= 25 * kLdsStep, "five wavefronts per CU");
 
-// bits of DF_GWF's second word
+// bits of DF_GWF's second word, whose upper half holds G_Rgmax
 enum { DB_ARID = 1, DB_CUT = 2, DB_LDD = 4, DB_CONT = 8, DB_LAKE = 16, DB_RES = 32, DB_FULL_LAKE = 64 };
 
 struct WordPair {
@@ -65,29 +76,29 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
   const WgDayWave wv = waves[blockIdx.x];
   const int lane = threadIdx.x;
   const WgDaySlot slot = slots[blockIdx.x * 64 + lane];
-  const int p = slot.cell;
-  if (p < 0) return;
+  if (slot.cell < 0) return;
+  const uint32_t p = uint32_t(slot.cell);
   const int m = blockIdx.y;
   const int n = S.n;
-  const int64_t mp = int64_t(m) * n + p;
+  member_rows(X, m, n);
   double *F = wg_lds + WG_EXP2_LDS_BYTES / sizeof(double) + lane;
   auto fld = [&](int f) -> double { return F[f * 64]; };
 
   const WgChainLink link = load_link(S, p);
   const int rank = ranks[blockIdx.x * 64 + lane];
-  auto near_lane = [&](int u) -> int { return int((u < 4 ? slot.near_lo : slot.near_hi) >> (8 * (u & 3)) & 0xffu); };
+  F[DF_NEAR * 64] = __builtin_bit_cast(double, WordPair{int32_t(slot.near_lo), int32_t(slot.near_hi)});
   int bits = 0;
   {
     DayStatA a;
     DayStatB b;
     DayStatEnd e;
     load_stat_a(S, T, p, a);
-    load_stat_b(S, X, mp, p, b);
+    load_stat_b(S, X, p, b);
     load_stat_end(S, p, e);
     const WgChainStatic cs = load_cstat(S, p);
     bits = (b.arid ? DB_ARID : 0) | (b.recharge_cut ? DB_CUT : 0) | (b.ldd >= 0 ? DB_LDD : 0) |
            (e.contcell ? DB_CONT : 0) | (e.lake_area > 0. ? DB_LAKE : 0) | (e.reservoir_area > 0. ? DB_RES : 0) |
-           (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0);
+           (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0) | int(uint32_t(uint16_t(at(S.rgmax, p))) << 16);
     F[DF_M_PREC * 64] = a.m_prec;
     F[DF_ALPHA * 64] = a.alpha;
     F[DF_PET_MXDY * 64] = a.pet_mxdy;
@@ -109,7 +120,6 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
     F[DF_GAMMA * 64] = b.gamma;
     F[DF_CFA * 64] = b.cfa;
     F[DF_PCRIT * 64] = b.pcritgwa;
-    F[DF_RGMAX * 64] = b.rgmax;
     F[DF_AREA * 64] = b.area;
     F[DF_AREA_M * 64] = b.area_m;
     F[DF_CF100 * 64] = b.cf100;
@@ -129,7 +139,6 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
     F[DF_LW100 * 64] = b.lw100;
     F[DF_LW_MAX * 64] = b.lw_max;
     F[DF_GW * 64] = b.glo_wetland;
-    F[DF_GW100 * 64] = b.gw100;
     F[DF_GW_MAX * 64] = b.gw_max;
     F[DF_LENGTH * 64] = b.river_length;
     F[DF_BOTTOM * 64] = b.bottom;
@@ -149,21 +158,35 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
   if (cont) {
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      if (u < link.nu && near_lane(u) == 0xff) ext |= 1u << u;
+      if (u < link.nu && ((u < 4 ? slot.near_lo : slot.near_hi) >> (8 * (u & 3)) & 0xffu) == 0xffu) ext |= 1u << u;
   }
 
   CellState s;
-  load_state_a(X, mp, s);
-  load_state_b(X, mp, s);
-  load_state_end(X, mp, s);
-  s.laf_prev = X.laf_prev[mp];
-  s.red_gl = X.red_gl[mp];
-  s.red_res = X.red_res[mp];
-  WgD2 *sp = X.snow2 + int64_t(m) * WG_DEV_NPAIR * n + p;
-  const int32_t *ep = S.elev_pairs + p;
+  load_state_a(X, p, s);
+  load_state_b(X, p, s);
+  load_state_end(X, p, s);
+  s.laf_prev = at(X.laf_prev, p);
+  s.red_gl = at(X.red_gl, p);
+  s.red_res = at(X.red_res, p);
+  F[DF_LAI_PREC * 64] = s.lai_precsum;
+  F[DF_TRANSFER * 64] = s.transfer;
+  F[DF_GLO_LAKE * 64] = s.glo_lake;
+  F[DF_RES * 64] = s.res;
+  F[DF_K_RELEASE * 64] = s.k_release;
+  F[DF_RED_GL * 64] = s.red_gl;
+  F[DF_RED_RES * 64] = s.red_res;
+  F[DF_RED_RIVER * 64] = s.red_river;
+  F[DF_FRAC_CHANGE * 64] = s.river_frac_change;
+  const ElevRange er = load_elev_range(S, p);
   const int64_t ring_stride = int64_t(S.n_members) * n;
-  const float *fd = forcing + fday0 * 4 * int64_t(n) + p;
-  float f0 = fd[0], f1 = fd[n], f2 = fd[2 * int64_t(n)], f3 = fd[3 * int64_t(n)];
+  const float *fd = forcing + fday0 * 4 * int64_t(n);
+  float f0 = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
+  if (!kUse) {
+    f0 = at(fd, p);
+    f1 = at(fd + n, p);
+    f2 = at(fd + 2 * int64_t(n), p);
+    f3 = at(fd + 3 * int64_t(n), p);
+  }
 
 #pragma unroll 1
   for (int k = 0; k < days; k++) {
@@ -179,22 +202,22 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
     if (!cont) {
       // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
       // routing.cpp:1876); other cells keep a zero transported volume.
-      __hip_atomic_store(rrow + p, sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&at(rrow, p), sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (link.station >= 0) daily[link.station] = 0.;
     } else {
-      float tf = f0, pf = f1;
-      const float swf = f2, lwf = f3;
-      if (k + 1 < days) {
+      // the next day's forcing is loaded a day ahead (with water use there is no
+      // register to hold it)
+      float tf = kUse ? at(fd, p) : f0, pf = kUse ? at(fd + n, p) : f1;
+      const float swf = kUse ? at(fd + 2 * int64_t(n), p) : f2, lwf = kUse ? at(fd + 3 * int64_t(n), p) : f3;
+      if (kUse) fd += 4 * int64_t(n);
+      if (!kUse && k + 1 < days) {
         fd += 4 * int64_t(n);
-        f0 = fd[0];
-        f1 = fd[n];
-        f2 = fd[2 * int64_t(n)];
-        f3 = fd[3 * int64_t(n)];
+        f0 = at(fd, p);
+        f1 = at(fd + n, p);
+        f2 = at(fd + 2 * int64_t(n), p);
+        f3 = at(fd + 3 * int64_t(n), p);
       }
       if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
-      double use_desired = 0., use_nag = 0.;
-      int64_t use_t = 0;
-      if (kUse) use_t = day_use(S, X, mp, p, fday, di.month, use_desired, use_nag);
       const double laf_prev = (started0 || k > 0) ? s.laf_prev : s.laf;  // daily.cpp:159-169
       DayFlux v;
       {
@@ -218,8 +241,13 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         a.lct = cl.b & 0xff;
         a.elev0 = cl.b >> 8;
         a.arid = (bits & DB_ARID) != 0;
+        s.lai_precsum = fld(DF_LAI_PREC);
+        s.transfer = fld(DF_TRANSFER);
         day_pet_canopy(a, s, v, tf, pf, swf, lwf, laf_prev);
-        day_snow<5>(a, s, v, laf_prev, sp, ep, n);
+        F[DF_LAI_PREC * 64] = s.lai_precsum;
+        if (s.laf <= 0.) day_snow_no_land(s, v, X.snow2, p, n);
+        F[DF_TRANSFER * 64] = s.transfer;
+        if (s.laf > 0.) day_snow<5>(a, s, v, laf_prev, er, X.snow2, S.elev_pairs, p, n);
       }
       ChainRec c;
       {
@@ -233,18 +261,23 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         b.pet_mxdy = fld(DF_PET_MXDY);
         b.t_snowfz = fld(DF_SNOWFZ);
         b.pcritgwa = fld(DF_PCRIT);
-        b.rgmax = fld(DF_RGMAX);
+        b.rgmax = (gf.b >> 16) / 100.;  // G_Rgmax, an int16
         b.recharge_cut = (bits & DB_CUT) != 0;
         b.arid = (bits & DB_ARID) != 0;
         b.ldd = (bits & DB_LDD) ? 0 : -1;
+        s.transfer = fld(DF_TRANSFER);
         day_soil(b, s, v, laf_prev);
+        F[DF_TRANSFER * 64] = s.transfer;
         if (k == days - 1) {
-          X.d_surf[mp] = v.surf_runoff;
-          X.d_recharge[mp] = v.recharge;
-          X.d_ow_pet[mp] = v.ow_pet;
-          X.d_aet[mp] = v.aet;
-          X.d_prec[mp] = v.prec;
+          at(X.d_surf, p) = v.surf_runoff;
+          at(X.d_recharge, p) = v.recharge;
+          at(X.d_ow_pet, p) = v.ow_pet;
+          at(X.d_aet, p) = v.aet;
+          at(X.d_prec, p) = v.prec;
         }
+        double use_desired = 0., use_nag = 0.;
+        int64_t use_t = 0;
+        if (kUse) use_t = day_use(S, X, p, fday, di.month, use_desired, use_nag);
         b.area = fld(DF_AREA);
         b.area_m = fld(DF_AREA_M);
         b.cf100 = fld(DF_CF100);
@@ -262,7 +295,7 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         b.lw100 = fld(DF_LW100);
         b.lw_max = fld(DF_LW_MAX);
         b.glo_wetland = fld(DF_GW);
-        b.gw100 = fld(DF_GW100);
+        b.gw100 = b.glo_wetland / 100.;
         b.gw_max = fld(DF_GW_MAX);
         b.river_length = fld(DF_LENGTH);
         b.bottom = fld(DF_BOTTOM);
@@ -272,9 +305,15 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         b.vel_c2 = fld(DF_VEL_C2);
         // global lakes and reservoirs (one cell in a hundred) read their statics here
         DayStatLake lake{0., 0., 0., 0., 0., 0.};
+        s.glo_lake = s.red_gl = s.res = s.red_res = s.k_release = 0.;
         if ((bits & (DB_LAKE | DB_RES)) || (link.flags & (CFL_LAKE | CFL_RES))) {
           load_stat_lake(S, p, lake);
-          if (kUse) lake.prov_rel = S.use_provrel[use_t];
+          s.glo_lake = fld(DF_GLO_LAKE);
+          s.red_gl = fld(DF_RED_GL);
+          s.res = fld(DF_RES);
+          s.red_res = fld(DF_RED_RES);
+          s.k_release = fld(DF_K_RELEASE);
+          if (kUse) lake.prov_rel = at(S.use_provrel + use_t, p);
         }
         c.inv_ksw = fld(DF_INV_KSW);
         c.ome_sw = fld(DF_OME_SW);
@@ -286,8 +325,8 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         PotTerms pot;
         day_local_routing<kUse>(b, lake, s, v, use_desired, use_nag, c, pot);
         if (X.pot_base) {
-          X.pot_base[mp] = pot.base;
-          X.pot_ow[mp] = pot.ow;
+          at(X.pot_base, p) = pot.base;
+          at(X.pot_ow, p) = pot.ow;
         }
       }
       // transported volumes of upstream cells in earlier wavefronts: wait for the
@@ -299,7 +338,7 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
 #pragma unroll
         for (int u = 0; u < 8; u++)
           if (u < wv.nu && (ext >> u & 1)) {
-            t[u] = __hip_atomic_load(rrow + slot.group + uint16_t(link.up[u]), __ATOMIC_RELAXED,
+            t[u] = __hip_atomic_load(&at(rrow, uint32_t(slot.group) + uint16_t(link.up[u])), __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
             ready = ready && ((t[u] ^ sign) >> 63) == 0;
           }
@@ -319,11 +358,12 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         if (rank == r) {
           // gather in routing order (the serial += of routing.cpp:3955-3958)
           double up = 0.;
+          const WordPair lanes = __builtin_bit_cast(WordPair, fld(DF_NEAR));
 #pragma unroll
           for (int u = 0; u < 8; u++)
             if (u < wv.nu) {
-              const double near =
-                  wg_lds[WG_EXP2_LDS_BYTES / sizeof(double) + DF_TV * 64 + (near_lane(u) & 63)];
+              const int near_lane = int(uint32_t(u < 4 ? lanes.a : lanes.b) >> (8 * (u & 3))) & 63;
+              const double near = wg_lds[WG_EXP2_LDS_BYTES / sizeof(double) + DF_TV * 64 + near_lane];
               const double far = __builtin_bit_cast(double, t[u] & 0x7fffffffffffffffull);
               const double q = (ext >> u & 1) ? far : near;
               up += (u < link.nu) ? q : 0.;
@@ -332,24 +372,24 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
           o = step_fast<kUse>(c, pre, up, slow);
           if (slow) o = chain_step<kUse>(c, up, di);
           const unsigned long long w = __builtin_bit_cast(unsigned long long, o.tv) & 0x7fffffffffffffffull;
-          __hip_atomic_store(rrow + p, w | sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(&at(rrow, p), w | sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           F[DF_TV * 64] = o.tv;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
       }
-      if (c.flags & CFL_LAKE) s.glo_lake = o.glo_lake;
+      if (c.flags & CFL_LAKE) F[DF_GLO_LAKE * 64] = o.glo_lake;
       if (c.flags & CFL_RES) {
-        s.res = o.res;
-        s.k_release = o.k_release;
+        F[DF_RES * 64] = o.res;
+        F[DF_K_RELEASE * 64] = o.k_release;
       }
       if (c.flags & CFL_GWET) s.glo_wetl = o.glo_wetl;
       if (c.flags & CFL_ARID) s.gw = o.gw;
-      if ((c.flags & CFL_ARID) && X.pot_lgw) X.pot_lgw[mp] = o.lgw;
+      if ((c.flags & CFL_ARID) && X.pot_lgw) at(X.pot_lgw, p) = o.lgw;
       s.river = o.river;
       rem = o.rem;
       if (link.station >= 0) daily[link.station] = (c.flags & CFL_LDD) ? o.tv : 0.;
-      if (k == days - 1) X.tv[mp] = o.tv;
-      if (X.pot_acc) add_pot_runoff(S, X, mp, p);
+      if (k == days - 1) at(X.tv, p) = o.tv;
+      if (X.pot_acc) add_pot_runoff(S, X, p);
     }
     {
       DayStatEnd e;
@@ -372,47 +412,59 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
       e.reservoir_area = 0.;
       e.stor_cap = 0.;
       if (bits & (DB_LAKE | DB_RES)) {
-        e.lake_area = S.lake_area[p];
-        e.lake_max = e.lake_area * S.lake_depth[p];
-        e.reservoir_area = S.reservoir_area[p];
-        e.stor_cap = S.stor_cap[p];
+        e.lake_area = at(S.lake_area, p);
+        e.lake_max = e.lake_area * at(S.lake_depth, p);
+        e.reservoir_area = at(S.reservoir_area, p);
+        e.stor_cap = at(S.stor_cap, p);
+        s.glo_lake = fld(DF_GLO_LAKE);
+        s.red_gl = fld(DF_RED_GL);
+        s.res = fld(DF_RES);
+        s.red_res = fld(DF_RED_RES);
       }
       e.contcell = cont;
+      s.red_river = fld(DF_RED_RIVER);
+      s.river_frac_change = fld(DF_FRAC_CHANGE);
       if (kUse && cont) {
         const int fin_ym = int((fday - S.use_day0) / 365) * 12 + di.month;
-        day_end_use(S, X.use + mp, p, s, rem, e.loc_lake, fld(DF_LL_MAX), e.red_exp, fin_ym, doy == 365);
+        day_end_use(S, X.use, p, s, rem, e.loc_lake, fld(DF_LL_MAX), e.red_exp, fin_ym, doy == 365);
       }
       day_end(e, s);
+      F[DF_RED_RIVER * 64] = s.red_river;
+      F[DF_FRAC_CHANGE * 64] = s.river_frac_change;
+      if (bits & (DB_LAKE | DB_RES)) {
+        F[DF_RED_GL * 64] = s.red_gl;
+        F[DF_RED_RES * 64] = s.red_res;
+      }
     }
   }
 
-  X.canopy[mp] = s.canopy;
-  X.soil[mp] = s.soil;
-  X.snow[mp] = s.snow;
-  X.transfer[mp] = s.transfer;
-  X.lai_precsum[mp] = s.lai_precsum;
-  X.lai_days[mp] = s.lai_days;
-  X.lai_status[mp] = s.lai_status;
-  X.snow_any[mp] = s.snow_any ? 1 : 0;
-  X.gw[mp] = s.gw;
-  X.loc_lake[mp] = s.loc_lake;
-  X.loc_wetl[mp] = s.loc_wetl;
-  X.glo_lake[mp] = s.glo_lake;
-  X.glo_wetl[mp] = s.glo_wetl;
-  X.res[mp] = s.res;
-  X.river[mp] = s.river;
-  X.red_ll[mp] = s.red_ll;
-  X.red_lw[mp] = s.red_lw;
-  X.red_gl[mp] = s.red_gl;
-  X.red_gw[mp] = s.red_gw;
-  X.red_res[mp] = s.red_res;
-  X.red_river[mp] = s.red_river;
-  X.river_frac_next[mp] = s.river_frac_next;
-  X.river_frac_change[mp] = s.river_frac_change;
-  X.fswb_next[mp] = s.fswb_next;
-  X.laf[mp] = s.laf;
-  X.laf_prev[mp] = s.laf_prev;
-  X.k_release[mp] = s.k_release;
+  at(X.canopy, p) = s.canopy;
+  at(X.soil, p) = s.soil;
+  at(X.snow, p) = s.snow;
+  at(X.transfer, p) = fld(DF_TRANSFER);
+  at(X.lai_precsum, p) = fld(DF_LAI_PREC);
+  at(X.lai_days, p) = s.lai_days;
+  at(X.lai_status, p) = s.lai_status;
+  at(X.snow_any, p) = s.snow_any ? 1 : 0;
+  at(X.gw, p) = s.gw;
+  at(X.loc_lake, p) = s.loc_lake;
+  at(X.loc_wetl, p) = s.loc_wetl;
+  at(X.glo_lake, p) = fld(DF_GLO_LAKE);
+  at(X.glo_wetl, p) = s.glo_wetl;
+  at(X.res, p) = fld(DF_RES);
+  at(X.river, p) = s.river;
+  at(X.red_ll, p) = s.red_ll;
+  at(X.red_lw, p) = s.red_lw;
+  at(X.red_gl, p) = fld(DF_RED_GL);
+  at(X.red_gw, p) = s.red_gw;
+  at(X.red_res, p) = fld(DF_RED_RES);
+  at(X.red_river, p) = fld(DF_RED_RIVER);
+  at(X.river_frac_next, p) = s.river_frac_next;
+  at(X.river_frac_change, p) = fld(DF_FRAC_CHANGE);
+  at(X.fswb_next, p) = s.fswb_next;
+  at(X.laf, p) = s.laf;
+  at(X.laf_prev, p) = s.laf_prev;
+  at(X.k_release, p) = fld(DF_K_RELEASE);
 }
 
 #endif  // WG_DAYS_KERNEL_H

@@ -91,6 +91,7 @@ struct WgStatic {
   const float *built_up, *gw_factor, *lai_max;
   const int16_t *elev0;         // [N] mean cell elevation (channel 0 of G_Elevation)
   const int32_t *elev_pairs;    // [50][N] sub-cell elevations 2k+1 (low half) and 2k+2 (high half)
+  const int32_t *elev_range;    // [N] lowest (low half) and highest (high half) sub-cell elevation
   // calibration parameters used by the day loop
   const double *alpha, *pet_mxdy, *m_prec, *m_netrad, *mcwh, *t_snowfz, *t_snowmt, *t_gradnt,
       *degday, *pcritgwa, *evarexp, *m_rivrgh;

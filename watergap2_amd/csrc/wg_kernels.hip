@@ -22,6 +22,8 @@
 // pow are the deterministic ones of wg_libm.h, shared with the CPU oracle.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "wg_device.h"
 // The exp/log/pow table lives in LDS, one copy per wavefront at the front of the
 // workgroup's dynamic LDS (WG_EXP2_LDS_BYTES per wavefront): a lane-varying index
@@ -80,9 +82,20 @@ __device__ inline void normal_pair(uint64_t seed, uint32_t cell, uint32_t day, d
   z1 = r * sn;
 }
 
+// Element i of a row that is the same for the whole wavefront: a scalar base and a
+// 32-bit byte offset (rows hold fewer than 2^27 elements of up to 16 bytes).  The
+// empty asm keeps the offset a 32-bit value of the block that uses it; otherwise the
+// compiler forms every row's 64-bit address ahead of the day loop and spills them.
+template <class T>
+__device__ __forceinline__ T &at(T *row, uint32_t i) {
+  uint32_t o = i * uint32_t(sizeof(T));
+  asm volatile("" : "+v"(o));
+  return *reinterpret_cast<T *>(reinterpret_cast<char *>(const_cast<std::remove_const_t<T> *>(row)) + o);
+}
+
 // Device accessors of the routing links and chain constants ([k][N] x 16 bytes).
-__device__ inline WgChainLink load_link(const WgStatic &S, int p) {
-  const WgI4 a = S.clink[p], b = S.clink[int64_t(S.n) + p];
+__device__ inline WgChainLink load_link(const WgStatic &S, uint32_t p) {
+  const WgI4 a = at(S.clink, p), b = at(S.clink + S.n, p);
   WgChainLink lk;
   lk.flags = a.x;
   lk.station = a.y;
@@ -98,30 +111,50 @@ __device__ inline WgChainLink load_link(const WgStatic &S, int p) {
   return lk;
 }
 
-__device__ inline WgChainStatic load_cstat(const WgStatic &S, int p) {
+__device__ inline WgChainStatic load_cstat(const WgStatic &S, uint32_t p) {
   const int64_t n = S.n;
-  const WgD2 a = S.cstat[p], b = S.cstat[n + p], c = S.cstat[2 * n + p];
+  const WgD2 a = at(S.cstat, p), b = at(S.cstat + n, p), c = at(S.cstat + 2 * n, p);
   return WgChainStatic{a.x, a.y, b.x, b.y, c.x, c.y};
 }
 
-// Pair 0 of the routing record of (member m, cell p); pair k is at [k * N].
-__device__ inline WgD2 *rec_at(const WgState &X, int n, int m, int p) {
-  return X.crec + int64_t(m) * (WG_DEV_NREC / 2) * n + p;
+// Moves a state's pointers to the rows of member m.
+__device__ __forceinline__ void member_rows(WgState &X, int m, int n) {
+  const int64_t o = int64_t(m) * n;
+  double **rows[] = {&X.canopy, &X.soil, &X.snow, &X.transfer, &X.lai_precsum, &X.gw, &X.loc_lake, &X.loc_wetl,
+                     &X.glo_lake, &X.glo_wetl, &X.res, &X.river, &X.red_ll, &X.red_lw, &X.red_gl, &X.red_gw,
+                     &X.red_res, &X.red_river, &X.river_frac_next, &X.river_frac_change, &X.fswb_next, &X.laf,
+                     &X.laf_prev, &X.k_release, &X.gamma, &X.cfa, &X.tv, &X.d_surf, &X.d_recharge, &X.d_ow_pet,
+                     &X.d_aet, &X.d_prec};
+#pragma unroll
+  for (size_t k = 0; k < sizeof(rows) / sizeof(rows[0]); k++) *rows[k] += o;
+  X.lai_days += o;
+  X.lai_status += o;
+  X.snow_any += o;
+  X.smax += o;
+  X.snow2 += o * WG_DEV_NPAIR;
+  X.crec += o * (WG_DEV_NREC / 2);
+  // optional arrays stay NULL when off
+  if (X.pot_acc) X.pot_acc += o;
+  if (X.pot_base) X.pot_base += o;
+  if (X.pot_ow) X.pot_ow += o;
+  if (X.pot_lgw) X.pot_lgw += o;
+  if (X.use) X.use += o;
+  if (X.use_rem) X.use_rem += o;
 }
 
-// Writes what chain_step changed.
-__device__ inline void store_chain(const WgState &X, int64_t mp, int flags, const ChainOut &o) {
-  if (flags & CFL_LAKE) X.glo_lake[mp] = o.glo_lake;
+// Writes what chain_step changed; X holds the member's rows.
+__device__ inline void store_chain(const WgState &X, uint32_t p, int flags, const ChainOut &o) {
+  if (flags & CFL_LAKE) at(X.glo_lake, p) = o.glo_lake;
   if (flags & CFL_RES) {
-    X.res[mp] = o.res;
-    X.k_release[mp] = o.k_release;
+    at(X.res, p) = o.res;
+    at(X.k_release, p) = o.k_release;
   }
-  if (flags & CFL_GWET) X.glo_wetl[mp] = o.glo_wetl;
-  if (flags & CFL_ARID) X.gw[mp] = o.gw;
-  if ((flags & CFL_ARID) && X.pot_lgw) X.pot_lgw[mp] = o.lgw;
-  X.river[mp] = o.river;
-  X.tv[mp] = o.tv;
-  if (X.use_rem) X.use_rem[mp] = o.rem;
+  if (flags & CFL_GWET) at(X.glo_wetl, p) = o.glo_wetl;
+  if (flags & CFL_ARID) at(X.gw, p) = o.gw;
+  if ((flags & CFL_ARID) && X.pot_lgw) at(X.pot_lgw, p) = o.lgw;
+  at(X.river, p) = o.river;
+  at(X.tv, p) = o.tv;
+  if (X.use_rem) at(X.use_rem, p) = o.rem;
 }
 
 #include "wg_cell_day.h"
@@ -135,18 +168,18 @@ namespace {
 // that they are in flight together (after a store the compiler must keep later
 // loads behind it).  Every array covers all cells, so the loads of fields a cell
 // does not use are in bounds.
-__device__ __forceinline__ void load_stat_a(const WgStatic &S, const WgTables &T, int p, DayStatA &a) {
-  const int l = S.land_cover[p] - 1;
-  const float lmax_f = S.lai_max[p];
-  a.m_prec = S.m_prec[p];
-  a.alpha = S.alpha[p];
-  a.pet_mxdy = S.pet_mxdy[p];
-  a.m_netrad = S.m_netrad[p];
-  a.mcwh = S.mcwh[p];
-  a.t_snowfz = S.t_snowfz[p];
-  a.t_snowmt = S.t_snowmt[p];
-  a.t_gradnt = S.t_gradnt[p];
-  a.melt_factor = S.degday[p] * T.ddf[l];
+__device__ __forceinline__ void load_stat_a(const WgStatic &S, const WgTables &T, uint32_t p, DayStatA &a) {
+  const int l = at(S.land_cover, p) - 1;
+  const float lmax_f = at(S.lai_max, p);
+  a.m_prec = at(S.m_prec, p);
+  a.alpha = at(S.alpha, p);
+  a.pet_mxdy = at(S.pet_mxdy, p);
+  a.m_netrad = at(S.m_netrad, p);
+  a.mcwh = at(S.mcwh, p);
+  a.t_snowfz = at(S.t_snowfz, p);
+  a.t_snowmt = at(S.t_snowmt, p);
+  a.t_gradnt = at(S.t_gradnt, p);
+  a.melt_factor = at(S.degday, p) * T.ddf[l];
   a.albedo = T.albedo[l];
   a.albedo_snow = T.albedo_snow[l];
   a.emis = T.emissivity[l] * 0.000000004903;
@@ -154,148 +187,153 @@ __device__ __forceinline__ void load_stat_a(const WgStatic &S, const WgTables &T
   a.lmax = lmax_f;
   a.initial_days = T.initial_days[l];
   a.lct = l + 1;
-  a.elev0 = S.elev0[p];
-  a.arid = S.aindex[p] == 1;
+  a.elev0 = at(S.elev0, p);
+  a.arid = at(S.aindex, p) == 1;
 }
 
-__device__ __forceinline__ void load_stat_b(const WgStatic &S, const WgState &X, int64_t mp, int p, DayStatB &b) {
-  b.built_up = S.built_up[p];
-  b.smax = X.smax[mp];
-  b.gw_factor = S.gw_factor[p];
-  b.gamma = X.gamma[mp];
-  b.cfa = X.cfa[mp];
-  b.pet_mxdy = S.pet_mxdy[p];
-  b.t_snowfz = S.t_snowfz[p];
-  b.pcritgwa = S.pcritgwa[p];
-  const int16_t rgmax = S.rgmax[p];
+__device__ __forceinline__ void load_stat_b(const WgStatic &S, const WgState &X, uint32_t p, DayStatB &b) {
+  b.built_up = at(S.built_up, p);
+  b.smax = at(X.smax, p);
+  b.gw_factor = at(S.gw_factor, p);
+  b.gamma = at(X.gamma, p);
+  b.cfa = at(X.cfa, p);
+  b.pet_mxdy = at(S.pet_mxdy, p);
+  b.t_snowfz = at(S.t_snowfz, p);
+  b.pcritgwa = at(S.pcritgwa, p);
+  const int16_t rgmax = at(S.rgmax, p);
   b.rgmax = rgmax / 100.;
-  b.arid = S.aindex[p] == 1;
-  b.ldd = S.ldd[p];
-  b.recharge_cut = (b.arid && (S.texture[p] < 21)) && (b.ldd >= 0);
-  b.area = S.cell_area[p];
+  b.arid = at(S.aindex, p) == 1;
+  b.ldd = at(S.ldd, p);
+  b.recharge_cut = (b.arid && (at(S.texture, p) < 21)) && (b.ldd >= 0);
+  b.area = at(S.cell_area, p);
   b.area_m = b.area / 1000000.;
-  b.cf100 = S.contfreq[p] / 100.;
-  double f = S.fswb_init[p] * 20.;
+  b.cf100 = at(S.contfreq, p) / 100.;
+  double f = at(S.fswb_init, p) * 20.;
   if (f > 1.) f = 1.;
   b.fswb_catchment = f;
-  b.e_gw = S.e_gw[p];
-  b.inv_kgw = S.inv_kgw[p];
-  b.ome_gw = S.ome_gw[p];
-  b.e_sw = S.e_sw[p];
-  b.k_sw = S.k_sw[p];
-  b.red_exp = S.evarexp[p] * kEvapoRedExp;
-  const double lake_depth = S.lake_depth[p], wetl_depth = S.wetl_depth[p];
-  b.loc_lake = S.loc_lake[p];
+  b.e_gw = at(S.e_gw, p);
+  b.inv_kgw = at(S.inv_kgw, p);
+  b.ome_gw = at(S.ome_gw, p);
+  b.e_sw = at(S.e_sw, p);
+  b.k_sw = at(S.k_sw, p);
+  b.red_exp = at(S.evarexp, p) * kEvapoRedExp;
+  const double lake_depth = at(S.lake_depth, p), wetl_depth = at(S.wetl_depth, p);
+  b.loc_lake = at(S.loc_lake, p);
   b.ll100 = b.loc_lake / 100.;
   b.ll_max = b.ll100 * b.area * lake_depth;
-  b.loc_wetland = S.loc_wetland[p];
+  b.loc_wetland = at(S.loc_wetland, p);
   b.lw100 = b.loc_wetland / 100.;
   b.lw_max = b.lw100 * b.area * wetl_depth;
-  b.glo_wetland = S.glo_wetland[p];
+  b.glo_wetland = at(S.glo_wetland, p);
   b.gw100 = b.glo_wetland / 100.;
   b.gw_max = b.gw100 * b.area * wetl_depth;
-  b.river_length = S.river_length[p];
-  b.bottom = S.bottom_width[p];
+  b.river_length = at(S.river_length, p);
+  b.bottom = at(S.bottom_width, p);
   b.vel_b4 = -b.bottom / 4.0;
   b.vel_b16 = b.bottom * b.bottom / 16.0;
-  b.vel_c1 = S.vel_c1[p];
-  b.vel_c2 = S.vel_c2[p];
+  b.vel_c1 = at(S.vel_c1, p);
+  b.vel_c2 = at(S.vel_c2, p);
 }
 
-__device__ __forceinline__ void load_stat_lake(const WgStatic &S, int p, DayStatLake &k) {
-  k.lake_area = S.lake_area[p];
-  k.lake_depth = S.lake_depth[p];
-  k.reservoir_area = S.reservoir_area[p];
-  k.stor_cap = S.stor_cap[p];
-  k.mean_outflow = S.mean_outflow[p];
-  k.prov_rel = S.res_prov_rel[p];
+__device__ __forceinline__ void load_stat_lake(const WgStatic &S, uint32_t p, DayStatLake &k) {
+  k.lake_area = at(S.lake_area, p);
+  k.lake_depth = at(S.lake_depth, p);
+  k.reservoir_area = at(S.reservoir_area, p);
+  k.stor_cap = at(S.stor_cap, p);
+  k.mean_outflow = at(S.mean_outflow, p);
+  k.prov_rel = at(S.res_prov_rel, p);
 }
 
-__device__ __forceinline__ void load_stat_end(const WgStatic &S, int p, DayStatEnd &e) {
-  e.red_exp = S.evarexp[p] * kEvapoRedExp;
-  e.area = S.cell_area[p];
-  e.river_length = S.river_length[p];
-  e.rw_c0 = S.rw_c0[p];
-  e.rw_c1 = S.rw_c1[p];
-  e.rw_c2 = S.rw_c2[p];
-  e.rw_c3 = S.rw_c3[p];
-  e.river_stor_max = S.river_stor_max[p];
-  e.f_glo_lake = S.f_glo_lake[p];
-  e.max_raf = S.contfreq[p] / 100. - e.f_glo_lake;
-  e.loc_lake = S.loc_lake[p];
-  e.loc_wetland = S.loc_wetland[p];
-  e.glo_wetland = S.glo_wetland[p];
-  e.gw_max = e.glo_wetland / 100. * e.area * S.wetl_depth[p];
-  e.lake_area = S.lake_area[p];
-  e.lake_max = e.lake_area * S.lake_depth[p];
-  e.reservoir_area = S.reservoir_area[p];
-  e.stor_cap = S.stor_cap[p];
-  e.contcell = S.contcell[p] != 0;
+__device__ __forceinline__ void load_stat_end(const WgStatic &S, uint32_t p, DayStatEnd &e) {
+  e.red_exp = at(S.evarexp, p) * kEvapoRedExp;
+  e.area = at(S.cell_area, p);
+  e.river_length = at(S.river_length, p);
+  e.rw_c0 = at(S.rw_c0, p);
+  e.rw_c1 = at(S.rw_c1, p);
+  e.rw_c2 = at(S.rw_c2, p);
+  e.rw_c3 = at(S.rw_c3, p);
+  e.river_stor_max = at(S.river_stor_max, p);
+  e.f_glo_lake = at(S.f_glo_lake, p);
+  e.max_raf = at(S.contfreq, p) / 100. - e.f_glo_lake;
+  e.loc_lake = at(S.loc_lake, p);
+  e.loc_wetland = at(S.loc_wetland, p);
+  e.glo_wetland = at(S.glo_wetland, p);
+  e.gw_max = e.glo_wetland / 100. * e.area * at(S.wetl_depth, p);
+  e.lake_area = at(S.lake_area, p);
+  e.lake_max = e.lake_area * at(S.lake_depth, p);
+  e.reservoir_area = at(S.reservoir_area, p);
+  e.stor_cap = at(S.stor_cap, p);
+  e.contcell = at(S.contcell, p) != 0;
+}
+
+__device__ __forceinline__ ElevRange load_elev_range(const WgStatic &S, uint32_t p) {
+  const int32_t r = at(S.elev_range, p), e = at(S.elev_pairs, p);
+  return ElevRange{int16_t(r & 0xffff), int16_t(r >> 16), int16_t(e & 0xffff)};
 }
 
 // State read by PET, LAI, canopy and snow.
-__device__ __forceinline__ void load_state_a(const WgState &X, int64_t mp, CellState &s) {
-  s.canopy = X.canopy[mp];
-  s.lai_days = X.lai_days[mp];
-  s.lai_precsum = X.lai_precsum[mp];
-  s.lai_status = X.lai_status[mp];
-  s.snow = X.snow[mp];
-  s.snow_any = X.snow_any[mp] != 0;
-  s.transfer = X.transfer[mp];
+__device__ __forceinline__ void load_state_a(const WgState &X, uint32_t p, CellState &s) {
+  s.canopy = at(X.canopy, p);
+  s.lai_days = at(X.lai_days, p);
+  s.lai_precsum = at(X.lai_precsum, p);
+  s.lai_status = at(X.lai_status, p);
+  s.snow = at(X.snow, p);
+  s.snow_any = at(X.snow_any, p) != 0;
+  s.transfer = at(X.transfer, p);
 }
 
 // State read by soil and local routing.
-__device__ __forceinline__ void load_state_b(const WgState &X, int64_t mp, CellState &s) {
-  s.soil = X.soil[mp];
-  s.gw = X.gw[mp];
-  s.loc_lake = X.loc_lake[mp];
-  s.loc_wetl = X.loc_wetl[mp];
-  s.glo_lake = X.glo_lake[mp];
-  s.glo_wetl = X.glo_wetl[mp];
-  s.res = X.res[mp];
-  s.river = X.river[mp];
-  s.k_release = X.k_release[mp];
+__device__ __forceinline__ void load_state_b(const WgState &X, uint32_t p, CellState &s) {
+  s.soil = at(X.soil, p);
+  s.gw = at(X.gw, p);
+  s.loc_lake = at(X.loc_lake, p);
+  s.loc_wetl = at(X.loc_wetl, p);
+  s.glo_lake = at(X.glo_lake, p);
+  s.glo_wetl = at(X.glo_wetl, p);
+  s.res = at(X.res, p);
+  s.river = at(X.river, p);
+  s.k_release = at(X.k_release, p);
 }
 
 // State read by the day's end (with loc_lake for the water use).
-__device__ __forceinline__ void load_state_end(const WgState &X, int64_t mp, CellState &s) {
-  s.glo_lake = X.glo_lake[mp];
-  s.glo_wetl = X.glo_wetl[mp];
-  s.res = X.res[mp];
-  s.river = X.river[mp];
-  s.red_ll = X.red_ll[mp];
-  s.red_lw = X.red_lw[mp];
+__device__ __forceinline__ void load_state_end(const WgState &X, uint32_t p, CellState &s) {
+  s.glo_lake = at(X.glo_lake, p);
+  s.glo_wetl = at(X.glo_wetl, p);
+  s.res = at(X.res, p);
+  s.river = at(X.river, p);
+  s.red_ll = at(X.red_ll, p);
+  s.red_lw = at(X.red_lw, p);
   s.red_gl = 0.;
-  s.red_gw = X.red_gw[mp];
+  s.red_gw = at(X.red_gw, p);
   s.red_res = 0.;
-  s.red_river = X.red_river[mp];
-  s.river_frac_next = X.river_frac_next[mp];
-  s.river_frac_change = X.river_frac_change[mp];
-  s.fswb_next = X.fswb_next[mp];
-  s.laf = X.laf[mp];
+  s.red_river = at(X.red_river, p);
+  s.river_frac_next = at(X.river_frac_next, p);
+  s.river_frac_change = at(X.river_frac_change, p);
+  s.fswb_next = at(X.fswb_next, p);
+  s.laf = at(X.laf, p);
 }
 
 // Writes what the day's end changed.
-__device__ __forceinline__ void store_state_end(const WgState &X, int64_t mp, const DayStatEnd &e,
+__device__ __forceinline__ void store_state_end(const WgState &X, uint32_t p, const DayStatEnd &e,
                                                 const CellState &s) {
-  if (e.lake_area > 0.) X.red_gl[mp] = s.red_gl;
-  if (e.reservoir_area > 0.) X.red_res[mp] = s.red_res;
-  X.laf_prev[mp] = s.laf_prev;
-  X.laf[mp] = s.laf;
-  X.fswb_next[mp] = s.fswb_next;
-  X.red_ll[mp] = s.red_ll;
-  X.red_lw[mp] = s.red_lw;
-  X.red_gw[mp] = s.red_gw;
-  X.red_river[mp] = s.red_river;
-  X.river_frac_next[mp] = s.river_frac_next;
-  X.river_frac_change[mp] = s.river_frac_change;
+  if (e.lake_area > 0.) at(X.red_gl, p) = s.red_gl;
+  if (e.reservoir_area > 0.) at(X.red_res, p) = s.red_res;
+  at(X.laf_prev, p) = s.laf_prev;
+  at(X.laf, p) = s.laf;
+  at(X.fswb_next, p) = s.fswb_next;
+  at(X.red_ll, p) = s.red_ll;
+  at(X.red_lw, p) = s.red_lw;
+  at(X.red_gw, p) = s.red_gw;
+  at(X.red_river, p) = s.red_river;
+  at(X.river_frac_next, p) = s.river_frac_next;
+  at(X.river_frac_change, p) = s.river_frac_change;
 }
 
 // The day's perturbed temperature and precipitation of one (member, cell).
-__device__ __forceinline__ void perturb_forcing(const WgStatic &S, const WgState &X, int m, int p, int64_t fday,
+__device__ __forceinline__ void perturb_forcing(const WgStatic &S, const WgState &X, int m, uint32_t p, int64_t fday,
                                                 float &tf, float &pf) {
   const uint64_t seed = X.member_seed[m];
-  const uint32_t ref = uint32_t(S.ref_index[p]);
+  const uint32_t ref = uint32_t(at(S.ref_index, p));
   double zp, zt;
   normal_pair(seed, ref, uint32_t(fday), zp, zt);
   pf = float(double(pf) * wg_exp(X.prec_sigma * zp));
@@ -307,16 +345,16 @@ __device__ __forceinline__ void perturb_forcing(const WgStatic &S, const WgState
 // updateNetAbstractionGW in every groundwater branch when the last day left a
 // remaining use; the adaptation reads only the last day's state, so it is done
 // here for (semi-)arid cells too, whose groundwater step the chain runs).
-// Returns the index of the day's tables.
-__device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, int64_t mp, int p, int64_t fday,
+// Returns the offset of the day's rows in the tables.
+__device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, uint32_t p, int64_t fday,
                                            int month, double &desired, double &nag) {
-  const int64_t t = (int64_t((fday - S.use_day0) / 365) * 12 + month) * S.n + p;
+  const int64_t t = (int64_t((fday - S.use_day0) / 365) * 12 + month) * S.n;
   const int64_t us = S.use_stride;
-  double *U = X.use + mp;
-  nag = S.use_nug[t];
-  if (U[WG_USE_DAILY_REMAINING * us] != 0.) nag = update_net_abstraction_gw(U, us, S.use_frgi[p], nag);
-  desired = S.use_nus[t];
-  if (S.use_delayed == 1) desired += U[WG_USE_TOTAL_UNSAT * us];
+  double *U = X.use;
+  nag = at(S.use_nug + t, p);
+  if (at(U + WG_USE_DAILY_REMAINING * us, p) != 0.) nag = update_net_abstraction_gw(U, us, p, at(S.use_frgi, p), nag);
+  desired = at(S.use_nus + t, p);
+  if (S.use_delayed == 1) desired += at(U + WG_USE_TOTAL_UNSAT * us, p);
   return t;
 }
 
@@ -324,14 +362,14 @@ __device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, 
 // G_potCellRunoff[n] += potCellRunoff (routing.cpp:1970, 2053, 2187, 3379): the
 // local runoff terms, then the arid groundwater step's runoff where that step ran,
 // then the open-water balance, in the reference's order of addition.
-__device__ __forceinline__ void add_pot_runoff(const WgStatic &S, const WgState &X, int64_t mp, int p) {
-  const double base = X.pot_base[mp];
-  const double lake_balance = X.pot_ow[mp] * X.cfa[mp];  // (dailyPrec - dailyOpenWaterPET) * CFA
+__device__ __forceinline__ void add_pot_runoff(const WgStatic &S, const WgState &X, uint32_t p) {
+  const double base = at(X.pot_base, p);
+  const double lake_balance = at(X.pot_ow, p) * at(X.cfa, p);  // (dailyPrec - dailyOpenWaterPET) * CFA
   const double ow = (lake_balance / 1000000.0) *
-                    ((S.lake_area[p] + S.reservoir_area[p]) +
-                     ((S.cell_area[p] / 100.0) * ((S.loc_lake[p] + S.loc_wetland[p]) + S.glo_wetland[p])));
-  const double pot = (S.cflags[p] & CFL_ARID) ? (base + X.pot_lgw[mp]) + ow : base + ow;
-  X.pot_acc[mp] += pot;
+                    ((at(S.lake_area, p) + at(S.reservoir_area, p)) +
+                     ((at(S.cell_area, p) / 100.0) * ((at(S.loc_lake, p) + at(S.loc_wetland, p)) + at(S.glo_wetland, p))));
+  const double pot = (at(S.cflags, p) & CFL_ARID) ? (base + at(X.pot_lgw, p)) + ow : base + ow;
+  at(X.pot_acc, p) += pot;
 }
 
 }  // namespace
@@ -358,50 +396,52 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   load_exp2_table();
   const int t0 = S.tile_start[blockIdx.x];
   if (t0 < 0) return;
-  const int p = t0 + int(threadIdx.x);
-  if (p >= S.tile_end[blockIdx.x]) return;
+  const uint32_t p = uint32_t(t0) + threadIdx.x;
+  if (int(p) >= S.tile_end[blockIdx.x]) return;
   const int m = blockIdx.y;
   const int n = S.n;
-  const int64_t mp = int64_t(m) * n + p;
+  member_rows(X, m, n);
 
   DayStatA sa;
   CellState s;
+  ElevRange er{0, 0, 0};
   if (do_vertical) {
+    er = load_elev_range(S, p);
     load_stat_a(S, T, p, sa);
-    load_state_a(X, mp, s);
+    load_state_a(X, p, s);
   }
   if (do_post) {
     DayStatEnd e;
     load_stat_end(S, p, e);
-    load_state_end(X, mp, s);
+    load_state_end(X, p, s);
     if (kUse && e.contcell) {
       // the finished day is day k - 1 of the block (the closing pass runs with k = days)
       const int64_t fin = clock->day0 + k - 1;
       const int fin_doy = int((clock->doy0 - 1 + k - 1) % 365) + 1;
       const int fin_ym = int((fin - S.use_day0) / 365) * 12 + day_info(fin_doy).month;
-      s.loc_lake = X.loc_lake[mp];
-      day_end_use(S, X.use + mp, p, s, X.use_rem[mp], e.loc_lake,
-                  e.loc_lake / 100. * e.area * S.lake_depth[p], e.red_exp, fin_ym, fin_doy == 365);
-      X.loc_lake[mp] = s.loc_lake;
-      X.use_rem[mp] = 0.;
+      s.loc_lake = at(X.loc_lake, p);
+      day_end_use(S, X.use, p, s, at(X.use_rem, p), e.loc_lake,
+                  e.loc_lake / 100. * e.area * at(S.lake_depth, p), e.red_exp, fin_ym, fin_doy == 365);
+      at(X.loc_lake, p) = s.loc_lake;
+      at(X.use_rem, p) = 0.;
     }
     day_end(e, s);
-    store_state_end(X, mp, e, s);
+    store_state_end(X, p, e, s);
   } else if (do_vertical) {
-    s.laf = X.laf[mp];
-    s.laf_prev = X.laf_prev[mp];
-    s.red_ll = X.red_ll[mp];
-    s.red_lw = X.red_lw[mp];
-    s.red_gw = X.red_gw[mp];
-    s.red_gl = X.red_gl[mp];
-    s.red_res = X.red_res[mp];
-    s.river_frac_next = X.river_frac_next[mp];
+    s.laf = at(X.laf, p);
+    s.laf_prev = at(X.laf_prev, p);
+    s.red_ll = at(X.red_ll, p);
+    s.red_lw = at(X.red_lw, p);
+    s.red_gw = at(X.red_gw, p);
+    s.red_gl = at(X.red_gl, p);
+    s.red_res = at(X.red_res, p);
+    s.river_frac_next = at(X.river_frac_next, p);
   }
   // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
   // routing.cpp:1876); other cells keep a zero transported volume.
   if (!do_vertical) return;
-  if (!S.contcell[p]) {
-    const int st = S.station[p];
+  if (!at(S.contcell, p)) {
+    const int st = at(S.station, p);
     if (st >= 0) X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + st] = 0.;
     return;
   }
@@ -411,40 +451,43 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   const bool started = (clock->started != 0) || (k > 0) || (do_post != 0);
   if (fday < 0 || fday >= n_forcing_days) return;
   const float *f = forcing + fday * 4 * int64_t(n);
-  float tf = f[p], pf = f[n + p];
-  const float swf = f[2 * n + p], lwf = f[3 * n + p];
+  float tf = at(f, p), pf = at(f + n, p);
+  const float swf = at(f + 2 * int64_t(n), p), lwf = at(f + 3 * int64_t(n), p);
   if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
   double use_desired = 0., use_nag = 0.;
   int64_t use_t = 0;
-  if (kUse) use_t = day_use(S, X, mp, p, fday, day_info(doy).month, use_desired, use_nag);
+  if (kUse) use_t = day_use(S, X, p, fday, day_info(doy).month, use_desired, use_nag);
 
   const double laf_prev = started ? s.laf_prev : s.laf;  // daily.cpp:159-169
   DayFlux v;
   day_pet_canopy(sa, s, v, tf, pf, swf, lwf, laf_prev);
-  X.lai_days[mp] = s.lai_days;
-  X.lai_status[mp] = s.lai_status;
-  X.lai_precsum[mp] = s.lai_precsum;
-  X.canopy[mp] = s.canopy;
-  day_snow<kSnowChunk>(sa, s, v, laf_prev, X.snow2 + int64_t(m) * WG_DEV_NPAIR * n + p, S.elev_pairs + p, n);
-  X.snow_any[mp] = s.snow_any ? 1 : 0;
+  at(X.lai_days, p) = s.lai_days;
+  at(X.lai_status, p) = s.lai_status;
+  at(X.lai_precsum, p) = s.lai_precsum;
+  at(X.canopy, p) = s.canopy;
+  if (s.laf <= 0.)
+    day_snow_no_land(s, v, X.snow2, p, n);
+  else
+    day_snow<kSnowChunk>(sa, s, v, laf_prev, er, X.snow2, S.elev_pairs, p, n);
+  at(X.snow_any, p) = s.snow_any ? 1 : 0;
   DayStatB sb;
   DayStatLake lake;
-  load_stat_b(S, X, mp, p, sb);
+  load_stat_b(S, X, p, sb);
   load_stat_lake(S, p, lake);
-  load_state_b(X, mp, s);
+  load_state_b(X, p, s);
   const WgChainLink lk = load_link(S, p);
   const WgChainStatic cs = load_cstat(S, p);
-  if (kUse) lake.prov_rel = S.use_provrel[use_t];
-  X.snow[mp] = s.snow;
+  if (kUse) lake.prov_rel = at(S.use_provrel + use_t, p);
+  at(X.snow, p) = s.snow;
   day_soil(sb, s, v, laf_prev);
-  X.soil[mp] = s.soil;
-  X.transfer[mp] = s.transfer;
+  at(X.soil, p) = s.soil;
+  at(X.transfer, p) = s.transfer;
   if (write_diag) {
-    X.d_surf[mp] = v.surf_runoff;
-    X.d_recharge[mp] = v.recharge;
-    X.d_ow_pet[mp] = v.ow_pet;
-    X.d_aet[mp] = v.aet;
-    X.d_prec[mp] = v.prec;
+    at(X.d_surf, p) = v.surf_runoff;
+    at(X.d_recharge, p) = v.recharge;
+    at(X.d_ow_pet, p) = v.ow_pet;
+    at(X.d_aet, p) = v.aet;
+    at(X.d_prec, p) = v.prec;
   }
   ChainRec c;
   double *w = c.v;
@@ -457,37 +500,36 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   c.flags = lk.flags;
   PotTerms pot;
   day_local_routing<kUse>(sb, lake, s, v, use_desired, use_nag, c, pot);
-  if (!(sb.arid && (sb.ldd >= 0))) X.gw[mp] = s.gw;
+  if (!(sb.arid && (sb.ldd >= 0))) at(X.gw, p) = s.gw;
   if (X.pot_base) {
-    X.pot_base[mp] = pot.base;  // wg_pot_runoff_kernel completes the terms
-    X.pot_ow[mp] = pot.ow;
+    at(X.pot_base, p) = pot.base;  // wg_pot_runoff_kernel completes the terms
+    at(X.pot_ow, p) = pot.ow;
   }
   if (sb.loc_lake > 0.) {
-    X.loc_lake[mp] = s.loc_lake;
-    X.red_ll[mp] = s.red_ll;
+    at(X.loc_lake, p) = s.loc_lake;
+    at(X.red_ll, p) = s.red_ll;
   }
   if (sb.loc_wetland > 0.) {
-    X.loc_wetl[mp] = s.loc_wetl;
-    X.red_lw[mp] = s.red_lw;
+    at(X.loc_wetl, p) = s.loc_wetl;
+    at(X.red_lw, p) = s.red_lw;
   }
   if (lk.nu == 0) {
     // no upstream cell: G_riverInflow[n] is still 0 when the cell is routed
     const ChainOut o = chain_step<kUse>(c, 0.0, day_info(doy));
-    store_chain(X, mp, c.flags, o);
+    store_chain(X, p, c.flags, o);
     if (lk.station >= 0)
       X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + lk.station] = (sb.ldd >= 0) ? o.tv : 0.;
   } else {
     // the pairs holding the prefix for every routed cell (the last of them also
     // holds the first suffix field), the rest for cells with a lake or reservoir
-    WgD2 *dst = rec_at(X, n, m, p);
     constexpr int kPrefixPairs = (CF_PREFIX + 1) / 2;
 #pragma unroll
-    for (int k = 0; k < kPrefixPairs; k++) dst[int64_t(k) * n] = WgD2{w[2 * k], w[2 * k + 1]};
+    for (int k = 0; k < kPrefixPairs; k++) at(X.crec + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
     if (lk.flags & (CFL_LAKE | CFL_RES)) {
 #pragma unroll
-      for (int k = kPrefixPairs; k < CF_USE / 2; k++) dst[int64_t(k) * n] = WgD2{w[2 * k], w[2 * k + 1]};
+      for (int k = kPrefixPairs; k < CF_USE / 2; k++) at(X.crec + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
     }
-    if (kUse) dst[int64_t(CF_USE / 2) * n] = WgD2{w[CF_USE], w[CF_A_NUG]};
+    if (kUse) at(X.crec + int64_t(CF_USE / 2) * n, p) = WgD2{w[CF_USE], w[CF_A_NUG]};
   }
 }
 
@@ -1059,6 +1101,8 @@ __global__ __launch_bounds__(256) void wg_chain_flow_kernel(WgStatic S, WgState 
   const int depth = l1 - l0;
   const int gs = group_level_off[l0], ge = group_level_off[l1];
   const int lvl0_end = group_level_off[l0 + 1];
+  WgState Xm = X;
+  member_rows(Xm, m, n);
   const int64_t base = int64_t(m) * n;
   for (int i = tid; i <= depth; i += nt) s_lo[i] = group_level_off[l0 + i];
   volatile unsigned long long *vtv = reinterpret_cast<volatile unsigned long long *>(s_tv);
@@ -1104,12 +1148,11 @@ __global__ __launch_bounds__(256) void wg_chain_flow_kernel(WgStatic S, WgState 
 #pragma unroll
       for (int u = 0; u < 8; u++)
         if (u < cur.nu) up += __longlong_as_double(vtv[(cur.up[u >> 1] >> ((u & 1) * 16)) & 0xffff]);
-      const int64_t mp = base + p;
       ChainRec c;
       slot_record(cur, c);
       const ChainOut o = chain_step<kUse>(c, up, d);
       vtv[p - gs] = __double_as_longlong(o.tv);
-      store_chain(X, mp, cur.flags, o);
+      store_chain(Xm, p, cur.flags, o);
       qq = (cur.flags & CFL_LDD) ? o.tv : 0.;
     }
     if (cur.station >= 0)
@@ -1150,7 +1193,8 @@ __global__ void wg_pot_runoff_kernel(WgStatic S, WgState X, int32_t p0, int32_t 
   const int p = p0 + int(blockIdx.x * blockDim.x + threadIdx.x);
   if (p >= p1) return;
   if (!(S.cflags[p] & CFL_CONT)) return;
-  add_pot_runoff(S, X, int64_t(blockIdx.y) * S.n + p, p);
+  member_rows(X, blockIdx.y, S.n);
+  add_pot_runoff(S, X, p);
 }
 
 // Sets the day clock read by the kernels of a captured block of days; launched
