@@ -1646,9 +1646,11 @@ int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int day
   for (int done = 0; done < days;) {
     const int k = std::min(days - done, h->ring_slots);
     auto *kern = h->S.use_on ? wg_days_kernel<true> : wg_days_kernel<false>;
-    hipLaunchKernelGGL(kern, dim3(t.n_waves, h->m), dim3(64), kDaysLdsBytes, h->stream, h->S, h->X, h->T,
-                       h->d_forcing, t.waves, t.slots, t.ranks, h->d_ring, h->ring_slots, h->ring_day, day + done,
-                       (doy - 1 + done) % 365 + 1, (h->started || done > 0) ? 1 : 0, k, done);
+    const DaysArgs args{h->S, h->X, h->T, h->d_forcing, t.waves, t.slots, t.ranks, h->d_ring, day + done,
+                        h->ring_slots, int32_t(h->ring_day % h->ring_slots),
+                        int32_t(h->ring_day / h->ring_slots % 2), (doy - 1 + done) % 365 + 1,
+                        (h->started || done > 0) ? 1 : 0, k, done};
+    hipLaunchKernelGGL(kern, dim3(t.n_waves, h->m), dim3(64), kDaysLdsBytes, h->stream, args);
     HIP_CHECK(h, hipGetLastError());
     h->ring_day += k;
     done += k;

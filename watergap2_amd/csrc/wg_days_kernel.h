@@ -63,42 +63,83 @@ constexpr int kDaysSpinLimit = 1 << 22;
 
 }  // namespace
 
+// The kernel's arguments, read where they are used: each DAYS_ARGS makes the compiler
+// load those that follow anew (scalar loads).  Held in scalar registers from the
+// start they would take ten times what there is, spilled lane by lane (a sixth of
+// the vector instructions of a day).
+struct DaysArgs {
+  WgStatic stat;
+  WgState state;
+  WgTables tables;
+  const float *forcing;
+  const WgDayWave *waves;
+  const WgDaySlot *slots;
+  const uint8_t *ranks;
+  unsigned long long *ring;
+  int64_t fday0;
+  int32_t ring_slots, ring_slot0, ring_turn;  // the first day's slot, and its turn's parity
+  int32_t doy0, started0, days, slot0;
+};
+typedef const __attribute__((address_space(4))) DaysArgs *DaysArgsPtr;
+#define DAYS_ARGS(A, S, X)                                              \
+  DaysArgsPtr A##_ = (DaysArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(); \
+  asm volatile("" : "+s"(A##_));                                        \
+  const DaysArgs &A = *(const DaysArgs *)A##_;                          \
+  const WgStatic &S = A.stat;                                              \
+  const WgState &X = A.state;                                               \
+  (void)S;                                                              \
+  (void)X
+
+namespace {
+
+__device__ __forceinline__ int days_doy(const DaysArgs &A, int k) { return int((A.doy0 - 1 + k) % 365) + 1; }
+__device__ __forceinline__ DayInfo days_info(const DaysArgs &A, int k) { return day_info(days_doy(A, k)); }
+
+// The member's row of day k in the ring, and the sign bit of its turn.
+__device__ __forceinline__ unsigned long long *days_ring_row(const DaysArgs &A, int k, int64_t o,
+                                                             unsigned long long &sign) {
+  const uint32_t slots = uint32_t(A.ring_slots), at0 = uint32_t(A.ring_slot0) + uint32_t(k);
+  const bool wrapped = at0 >= slots;  // at most once in a launch
+  sign = (wrapped != (A.ring_turn != 0)) ? 0ull : 0x8000000000000000ull;
+  return A.ring + int64_t(wrapped ? at0 - slots : at0) * A.stat.n_members * A.stat.n + o;
+}
+
+__device__ __forceinline__ double *days_station_row(const DaysArgs &A, int k, int m) {
+  return A.state.st_daily + (int64_t(m) * WG_DAILY_SLOTS + A.slot0 + k) * A.stat.n_stations;
+}
+
+}  // namespace
+
 template <bool kUse>
-__global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, WgTables T,
-                                                        const float *__restrict__ forcing,
-                                                        const WgDayWave *__restrict__ waves,
-                                                        const WgDaySlot *__restrict__ slots,
-                                                        const uint8_t *__restrict__ ranks,
-                                                        unsigned long long *ring, int32_t ring_slots,
-                                                        int64_t ring_day, int64_t fday0, int32_t doy0,
-                                                        int32_t started0, int32_t days, int32_t slot0) {
+__global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
   load_exp2_table();
-  const WgDayWave wv = waves[blockIdx.x];
   const int lane = threadIdx.x;
-  const WgDaySlot slot = slots[blockIdx.x * 64 + lane];
+  const int m = blockIdx.y;
+  DAYS_ARGS(A0, S0, X0);
+  const WgDayWave wv = A0.waves[blockIdx.x];
+  const WgDaySlot slot = A0.slots[blockIdx.x * 64 + lane];
   if (slot.cell < 0) return;
   const uint32_t p = uint32_t(slot.cell);
-  const int m = blockIdx.y;
-  const int n = S.n;
-  member_rows(X, m, n);
+  const int n = S0.n;
+  const int64_t o = int64_t(m) * n;  // the member's rows
   double *F = wg_lds + WG_EXP2_LDS_BYTES / sizeof(double) + lane;
   auto fld = [&](int f) -> double { return F[f * 64]; };
 
-  const WgChainLink link = load_link(S, p);
-  const int rank = ranks[blockIdx.x * 64 + lane];
+  const WgChainLink link = load_link(S0, p);
+  const int rank = A0.ranks[blockIdx.x * 64 + lane];
   F[DF_NEAR * 64] = __builtin_bit_cast(double, WordPair{int32_t(slot.near_lo), int32_t(slot.near_hi)});
   int bits = 0;
   {
     DayStatA a;
     DayStatB b;
     DayStatEnd e;
-    load_stat_a(S, T, p, a);
-    load_stat_b(S, X, p, b);
-    load_stat_end(S, p, e);
-    const WgChainStatic cs = load_cstat(S, p);
+    load_stat_a(S0, A0.tables, p, a);
+    load_stat_b(S0, X0, o, p, b);
+    load_stat_end(S0, p, e);
+    const WgChainStatic cs = load_cstat(S0, p);
     bits = (b.arid ? DB_ARID : 0) | (b.recharge_cut ? DB_CUT : 0) | (b.ldd >= 0 ? DB_LDD : 0) |
            (e.contcell ? DB_CONT : 0) | (e.lake_area > 0. ? DB_LAKE : 0) | (e.reservoir_area > 0. ? DB_RES : 0) |
-           (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0) | int(uint32_t(uint16_t(at(S.rgmax, p))) << 16);
+           (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0) | int(uint32_t(uint16_t(at(S0.rgmax, p))) << 16);
     F[DF_M_PREC * 64] = a.m_prec;
     F[DF_ALPHA * 64] = a.alpha;
     F[DF_PET_MXDY * 64] = a.pet_mxdy;
@@ -162,12 +203,12 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
   }
 
   CellState s;
-  load_state_a(X, p, s);
-  load_state_b(X, p, s);
-  load_state_end(X, p, s);
-  s.laf_prev = at(X.laf_prev, p);
-  s.red_gl = at(X.red_gl, p);
-  s.red_res = at(X.red_res, p);
+  load_state_a(X0, o, p, s);
+  load_state_b(X0, o, p, s);
+  load_state_end(X0, o, p, s);
+  s.laf_prev = at(X0.laf_prev + o, p);
+  s.red_gl = at(X0.red_gl + o, p);
+  s.red_res = at(X0.red_res + o, p);
   F[DF_LAI_PREC * 64] = s.lai_precsum;
   F[DF_TRANSFER * 64] = s.transfer;
   F[DF_GLO_LAKE * 64] = s.glo_lake;
@@ -177,9 +218,9 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
   F[DF_RED_RES * 64] = s.red_res;
   F[DF_RED_RIVER * 64] = s.red_river;
   F[DF_FRAC_CHANGE * 64] = s.river_frac_change;
-  const ElevRange er = load_elev_range(S, p);
-  const int64_t ring_stride = int64_t(S.n_members) * n;
-  const float *fd = forcing + fday0 * 4 * int64_t(n);
+  const ElevRange er = load_elev_range(S0, p);
+  const float *fd = A0.forcing + A0.fday0 * 4 * int64_t(n);
+  const int days = A0.days;
   float f0 = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
   if (!kUse) {
     f0 = at(fd, p);
@@ -190,20 +231,15 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
 
 #pragma unroll 1
   for (int k = 0; k < days; k++) {
-    const int64_t fday = fday0 + k;
-    const int doy = int((doy0 - 1 + k) % 365) + 1;
-    const DayInfo di = day_info(doy);
-    const int64_t gday = ring_day + k;
-    const int64_t turn = gday / ring_slots;
-    unsigned long long *rrow = ring + (gday - turn * ring_slots) * ring_stride + int64_t(m) * n;
-    const unsigned long long sign = (turn & 1) ? 0ull : 0x8000000000000000ull;
-    double *daily = X.st_daily + (int64_t(m) * WG_DAILY_SLOTS + slot0 + k) * S.n_stations;
     double rem = 0.;
     if (!cont) {
+      DAYS_ARGS(A, S, X);
+      unsigned long long sign;
+      unsigned long long *rrow = days_ring_row(A, k, o, sign);
       // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
       // routing.cpp:1876); other cells keep a zero transported volume.
       __hip_atomic_store(&at(rrow, p), sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (link.station >= 0) daily[link.station] = 0.;
+      if (link.station >= 0) days_station_row(A, k, m)[link.station] = 0.;
     } else {
       // the next day's forcing is loaded a day ahead (with water use there is no
       // register to hold it)
@@ -217,8 +253,13 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         f2 = at(fd + 2 * int64_t(n), p);
         f3 = at(fd + 3 * int64_t(n), p);
       }
-      if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
-      const double laf_prev = (started0 || k > 0) ? s.laf_prev : s.laf;  // daily.cpp:159-169
+      bool started;
+      {
+        DAYS_ARGS(A, S, X);
+        if (X.perturb) perturb_forcing(S, X, m, p, A.fday0 + k, tf, pf);
+        started = A.started0 || k > 0;
+      }
+      const double laf_prev = started ? s.laf_prev : s.laf;  // daily.cpp:159-169
       DayFlux v;
       {
         DayStatA a;
@@ -245,9 +286,11 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         s.transfer = fld(DF_TRANSFER);
         day_pet_canopy(a, s, v, tf, pf, swf, lwf, laf_prev);
         F[DF_LAI_PREC * 64] = s.lai_precsum;
-        if (s.laf <= 0.) day_snow_no_land(s, v, X.snow2, p, n);
+        DAYS_ARGS(A, S, X);
+        WgD2 *sub = X.snow2 + o * WG_DEV_NPAIR;
+        if (s.laf <= 0.) day_snow_no_land(s, v, sub, p, n);
         F[DF_TRANSFER * 64] = s.transfer;
-        if (s.laf > 0.) day_snow<5>(a, s, v, laf_prev, er, X.snow2, S.elev_pairs, p, n);
+        if (s.laf > 0.) day_snow<5>(a, s, v, laf_prev, er, sub, S.elev_pairs, p, n);
       }
       ChainRec c;
       {
@@ -269,15 +312,17 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         day_soil(b, s, v, laf_prev);
         F[DF_TRANSFER * 64] = s.transfer;
         if (k == days - 1) {
-          at(X.d_surf, p) = v.surf_runoff;
-          at(X.d_recharge, p) = v.recharge;
-          at(X.d_ow_pet, p) = v.ow_pet;
-          at(X.d_aet, p) = v.aet;
-          at(X.d_prec, p) = v.prec;
+          DAYS_ARGS(A, S, X);
+          at(X.d_surf + o, p) = v.surf_runoff;
+          at(X.d_recharge + o, p) = v.recharge;
+          at(X.d_ow_pet + o, p) = v.ow_pet;
+          at(X.d_aet + o, p) = v.aet;
+          at(X.d_prec + o, p) = v.prec;
         }
+        DAYS_ARGS(A, S, X);
         double use_desired = 0., use_nag = 0.;
         int64_t use_t = 0;
-        if (kUse) use_t = day_use(S, X, p, fday, di.month, use_desired, use_nag);
+        if (kUse) use_t = day_use(S, X, o, p, A.fday0 + k, days_info(A, k).month, use_desired, use_nag);
         b.area = fld(DF_AREA);
         b.area_m = fld(DF_AREA_M);
         b.cf100 = fld(DF_CF100);
@@ -325,12 +370,15 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         PotTerms pot;
         day_local_routing<kUse>(b, lake, s, v, use_desired, use_nag, c, pot);
         if (X.pot_base) {
-          at(X.pot_base, p) = pot.base;
-          at(X.pot_ow, p) = pot.ow;
+          at(X.pot_base + o, p) = pot.base;
+          at(X.pot_ow + o, p) = pot.ow;
         }
       }
       // transported volumes of upstream cells in earlier wavefronts: wait for the
       // day's values (they are there already unless this wavefront has caught up)
+      DAYS_ARGS(A, S, X);
+      unsigned long long sign;
+      unsigned long long *rrow = days_ring_row(A, k, o, sign);
       unsigned long long t[8];
       int spins = 0;
       for (;;) {
@@ -353,9 +401,9 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
         __builtin_amdgcn_s_sleep(1);
       }
       const StepPre pre = step_pre<kUse>(c);
-      ChainOut o = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
-      for (int r = 0; r < wv.passes; r++) {
-        if (rank == r) {
+      ChainOut r = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
+      for (int pass = 0; pass < wv.passes; pass++) {
+        if (rank == pass) {
           // gather in routing order (the serial += of routing.cpp:3955-3958)
           double up = 0.;
           const WordPair lanes = __builtin_bit_cast(WordPair, fld(DF_NEAR));
@@ -369,27 +417,35 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
               up += (u < link.nu) ? q : 0.;
             }
           bool slow;
-          o = step_fast<kUse>(c, pre, up, slow);
-          if (slow) o = chain_step<kUse>(c, up, di);
-          const unsigned long long w = __builtin_bit_cast(unsigned long long, o.tv) & 0x7fffffffffffffffull;
+          r = step_fast<kUse>(c, pre, up, slow);
+          if (slow) {
+            DAYS_ARGS(A, S, X);
+            r = chain_step<kUse>(c, up, days_info(A, k));
+          }
+          const unsigned long long w = __builtin_bit_cast(unsigned long long, r.tv) & 0x7fffffffffffffffull;
           __hip_atomic_store(&at(rrow, p), w | sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          F[DF_TV * 64] = o.tv;
+          F[DF_TV * 64] = r.tv;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
       }
-      if (c.flags & CFL_LAKE) F[DF_GLO_LAKE * 64] = o.glo_lake;
+      if (c.flags & CFL_LAKE) F[DF_GLO_LAKE * 64] = r.glo_lake;
       if (c.flags & CFL_RES) {
-        F[DF_RES * 64] = o.res;
-        F[DF_K_RELEASE * 64] = o.k_release;
+        F[DF_RES * 64] = r.res;
+        F[DF_K_RELEASE * 64] = r.k_release;
       }
-      if (c.flags & CFL_GWET) s.glo_wetl = o.glo_wetl;
-      if (c.flags & CFL_ARID) s.gw = o.gw;
-      if ((c.flags & CFL_ARID) && X.pot_lgw) at(X.pot_lgw, p) = o.lgw;
-      s.river = o.river;
-      rem = o.rem;
-      if (link.station >= 0) daily[link.station] = (c.flags & CFL_LDD) ? o.tv : 0.;
-      if (k == days - 1) at(X.tv, p) = o.tv;
-      if (X.pot_acc) add_pot_runoff(S, X, p);
+      if (c.flags & CFL_GWET) s.glo_wetl = r.glo_wetl;
+      if (c.flags & CFL_ARID) s.gw = r.gw;
+      s.river = r.river;
+      rem = r.rem;
+      {
+        DAYS_ARGS(B, SB, XB);
+        if (link.station >= 0) days_station_row(B, k, m)[link.station] = (c.flags & CFL_LDD) ? r.tv : 0.;
+        if (k == days - 1) at(XB.tv + o, p) = r.tv;
+        if (XB.pot_acc) {
+          if (c.flags & CFL_ARID) at(XB.pot_lgw + o, p) = r.lgw;
+          add_pot_runoff(SB, XB, o, p);
+        }
+      }
     }
     {
       DayStatEnd e;
@@ -412,6 +468,7 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
       e.reservoir_area = 0.;
       e.stor_cap = 0.;
       if (bits & (DB_LAKE | DB_RES)) {
+        DAYS_ARGS(A, S, X);
         e.lake_area = at(S.lake_area, p);
         e.lake_max = e.lake_area * at(S.lake_depth, p);
         e.reservoir_area = at(S.reservoir_area, p);
@@ -425,8 +482,10 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
       s.red_river = fld(DF_RED_RIVER);
       s.river_frac_change = fld(DF_FRAC_CHANGE);
       if (kUse && cont) {
-        const int fin_ym = int((fday - S.use_day0) / 365) * 12 + di.month;
-        day_end_use(S, X.use, p, s, rem, e.loc_lake, fld(DF_LL_MAX), e.red_exp, fin_ym, doy == 365);
+        DAYS_ARGS(A, S, X);
+        const int fin_ym = int((A.fday0 + k - S.use_day0) / 365) * 12 + days_info(A, k).month;
+        day_end_use(S, X.use + o, p, s, rem, e.loc_lake, fld(DF_LL_MAX), e.red_exp, fin_ym,
+                    days_doy(A, k) == 365);
       }
       day_end(e, s);
       F[DF_RED_RIVER * 64] = s.red_river;
@@ -438,33 +497,34 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(WgStatic S, WgState X, W
     }
   }
 
-  at(X.canopy, p) = s.canopy;
-  at(X.soil, p) = s.soil;
-  at(X.snow, p) = s.snow;
-  at(X.transfer, p) = fld(DF_TRANSFER);
-  at(X.lai_precsum, p) = fld(DF_LAI_PREC);
-  at(X.lai_days, p) = s.lai_days;
-  at(X.lai_status, p) = s.lai_status;
-  at(X.snow_any, p) = s.snow_any ? 1 : 0;
-  at(X.gw, p) = s.gw;
-  at(X.loc_lake, p) = s.loc_lake;
-  at(X.loc_wetl, p) = s.loc_wetl;
-  at(X.glo_lake, p) = fld(DF_GLO_LAKE);
-  at(X.glo_wetl, p) = s.glo_wetl;
-  at(X.res, p) = fld(DF_RES);
-  at(X.river, p) = s.river;
-  at(X.red_ll, p) = s.red_ll;
-  at(X.red_lw, p) = s.red_lw;
-  at(X.red_gl, p) = fld(DF_RED_GL);
-  at(X.red_gw, p) = s.red_gw;
-  at(X.red_res, p) = fld(DF_RED_RES);
-  at(X.red_river, p) = fld(DF_RED_RIVER);
-  at(X.river_frac_next, p) = s.river_frac_next;
-  at(X.river_frac_change, p) = fld(DF_FRAC_CHANGE);
-  at(X.fswb_next, p) = s.fswb_next;
-  at(X.laf, p) = s.laf;
-  at(X.laf_prev, p) = s.laf_prev;
-  at(X.k_release, p) = fld(DF_K_RELEASE);
+  DAYS_ARGS(A, S, X);
+  at(X.canopy + o, p) = s.canopy;
+  at(X.soil + o, p) = s.soil;
+  at(X.snow + o, p) = s.snow;
+  at(X.transfer + o, p) = fld(DF_TRANSFER);
+  at(X.lai_precsum + o, p) = fld(DF_LAI_PREC);
+  at(X.lai_days + o, p) = s.lai_days;
+  at(X.lai_status + o, p) = s.lai_status;
+  at(X.snow_any + o, p) = s.snow_any ? 1 : 0;
+  at(X.gw + o, p) = s.gw;
+  at(X.loc_lake + o, p) = s.loc_lake;
+  at(X.loc_wetl + o, p) = s.loc_wetl;
+  at(X.glo_lake + o, p) = fld(DF_GLO_LAKE);
+  at(X.glo_wetl + o, p) = s.glo_wetl;
+  at(X.res + o, p) = fld(DF_RES);
+  at(X.river + o, p) = s.river;
+  at(X.red_ll + o, p) = s.red_ll;
+  at(X.red_lw + o, p) = s.red_lw;
+  at(X.red_gl + o, p) = fld(DF_RED_GL);
+  at(X.red_gw + o, p) = s.red_gw;
+  at(X.red_res + o, p) = fld(DF_RED_RES);
+  at(X.red_river + o, p) = fld(DF_RED_RIVER);
+  at(X.river_frac_next + o, p) = s.river_frac_next;
+  at(X.river_frac_change + o, p) = fld(DF_FRAC_CHANGE);
+  at(X.fswb_next + o, p) = s.fswb_next;
+  at(X.laf + o, p) = s.laf;
+  at(X.laf_prev + o, p) = s.laf_prev;
+  at(X.k_release + o, p) = fld(DF_K_RELEASE);
 }
 
 #endif  // WG_DAYS_KERNEL_H

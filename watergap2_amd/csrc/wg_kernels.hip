@@ -117,44 +117,19 @@ __device__ inline WgChainStatic load_cstat(const WgStatic &S, uint32_t p) {
   return WgChainStatic{a.x, a.y, b.x, b.y, c.x, c.y};
 }
 
-// Moves a state's pointers to the rows of member m.
-__device__ __forceinline__ void member_rows(WgState &X, int m, int n) {
-  const int64_t o = int64_t(m) * n;
-  double **rows[] = {&X.canopy, &X.soil, &X.snow, &X.transfer, &X.lai_precsum, &X.gw, &X.loc_lake, &X.loc_wetl,
-                     &X.glo_lake, &X.glo_wetl, &X.res, &X.river, &X.red_ll, &X.red_lw, &X.red_gl, &X.red_gw,
-                     &X.red_res, &X.red_river, &X.river_frac_next, &X.river_frac_change, &X.fswb_next, &X.laf,
-                     &X.laf_prev, &X.k_release, &X.gamma, &X.cfa, &X.tv, &X.d_surf, &X.d_recharge, &X.d_ow_pet,
-                     &X.d_aet, &X.d_prec};
-#pragma unroll
-  for (size_t k = 0; k < sizeof(rows) / sizeof(rows[0]); k++) *rows[k] += o;
-  X.lai_days += o;
-  X.lai_status += o;
-  X.snow_any += o;
-  X.smax += o;
-  X.snow2 += o * WG_DEV_NPAIR;
-  X.crec += o * (WG_DEV_NREC / 2);
-  // optional arrays stay NULL when off
-  if (X.pot_acc) X.pot_acc += o;
-  if (X.pot_base) X.pot_base += o;
-  if (X.pot_ow) X.pot_ow += o;
-  if (X.pot_lgw) X.pot_lgw += o;
-  if (X.use) X.use += o;
-  if (X.use_rem) X.use_rem += o;
-}
-
-// Writes what chain_step changed; X holds the member's rows.
-__device__ inline void store_chain(const WgState &X, uint32_t p, int flags, const ChainOut &o) {
-  if (flags & CFL_LAKE) at(X.glo_lake, p) = o.glo_lake;
+// Writes what chain_step changed; o: the offset of the member's rows.
+__device__ inline void store_chain(const WgState &X, int64_t o, uint32_t p, int flags, const ChainOut &r) {
+  if (flags & CFL_LAKE) at(X.glo_lake + o, p) = r.glo_lake;
   if (flags & CFL_RES) {
-    at(X.res, p) = o.res;
-    at(X.k_release, p) = o.k_release;
+    at(X.res + o, p) = r.res;
+    at(X.k_release + o, p) = r.k_release;
   }
-  if (flags & CFL_GWET) at(X.glo_wetl, p) = o.glo_wetl;
-  if (flags & CFL_ARID) at(X.gw, p) = o.gw;
-  if ((flags & CFL_ARID) && X.pot_lgw) at(X.pot_lgw, p) = o.lgw;
-  at(X.river, p) = o.river;
-  at(X.tv, p) = o.tv;
-  if (X.use_rem) at(X.use_rem, p) = o.rem;
+  if (flags & CFL_GWET) at(X.glo_wetl + o, p) = r.glo_wetl;
+  if (flags & CFL_ARID) at(X.gw + o, p) = r.gw;
+  if ((flags & CFL_ARID) && X.pot_lgw) at(X.pot_lgw + o, p) = r.lgw;
+  at(X.river + o, p) = r.river;
+  at(X.tv + o, p) = r.tv;
+  if (X.use_rem) at(X.use_rem + o, p) = r.rem;
 }
 
 #include "wg_cell_day.h"
@@ -191,12 +166,12 @@ __device__ __forceinline__ void load_stat_a(const WgStatic &S, const WgTables &T
   a.arid = at(S.aindex, p) == 1;
 }
 
-__device__ __forceinline__ void load_stat_b(const WgStatic &S, const WgState &X, uint32_t p, DayStatB &b) {
+__device__ __forceinline__ void load_stat_b(const WgStatic &S, const WgState &X, int64_t o, uint32_t p, DayStatB &b) {
   b.built_up = at(S.built_up, p);
-  b.smax = at(X.smax, p);
+  b.smax = at(X.smax + o, p);
   b.gw_factor = at(S.gw_factor, p);
-  b.gamma = at(X.gamma, p);
-  b.cfa = at(X.cfa, p);
+  b.gamma = at(X.gamma + o, p);
+  b.cfa = at(X.cfa + o, p);
   b.pet_mxdy = at(S.pet_mxdy, p);
   b.t_snowfz = at(S.t_snowfz, p);
   b.pcritgwa = at(S.pcritgwa, p);
@@ -272,61 +247,61 @@ __device__ __forceinline__ ElevRange load_elev_range(const WgStatic &S, uint32_t
 }
 
 // State read by PET, LAI, canopy and snow.
-__device__ __forceinline__ void load_state_a(const WgState &X, uint32_t p, CellState &s) {
-  s.canopy = at(X.canopy, p);
-  s.lai_days = at(X.lai_days, p);
-  s.lai_precsum = at(X.lai_precsum, p);
-  s.lai_status = at(X.lai_status, p);
-  s.snow = at(X.snow, p);
-  s.snow_any = at(X.snow_any, p) != 0;
-  s.transfer = at(X.transfer, p);
+__device__ __forceinline__ void load_state_a(const WgState &X, int64_t o, uint32_t p, CellState &s) {
+  s.canopy = at(X.canopy + o, p);
+  s.lai_days = at(X.lai_days + o, p);
+  s.lai_precsum = at(X.lai_precsum + o, p);
+  s.lai_status = at(X.lai_status + o, p);
+  s.snow = at(X.snow + o, p);
+  s.snow_any = at(X.snow_any + o, p) != 0;
+  s.transfer = at(X.transfer + o, p);
 }
 
 // State read by soil and local routing.
-__device__ __forceinline__ void load_state_b(const WgState &X, uint32_t p, CellState &s) {
-  s.soil = at(X.soil, p);
-  s.gw = at(X.gw, p);
-  s.loc_lake = at(X.loc_lake, p);
-  s.loc_wetl = at(X.loc_wetl, p);
-  s.glo_lake = at(X.glo_lake, p);
-  s.glo_wetl = at(X.glo_wetl, p);
-  s.res = at(X.res, p);
-  s.river = at(X.river, p);
-  s.k_release = at(X.k_release, p);
+__device__ __forceinline__ void load_state_b(const WgState &X, int64_t o, uint32_t p, CellState &s) {
+  s.soil = at(X.soil + o, p);
+  s.gw = at(X.gw + o, p);
+  s.loc_lake = at(X.loc_lake + o, p);
+  s.loc_wetl = at(X.loc_wetl + o, p);
+  s.glo_lake = at(X.glo_lake + o, p);
+  s.glo_wetl = at(X.glo_wetl + o, p);
+  s.res = at(X.res + o, p);
+  s.river = at(X.river + o, p);
+  s.k_release = at(X.k_release + o, p);
 }
 
 // State read by the day's end (with loc_lake for the water use).
-__device__ __forceinline__ void load_state_end(const WgState &X, uint32_t p, CellState &s) {
-  s.glo_lake = at(X.glo_lake, p);
-  s.glo_wetl = at(X.glo_wetl, p);
-  s.res = at(X.res, p);
-  s.river = at(X.river, p);
-  s.red_ll = at(X.red_ll, p);
-  s.red_lw = at(X.red_lw, p);
+__device__ __forceinline__ void load_state_end(const WgState &X, int64_t o, uint32_t p, CellState &s) {
+  s.glo_lake = at(X.glo_lake + o, p);
+  s.glo_wetl = at(X.glo_wetl + o, p);
+  s.res = at(X.res + o, p);
+  s.river = at(X.river + o, p);
+  s.red_ll = at(X.red_ll + o, p);
+  s.red_lw = at(X.red_lw + o, p);
   s.red_gl = 0.;
-  s.red_gw = at(X.red_gw, p);
+  s.red_gw = at(X.red_gw + o, p);
   s.red_res = 0.;
-  s.red_river = at(X.red_river, p);
-  s.river_frac_next = at(X.river_frac_next, p);
-  s.river_frac_change = at(X.river_frac_change, p);
-  s.fswb_next = at(X.fswb_next, p);
-  s.laf = at(X.laf, p);
+  s.red_river = at(X.red_river + o, p);
+  s.river_frac_next = at(X.river_frac_next + o, p);
+  s.river_frac_change = at(X.river_frac_change + o, p);
+  s.fswb_next = at(X.fswb_next + o, p);
+  s.laf = at(X.laf + o, p);
 }
 
 // Writes what the day's end changed.
-__device__ __forceinline__ void store_state_end(const WgState &X, uint32_t p, const DayStatEnd &e,
+__device__ __forceinline__ void store_state_end(const WgState &X, int64_t o, uint32_t p, const DayStatEnd &e,
                                                 const CellState &s) {
-  if (e.lake_area > 0.) at(X.red_gl, p) = s.red_gl;
-  if (e.reservoir_area > 0.) at(X.red_res, p) = s.red_res;
-  at(X.laf_prev, p) = s.laf_prev;
-  at(X.laf, p) = s.laf;
-  at(X.fswb_next, p) = s.fswb_next;
-  at(X.red_ll, p) = s.red_ll;
-  at(X.red_lw, p) = s.red_lw;
-  at(X.red_gw, p) = s.red_gw;
-  at(X.red_river, p) = s.red_river;
-  at(X.river_frac_next, p) = s.river_frac_next;
-  at(X.river_frac_change, p) = s.river_frac_change;
+  if (e.lake_area > 0.) at(X.red_gl + o, p) = s.red_gl;
+  if (e.reservoir_area > 0.) at(X.red_res + o, p) = s.red_res;
+  at(X.laf_prev + o, p) = s.laf_prev;
+  at(X.laf + o, p) = s.laf;
+  at(X.fswb_next + o, p) = s.fswb_next;
+  at(X.red_ll + o, p) = s.red_ll;
+  at(X.red_lw + o, p) = s.red_lw;
+  at(X.red_gw + o, p) = s.red_gw;
+  at(X.red_river + o, p) = s.red_river;
+  at(X.river_frac_next + o, p) = s.river_frac_next;
+  at(X.river_frac_change + o, p) = s.river_frac_change;
 }
 
 // The day's perturbed temperature and precipitation of one (member, cell).
@@ -346,11 +321,11 @@ __device__ __forceinline__ void perturb_forcing(const WgStatic &S, const WgState
 // remaining use; the adaptation reads only the last day's state, so it is done
 // here for (semi-)arid cells too, whose groundwater step the chain runs).
 // Returns the offset of the day's rows in the tables.
-__device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, uint32_t p, int64_t fday,
+__device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, int64_t o, uint32_t p, int64_t fday,
                                            int month, double &desired, double &nag) {
   const int64_t t = (int64_t((fday - S.use_day0) / 365) * 12 + month) * S.n;
   const int64_t us = S.use_stride;
-  double *U = X.use;
+  double *U = X.use + o;
   nag = at(S.use_nug + t, p);
   if (at(U + WG_USE_DAILY_REMAINING * us, p) != 0.) nag = update_net_abstraction_gw(U, us, p, at(S.use_frgi, p), nag);
   desired = at(S.use_nus + t, p);
@@ -362,14 +337,14 @@ __device__ __forceinline__ int64_t day_use(const WgStatic &S, const WgState &X, 
 // G_potCellRunoff[n] += potCellRunoff (routing.cpp:1970, 2053, 2187, 3379): the
 // local runoff terms, then the arid groundwater step's runoff where that step ran,
 // then the open-water balance, in the reference's order of addition.
-__device__ __forceinline__ void add_pot_runoff(const WgStatic &S, const WgState &X, uint32_t p) {
-  const double base = at(X.pot_base, p);
-  const double lake_balance = at(X.pot_ow, p) * at(X.cfa, p);  // (dailyPrec - dailyOpenWaterPET) * CFA
+__device__ __forceinline__ void add_pot_runoff(const WgStatic &S, const WgState &X, int64_t o, uint32_t p) {
+  const double base = at(X.pot_base + o, p);
+  const double lake_balance = at(X.pot_ow + o, p) * at(X.cfa + o, p);  // (dailyPrec - dailyOpenWaterPET) * CFA
   const double ow = (lake_balance / 1000000.0) *
                     ((at(S.lake_area, p) + at(S.reservoir_area, p)) +
                      ((at(S.cell_area, p) / 100.0) * ((at(S.loc_lake, p) + at(S.loc_wetland, p)) + at(S.glo_wetland, p))));
-  const double pot = (at(S.cflags, p) & CFL_ARID) ? (base + at(X.pot_lgw, p)) + ow : base + ow;
-  at(X.pot_acc, p) += pot;
+  const double pot = (at(S.cflags, p) & CFL_ARID) ? (base + at(X.pot_lgw + o, p)) + ow : base + ow;
+  at(X.pot_acc + o, p) += pot;
 }
 
 }  // namespace
@@ -400,7 +375,7 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   if (int(p) >= S.tile_end[blockIdx.x]) return;
   const int m = blockIdx.y;
   const int n = S.n;
-  member_rows(X, m, n);
+  const int64_t o = int64_t(m) * n;
 
   DayStatA sa;
   CellState s;
@@ -408,34 +383,34 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   if (do_vertical) {
     er = load_elev_range(S, p);
     load_stat_a(S, T, p, sa);
-    load_state_a(X, p, s);
+    load_state_a(X, o, p, s);
   }
   if (do_post) {
     DayStatEnd e;
     load_stat_end(S, p, e);
-    load_state_end(X, p, s);
+    load_state_end(X, o, p, s);
     if (kUse && e.contcell) {
       // the finished day is day k - 1 of the block (the closing pass runs with k = days)
       const int64_t fin = clock->day0 + k - 1;
       const int fin_doy = int((clock->doy0 - 1 + k - 1) % 365) + 1;
       const int fin_ym = int((fin - S.use_day0) / 365) * 12 + day_info(fin_doy).month;
-      s.loc_lake = at(X.loc_lake, p);
-      day_end_use(S, X.use, p, s, at(X.use_rem, p), e.loc_lake,
+      s.loc_lake = at(X.loc_lake + o, p);
+      day_end_use(S, X.use + o, p, s, at(X.use_rem + o, p), e.loc_lake,
                   e.loc_lake / 100. * e.area * at(S.lake_depth, p), e.red_exp, fin_ym, fin_doy == 365);
-      at(X.loc_lake, p) = s.loc_lake;
-      at(X.use_rem, p) = 0.;
+      at(X.loc_lake + o, p) = s.loc_lake;
+      at(X.use_rem + o, p) = 0.;
     }
     day_end(e, s);
-    store_state_end(X, p, e, s);
+    store_state_end(X, o, p, e, s);
   } else if (do_vertical) {
-    s.laf = at(X.laf, p);
-    s.laf_prev = at(X.laf_prev, p);
-    s.red_ll = at(X.red_ll, p);
-    s.red_lw = at(X.red_lw, p);
-    s.red_gw = at(X.red_gw, p);
-    s.red_gl = at(X.red_gl, p);
-    s.red_res = at(X.red_res, p);
-    s.river_frac_next = at(X.river_frac_next, p);
+    s.laf = at(X.laf + o, p);
+    s.laf_prev = at(X.laf_prev + o, p);
+    s.red_ll = at(X.red_ll + o, p);
+    s.red_lw = at(X.red_lw + o, p);
+    s.red_gw = at(X.red_gw + o, p);
+    s.red_gl = at(X.red_gl + o, p);
+    s.red_res = at(X.red_res + o, p);
+    s.river_frac_next = at(X.river_frac_next + o, p);
   }
   // calcNewDay and routing run for continental cells only (integrateWGHM.cpp:770,
   // routing.cpp:1876); other cells keep a zero transported volume.
@@ -456,38 +431,38 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   if (X.perturb) perturb_forcing(S, X, m, p, fday, tf, pf);
   double use_desired = 0., use_nag = 0.;
   int64_t use_t = 0;
-  if (kUse) use_t = day_use(S, X, p, fday, day_info(doy).month, use_desired, use_nag);
+  if (kUse) use_t = day_use(S, X, o, p, fday, day_info(doy).month, use_desired, use_nag);
 
   const double laf_prev = started ? s.laf_prev : s.laf;  // daily.cpp:159-169
   DayFlux v;
   day_pet_canopy(sa, s, v, tf, pf, swf, lwf, laf_prev);
-  at(X.lai_days, p) = s.lai_days;
-  at(X.lai_status, p) = s.lai_status;
-  at(X.lai_precsum, p) = s.lai_precsum;
-  at(X.canopy, p) = s.canopy;
+  at(X.lai_days + o, p) = s.lai_days;
+  at(X.lai_status + o, p) = s.lai_status;
+  at(X.lai_precsum + o, p) = s.lai_precsum;
+  at(X.canopy + o, p) = s.canopy;
   if (s.laf <= 0.)
-    day_snow_no_land(s, v, X.snow2, p, n);
+    day_snow_no_land(s, v, X.snow2 + o * WG_DEV_NPAIR, p, n);
   else
-    day_snow<kSnowChunk>(sa, s, v, laf_prev, er, X.snow2, S.elev_pairs, p, n);
-  at(X.snow_any, p) = s.snow_any ? 1 : 0;
+    day_snow<kSnowChunk>(sa, s, v, laf_prev, er, X.snow2 + o * WG_DEV_NPAIR, S.elev_pairs, p, n);
+  at(X.snow_any + o, p) = s.snow_any ? 1 : 0;
   DayStatB sb;
   DayStatLake lake;
-  load_stat_b(S, X, p, sb);
+  load_stat_b(S, X, o, p, sb);
   load_stat_lake(S, p, lake);
-  load_state_b(X, p, s);
+  load_state_b(X, o, p, s);
   const WgChainLink lk = load_link(S, p);
   const WgChainStatic cs = load_cstat(S, p);
   if (kUse) lake.prov_rel = at(S.use_provrel + use_t, p);
-  at(X.snow, p) = s.snow;
+  at(X.snow + o, p) = s.snow;
   day_soil(sb, s, v, laf_prev);
-  at(X.soil, p) = s.soil;
-  at(X.transfer, p) = s.transfer;
+  at(X.soil + o, p) = s.soil;
+  at(X.transfer + o, p) = s.transfer;
   if (write_diag) {
-    at(X.d_surf, p) = v.surf_runoff;
-    at(X.d_recharge, p) = v.recharge;
-    at(X.d_ow_pet, p) = v.ow_pet;
-    at(X.d_aet, p) = v.aet;
-    at(X.d_prec, p) = v.prec;
+    at(X.d_surf + o, p) = v.surf_runoff;
+    at(X.d_recharge + o, p) = v.recharge;
+    at(X.d_ow_pet + o, p) = v.ow_pet;
+    at(X.d_aet + o, p) = v.aet;
+    at(X.d_prec + o, p) = v.prec;
   }
   ChainRec c;
   double *w = c.v;
@@ -500,36 +475,36 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   c.flags = lk.flags;
   PotTerms pot;
   day_local_routing<kUse>(sb, lake, s, v, use_desired, use_nag, c, pot);
-  if (!(sb.arid && (sb.ldd >= 0))) at(X.gw, p) = s.gw;
+  if (!(sb.arid && (sb.ldd >= 0))) at(X.gw + o, p) = s.gw;
   if (X.pot_base) {
-    at(X.pot_base, p) = pot.base;  // wg_pot_runoff_kernel completes the terms
-    at(X.pot_ow, p) = pot.ow;
+    at(X.pot_base + o, p) = pot.base;  // wg_pot_runoff_kernel completes the terms
+    at(X.pot_ow + o, p) = pot.ow;
   }
   if (sb.loc_lake > 0.) {
-    at(X.loc_lake, p) = s.loc_lake;
-    at(X.red_ll, p) = s.red_ll;
+    at(X.loc_lake + o, p) = s.loc_lake;
+    at(X.red_ll + o, p) = s.red_ll;
   }
   if (sb.loc_wetland > 0.) {
-    at(X.loc_wetl, p) = s.loc_wetl;
-    at(X.red_lw, p) = s.red_lw;
+    at(X.loc_wetl + o, p) = s.loc_wetl;
+    at(X.red_lw + o, p) = s.red_lw;
   }
   if (lk.nu == 0) {
     // no upstream cell: G_riverInflow[n] is still 0 when the cell is routed
-    const ChainOut o = chain_step<kUse>(c, 0.0, day_info(doy));
-    store_chain(X, p, c.flags, o);
+    const ChainOut r = chain_step<kUse>(c, 0.0, day_info(doy));
+    store_chain(X, o, p, c.flags, r);
     if (lk.station >= 0)
-      X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + lk.station] = (sb.ldd >= 0) ? o.tv : 0.;
+      X.st_daily[(int64_t(m) * WG_DAILY_SLOTS + daily_slot) * S.n_stations + lk.station] = (sb.ldd >= 0) ? r.tv : 0.;
   } else {
     // the pairs holding the prefix for every routed cell (the last of them also
     // holds the first suffix field), the rest for cells with a lake or reservoir
     constexpr int kPrefixPairs = (CF_PREFIX + 1) / 2;
 #pragma unroll
-    for (int k = 0; k < kPrefixPairs; k++) at(X.crec + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
+    for (int k = 0; k < kPrefixPairs; k++) at(X.crec + o * (WG_DEV_NREC / 2) + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
     if (lk.flags & (CFL_LAKE | CFL_RES)) {
 #pragma unroll
-      for (int k = kPrefixPairs; k < CF_USE / 2; k++) at(X.crec + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
+      for (int k = kPrefixPairs; k < CF_USE / 2; k++) at(X.crec + o * (WG_DEV_NREC / 2) + int64_t(k) * n, p) = WgD2{w[2 * k], w[2 * k + 1]};
     }
-    if (kUse) at(X.crec + int64_t(CF_USE / 2) * n, p) = WgD2{w[CF_USE], w[CF_A_NUG]};
+    if (kUse) at(X.crec + o * (WG_DEV_NREC / 2) + int64_t(CF_USE / 2) * n, p) = WgD2{w[CF_USE], w[CF_A_NUG]};
   }
 }
 
@@ -1101,8 +1076,6 @@ __global__ __launch_bounds__(256) void wg_chain_flow_kernel(WgStatic S, WgState 
   const int depth = l1 - l0;
   const int gs = group_level_off[l0], ge = group_level_off[l1];
   const int lvl0_end = group_level_off[l0 + 1];
-  WgState Xm = X;
-  member_rows(Xm, m, n);
   const int64_t base = int64_t(m) * n;
   for (int i = tid; i <= depth; i += nt) s_lo[i] = group_level_off[l0 + i];
   volatile unsigned long long *vtv = reinterpret_cast<volatile unsigned long long *>(s_tv);
@@ -1152,7 +1125,7 @@ __global__ __launch_bounds__(256) void wg_chain_flow_kernel(WgStatic S, WgState 
       slot_record(cur, c);
       const ChainOut o = chain_step<kUse>(c, up, d);
       vtv[p - gs] = __double_as_longlong(o.tv);
-      store_chain(Xm, p, cur.flags, o);
+      store_chain(X, base, p, cur.flags, o);
       qq = (cur.flags & CFL_LDD) ? o.tv : 0.;
     }
     if (cur.station >= 0)
@@ -1193,8 +1166,7 @@ __global__ void wg_pot_runoff_kernel(WgStatic S, WgState X, int32_t p0, int32_t 
   const int p = p0 + int(blockIdx.x * blockDim.x + threadIdx.x);
   if (p >= p1) return;
   if (!(S.cflags[p] & CFL_CONT)) return;
-  member_rows(X, blockIdx.y, S.n);
-  add_pot_runoff(S, X, p);
+  add_pot_runoff(S, X, int64_t(blockIdx.y) * S.n, p);
 }
 
 // Sets the day clock read by the kernels of a captured block of days; launched

@@ -62,6 +62,36 @@ __constant__ static const double wg_exp2_tab_d[128] = {WG_EXP2_TAB_VALUES};
 #define WG_EXP2_TAB wg_exp2_tab_h
 #endif
 
+/* Coefficients of exp and log.  On the device each call reads them from constant
+ * memory through a pointer the compiler cannot see through: written as literals,
+ * the ten powers of a cell's day share them, which keeps all of them in scalar
+ * registers for the whole day and spills them lane by lane. */
+#define WG_COEF_VALUES                                                                                    \
+  WG_INV_LN2_64, WG_LN2_64_1, WG_LN2_64_2, WG_LN2_64_3, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0, 1.0 / 720.0, \
+      1.0 / 5040.0, 1.0 / 40320.0, WG_LN2_HI, 1.0 / 3.0, 1.0 / 5.0, 1.0 / 7.0, 1.0 / 9.0, 1.0 / 11.0,    \
+      1.0 / 13.0, 1.0 / 15.0
+enum {
+  WG_C_INV, WG_C_L1, WG_C_L2, WG_C_L3, WG_C_E3, WG_C_E4, WG_C_E5, WG_C_E6, WG_C_E7, WG_C_E8, WG_C_LN2,
+  WG_C_A3, WG_C_A5, WG_C_A7, WG_C_A9, WG_C_A11, WG_C_A13, WG_C_A15, WG_C_COUNT
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+__constant__ static const double wg_coef_d[WG_C_COUNT] = {WG_COEF_VALUES};
+typedef const __attribute__((address_space(4))) double *wg_coef_ptr;
+#else
+static const double wg_coef_h[WG_C_COUNT] = {WG_COEF_VALUES};
+typedef const double *wg_coef_ptr;
+#endif
+
+WG_FN wg_coef_ptr wg_coef(void) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  wg_coef_ptr c = (wg_coef_ptr)wg_coef_d;
+  asm volatile("" : "+s"(c));
+  return c;
+#else
+  return wg_coef_h;
+#endif
+}
+
 typedef struct wg_dd {
   double hi, lo;
 } wg_dd;
@@ -91,20 +121,20 @@ WG_FN wg_dd wg_two_prod(double a, double b) {
 }
 
 /* e^(xh + xl) as a double-double; xh in [-745.2, 709.8], |xl| <= ulp(xh). */
-WG_FN wg_dd wg_exp_dd(double xh, double xl) {
-  const double kk = WG_FLOOR(xh * WG_INV_LN2_64 + 0.5);
+WG_FN wg_dd wg_exp_dd(double xh, double xl, wg_coef_ptr co) {
+  const double kk = WG_FLOOR(xh * co[WG_C_INV] + 0.5);
   const int ik = (int)kk;
   const int j = ik & 63;
   const int k = (ik - j) / 64;
-  const double r1 = xh - kk * WG_LN2_64_1; /* exact: kk has < 18 bits, the constant 36 */
-  wg_dd a = wg_two_sum(r1, -(kk * WG_LN2_64_2));
-  const double rl = a.lo + (xl - kk * WG_LN2_64_3);
+  const double r1 = xh - kk * co[WG_C_L1]; /* exact: kk has < 18 bits, the constant 36 */
+  wg_dd a = wg_two_sum(r1, -(kk * co[WG_C_L2]));
+  const double rl = a.lo + (xl - kk * co[WG_C_L3]);
   wg_dd r = wg_fast_two_sum(a.hi, rl);
   const double rh = r.hi;
   const double q =
       rh * rh *
-      (0.5 + rh * (1.0 / 6.0 + rh * (1.0 / 24.0 + rh * (1.0 / 120.0 + rh * (1.0 / 720.0 +
-                                                                             rh * (1.0 / 5040.0 + rh * (1.0 / 40320.0)))))));
+      (0.5 + rh * (co[WG_C_E3] + rh * (co[WG_C_E4] + rh * (co[WG_C_E5] + rh * (co[WG_C_E6] +
+                                                                             rh * (co[WG_C_E7] + rh * (co[WG_C_E8])))))));
   wg_dd p = wg_fast_two_sum(rh, r.lo + q);
   const double th = WG_EXP2_TAB[2 * j], tl = WG_EXP2_TAB[2 * j + 1];
   wg_dd tp = wg_two_prod(th, p.hi);
@@ -120,12 +150,12 @@ WG_FN double wg_exp(double x) {
   if (x != x) return x;
   if (x > 709.782712893384) return 1.0 / 0.0;
   if (x < -745.1332191019412) return 0.0;
-  wg_dd r = wg_exp_dd(x, 0.0);
+  wg_dd r = wg_exp_dd(x, 0.0, wg_coef());
   return r.hi + r.lo;
 }
 
 /* log(x) as a double-double for finite x > 0. */
-WG_FN wg_dd wg_log_dd(double x) {
+WG_FN wg_dd wg_log_dd(double x, wg_coef_ptr co) {
   int e;
   double m = WG_FREXP(x, &e);
   if (m < 0.70710678118654752) {
@@ -135,11 +165,11 @@ WG_FN wg_dd wg_log_dd(double x) {
   const double s = (m - 1.0) / (m + 1.0);
   const double s2 = s * s;
   const double y0 =
-      e * WG_LN2_HI +
+      e * co[WG_C_LN2] +
       2.0 * s *
-          (1.0 + s2 * (1.0 / 3.0 + s2 * (1.0 / 5.0 + s2 * (1.0 / 7.0 + s2 * (1.0 / 9.0 + s2 * (1.0 / 11.0 +
-                                                                                              s2 * (1.0 / 13.0 + s2 * (1.0 / 15.0))))))));
-  wg_dd E = wg_exp_dd(-y0, 0.0);
+          (1.0 + s2 * (co[WG_C_A3] + s2 * (co[WG_C_A5] + s2 * (co[WG_C_A7] + s2 * (co[WG_C_A9] + s2 * (co[WG_C_A11] +
+                                                                                              s2 * (co[WG_C_A13] + s2 * (co[WG_C_A15]))))))));
+  wg_dd E = wg_exp_dd(-y0, 0.0, co);
   const double t = WG_FMA(x, E.hi, -1.0) + x * E.lo;
   return wg_fast_two_sum(y0, t - 0.5 * t * t);
 }
@@ -149,7 +179,7 @@ WG_FN double wg_log(double x) {
   if (x == 0.0) return -1.0 / 0.0;
   if (x == 1.0 / 0.0) return x;
   if (x == 1.0) return 0.0;
-  wg_dd l = wg_log_dd(x);
+  wg_dd l = wg_log_dd(x, wg_coef());
   return l.hi + l.lo;
 }
 
@@ -168,12 +198,13 @@ WG_FN double wg_pow(double x, double y) {
   }
   if (x == 0.0) return y > 0.0 ? 0.0 : sign / 0.0;
   if (x == 1.0 / 0.0) return y > 0.0 ? sign * x : 0.0;
-  wg_dd l = wg_log_dd(x);
+  const wg_coef_ptr co = wg_coef();
+  wg_dd l = wg_log_dd(x, co);
   wg_dd z = wg_two_prod(y, l.hi);
   z = wg_fast_two_sum(z.hi, z.lo + y * l.lo);
   if (z.hi > 709.782712893384) return sign / 0.0;
   if (z.hi < -745.1332191019412) return sign * 0.0;
-  wg_dd r = wg_exp_dd(z.hi, z.lo);
+  wg_dd r = wg_exp_dd(z.hi, z.lo, co);
   return sign * (r.hi + r.lo);
 }
 
