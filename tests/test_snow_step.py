@@ -99,8 +99,9 @@ int main(int argc, char **argv) {
     deep += acc.thresh != 0;
     odd += kind >= 0.9;
     const ElevRange er{int16_t(lo), int16_t(hi), int16_t(first)};
-    if (it & 1) day_snow<5>(a, s, v, laf_prev, er, sub, elev, 0, 1);
-    else day_snow<10>(a, s, v, laf_prev, er, sub, elev, 0, 1);
+    if (it % 3 == 0) day_snow<5, true>(a, s, v, laf_prev, er, sub, elev, 0, 1);
+    else if (it % 3 == 1) day_snow<5, false>(a, s, v, laf_prev, er, sub, elev, 0, 1);
+    else day_snow<10, false>(a, s, v, laf_prev, er, sub, elev, 0, 1);
     bool ok = same(s.snow, acc.snow_sum / 100.) && same(v.eff_prec, acc.eff / 100.) &&
               same(v.snow_evapo, acc.evapo / 100.) && same(v.land_change, 0. + acc.change / 100.) &&
               same(v.temp_elev_max, acc.temp_max) && s.snow_any == any;

@@ -692,19 +692,23 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
   return WG_E_NOMEM;
 }
 
-// Chooses the wavefronts of a launch of `days` days: more levels per wavefront cost
-// each day a pass per level in the deepest-packed wavefront, fewer cost a hand over
-// between wavefronts per level once per launch.  Only plans whose wavefronts all
-// fit on the chip at once are taken: with more of them a day costs each its share
-// of the chip, and one launch per day and part, which keeps three wavefronts per
-// SIMD, was faster (64 members of the global grid: 1.99 ms a day against 2.6).
-// Calls of few days stay with it too: the hand overs along the deepest basin are
-// paid once per launch (one day of the global grid: 359 us a call against 502).
+// Chooses the wavefronts of a launch of `days` days.  While they all fit on the chip
+// at once, more levels per wavefront cost each day a pass of the routing step per
+// level, fewer cost a hand over between wavefronts per level once per launch (us,
+// measured on grids of 56, 104 and 352 levels).  With more wavefronts than fit, all
+// of them cost chip time, and eight levels per wavefront is nearly the least (64
+// members of the global grid: 1.21 ms a day against 1.32 with one level).
+// Calls of fewer than kManyDaysMin days run one launch per day and part: there the
+// hand overs along the deepest basin, paid once per launch, outweigh the rest.  Per
+// day, that path against this one:    1 day       2 days      3 days      6 days
+//   global grid, 104 levels (us)    189 / 311   143 / 176   132 / 130   120 / 84
+//   2,000 cells, 56 levels          102 / 122    89 / 78     84 / 63     78 / 47
+//   global grid, 352 levels         305 / 533   276 / 291   263 / 211   246 / 127
 // The chosen table is built by the first call that needs it and kept.  Returns NULL
-// when no plan fits or the memory for its tables is not there.
-constexpr int32_t kManyDaysMin = 8;
+// when the memory for it is not there.
+constexpr int32_t kManyDaysMin = 3;
 const WgDayTable *day_table(wg_handle *h, int32_t days) {
-  constexpr double kHandOver = 2.5, kPass = 0.7;  // us
+  constexpr double kHandOver = 1.2, kPass = 1.1;
   if (days < kManyDaysMin || h->day_capacity <= 0) return nullptr;
   if (h->day_level_cells.empty()) {
     h->day_level_cells.assign(size_t(h->max_depth), 0);
@@ -715,13 +719,13 @@ const WgDayTable *day_table(wg_handle *h, int32_t days) {
   for (int32_t span : {1, 2, 4, 8, 16, 64}) {
     const DayPlan d = day_plan(h->day_level_cells, span);
     if (int64_t(d.n_waves) * h->m > h->day_capacity) continue;
-    const double c = kHandOver * h->max_depth / span + kPass * (double(days) * (d.max_levels - 1) + h->max_depth);
+    const double c = kHandOver * h->max_depth / span + kPass * double(days) * (d.max_levels - 1);
     if (!best.span || c < cost) {
       best = d;
       cost = c;
     }
   }
-  if (!best.span) return nullptr;
+  if (!best.span) best = day_plan(h->day_level_cells, 8);
   auto it = h->day_tables.find(best.span);
   if (it == h->day_tables.end()) {
     WgDayTable t;
@@ -1105,14 +1109,18 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
       }
     }
     {
+      const int waves = M > 1 ? 2 : 1;
       int per_cu = 0, cus = 0, lds_cu = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wg_days_kernel<false>, 64, kDaysLdsBytes) ==
-              hipSuccess &&
+      const hipError_t q = waves == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wg_days_kernel<false, 2>,
+                                                                                    128, days_lds_bytes(2))
+                                      : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wg_days_kernel<false, 1>,
+                                                                                    64, days_lds_bytes(1));
+      if (q == hipSuccess &&
           hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, H->device) ==
               hipSuccess &&
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, H->device) == hipSuccess) {
-        constexpr int kGiven = (kDaysLdsBytes + kLdsStep - 1) / kLdsStep * kLdsStep;
-        H->day_capacity = int64_t(std::min(per_cu, lds_cu / kGiven)) * cus;
+        const int given = (days_lds_bytes(waves) + kLdsStep - 1) / kLdsStep * kLdsStep;
+        H->day_capacity = int64_t(std::min(per_cu, lds_cu / given)) * waves * cus;
       }
     }
     // the largest upstream count of each level
@@ -1645,12 +1653,15 @@ bool ensure_ring(wg_handle *h, int32_t days) {
 int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int days) {
   for (int done = 0; done < days;) {
     const int k = std::min(days - done, h->ring_slots);
-    auto *kern = h->S.use_on ? wg_days_kernel<true> : wg_days_kernel<false>;
+    const int waves = h->m > 1 ? 2 : 1;  // members of a workgroup
+    auto *kern = waves == 2 ? (h->S.use_on ? wg_days_kernel<true, 2> : wg_days_kernel<false, 2>)
+                            : (h->S.use_on ? wg_days_kernel<true, 1> : wg_days_kernel<false, 1>);
     const DaysArgs args{h->S, h->X, h->T, h->d_forcing, t.waves, t.slots, t.ranks, h->d_ring, day + done,
                         h->ring_slots, int32_t(h->ring_day % h->ring_slots),
                         int32_t(h->ring_day / h->ring_slots % 2), (doy - 1 + done) % 365 + 1,
                         (h->started || done > 0) ? 1 : 0, k, done};
-    hipLaunchKernelGGL(kern, dim3(t.n_waves, h->m), dim3(64), kDaysLdsBytes, h->stream, args);
+    hipLaunchKernelGGL(kern, dim3(t.n_waves, (h->m + waves - 1) / waves), dim3(64 * waves), days_lds_bytes(waves),
+                       h->stream, args);
     HIP_CHECK(h, hipGetLastError());
     h->ring_day += k;
     done += k;

@@ -446,7 +446,9 @@ __device__ __forceinline__ double snow_subcell_fast(double q, double temp_elev, 
 // stepped, so that a wavefront keeps many 16-byte loads in flight.  sub, elev: the member's pairs [k][n], cell p.
 // What bounds it is VALU issue: a sub-cell is 38 instructions (61 before the minima
 // and maxima of snow_subcell_fast), a bare one 2 additions' share.
-template <int kSnowChunk>
+// kTwo: two load buffers, a chunk's loads out for the whole step of the chunk before
+// (25 registers more); else one, refilled when its storages are rescaled.
+template <int kSnowChunk, bool kTwo>
 __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlux &v, double laf_prev,
                                          const ElevRange &er, WgD2 *sub, const int32_t *elev, uint32_t p, int n) {
   auto sp = [&](int k) -> WgD2 & { return at(sub + int64_t(k) * n, p); };
@@ -492,23 +494,22 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
   } else {
     // snow_subcell_fast needs a number for the precipitation and a melt factor >= 0
     const bool usual = sd.melt_ok && sd.prec_to_soil == sd.prec_to_soil;
-    WgD2 in[kSnowChunk];
-    int32_t en[kSnowChunk];
+    WgD2 ia[kSnowChunk], ib[kSnowChunk];
+    int32_t ea[kSnowChunk], eb[kSnowChunk];
+    auto fetch = [&](int c, WgD2 *in, int32_t *en) {
 #pragma unroll
-    for (int j = 0; j < kSnowChunk; j++) {
-      in[j] = snow_any ? sp(j) : WgD2{0., 0.};
-      en[j] = ep(j);
-    }
-#pragma unroll 1
-    for (int c = 0; c < WG_DEV_NPAIR / kSnowChunk; c++) {
+      for (int j = 0; j < kSnowChunk; j++) {
+        in[j] = snow_any ? sp(c * kSnowChunk + j) : WgD2{0., 0.};
+        en[j] = ep(c * kSnowChunk + j);
+      }
+    };
+    auto rescale = [&](const WgD2 *in, WgD2 *q) -> uint32_t {
       // The land-area rescaling s * scale_num / laf with the reused reciprocal:
       // q0 = x (1/laf), one exact residual and one correction give the correctly
       // rounded quotient (as in snow_subcell).  Storages in [0, 1000) mm, by the
       // high word of q, are the usual case; larger finite ones take the step with
       // the threshold elevation, anything else (negative, NaN, infinite, -0, or
       // not `usual`) the general step.
-      WgD2 q[kSnowChunk];
-      int32_t e2[kSnowChunk];
       uint32_t top = usual ? 0u : 0xffffffffu;
 #pragma unroll
       for (int j = 0; j < kSnowChunk; j++) {
@@ -517,16 +518,10 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
         q[j].x = fma(fma(-rx, sd.laf, x0), sd.inv_laf, rx);
         q[j].y = fma(fma(-ry, sd.laf, y0), sd.inv_laf, ry);
         top = max(top, max(uint32_t(__double2hiint(q[j].x)), uint32_t(__double2hiint(q[j].y))));
-        e2[j] = en[j];
       }
-      // the next chunk's loads fly while this chunk is stepped
-      if (c + 1 < WG_DEV_NPAIR / kSnowChunk) {
-#pragma unroll
-        for (int j = 0; j < kSnowChunk; j++) {
-          in[j] = snow_any ? sp((c + 1) * kSnowChunk + j) : WgD2{0., 0.};
-          en[j] = ep((c + 1) * kSnowChunk + j);
-        }
-      }
+      return top;
+    };
+    auto finish = [&](int c, WgD2 *q, const int32_t *en, uint32_t top) {
       if (__builtin_amdgcn_ballot_w64(top >= 0x7ff00000u) != 0) {
 #pragma unroll 1
         for (int j = 0; j < kSnowChunk; j++) {
@@ -540,31 +535,52 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
           any_after |= nz;
           if (snow_any || nz) sp(c * kSnowChunk + j) = w;
         }
-      } else {
-        const bool thresh = __builtin_amdgcn_ballot_w64(top >= 0x408f4000u) != 0;
-        if (thresh) {
-#pragma unroll
-          for (int j = 0; j < kSnowChunk; j++) {
-            const int e0 = int(int16_t(e2[j] & 0xffff)), e1 = int(int16_t(e2[j] >> 16));
-            q[j].x = snow_subcell_fast<true>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0,
-                                             sd, acc);
-            q[j].y = snow_subcell_fast<true>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < kSnowChunk; j++) {
-            const int e0 = int(int16_t(e2[j] & 0xffff)), e1 = int(int16_t(e2[j] >> 16));
-            q[j].x = snow_subcell_fast<false>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0,
-                                              sd, acc);
-            q[j].y = snow_subcell_fast<false>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
-          }
-        }
+        return;
+      }
+      if (__builtin_amdgcn_ballot_w64(top >= 0x408f4000u) != 0) {
 #pragma unroll
         for (int j = 0; j < kSnowChunk; j++) {
-          const bool nz = q[j].x != 0. || q[j].y != 0.;
-          any_after |= nz;
-          if (snow_any || nz) sp(c * kSnowChunk + j) = q[j];
+          const int e0 = int(int16_t(en[j] & 0xffff)), e1 = int(int16_t(en[j] >> 16));
+          q[j].x = snow_subcell_fast<true>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0, sd,
+                                           acc);
+          q[j].y = snow_subcell_fast<true>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
         }
+      } else {
+#pragma unroll
+        for (int j = 0; j < kSnowChunk; j++) {
+          const int e0 = int(int16_t(en[j] & 0xffff)), e1 = int(int16_t(en[j] >> 16));
+          q[j].x = snow_subcell_fast<false>(q[j].x, sd.tempC - ((e0 - sd.elev0) * sd.gradnt), e0, c == 0 && j == 0,
+                                            sd, acc);
+          q[j].y = snow_subcell_fast<false>(q[j].y, sd.tempC - ((e1 - sd.elev0) * sd.gradnt), e1, false, sd, acc);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kSnowChunk; j++) {
+        const bool nz = q[j].x != 0. || q[j].y != 0.;
+        any_after |= nz;
+        if (snow_any || nz) sp(c * kSnowChunk + j) = q[j];
+      }
+    };
+    constexpr int kChunks = WG_DEV_NPAIR / kSnowChunk;
+    WgD2 q[kSnowChunk];
+    fetch(0, ia, ea);
+    if (kTwo) {
+      static_assert(!kTwo || kChunks % 2 == 0, "chunks in pairs");
+#pragma unroll 1
+      for (int c = 0; c < kChunks; c += 2) {
+        fetch(c + 1, ib, eb);
+        finish(c, q, ea, rescale(ia, q));
+        if (c + 2 < kChunks) fetch(c + 2, ia, ea);
+        finish(c + 1, q, eb, rescale(ib, q));
+      }
+    } else {
+#pragma unroll 1
+      for (int c = 0; c < kChunks; c++) {
+        const uint32_t top = rescale(ia, q);
+#pragma unroll
+        for (int j = 0; j < kSnowChunk; j++) eb[j] = ea[j];
+        if (c + 1 < kChunks) fetch(c + 1, ia, ea);
+        finish(c, q, eb, top);
       }
     }
   }

@@ -34,23 +34,33 @@ namespace {
 // because this compiler can place a spill's store before the point where a branch's
 // lanes rejoin.
 enum DayField : int {
+  // the same for every member
   DF_M_PREC, DF_ALPHA, DF_PET_MXDY, DF_M_NETRAD, DF_MCWH, DF_SNOWFZ, DF_SNOWMT, DF_GRADNT, DF_MELT, DF_ALBEDO,
-  DF_ALBEDO_SNOW, DF_EMIS, DF_LAI, DF_CLASS, DF_SMAX, DF_GWF, DF_GAMMA, DF_CFA, DF_PCRIT, DF_AREA,
-  DF_AREA_M, DF_CF100, DF_FSWB, DF_E_GW, DF_INV_KGW, DF_OME_GW, DF_E_SW, DF_K_SW, DF_INV_KSW, DF_OME_SW,
-  DF_RED_EXP, DF_LL, DF_LL100, DF_LL_MAX, DF_LW, DF_LW100, DF_LW_MAX, DF_GW, DF_GW_MAX, DF_LENGTH,
-  DF_BOTTOM, DF_VEL_C1, DF_VEL_C2, DF_RW_C0, DF_RW_C1, DF_RW_C2, DF_RW_C3, DF_RIVER_MAX, DF_MAX_RAF,
-  // state that a day reads once or few cells have
-  DF_LAI_PREC, DF_TRANSFER, DF_GLO_LAKE, DF_RES, DF_K_RELEASE, DF_RED_GL, DF_RED_RES, DF_RED_RIVER, DF_FRAC_CHANGE,
+  DF_ALBEDO_SNOW, DF_EMIS, DF_LAI, DF_CLASS, DF_GWF, DF_PCRIT, DF_AREA, DF_AREA_M, DF_CF100, DF_FSWB, DF_E_GW,
+  DF_INV_KGW, DF_OME_GW, DF_E_SW, DF_K_SW, DF_INV_KSW, DF_OME_SW, DF_RED_EXP, DF_LL, DF_LL100, DF_LL_MAX, DF_LW,
+  DF_LW100, DF_LW_MAX, DF_GW, DF_GW_MAX, DF_LENGTH, DF_BOTTOM, DF_VEL_C1, DF_VEL_C2, DF_RW_C0, DF_RW_C1, DF_RW_C2,
+  DF_RW_C3, DF_RIVER_MAX, DF_MAX_RAF,
   DF_NEAR,  // WgDaySlot's near_lo and near_hi
-  DF_TV,    // the day's transported volumes of the wavefront's cells
+  DF_SHARED,
+  // a member's own: parameters, and state that a day reads once or few cells have
+  DF_SMAX = DF_SHARED, DF_GAMMA, DF_CFA, DF_LAI_PREC, DF_TRANSFER, DF_GLO_LAKE, DF_RES, DF_K_RELEASE, DF_RED_GL,
+  DF_RED_RES, DF_RED_RIVER, DF_FRAC_CHANGE,
+  DF_TV,  // the day's transported volumes of the wavefront's cells
   DF_ROWS
 };
-constexpr int kDaysLdsBytes = WG_EXP2_LDS_BYTES + DF_ROWS * 64 * int(sizeof(double));
-// LDS is given out in steps of 1,280 bytes: 25 of them, so that a CU's 160 KB hold the
-// rows of five wavefronts (with 32,768 bytes only four started, whatever the occupancy
-// query says, and the rest of the grid waited for whole launches)
+// A workgroup is one wavefront, or two that hold the same cells of two members and
+// share the members' common rows (both write them, with the same values).
+constexpr int days_lds_bytes(int waves) {
+  return waves * WG_EXP2_LDS_BYTES + (DF_SHARED + waves * (DF_ROWS - DF_SHARED)) * 64 * int(sizeof(double));
+}
+// LDS is given out in steps of 1,280 bytes.  One wavefront's rows take 25 of them, so
+// that a CU's 160 KB hold five (with 32,768 bytes only four started, whatever the
+// occupancy query says, and the rest of the grid waited for whole launches); two
+// members' take 32, so that they hold four workgroups, the eight wavefronts that the
+// registers allow.
 constexpr int kLdsStep = 1280;
-static_assert(kDaysLdsBytes <= 25 * kLdsStep, "five wavefronts per CU");
+static_assert(days_lds_bytes(1) <= 25 * kLdsStep, "five wavefronts per CU");
+static_assert(days_lds_bytes(2) <= 32 * kLdsStep, "four workgroups of two wavefronts per CU");
 
 // bits of DF_GWF's second word, whose upper half holds G_Rgmax
 enum { DB_ARID = 1, DB_CUT = 2, DB_LDD = 4, DB_CONT = 8, DB_LAKE = 16, DB_RES = 32, DB_FULL_LAKE = 64 };
@@ -60,6 +70,7 @@ struct WordPair {
 };
 
 constexpr int kDaysSpinLimit = 1 << 22;
+constexpr int kEarly = 3;  // upstream cells whose volumes are loaded ahead (few cells have more)
 
 }  // namespace
 
@@ -95,6 +106,13 @@ namespace {
 __device__ __forceinline__ int days_doy(const DaysArgs &A, int k) { return int((A.doy0 - 1 + k) % 365) + 1; }
 __device__ __forceinline__ DayInfo days_info(const DaysArgs &A, int k) { return day_info(days_doy(A, k)); }
 
+// Upstream cell u's volume of the day, as it stands in the ring.
+__device__ __forceinline__ unsigned long long days_volume(unsigned long long *row, int group, const WgChainLink &link,
+                                                          int u) {
+  return __hip_atomic_load(&at(row, uint32_t(group) + uint16_t(link.up[u])), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The member's row of day k in the ring, and the sign bit of its turn.
 __device__ __forceinline__ unsigned long long *days_ring_row(const DaysArgs &A, int k, int64_t o,
                                                              unsigned long long &sign) {
@@ -110,24 +128,28 @@ __device__ __forceinline__ double *days_station_row(const DaysArgs &A, int k, in
 
 }  // namespace
 
-template <bool kUse>
-__global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
+template <bool kUse, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, 2) void wg_days_kernel(DaysArgs) {
   load_exp2_table();
-  const int lane = threadIdx.x;
-  const int m = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = blockIdx.y * kWaves + wave;
   DAYS_ARGS(A0, S0, X0);
+  if (kWaves > 1 && m >= S0.n_members) return;
   const WgDayWave wv = A0.waves[blockIdx.x];
   const WgDaySlot slot = A0.slots[blockIdx.x * 64 + lane];
   if (slot.cell < 0) return;
   const uint32_t p = uint32_t(slot.cell);
   const int n = S0.n;
   const int64_t o = int64_t(m) * n;  // the member's rows
-  double *F = wg_lds + WG_EXP2_LDS_BYTES / sizeof(double) + lane;
-  auto fld = [&](int f) -> double { return F[f * 64]; };
+  double *Fs = wg_lds + kWaves * WG_EXP2_LDS_BYTES / sizeof(double) + lane;
+  double *Fm = Fs + wave * (DF_ROWS - DF_SHARED) * 64;
+  auto row = [&](int f) -> double & { return f < DF_SHARED ? Fs[f * 64] : Fm[f * 64]; };
+  auto fld = [&](int f) -> double { return row(f); };
 
   const WgChainLink link = load_link(S0, p);
   const int rank = A0.ranks[blockIdx.x * 64 + lane];
-  F[DF_NEAR * 64] = __builtin_bit_cast(double, WordPair{int32_t(slot.near_lo), int32_t(slot.near_hi)});
+  row(DF_NEAR) = __builtin_bit_cast(double, WordPair{int32_t(slot.near_lo), int32_t(slot.near_hi)});
   int bits = 0;
   {
     DayStatA a;
@@ -140,58 +162,58 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
     bits = (b.arid ? DB_ARID : 0) | (b.recharge_cut ? DB_CUT : 0) | (b.ldd >= 0 ? DB_LDD : 0) |
            (e.contcell ? DB_CONT : 0) | (e.lake_area > 0. ? DB_LAKE : 0) | (e.reservoir_area > 0. ? DB_RES : 0) |
            (e.f_glo_lake == 1. ? DB_FULL_LAKE : 0) | int(uint32_t(uint16_t(at(S0.rgmax, p))) << 16);
-    F[DF_M_PREC * 64] = a.m_prec;
-    F[DF_ALPHA * 64] = a.alpha;
-    F[DF_PET_MXDY * 64] = a.pet_mxdy;
-    F[DF_M_NETRAD * 64] = a.m_netrad;
-    F[DF_MCWH * 64] = a.mcwh;
-    F[DF_SNOWFZ * 64] = a.t_snowfz;
-    F[DF_SNOWMT * 64] = a.t_snowmt;
-    F[DF_GRADNT * 64] = a.t_gradnt;
-    F[DF_MELT * 64] = a.melt_factor;
-    F[DF_ALBEDO * 64] = a.albedo;
-    F[DF_ALBEDO_SNOW * 64] = a.albedo_snow;
-    F[DF_EMIS * 64] = a.emis;
-    F[DF_LAI * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, float(a.lmin)),
+    row(DF_M_PREC) = a.m_prec;
+    row(DF_ALPHA) = a.alpha;
+    row(DF_PET_MXDY) = a.pet_mxdy;
+    row(DF_M_NETRAD) = a.m_netrad;
+    row(DF_MCWH) = a.mcwh;
+    row(DF_SNOWFZ) = a.t_snowfz;
+    row(DF_SNOWMT) = a.t_snowmt;
+    row(DF_GRADNT) = a.t_gradnt;
+    row(DF_MELT) = a.melt_factor;
+    row(DF_ALBEDO) = a.albedo;
+    row(DF_ALBEDO_SNOW) = a.albedo_snow;
+    row(DF_EMIS) = a.emis;
+    row(DF_LAI) = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, float(a.lmin)),
                                                          __builtin_bit_cast(int32_t, float(a.lmax))});
-    F[DF_CLASS * 64] = __builtin_bit_cast(double, WordPair{a.initial_days, a.lct | (a.elev0 << 8)});
-    F[DF_SMAX * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.smax),
+    row(DF_CLASS) = __builtin_bit_cast(double, WordPair{a.initial_days, a.lct | (a.elev0 << 8)});
+    row(DF_SMAX) = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.smax),
                                                           __builtin_bit_cast(int32_t, b.built_up)});
-    F[DF_GWF * 64] = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.gw_factor), bits});
-    F[DF_GAMMA * 64] = b.gamma;
-    F[DF_CFA * 64] = b.cfa;
-    F[DF_PCRIT * 64] = b.pcritgwa;
-    F[DF_AREA * 64] = b.area;
-    F[DF_AREA_M * 64] = b.area_m;
-    F[DF_CF100 * 64] = b.cf100;
-    F[DF_FSWB * 64] = b.fswb_catchment;
-    F[DF_E_GW * 64] = b.e_gw;
-    F[DF_INV_KGW * 64] = cs.inv_kgw;
-    F[DF_OME_GW * 64] = cs.ome_gw;
-    F[DF_E_SW * 64] = b.e_sw;
-    F[DF_K_SW * 64] = b.k_sw;
-    F[DF_INV_KSW * 64] = cs.inv_ksw;
-    F[DF_OME_SW * 64] = cs.ome_sw;
-    F[DF_RED_EXP * 64] = b.red_exp;
-    F[DF_LL * 64] = b.loc_lake;
-    F[DF_LL100 * 64] = b.ll100;
-    F[DF_LL_MAX * 64] = b.ll_max;
-    F[DF_LW * 64] = b.loc_wetland;
-    F[DF_LW100 * 64] = b.lw100;
-    F[DF_LW_MAX * 64] = b.lw_max;
-    F[DF_GW * 64] = b.glo_wetland;
-    F[DF_GW_MAX * 64] = b.gw_max;
-    F[DF_LENGTH * 64] = b.river_length;
-    F[DF_BOTTOM * 64] = b.bottom;
-    F[DF_VEL_C1 * 64] = b.vel_c1;
-    F[DF_VEL_C2 * 64] = b.vel_c2;
-    F[DF_RW_C0 * 64] = e.rw_c0;
-    F[DF_RW_C1 * 64] = e.rw_c1;
-    F[DF_RW_C2 * 64] = e.rw_c2;
-    F[DF_RW_C3 * 64] = e.rw_c3;
-    F[DF_RIVER_MAX * 64] = e.river_stor_max;
-    F[DF_MAX_RAF * 64] = e.max_raf;
-    F[DF_TV * 64] = 0.;
+    row(DF_GWF) = __builtin_bit_cast(double, WordPair{__builtin_bit_cast(int32_t, b.gw_factor), bits});
+    row(DF_GAMMA) = b.gamma;
+    row(DF_CFA) = b.cfa;
+    row(DF_PCRIT) = b.pcritgwa;
+    row(DF_AREA) = b.area;
+    row(DF_AREA_M) = b.area_m;
+    row(DF_CF100) = b.cf100;
+    row(DF_FSWB) = b.fswb_catchment;
+    row(DF_E_GW) = b.e_gw;
+    row(DF_INV_KGW) = cs.inv_kgw;
+    row(DF_OME_GW) = cs.ome_gw;
+    row(DF_E_SW) = b.e_sw;
+    row(DF_K_SW) = b.k_sw;
+    row(DF_INV_KSW) = cs.inv_ksw;
+    row(DF_OME_SW) = cs.ome_sw;
+    row(DF_RED_EXP) = b.red_exp;
+    row(DF_LL) = b.loc_lake;
+    row(DF_LL100) = b.ll100;
+    row(DF_LL_MAX) = b.ll_max;
+    row(DF_LW) = b.loc_wetland;
+    row(DF_LW100) = b.lw100;
+    row(DF_LW_MAX) = b.lw_max;
+    row(DF_GW) = b.glo_wetland;
+    row(DF_GW_MAX) = b.gw_max;
+    row(DF_LENGTH) = b.river_length;
+    row(DF_BOTTOM) = b.bottom;
+    row(DF_VEL_C1) = b.vel_c1;
+    row(DF_VEL_C2) = b.vel_c2;
+    row(DF_RW_C0) = e.rw_c0;
+    row(DF_RW_C1) = e.rw_c1;
+    row(DF_RW_C2) = e.rw_c2;
+    row(DF_RW_C3) = e.rw_c3;
+    row(DF_RIVER_MAX) = e.river_stor_max;
+    row(DF_MAX_RAF) = e.max_raf;
+    row(DF_TV) = 0.;
   }
   const bool cont = (bits & DB_CONT) != 0;
   // upstream cells: bit u of ext when upstream cell u belongs to an earlier wavefront
@@ -209,15 +231,15 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
   s.laf_prev = at(X0.laf_prev + o, p);
   s.red_gl = at(X0.red_gl + o, p);
   s.red_res = at(X0.red_res + o, p);
-  F[DF_LAI_PREC * 64] = s.lai_precsum;
-  F[DF_TRANSFER * 64] = s.transfer;
-  F[DF_GLO_LAKE * 64] = s.glo_lake;
-  F[DF_RES * 64] = s.res;
-  F[DF_K_RELEASE * 64] = s.k_release;
-  F[DF_RED_GL * 64] = s.red_gl;
-  F[DF_RED_RES * 64] = s.red_res;
-  F[DF_RED_RIVER * 64] = s.red_river;
-  F[DF_FRAC_CHANGE * 64] = s.river_frac_change;
+  row(DF_LAI_PREC) = s.lai_precsum;
+  row(DF_TRANSFER) = s.transfer;
+  row(DF_GLO_LAKE) = s.glo_lake;
+  row(DF_RES) = s.res;
+  row(DF_K_RELEASE) = s.k_release;
+  row(DF_RED_GL) = s.red_gl;
+  row(DF_RED_RES) = s.red_res;
+  row(DF_RED_RIVER) = s.red_river;
+  row(DF_FRAC_CHANGE) = s.river_frac_change;
   const ElevRange er = load_elev_range(S0, p);
   const float *fd = A0.forcing + A0.fday0 * 4 * int64_t(n);
   const int days = A0.days;
@@ -285,13 +307,23 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
         s.lai_precsum = fld(DF_LAI_PREC);
         s.transfer = fld(DF_TRANSFER);
         day_pet_canopy(a, s, v, tf, pf, swf, lwf, laf_prev);
-        F[DF_LAI_PREC * 64] = s.lai_precsum;
+        row(DF_LAI_PREC) = s.lai_precsum;
         DAYS_ARGS(A, S, X);
         WgD2 *sub = X.snow2 + o * WG_DEV_NPAIR;
         if (s.laf <= 0.) day_snow_no_land(s, v, sub, p, n);
-        F[DF_TRANSFER * 64] = s.transfer;
-        if (s.laf > 0.) day_snow<5>(a, s, v, laf_prev, er, sub, S.elev_pairs, p, n);
+        row(DF_TRANSFER) = s.transfer;
+        if (s.laf > 0.) day_snow<5, true>(a, s, v, laf_prev, er, sub, S.elev_pairs, p, n);
       }
+      // Transported volumes of upstream cells in earlier wavefronts: they are there
+      // already unless this wavefront has caught up, so those of the first kEarly
+      // upstream cells are loaded before soil and local routing and looked at after.
+      DAYS_ARGS(A, S, X);
+      unsigned long long sign;
+      unsigned long long *rrow = days_ring_row(A, k, o, sign);
+      unsigned long long t[8];
+#pragma unroll
+      for (int u = 0; u < kEarly; u++)
+        if (u < wv.nu && (ext >> u & 1)) t[u] = days_volume(rrow, slot.group, link, u);
       ChainRec c;
       {
         DayStatB b;
@@ -310,7 +342,7 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
         b.ldd = (bits & DB_LDD) ? 0 : -1;
         s.transfer = fld(DF_TRANSFER);
         day_soil(b, s, v, laf_prev);
-        F[DF_TRANSFER * 64] = s.transfer;
+        row(DF_TRANSFER) = s.transfer;
         if (k == days - 1) {
           DAYS_ARGS(A, S, X);
           at(X.d_surf + o, p) = v.surf_runoff;
@@ -374,20 +406,15 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
           at(X.pot_ow + o, p) = pot.ow;
         }
       }
-      // transported volumes of upstream cells in earlier wavefronts: wait for the
-      // day's values (they are there already unless this wavefront has caught up)
-      DAYS_ARGS(A, S, X);
-      unsigned long long sign;
-      unsigned long long *rrow = days_ring_row(A, k, o, sign);
-      unsigned long long t[8];
+      // wait for the volumes that were not there yet, and load those past the first
+      // kEarly upstream cells
       int spins = 0;
       for (;;) {
         bool ready = true;
 #pragma unroll
         for (int u = 0; u < 8; u++)
           if (u < wv.nu && (ext >> u & 1)) {
-            t[u] = __hip_atomic_load(&at(rrow, uint32_t(slot.group) + uint16_t(link.up[u])), __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
+            if (u >= kEarly || spins > 0) t[u] = days_volume(rrow, slot.group, link, u);
             ready = ready && ((t[u] ^ sign) >> 63) == 0;
           }
         if (__builtin_amdgcn_ballot_w64(!ready) == 0) break;
@@ -411,7 +438,7 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
           for (int u = 0; u < 8; u++)
             if (u < wv.nu) {
               const int near_lane = int(uint32_t(u < 4 ? lanes.a : lanes.b) >> (8 * (u & 3))) & 63;
-              const double near = wg_lds[WG_EXP2_LDS_BYTES / sizeof(double) + DF_TV * 64 + near_lane];
+              const double near = (&row(DF_TV))[near_lane - lane];
               const double far = __builtin_bit_cast(double, t[u] & 0x7fffffffffffffffull);
               const double q = (ext >> u & 1) ? far : near;
               up += (u < link.nu) ? q : 0.;
@@ -424,14 +451,14 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
           }
           const unsigned long long w = __builtin_bit_cast(unsigned long long, r.tv) & 0x7fffffffffffffffull;
           __hip_atomic_store(&at(rrow, p), w | sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          F[DF_TV * 64] = r.tv;
+          row(DF_TV) = r.tv;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
       }
-      if (c.flags & CFL_LAKE) F[DF_GLO_LAKE * 64] = r.glo_lake;
+      if (c.flags & CFL_LAKE) row(DF_GLO_LAKE) = r.glo_lake;
       if (c.flags & CFL_RES) {
-        F[DF_RES * 64] = r.res;
-        F[DF_K_RELEASE * 64] = r.k_release;
+        row(DF_RES) = r.res;
+        row(DF_K_RELEASE) = r.k_release;
       }
       if (c.flags & CFL_GWET) s.glo_wetl = r.glo_wetl;
       if (c.flags & CFL_ARID) s.gw = r.gw;
@@ -488,11 +515,11 @@ __global__ __launch_bounds__(64, 2) void wg_days_kernel(DaysArgs) {
                     days_doy(A, k) == 365);
       }
       day_end(e, s);
-      F[DF_RED_RIVER * 64] = s.red_river;
-      F[DF_FRAC_CHANGE * 64] = s.river_frac_change;
+      row(DF_RED_RIVER) = s.red_river;
+      row(DF_FRAC_CHANGE) = s.river_frac_change;
       if (bits & (DB_LAKE | DB_RES)) {
-        F[DF_RED_GL * 64] = s.red_gl;
-        F[DF_RED_RES * 64] = s.red_res;
+        row(DF_RED_GL) = s.red_gl;
+        row(DF_RED_RES) = s.red_res;
       }
     }
   }

@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256, kSnowChunk == 5 ? 3 : 1) void wg_cell_kernel(W
   if (s.laf <= 0.)
     day_snow_no_land(s, v, X.snow2 + o * WG_DEV_NPAIR, p, n);
   else
-    day_snow<kSnowChunk>(sa, s, v, laf_prev, er, X.snow2 + o * WG_DEV_NPAIR, S.elev_pairs, p, n);
+    day_snow<kSnowChunk, false>(sa, s, v, laf_prev, er, X.snow2 + o * WG_DEV_NPAIR, S.elev_pairs, p, n);
   at(X.snow_any + o, p) = s.snow_any ? 1 : 0;
   DayStatB sb;
   DayStatLake lake;
