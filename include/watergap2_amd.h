@@ -656,11 +656,9 @@ int wg_mlp_forward(wg_mlp *h, int32_t rows, const float *x, float *y);
  * under HIP graph capture, tight proposal loops).  No counterpart in the
  * reference.  x [rows][16] and y [rows] are device pointers on the handle's
  * device; the work is queued on `stream` (a hipStream_t of that device; NULL: the
- * handle's own stream) and not waited for.  The activations live in one static
- * scratch array per GPU of WG_MLP_NOALLOC_MAX_ROWS rows (6.5 MiB, held until the
- * process ends): 1 <= rows <= WG_MLP_NOALLOC_MAX_ROWS, else WG_E_ARG.  Every call
- * on a GPU shares that array, so calls that overlap on one GPU (other streams,
- * other handles) race.  Results are wg_mlp_forward's bits. */
+ * handle's own stream) and not waited for.  1 <= rows <= WG_MLP_NOALLOC_MAX_ROWS,
+ * else WG_E_ARG.  The activations live in the kernel's LDS and registers, so calls
+ * on other streams or handles may overlap.  Results are wg_mlp_forward's bits. */
 #define WG_MLP_NOALLOC_MAX_ROWS 8192
 int wg_mlp_forward_noalloc(wg_mlp *h, int32_t rows, const float *x, float *y, void *stream);
 /* Mean-squared-error loss and its gradient (flat, like the parameters) over rows. */

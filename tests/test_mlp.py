@@ -83,3 +83,33 @@ def test_gpu_training_fits_a_smooth_function(wg):
     assert losses[-1] < 0.05 * losses[0], losses
     y = net.forward(x[:512])
     assert float(np.mean((y - t[:512]) ** 2)) < 0.05 * float(np.var(t))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 1024, 1025, 2080, 8200])
+def test_gpu_row_tiles_and_sum_chunks(wg, rows):
+    """Sizes at the edges of the 16-row tiles and of the 1,024-row chunks of the sums
+    over rows: each row's output is the one it has alone, and loss and gradient are
+    the oracle's with the same BF16 rounding.  What is left between them is the FP32
+    accumulation and operands that it moves across a BF16 step, 2^-9 of a value: the
+    bounds of the 200-row test above."""
+    print("case: MLP rows", rows, flush=True)
+    from watergap2_amd.surrogate import MLP
+    net = MLP(seed=3)
+    p = small_net(6).astype(np.float32)
+    net.set_params(p)
+    rng = np.random.default_rng(rows)
+    x = rng.normal(size=(rows, mo.NIN)).astype(np.float32)
+    t = rng.normal(size=rows).astype(np.float32)
+    y = net.forward(x)
+    for r in {0, rows // 2, rows - 1}:
+        assert net.forward(x[r:r + 1])[0] == y[r], r
+    loss, g = net.gradient(x, t)
+    loss_ref, g_ref = mo.loss_and_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), bf=True)
+    assert abs(loss - loss_ref) <= 2e-3 * loss_ref
+    o = 0
+    for name, shape in mo.SIZES:
+        n = int(np.prod(shape))
+        e = rel_err(g[o:o + n], g_ref[o:o + n])
+        assert e < 2e-2, (name, e)
+        o += n

@@ -1,5 +1,5 @@
-"""wg_mlp_forward_noalloc (activations in the library's static scratch array)
-against wg_mlp_forward, through the C ABI: bit-identical outputs on two calls in
+"""wg_mlp_forward_noalloc (one kernel, activations in LDS and registers) against
+wg_mlp_forward, through the C ABI: bit-identical outputs on two calls in
 a row, the second with fewer rows, on a caller's stream and on the handle's own,
 nothing written past the last row, and sizes outside 1..WG_MLP_NOALLOC_MAX_ROWS
 refused without device work.  Device buffers and the stream come from the HIP
@@ -82,7 +82,7 @@ def test_forward_noalloc_matches_forward(wg):
             assert np.array_equal(y[:rows].view(np.uint32), y_ref.view(np.uint32))
             assert np.isnan(y[rows:]).all()  # nothing past the last row
             hip.free()
-        # sizes beyond the scratch array, or empty, are refused before any launch
+        # sizes beyond the entry point's limit, or empty, are refused before any launch
         for bad in (MAX_ROWS + 1, 0, -5):
             assert lib.wg_mlp_forward_noalloc(h, bad, C.c_void_p(16), C.c_void_p(16), stream) == WG_E_ARG
         assert b"rows must be 1..8192" in lib.wg_mlp_last_error(h)

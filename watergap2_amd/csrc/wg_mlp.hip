@@ -9,17 +9,23 @@
 //
 // All GEMMs are C[M][N] = sum_k A[m][k] * Bt[n][k] with both operands K-contiguous
 // BF16, on v_mfma_f32_16x16x32_bf16 (lane l: A row l%16 and B column l%16 with
-// k = (l/16)*8 .. +7; C column l%16, rows (l/16)*4 .. +3).  The backward pass
-// uses transposed copies written by the producing epilogues, so every operand
-// load is one 16-byte vector load.
+// k = (l/16)*8 .. +7; C column l%16, rows (l/16)*4 .. +3), accumulated in K order.
+//
+// A training step is two launches.  mlp_rows takes 16 batch rows per workgroup through
+// all layers and back, activations and deltas in LDS and registers; what the weight
+// gradients need goes to memory transposed ([unit][row]), so that every operand of
+// mlp_update, which forms the gradients and applies Adam, is K-contiguous too.  The
+// sums over rows (biases, output weights, loss) keep row order: mlp_update stages
+// their terms in LDS and adds them serially, one lane a sum.  (One launch per layer
+// and sum, the sums read from memory term by term, took 1,080 us a batch of 1,024.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
-#include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/watergap2_amd.h"
@@ -50,163 +56,310 @@ __device__ inline float gelu_grad(float z) {
   return 0.5f * (1.f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-struct Epilogue {
-  int mode;           // 0: C; 1: hidden forward; 2: delta of the previous layer
-  float *out_f32;     // mode 0: C; 1: z (may be null: forward only); 2: dz
-  const float *bias;  // mode 1
-  const float *zprev; // mode 2: pre-activation whose GELU derivative scales C
-  bf16 *out_b;        // modes 1, 2: bf16 [M][N]
-  bf16 *out_bt;       // modes 1, 2: bf16 [N][M] (mode 1: may be null)
+// Buffers of one batch of R rows (a multiple of 32), n of them valid, the rest zero
+// features and no loss; rows of xs and ts through idx, or in order when idx is NULL.
+struct RowBatch {
+  const float *xs, *ts;
+  const int32_t *idx;
+  int n, R;
+  bf16 *xt;           // [16][R] features
+  bf16 *ht[3];        // [128][R] hidden activations
+  bf16 *dt[3];        // [128][R] deltas
+  float *et[3];       // [128][R] deltas in FP32
+  float *y, *dy, *sq; // [R] output, its loss gradient, squared error
 };
 
-// One wavefront per 32 x 32 tile of C (2 x 2 MFMA blocks); M, N, K multiples of 32.
-__global__ __launch_bounds__(64) void mlp_gemm(const bf16 *__restrict__ A, const bf16 *__restrict__ Bt, int M,
-                                               int N, int K, Epilogue ep) {
-  const int l = threadIdx.x;
-  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  if (m0 >= M || n0 >= N) return;
-  f32x4 acc[2][2];
+// BF16 weights for mlp_rows and mlp_update, and the FP32 master parameters.
+struct Weights {
+  float *p;
+  bf16 *w1, *w1t, *w2, *w2t, *w3, *w3t, *w4;
+};
+
+constexpr int kRowTile = 16;
+constexpr int kLdA = kHid + 8;    // LDS rows padded by 16 bytes: the 16 rows that a
+constexpr int kLdX = kInPad + 8;  // wavefront reads together fall on different banks
+
+__device__ inline bf16x8 frag(const bf16 *row, int k) { return *reinterpret_cast<const bf16x8 *>(row + k); }
+
+// acc[j] += A (16 rows in LDS) x this wavefront's two column blocks; b: K / 32 x 2
+// operand fragments.
+template <int kSteps>
+__device__ inline void mma(const bf16 *a_row, int kq, const bf16x8 (&b)[kSteps][2], f32x4 (&acc)[2]) {
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int j = 0; j < 2; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r = l & 15, kq = (l >> 4) * 8;
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    bf16x8 a[2], b[2];
+  for (int k = 0; k < kSteps; k++) {
+    const bf16x8 a = frag(a_row, k * 32 + kq);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      a[i] = *reinterpret_cast<const bf16x8 *>(A + int64_t(m0 + 16 * i + r) * K + k0 + kq);
-      b[i] = *reinterpret_cast<const bf16x8 *>(Bt + int64_t(n0 + 16 * i + r) * K + k0 + kq);
+    for (int j = 0; j < 2; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[k][j], acc[j], 0, 0, 0);
+  }
+}
+
+template <int kSteps>
+__device__ inline void load_frags(const bf16 *w, int n0, int r, int kq, bf16x8 (&b)[kSteps][2]) {
+#pragma unroll
+  for (int k = 0; k < kSteps; k++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) b[k][j] = frag(w + (n0 + 16 * j + r) * (kSteps * 32), k * 32 + kq);
+}
+
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+
+// Forward pass of 16 rows per tile and, for training (kTrain), the backward pass to
+// the deltas of the first layer.  Four wavefronts, 32 units each; every weight
+// fragment a wavefront needs is loaded once, before the first tile.  Latency bounds a
+// batch: eight dependent stages of a few MFMAs between barriers; 16 rows a
+// workgroup put a batch of 1,024 on 64 CUs.  Without kTrain only y is written, and
+// workgroups take several tiles.
+template <bool kTrain>
+__global__ __launch_bounds__(256) void mlp_rows(RowBatch q, Weights w) {
+  __shared__ bf16 s_x[kRowTile * kLdX];
+  __shared__ bf16 s_a[2][kRowTile * kLdA];
+  __shared__ float s_w4[kHid];
+  __shared__ float s_dy[kRowTile];
+  const int tid = threadIdx.x, l = tid & 63;
+  const int n0 = (tid >> 6) * 32;  // first unit of this wavefront
+  const int r = l & 15, kq = (l >> 4) * 8, row4 = (l >> 4) * 4;
+  bf16x8 b1[1][2], b2[4][2], b3[4][2], c3[4][2], c2[4][2];
+  load_frags(w.w1, n0, r, kq, b1);
+  load_frags(w.w2, n0, r, kq, b2);
+  load_frags(w.w3, n0, r, kq, b3);
+  if (kTrain) {
+    load_frags(w.w3t, n0, r, kq, c3);
+    load_frags(w.w2t, n0, r, kq, c2);
+  }
+  float bias[3][2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int col = n0 + 16 * j + r;
+    bias[0][j] = w.p[kOffB1 + col];
+    bias[1][j] = w.p[kOffB2 + col];
+    bias[2][j] = w.p[kOffB3 + col];
+  }
+  const float b4 = w.p[kOffB4];
+  if (tid < kHid) s_w4[tid] = float(w.w4[tid]);
+  for (int t0 = blockIdx.x * kRowTile; t0 < q.R; t0 += gridDim.x * kRowTile) {
+    {
+      const int row = tid >> 4, k = tid & 15, g = t0 + row;
+      const bool ok = g < q.n;
+      const int64_t s = ok ? (q.idx ? q.idx[g] : g) : 0;
+      const bf16 v = bf16(ok ? q.xs[s * kIn + k] : 0.f);
+      s_x[row * kLdX + k] = v;
+      s_x[row * kLdX + kIn + k] = bf16(0.f);
+      if (kTrain) q.xt[int64_t(k) * q.R + g] = v;
     }
+    __syncthreads();
+    f32x4 acc[2], z[3][2];
+    auto layer = [&](int n, bf16 *out) {  // GELU of layer n + 1 from acc
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+      for (int j = 0; j < 2; j++) {
+        const int col = n0 + 16 * j + r;
+        bf16x4 h;
 #pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int row = m0 + 16 * i + (l >> 4) * 4 + e, col = n0 + 16 * j + r;
-        const int64_t o = int64_t(row) * N + col;
-        float c = acc[i][j][e];
-        if (ep.mode == 0) {
-          ep.out_f32[o] = c;
-        } else if (ep.mode == 1) {
-          const float z = c + ep.bias[col];
-          if (ep.out_f32) ep.out_f32[o] = z;
-          const bf16 h = bf16(gelu(z));
-          ep.out_b[o] = h;
-          if (ep.out_bt) ep.out_bt[int64_t(col) * M + row] = h;
-        } else {
-          const float dz = c * gelu_grad(ep.zprev[o]);
-          ep.out_f32[o] = dz;
-          const bf16 d = bf16(dz);
-          ep.out_b[o] = d;
-          ep.out_bt[int64_t(col) * M + row] = d;
+        for (int e = 0; e < 4; e++) {
+          z[n][j][e] = acc[j][e] + bias[n][j];
+          h[e] = bf16(gelu(z[n][j][e]));
+          out[(row4 + e) * kLdA + col] = h[e];
         }
+        if (kTrain) *reinterpret_cast<bf16x4 *>(q.ht[n] + int64_t(col) * q.R + t0 + row4) = h;
       }
-}
-
-// Batch rows from the resident sample set: X [R][32] bf16 (features padded with
-// zeros), its transpose [32][R], targets.  Rows beyond n_valid are zero.  A null
-// idx takes rows 0 .. n_valid - 1 in order; a null xt or tb is not written.
-__global__ void mlp_gather(const float *__restrict__ xs, const float *__restrict__ ts, const int32_t *__restrict__ idx,
-                           int n_valid, int R, bf16 *__restrict__ xb, bf16 *__restrict__ xt, float *__restrict__ tb) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  const bool ok = r < n_valid;
-  const int64_t s = ok ? (idx ? idx[r] : r) : 0;
-  for (int k = 0; k < kInPad; k++) {
-    const float v = (ok && k < kIn) ? xs[s * kIn + k] : 0.f;
-    const bf16 b = bf16(v);
-    xb[int64_t(r) * kInPad + k] = b;
-    if (xt) xt[int64_t(k) * R + r] = b;
-  }
-  if (tb) tb[r] = ok ? ts[s] : 0.f;
-}
-
-// Output layer forward: y = h3 . w4 + b4 (FP32, sequential over units), rows
-// 0 .. n_out - 1 of the batch.
-__global__ void mlp_out_fwd(const bf16 *__restrict__ h3, const bf16 *__restrict__ w4, const float *__restrict__ b4,
-                            int n_out, float *__restrict__ y) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n_out) return;
-  float s = 0.f;
-  for (int k = 0; k < kHid; k++) s += float(h3[int64_t(r) * kHid + k]) * float(w4[k]);
-  y[r] = s + b4[0];
-}
-
-// Loss gradient and the output layer's backward: dy = 2 (y - t) / n_valid,
-// dz3 = dy w4 * GELU'(z3) (FP32 and BF16 copies).
-__global__ void mlp_out_bwd(const float *__restrict__ y, const float *__restrict__ t, const bf16 *__restrict__ w4,
-                            const float *__restrict__ z3, int n_valid, int R, float *__restrict__ dy,
-                            float *__restrict__ dz, bf16 *__restrict__ dzb, bf16 *__restrict__ dzt) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  const float d = r < n_valid ? 2.f * (y[r] - t[r]) / float(n_valid) : 0.f;
-  dy[r] = d;
-  for (int k = 0; k < kHid; k++) {
-    const int64_t o = int64_t(r) * kHid + k;
-    const float v = d * float(w4[k]) * gelu_grad(z3[o]);
-    dz[o] = v;
-    const bf16 b = bf16(v);
-    dzb[o] = b;
-    dzt[int64_t(k) * R + r] = b;
-  }
-}
-
-// Column sums over the batch (biases, output weights), in row order.
-__global__ void mlp_colsum(const float *__restrict__ dz, int R, int N, float *__restrict__ out) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.f;
-  for (int r = 0; r < R; r++) s += dz[int64_t(r) * N + n];
-  out[n] = s;
-}
-
-__global__ void mlp_dw4(const float *__restrict__ dy, const bf16 *__restrict__ h3, int R, float *__restrict__ g) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > kHid) return;
-  float s = 0.f;
-  if (k < kHid) {
-    for (int r = 0; r < R; r++) s += dy[r] * float(h3[int64_t(r) * kHid + k]);
-    g[kOffW4 + k] = s;
-  } else {
-    for (int r = 0; r < R; r++) s += dy[r];
-    g[kOffB4] = s;
+      __syncthreads();
+    };
+    mma<1>(s_x + r * kLdX, kq, b1, acc);
+    layer(0, s_a[0]);
+    mma<4>(s_a[0] + r * kLdA, kq, b2, acc);
+    layer(1, s_a[1]);
+    mma<4>(s_a[1] + r * kLdA, kq, b3, acc);
+    layer(2, s_a[0]);
+    // output layer: y = h3 . w4 + b4 (FP32, sequential over units), one lane a row
+    if (tid < kRowTile) {
+      float s = 0.f;
+#pragma unroll 4
+      for (int k = 0; k < kHid; k += 8) {
+        const bf16x8 h = frag(s_a[0] + tid * kLdA, k);
+#pragma unroll
+        for (int e = 0; e < 8; e++) s += float(h[e]) * s_w4[k + e];
+      }
+      const float y = s + b4;
+      const int g = t0 + tid;
+      if (kTrain) {
+        const bool ok = g < q.n;
+        const float t = ok ? q.ts[q.idx ? q.idx[g] : g] : 0.f;
+        const float d = ok ? 2.f * (y - t) / float(q.n) : 0.f;
+        s_dy[tid] = d;
+        q.dy[g] = d;
+        q.sq[g] = (y - t) * (y - t);
+      } else if (g < q.n) {
+        q.y[g] = y;
+      }
+    }
+    __syncthreads();
+    if (kTrain) {
+      auto delta = [&](int n, auto value, bf16 *out) {  // deltas of layer n + 1
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          const int col = n0 + 16 * j + r;
+          bf16x4 h;
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            v[e] = value(j, e, col);
+            h[e] = bf16(v[e]);
+            if (out) out[(row4 + e) * kLdA + col] = h[e];
+          }
+          *reinterpret_cast<f32x4 *>(q.et[n] + int64_t(col) * q.R + t0 + row4) = v;
+          *reinterpret_cast<bf16x4 *>(q.dt[n] + int64_t(col) * q.R + t0 + row4) = h;
+        }
+        __syncthreads();
+      };
+      delta(2, [&](int j, int e, int col) { return s_dy[row4 + e] * s_w4[col] * gelu_grad(z[2][j][e]); }, s_a[1]);
+      mma<4>(s_a[1] + r * kLdA, kq, c3, acc);
+      delta(1, [&](int j, int e, int) { return acc[j][e] * gelu_grad(z[1][j][e]); }, s_a[0]);
+      mma<4>(s_a[0] + r * kLdA, kq, c2, acc);
+      delta(0, [&](int j, int e, int) { return acc[j][e] * gelu_grad(z[0][j][e]); }, nullptr);
+    }
   }
 }
 
-// First-layer weight gradient: the padded [128][32] GEMM result without the padding columns.
-__global__ void mlp_unpad_w1(const float *__restrict__ gpad, float *__restrict__ g) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kHid * kIn) return;
-  g[kOffW1 + i] = gpad[(i / kIn) * kInPad + (i % kIn)];
-}
+// Adam's constants of one step.
+struct AdamStep {
+  float lr, b1, b2, eps, c1, c2;
+};
 
-// Mean squared error of the valid rows (one thread, row order).
-__global__ void mlp_loss(const float *__restrict__ y, const float *__restrict__ t, int n_valid, float *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  float s = 0.f;
-  for (int r = 0; r < n_valid; r++) s += (y[r] - t[r]) * (y[r] - t[r]);
-  out[0] += s / float(n_valid);
-}
-
-// Adam step on the FP32 master parameters.
-__global__ void mlp_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m1,
-                         float *__restrict__ m2, int64_t n, float lr, float b1, float b2, float eps, float c1,
-                         float c2) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float a = b1 * m1[i] + (1.f - b1) * gi;
-  const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
+// Gradient g of parameter i: stored, or (kAdam) applied to the FP32 master parameter.
+// Returns the parameter's value afterwards.
+template <bool kAdam>
+__device__ inline float take_grad(float g, int64_t i, float *p, float *grad, float *m1, float *m2,
+                                  const AdamStep &st) {
+  if (!kAdam) {
+    grad[i] = g;
+    return 0.f;
+  }
+  const float a = st.b1 * m1[i] + (1.f - st.b1) * g;
+  const float b = st.b2 * m2[i] + (1.f - st.b2) * g * g;
   m1[i] = a;
   m2[i] = b;
-  p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+  const float v = p[i] - st.lr * (a / st.c1) / (sqrtf(b / st.c2) + st.eps);
+  p[i] = v;
+  return v;
+}
+
+// Work of mlp_update's workgroups, in order: 16 x 16 tiles of dW3, dW2 (64 each) and
+// dW1 (8), a wavefront a tile; then sums over rows, kSumCols columns a workgroup: the
+// biases (3 x 128), the output weights (128), and the output bias with the loss.
+constexpr int kTileBlocks = (64 + 64 + 8) / 4;
+constexpr int kSumCols = 32, kSumChunk = 1024, kSumLd = kSumChunk + 4;
+constexpr int kSumBlocks = 4 * (kHid / kSumCols) + 1;
+constexpr int kSumLdsBytes = kSumCols * kSumLd * int(sizeof(float));
+
+// Weight gradients dW[m][n] = sum_rows delta[row][m] act[row][n], bias and output
+// gradients, and the loss; with kAdam the parameters and their BF16 copies are
+// updated in place, by the owner of each gradient, and loss accumulates the mean
+// squared error of the batch.  The tiles take R / 32 dependent MFMAs, eight pairs of
+// loads in flight; a sum takes R dependent additions of terms read from LDS.
+template <bool kAdam>
+__global__ __launch_bounds__(256) void mlp_update(RowBatch q, Weights w, float *grad, float *m1, float *m2,
+                                                  AdamStep st, float *loss) {
+  extern __shared__ float s_t[];
+  const int tid = threadIdx.x, l = tid & 63, R = q.R;
+  if (blockIdx.x < kTileBlocks) {
+    int tile = blockIdx.x * 4 + (tid >> 6);
+    const bf16 *A, *B;
+    int64_t off;
+    int tn, ld;
+    bf16 *wb, *wt;  // BF16 copy and its transpose
+    if (tile < 64) {
+      A = q.dt[2], B = q.ht[1], off = kOffW3, tn = tile & 7, tile >>= 3, ld = kHid, wb = w.w3, wt = w.w3t;
+    } else if (tile < 128) {
+      tile -= 64;
+      A = q.dt[1], B = q.ht[0], off = kOffW2, tn = tile & 7, tile >>= 3, ld = kHid, wb = w.w2, wt = w.w2t;
+    } else {
+      tile -= 128;
+      A = q.dt[0], B = q.xt, off = kOffW1, tn = 0, ld = kIn, wb = w.w1, wt = w.w1t;
+    }
+    const int r = l & 15, kq = (l >> 4) * 8;
+    const bf16 *pa = A + int64_t(tile * 16 + r) * R + kq, *pb = B + int64_t(tn * 16 + r) * R + kq;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    int k0 = 0;
+    for (; k0 + 256 <= R; k0 += 256) {
+      bf16x8 a[8], b[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        a[u] = frag(pa, k0 + 32 * u);
+        b[u] = frag(pb, k0 + 32 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
+    }
+    for (; k0 < R; k0 += 32)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(pa, k0), frag(pb, k0), acc, 0, 0, 0);
+    const int n = tn * 16 + r;
+    const int ldb = ld == kIn ? kInPad : ld;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int m = tile * 16 + (l >> 4) * 4 + e;
+      const float v = take_grad<kAdam>(acc[e], off + int64_t(m) * ld + n, w.p, grad, m1, m2, st);
+      if (kAdam) {
+        const bf16 h = bf16(v);
+        wb[m * ldb + n] = h;
+        wt[n * kHid + m] = h;
+      }
+    }
+    return;
+  }
+  const int sb = blockIdx.x - kTileBlocks, kind = sb / (kHid / kSumCols);
+  const int c0 = (sb % (kHid / kSumCols)) * kSumCols;
+  const int cols = kind == 4 ? 2 : kSumCols;
+  float s = 0.f;
+  for (int r0 = 0; r0 < R; r0 += kSumChunk) {
+    const int m = R - r0 < kSumChunk ? R - r0 : kSumChunk;
+    // the chunk's terms, columns row-contiguous
+    for (int i = tid * 4; i < cols * m; i += 256 * 4) {
+      const int c = i / m, k = i - c * m;  // m is a multiple of 32
+      f32x4 v;
+      if (kind < 3) {
+        v = *reinterpret_cast<const f32x4 *>(q.et[kind] + int64_t(c0 + c) * R + r0 + k);
+      } else if (kind == 3) {
+        const f32x4 d = *reinterpret_cast<const f32x4 *>(q.dy + r0 + k);
+        const bf16x4 h = *reinterpret_cast<const bf16x4 *>(q.ht[2] + int64_t(c0 + c) * R + r0 + k);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = d[e] * float(h[e]);
+      } else {
+        v = *reinterpret_cast<const f32x4 *>((c == 0 ? q.dy : q.sq) + r0 + k);
+      }
+      *reinterpret_cast<f32x4 *>(s_t + c * kSumLd + k) = v;
+    }
+    __syncthreads();
+    if (tid < cols) {
+      const float *t = s_t + tid * kSumLd;
+      // the loss counts the valid rows only
+      const int end = kind == 4 && tid == 1 ? (q.n - r0 < m ? (q.n > r0 ? q.n - r0 : 0) : m) : m;
+      int k = 0;
+      for (; k + 16 <= end; k += 16) {
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const f32x4 *>(t + k + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) s += v[u][e];
+      }
+      for (; k < end; k++) s += t[k];
+    }
+    __syncthreads();
+  }
+  if (tid >= cols) return;
+  if (kind == 4 && tid == 1) {
+    loss[0] += s / float(q.n);
+    return;
+  }
+  constexpr int64_t kOff[5] = {kOffB1, kOffB2, kOffB3, kOffW4, kOffB4};
+  int64_t off = kOff[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (kind == k) off = kOff[k];
+  const float v = take_grad<kAdam>(s, off + c0 + tid, w.p, grad, m1, m2, st);
+  if (kAdam && kind == 3) w.w4[c0 + tid] = bf16(v);
 }
 
 // BF16 weight copies for the GEMMs: W1 padded [128][32] and its transpose [32][128],
@@ -232,32 +385,23 @@ __global__ void mlp_pack(const float *__restrict__ p, bf16 *__restrict__ w1, bf1
   if (i < kHid) w4[i] = bf16(p[kOffW4 + i]);
 }
 
-// Activations of wg_mlp_forward_noalloc: X [R][32] bf16 and the three hidden
-// layers [R][128] bf16 for up to WG_MLP_NOALLOC_MAX_ROWS rows (6.5 MiB), one copy
-// per GPU for the life of the process.  Host code uses the per-device address
-// that hipGetSymbolAddress returns, never this name.
-constexpr size_t kScratchXBytes = size_t(WG_MLP_NOALLOC_MAX_ROWS) * kInPad * sizeof(bf16);
-constexpr size_t kScratchHBytes = size_t(WG_MLP_NOALLOC_MAX_ROWS) * kHid * sizeof(bf16);
-constexpr size_t kScratchBytes = kScratchXBytes + 3 * kScratchHBytes;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
-
 }  // namespace
 
 struct wg_mlp {
   std::string err;
   hipStream_t stream = nullptr;
   int device = 0;
-  unsigned char *scratch = nullptr;  // this device's address of the scratch array
-  float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr, *gpad = nullptr;
-  bf16 *w1 = nullptr, *w1t = nullptr, *w2 = nullptr, *w2t = nullptr, *w3 = nullptr, *w3t = nullptr, *w4 = nullptr;
+  Weights w{};
+  float *g = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr;
   int64_t adam_t = 0;
-  // batch buffers (rows R)
+  // batch buffers of R rows, and the samples of a call with their host staging
+  // (pinned): kept and grown up to kKeepRows rows, larger ones live for one call
+  RowBatch q{};
+  void *batch = nullptr;
   int R = 0;
-  bf16 *xb = nullptr, *xt = nullptr, *h[3] = {}, *ht[3] = {}, *dzb = nullptr, *dzt = nullptr, *dzb2 = nullptr,
-       *dzt2 = nullptr;
-  float *z[3] = {}, *dz = nullptr, *dz2 = nullptr, *y = nullptr, *t = nullptr, *dy = nullptr, *loss = nullptr;
-  int32_t *idx = nullptr;
-  std::vector<void *> batch_bufs;
+  float *dx = nullptr, *dt = nullptr, *stage = nullptr;
+  int32_t *didx = nullptr;
+  int rows = 0;
 };
 
 namespace {
@@ -283,125 +427,122 @@ int mlp_alloc(wg_mlp *h, T **p, size_t n, std::vector<void *> *track = nullptr) 
   return WG_OK;
 }
 
+// Batch buffers for R rows (a multiple of 32) in one allocation.
 int ensure_batch(wg_mlp *h, int R) {
-  if (R <= h->R) return WG_OK;
-  MLP_CHECK(h, hipStreamSynchronize(h->stream));
-  for (void *q : h->batch_bufs) (void)hipFree(q);
-  h->batch_bufs.clear();
-  auto *t = &h->batch_bufs;
-  int rc = mlp_alloc(h, &h->xb, size_t(R) * kInPad, t);
-  if (!rc) rc = mlp_alloc(h, &h->xt, size_t(R) * kInPad, t);
-  for (int l = 0; l < 3 && !rc; l++) {
-    rc = mlp_alloc(h, &h->h[l], size_t(R) * kHid, t);
-    if (!rc) rc = mlp_alloc(h, &h->ht[l], size_t(R) * kHid, t);
-    if (!rc) rc = mlp_alloc(h, &h->z[l], size_t(R) * kHid, t);
+  if (R > h->R) {
+    MLP_CHECK(h, hipStreamSynchronize(h->stream));
+    if (h->batch) (void)hipFree(h->batch);
+    h->batch = nullptr;
+    h->R = 0;
+    const size_t per_row = kIn * sizeof(bf16) + 6 * kHid * sizeof(bf16) + (3 * kHid + 2) * sizeof(float);
+    if (hipMalloc(&h->batch, per_row * R) != hipSuccess) return mlp_fail(h, WG_E_NOMEM, "hipMalloc failed");
+    h->R = R;
   }
-  if (!rc) rc = mlp_alloc(h, &h->dzb, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->dzt, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->dzb2, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->dzt2, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->dz, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->dz2, size_t(R) * kHid, t);
-  if (!rc) rc = mlp_alloc(h, &h->y, size_t(R), t);
-  if (!rc) rc = mlp_alloc(h, &h->t, size_t(R), t);
-  if (!rc) rc = mlp_alloc(h, &h->dy, size_t(R), t);
-  if (!rc) rc = mlp_alloc(h, &h->idx, size_t(R), t);
-  if (rc) return rc;
-  h->R = R;
-  return WG_OK;
-}
-
-int launch_gemm_on(wg_mlp *h, hipStream_t stream, const bf16 *A, const bf16 *Bt, int M, int N, int K,
-                   const Epilogue &ep) {
-  if (M % 32 || N % 32 || K % 32) return mlp_fail(h, WG_E_ARG, "GEMM shape is not a multiple of 32");
-  hipLaunchKernelGGL(mlp_gemm, dim3(N / 32, M / 32), dim3(64), 0, stream, A, Bt, M, N, K, ep);
-  MLP_CHECK(h, hipGetLastError());
-  return WG_OK;
-}
-
-int launch_gemm(wg_mlp *h, const bf16 *A, const bf16 *Bt, int M, int N, int K, const Epilogue &ep) {
-  return launch_gemm_on(h, h->stream, A, Bt, M, N, K, ep);
-}
-
-// Per-device address of the scratch array, resolved once per device with that
-// device current (each GPU holds its own copy at its own address).
-std::mutex g_scratch_mu;
-unsigned char *g_scratch_addr[64] = {};
-
-int scratch_address(wg_mlp *h) {
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (h->device < 0 || h->device >= 64) return mlp_fail(h, WG_E_ARG, "device ordinal out of range");
-  if (!g_scratch_addr[h->device]) {
-    void *ptr = nullptr;
-    MLP_CHECK(h, hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
-    g_scratch_addr[h->device] = static_cast<unsigned char *>(ptr);
-  }
-  h->scratch = g_scratch_addr[h->device];
+  char *at = static_cast<char *>(h->batch);
+  auto take = [&](auto *&ptr, size_t n) {
+    ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(at);
+    at += n * sizeof(*ptr) * size_t(h->R);
+  };
+  for (int k = 0; k < 3; k++) take(h->q.et[k], kHid);
+  take(h->q.dy, 1);
+  take(h->q.sq, 1);
+  for (int k = 0; k < 3; k++) take(h->q.ht[k], kHid);
+  for (int k = 0; k < 3; k++) take(h->q.dt[k], kHid);
+  take(h->q.xt, kIn);
   return WG_OK;
 }
 
 int pack(wg_mlp *h) {
-  hipLaunchKernelGGL(mlp_pack, dim3((kHid * kHid + 255) / 256), dim3(256), 0, h->stream, h->p, h->w1, h->w1t, h->w2,
-                     h->w2t, h->w3, h->w3t, h->w4);
+  const Weights &w = h->w;
+  hipLaunchKernelGGL(mlp_pack, dim3((kHid * kHid + 255) / 256), dim3(256), 0, h->stream, w.p, w.w1, w.w1t, w.w2, w.w2t,
+                     w.w3, w.w3t, w.w4);
   MLP_CHECK(h, hipGetLastError());
   return WG_OK;
 }
 
-// Forward pass over R rows already in xb/xt.
-int forward(wg_mlp *h, int R) {
-  const bf16 *in[3] = {h->xb, nullptr, nullptr};
-  const bf16 *w[3] = {h->w1, h->w2, h->w3};
-  const float *b[3] = {h->p + kOffB1, h->p + kOffB2, h->p + kOffB3};
-  const int K[3] = {kInPad, kHid, kHid};
-  for (int l = 0; l < 3; l++) {
-    Epilogue ep{1, h->z[l], b[l], nullptr, h->h[l], h->ht[l]};
-    int rc = launch_gemm(h, l == 0 ? in[0] : h->h[l - 1], w[l], R, kHid, K[l], ep);
-    if (rc) return rc;
-  }
-  hipLaunchKernelGGL(mlp_out_fwd, dim3((R + 255) / 256), dim3(256), 0, h->stream, h->h[2], h->w4, h->p + kOffB4, R,
-                     h->y);
+// Forward pass of `rows` device rows x into y on a stream; workgroups beyond 512 (two
+// per CU) would only load the weights again.
+int launch_forward(wg_mlp *h, hipStream_t stream, const float *x, int rows, float *y) {
+  RowBatch q{};
+  q.xs = x;
+  q.n = rows;
+  q.R = (rows + kRowTile - 1) / kRowTile * kRowTile;
+  q.y = y;
+  hipLaunchKernelGGL(mlp_rows<false>, dim3(std::min(q.R / kRowTile, 512)), dim3(256), 0, stream, q, h->w);
   MLP_CHECK(h, hipGetLastError());
   return WG_OK;
 }
 
-// Backward pass for the rows of the last forward (targets in h->t); gradients into h->g.
-int backward(wg_mlp *h, int R, int n_valid) {
-  hipLaunchKernelGGL(mlp_out_bwd, dim3((R + 255) / 256), dim3(256), 0, h->stream, h->y, h->t, h->w4, h->z[2],
-                     n_valid, R, h->dy, h->dz, h->dzb, h->dzt);
-  MLP_CHECK(h, hipGetLastError());
-  hipLaunchKernelGGL(mlp_dw4, dim3(1), dim3(kHid + 64), 0, h->stream, h->dy, h->h[2], R, h->g);
-  MLP_CHECK(h, hipGetLastError());
-  // layer 3: dW3 = dz3^T h2, db3, dz2 = (dz3 W3) * GELU'(z2)
-  int rc = launch_gemm(h, h->dzt, h->ht[1], kHid, kHid, R, Epilogue{0, h->g + kOffW3, nullptr, nullptr, nullptr, nullptr});
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_colsum, dim3(1), dim3(kHid), 0, h->stream, h->dz, R, kHid, h->g + kOffB3);
-  rc = launch_gemm(h, h->dzb, h->w3t, R, kHid, kHid, Epilogue{2, h->dz2, nullptr, h->z[1], h->dzb2, h->dzt2});
-  if (rc) return rc;
-  // layer 2
-  rc = launch_gemm(h, h->dzt2, h->ht[0], kHid, kHid, R, Epilogue{0, h->g + kOffW2, nullptr, nullptr, nullptr, nullptr});
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_colsum, dim3(1), dim3(kHid), 0, h->stream, h->dz2, R, kHid, h->g + kOffB2);
-  rc = launch_gemm(h, h->dzb2, h->w2t, R, kHid, kHid, Epilogue{2, h->dz, nullptr, h->z[0], h->dzb, h->dzt});
-  if (rc) return rc;
-  // layer 1
-  rc = launch_gemm(h, h->dzt, h->xt, kHid, kInPad, R, Epilogue{0, h->gpad, nullptr, nullptr, nullptr, nullptr});
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_unpad_w1, dim3((kHid * kIn + 255) / 256), dim3(256), 0, h->stream, h->gpad, h->g);
-  hipLaunchKernelGGL(mlp_colsum, dim3(1), dim3(kHid), 0, h->stream, h->dz, R, kHid, h->g + kOffB1);
+// Forward and backward pass and the gradients of one batch (or Adam's step on them).
+int launch_batch(wg_mlp *h, const float *xs, const float *ts, const int32_t *idx, int n, int R, const AdamStep *st) {
+  RowBatch q = h->q;
+  q.xs = xs;
+  q.ts = ts;
+  q.idx = idx;
+  q.n = n;
+  q.R = R;
+  hipLaunchKernelGGL(mlp_rows<true>, dim3(R / kRowTile), dim3(256), 0, h->stream, q, h->w);
+  auto *update = st ? mlp_update<true> : mlp_update<false>;
+  hipLaunchKernelGGL(update, dim3(kTileBlocks + kSumBlocks), dim3(256), kSumLdsBytes, h->stream, q, h->w, h->g, h->m1,
+                     h->m2, st ? *st : AdamStep{}, h->loss);
   MLP_CHECK(h, hipGetLastError());
   return WG_OK;
 }
 
 int round32(int r) { return (r + 31) / 32 * 32; }
 
-// Uploads rows [r0, r0 + n) of host features/targets as a batch (identity index).
-int upload_rows(wg_mlp *h, const float *x, const float *t, int n, float **dx, float **dt) {
-  int rc = mlp_alloc(h, dx, size_t(n) * kIn);
-  if (!rc && t) rc = mlp_alloc(h, dt, size_t(n));
-  if (rc) return rc;
-  MLP_CHECK(h, hipMemcpyAsync(*dx, x, size_t(n) * kIn * sizeof(float), hipMemcpyHostToDevice, h->stream));
-  if (t) MLP_CHECK(h, hipMemcpyAsync(*dt, t, size_t(n) * sizeof(float), hipMemcpyHostToDevice, h->stream));
+constexpr int kKeepRows = 1 << 18;
+
+void free_samples(wg_mlp *h) {
+  void *bufs[] = {h->dx, h->dt, h->didx};
+  for (void *b : bufs)
+    if (b) (void)hipFree(b);
+  if (h->stage) (void)hipHostFree(h->stage);
+  h->dx = h->dt = h->stage = nullptr;
+  h->didx = nullptr;
+  h->rows = 0;
+}
+
+// Device copies of n samples: h->dx and, with targets, h->dt; up to kKeepRows through
+// the pinned staging buffer (free again: a call ends with the stream idle).
+int upload_samples(wg_mlp *h, const float *x, const float *t, int n) {
+  if (n > h->rows) {
+    MLP_CHECK(h, hipStreamSynchronize(h->stream));
+    free_samples(h);
+    // dt also holds the outputs of a forward pass
+    if (hipMalloc(&h->dx, size_t(n) * kIn * sizeof(float)) != hipSuccess ||
+        hipMalloc(&h->dt, size_t(n) * sizeof(float)) != hipSuccess ||
+        hipMalloc(&h->didx, size_t(n) * sizeof(int32_t)) != hipSuccess ||
+        (n <= kKeepRows &&
+         hipHostMalloc(&h->stage, size_t(n) * (kIn + 1) * sizeof(float), hipHostMallocDefault) != hipSuccess)) {
+      free_samples(h);
+      (void)hipGetLastError();
+      return mlp_fail(h, WG_E_NOMEM, "sample buffers: out of memory");
+    }
+    h->rows = n;
+  }
+  const size_t xb = size_t(n) * kIn * sizeof(float), tb = size_t(n) * sizeof(float);
+  if (h->stage) {
+    std::memcpy(h->stage, x, xb);
+    x = h->stage;
+    if (t) t = static_cast<const float *>(std::memcpy(h->stage + size_t(n) * kIn, t, tb));
+  }
+  MLP_CHECK(h, hipMemcpyAsync(h->dx, x, xb, hipMemcpyHostToDevice, h->stream));
+  if (t) MLP_CHECK(h, hipMemcpyAsync(h->dt, t, tb, hipMemcpyHostToDevice, h->stream));
   return WG_OK;
+}
+
+// Ends a call: the stream is idle and buffers beyond what a handle keeps are given back.
+int end_call(wg_mlp *h, int rc) {
+  const hipError_t e = hipStreamSynchronize(h->stream);
+  if (h->rows > kKeepRows) free_samples(h);
+  if (h->R > kKeepRows / 8) {
+    (void)hipFree(h->batch);
+    h->batch = nullptr;
+    h->R = 0;
+  }
+  if (!rc && e != hipSuccess) return mlp_fail(h, WG_E_HIP, std::string("stream: ") + hipGetErrorString(e));
+  return rc;
 }
 
 }  // namespace
@@ -414,19 +555,17 @@ extern "C" int wg_mlp_create(uint64_t seed, wg_mlp **out) {
   *out = h;
   MLP_CHECK(h, hipGetDevice(&h->device));
   MLP_CHECK(h, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  int rc = scratch_address(h);
-  if (!rc) rc = mlp_alloc(h, &h->p, kNParams);
+  int rc = mlp_alloc(h, &h->w.p, kNParams);
   if (!rc) rc = mlp_alloc(h, &h->g, kNParams);
   if (!rc) rc = mlp_alloc(h, &h->m1, kNParams);
   if (!rc) rc = mlp_alloc(h, &h->m2, kNParams);
-  if (!rc) rc = mlp_alloc(h, &h->gpad, size_t(kHid) * kInPad);
-  if (!rc) rc = mlp_alloc(h, &h->w1, size_t(kHid) * kInPad);
-  if (!rc) rc = mlp_alloc(h, &h->w1t, size_t(kHid) * kInPad);
-  if (!rc) rc = mlp_alloc(h, &h->w2, size_t(kHid) * kHid);
-  if (!rc) rc = mlp_alloc(h, &h->w2t, size_t(kHid) * kHid);
-  if (!rc) rc = mlp_alloc(h, &h->w3, size_t(kHid) * kHid);
-  if (!rc) rc = mlp_alloc(h, &h->w3t, size_t(kHid) * kHid);
-  if (!rc) rc = mlp_alloc(h, &h->w4, kHid);
+  if (!rc) rc = mlp_alloc(h, &h->w.w1, size_t(kHid) * kInPad);
+  if (!rc) rc = mlp_alloc(h, &h->w.w1t, size_t(kHid) * kInPad);
+  if (!rc) rc = mlp_alloc(h, &h->w.w2, size_t(kHid) * kHid);
+  if (!rc) rc = mlp_alloc(h, &h->w.w2t, size_t(kHid) * kHid);
+  if (!rc) rc = mlp_alloc(h, &h->w.w3, size_t(kHid) * kHid);
+  if (!rc) rc = mlp_alloc(h, &h->w.w3t, size_t(kHid) * kHid);
+  if (!rc) rc = mlp_alloc(h, &h->w.w4, kHid);
   if (!rc) rc = mlp_alloc(h, &h->loss, 1);
   if (rc) return rc;
   // He-uniform initial weights from a 64-bit LCG (host), zero biases
@@ -444,7 +583,7 @@ extern "C" int wg_mlp_create(uint64_t seed, wg_mlp **out) {
   fill(kOffW2, kHid, kHid);
   fill(kOffW3, kHid, kHid);
   fill(kOffW4, 1, kHid);
-  MLP_CHECK(h, hipMemcpyAsync(h->p, p.data(), kNParams * sizeof(float), hipMemcpyHostToDevice, h->stream));
+  MLP_CHECK(h, hipMemcpyAsync(h->w.p, p.data(), kNParams * sizeof(float), hipMemcpyHostToDevice, h->stream));
   rc = pack(h);
   if (rc) return rc;
   MLP_CHECK(h, hipStreamSynchronize(h->stream));
@@ -454,8 +593,9 @@ extern "C" int wg_mlp_create(uint64_t seed, wg_mlp **out) {
 extern "C" int wg_mlp_destroy(wg_mlp *h) {
   if (!h) return WG_E_ARG;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (void *q : h->batch_bufs) (void)hipFree(q);
-  void *bufs[] = {h->p, h->g, h->m1, h->m2, h->gpad, h->w1, h->w1t, h->w2, h->w2t, h->w3, h->w3t, h->w4, h->loss};
+  free_samples(h);
+  const Weights &w = h->w;
+  void *bufs[] = {w.p, w.w1, w.w1t, w.w2, w.w2t, w.w3, w.w3t, w.w4, h->g, h->m1, h->m2, h->loss, h->batch};
   for (void *q : bufs)
     if (q) (void)hipFree(q);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -469,14 +609,14 @@ extern "C" int64_t wg_mlp_n_params(void) { return kNParams; }
 
 extern "C" int wg_mlp_get_params(wg_mlp *h, float *out) {
   if (!h || !out) return WG_E_ARG;
-  MLP_CHECK(h, hipMemcpyAsync(out, h->p, kNParams * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  MLP_CHECK(h, hipMemcpyAsync(out, h->w.p, kNParams * sizeof(float), hipMemcpyDeviceToHost, h->stream));
   MLP_CHECK(h, hipStreamSynchronize(h->stream));
   return WG_OK;
 }
 
 extern "C" int wg_mlp_set_params(wg_mlp *h, const float *in) {
   if (!h || !in) return WG_E_ARG;
-  MLP_CHECK(h, hipMemcpyAsync(h->p, in, kNParams * sizeof(float), hipMemcpyHostToDevice, h->stream));
+  MLP_CHECK(h, hipMemcpyAsync(h->w.p, in, kNParams * sizeof(float), hipMemcpyHostToDevice, h->stream));
   int rc = pack(h);
   if (rc) return rc;
   MLP_CHECK(h, hipStreamSynchronize(h->stream));
@@ -485,103 +625,51 @@ extern "C" int wg_mlp_set_params(wg_mlp *h, const float *in) {
 
 extern "C" int wg_mlp_forward(wg_mlp *h, int32_t rows, const float *x, float *y) {
   if (!h || rows <= 0 || !x || !y) return WG_E_ARG;
-  const int chunk = 8192;
-  float *dx = nullptr;
-  int rc = upload_rows(h, x, nullptr, rows, &dx, nullptr);
-  if (rc) return rc;
-  rc = ensure_batch(h, std::min(round32(rows), chunk));
-  std::vector<int32_t> iota;
-  for (int r0 = 0; !rc && r0 < rows; r0 += chunk) {
-    const int n = std::min(chunk, rows - r0), R = round32(n);
-    iota.resize(n);
-    for (int i = 0; i < n; i++) iota[i] = r0 + i;
-    hipError_t e = hipMemcpyAsync(h->idx, iota.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, h->stream);
-    if (e != hipSuccess) { rc = mlp_fail(h, WG_E_HIP, "hipMemcpyAsync"); break; }
-    hipLaunchKernelGGL(mlp_gather, dim3((R + 255) / 256), dim3(256), 0, h->stream, dx, nullptr, h->idx, n, R, h->xb,
-                       h->xt, nullptr);
-    rc = forward(h, R);
-    if (rc) break;
-    e = hipMemcpyAsync(y + r0, h->y, n * sizeof(float), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) rc = mlp_fail(h, WG_E_HIP, "forward copy");
+  int rc = upload_samples(h, x, nullptr, rows);
+  if (!rc) rc = launch_forward(h, h->stream, h->dx, rows, h->dt);
+  // the outputs come back through the staging buffer's second part
+  float *st = rc || !h->stage ? y : h->stage + size_t(rows) * kIn;
+  if (!rc && hipMemcpyAsync(st, h->dt, size_t(rows) * sizeof(float), hipMemcpyDeviceToHost, h->stream) != hipSuccess)
+    rc = mlp_fail(h, WG_E_HIP, "forward copy");
+  if (!rc) {
+    const hipError_t e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) rc = mlp_fail(h, WG_E_HIP, std::string("forward: ") + hipGetErrorString(e));
   }
-  (void)hipStreamSynchronize(h->stream);
-  (void)hipFree(dx);
-  return rc;
+  if (!rc && st != y) std::memcpy(y, st, size_t(rows) * sizeof(float));
+  return end_call(h, rc);
 }
 
 extern "C" int wg_mlp_forward_noalloc(wg_mlp *h, int32_t rows, const float *x, float *y, void *stream) {
   if (!h || !x || !y) return WG_E_ARG;
   if (rows <= 0 || rows > WG_MLP_NOALLOC_MAX_ROWS)
     return mlp_fail(h, WG_E_ARG, "wg_mlp_forward_noalloc: rows must be 1.." + std::to_string(WG_MLP_NOALLOC_MAX_ROWS) +
-                                     " (the size of its scratch array), got " + std::to_string(rows));
-  if (!h->scratch) return mlp_fail(h, WG_E_STATE, "wg_mlp_forward_noalloc: scratch address not resolved");
-  hipStream_t s = stream ? static_cast<hipStream_t>(stream) : h->stream;
-  const int R = round32(rows);
-  bf16 *xb = reinterpret_cast<bf16 *>(h->scratch);
-  bf16 *hb[3];
-  for (int l = 0; l < 3; l++) hb[l] = reinterpret_cast<bf16 *>(h->scratch + kScratchXBytes + l * kScratchHBytes);
-  // every row of the batch, padding included, is written before it is read:
-  // nothing in the scratch array needs clearing between calls
-  hipLaunchKernelGGL(mlp_gather, dim3((R + 255) / 256), dim3(256), 0, s, x, nullptr, nullptr, rows, R, xb, nullptr,
-                     nullptr);
-  MLP_CHECK(h, hipGetLastError());
-  const bf16 *w[3] = {h->w1, h->w2, h->w3};
-  const float *b[3] = {h->p + kOffB1, h->p + kOffB2, h->p + kOffB3};
-  const int K[3] = {kInPad, kHid, kHid};
-  for (int l = 0; l < 3; l++) {
-    Epilogue ep{1, nullptr, b[l], nullptr, hb[l], nullptr};
-    int rc = launch_gemm_on(h, s, l == 0 ? xb : hb[l - 1], w[l], R, kHid, K[l], ep);
-    if (rc) return rc;
-  }
-  hipLaunchKernelGGL(mlp_out_fwd, dim3((rows + 255) / 256), dim3(256), 0, s, hb[2], h->w4, h->p + kOffB4, rows, y);
-  MLP_CHECK(h, hipGetLastError());
-  return WG_OK;
+                                     ", got " + std::to_string(rows));
+  return launch_forward(h, stream ? static_cast<hipStream_t>(stream) : h->stream, x, rows, y);
 }
 
 extern "C" int wg_mlp_gradient(wg_mlp *h, int32_t rows, const float *x, const float *t, float *loss, float *grad) {
   if (!h || rows <= 0 || !x || !t || !grad) return WG_E_ARG;
   const int R = round32(rows);
-  float *dx = nullptr, *dt = nullptr;
-  int rc = upload_rows(h, x, t, rows, &dx, &dt);
+  int rc = upload_samples(h, x, t, rows);
   if (!rc) rc = ensure_batch(h, R);
+  if (!rc && hipMemsetAsync(h->loss, 0, sizeof(float), h->stream) != hipSuccess) rc = mlp_fail(h, WG_E_HIP, "loss");
+  if (!rc) rc = launch_batch(h, h->dx, h->dt, nullptr, rows, R, nullptr);
   if (!rc) {
-    std::vector<int32_t> iota(rows);
-    for (int i = 0; i < rows; i++) iota[i] = i;
-    hipError_t e = hipMemcpyAsync(h->idx, iota.data(), rows * sizeof(int32_t), hipMemcpyHostToDevice, h->stream);
-    if (e != hipSuccess) rc = mlp_fail(h, WG_E_HIP, "hipMemcpyAsync");
-  }
-  if (!rc) {
-    hipLaunchKernelGGL(mlp_gather, dim3((R + 255) / 256), dim3(256), 0, h->stream, dx, dt, h->idx, rows, R, h->xb,
-                       h->xt, h->t);
-    rc = forward(h, R);
-  }
-  if (!rc) rc = backward(h, R, rows);
-  if (!rc) {
-    (void)hipMemsetAsync(h->loss, 0, sizeof(float), h->stream);
-    hipLaunchKernelGGL(mlp_loss, dim3(1), dim3(64), 0, h->stream, h->y, h->t, rows, h->loss);
     hipError_t e = hipMemcpyAsync(grad, h->g, kNParams * sizeof(float), hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess && loss) e = hipMemcpyAsync(loss, h->loss, sizeof(float), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) rc = mlp_fail(h, WG_E_HIP, "gradient copy");
   }
-  (void)hipStreamSynchronize(h->stream);
-  (void)hipFree(dx);
-  (void)hipFree(dt);
-  return rc;
+  return end_call(h, rc);
 }
 
 extern "C" int wg_mlp_train(wg_mlp *h, int32_t n_samples, const float *x, const float *t, int32_t epochs,
                             int32_t batch, float lr, uint64_t seed, float *epoch_loss) {
   if (!h || n_samples <= 0 || !x || !t || epochs <= 0 || batch < 32 || batch % 32) return WG_E_ARG;
-  float *dx = nullptr, *dt = nullptr;
-  int rc = upload_rows(h, x, t, n_samples, &dx, &dt);
-  if (!rc) rc = ensure_batch(h, batch);
+  int rc = upload_samples(h, x, t, n_samples);
+  if (!rc) rc = ensure_batch(h, std::min(batch, round32(n_samples)));
   std::vector<int32_t> perm(n_samples);
   for (int i = 0; i < n_samples; i++) perm[i] = i;
   uint64_t s = seed ^ 0x9E3779B97F4A7C15ULL;
-  int32_t *dperm = nullptr;
-  if (!rc) rc = mlp_alloc(h, &dperm, size_t(n_samples));
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int ep = 0; !rc && ep < epochs; ep++) {
     // Fisher-Yates shuffle of the sample order (host)
@@ -590,24 +678,16 @@ extern "C" int wg_mlp_train(wg_mlp *h, int32_t n_samples, const float *x, const 
       const int j = int((s >> 33) % uint64_t(i + 1));
       std::swap(perm[i], perm[j]);
     }
-    hipError_t e = hipMemcpyAsync(dperm, perm.data(), n_samples * sizeof(int32_t), hipMemcpyHostToDevice, h->stream);
+    hipError_t e = hipMemcpyAsync(h->didx, perm.data(), n_samples * sizeof(int32_t), hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess) e = hipMemsetAsync(h->loss, 0, sizeof(float), h->stream);
     if (e != hipSuccess) { rc = mlp_fail(h, WG_E_HIP, "epoch setup"); break; }
     int n_batches = 0;
     for (int r0 = 0; r0 < n_samples; r0 += batch) {
       const int n = std::min(batch, n_samples - r0);
-      const int R = round32(n);
-      hipLaunchKernelGGL(mlp_gather, dim3((R + 255) / 256), dim3(256), 0, h->stream, dx, dt, dperm + r0, n, R,
-                         h->xb, h->xt, h->t);
-      rc = forward(h, R);
-      if (!rc) rc = backward(h, R, n);
-      if (rc) break;
-      hipLaunchKernelGGL(mlp_loss, dim3(1), dim3(64), 0, h->stream, h->y, h->t, n, h->loss);
       h->adam_t++;
       const float c1 = 1.f - std::pow(b1, float(h->adam_t)), c2 = 1.f - std::pow(b2, float(h->adam_t));
-      hipLaunchKernelGGL(mlp_adam, dim3(unsigned((kNParams + 255) / 256)), dim3(256), 0, h->stream, h->p, h->g,
-                         h->m1, h->m2, kNParams, lr, b1, b2, eps, c1, c2);
-      rc = pack(h);
+      const AdamStep st{lr, b1, b2, eps, c1, c2};
+      rc = launch_batch(h, h->dx, h->dt, h->didx + r0, n, round32(n), &st);
       if (rc) break;
       n_batches++;
     }
@@ -618,9 +698,5 @@ extern "C" int wg_mlp_train(wg_mlp *h, int32_t n_samples, const float *x, const 
     if (e != hipSuccess) { rc = mlp_fail(h, WG_E_HIP, "loss copy"); break; }
     if (epoch_loss) epoch_loss[ep] = l / float(std::max(n_batches, 1));
   }
-  (void)hipStreamSynchronize(h->stream);
-  (void)hipFree(dx);
-  (void)hipFree(dt);
-  (void)hipFree(dperm);
-  return rc;
+  return end_call(h, rc);
 }
