@@ -53,6 +53,21 @@ def test_many_days_equals_eager(wg, rows, cols, members, calls):
     assert np.array_equal(a[3], b[3], equal_nan=True)
 
 
+@pytest.mark.parametrize("members, days", [(12, 9), (17, 9), (71, 4)])
+def test_members_one_by_one_and_in_twos(wg, members, days):
+    """Workgroups of one member while every wavefront has a SIMD of its own (12 members
+    of 80 wavefronts, 17 of 52 with two levels each), of two beyond, the last one half
+    empty (71)."""
+    print("case: many days, members", members, days, flush=True)
+    w = wg.World(wg.regional_spec(seed=6, nrows=40, ncols=50))
+    f = w.forcing(seed=3, day0=0, n_days=days)
+    a = run(wg, w, f, members, [days], False)
+    b = run(wg, w, f, members, [days], True)
+    for q in range(members):
+        assert all(np.array_equal(np.asarray(a[0][q][k]), np.asarray(b[0][q][k]), equal_nan=True) for k in b[0][q]), q
+    assert np.array_equal(a[2], b[2], equal_nan=True) and np.array_equal(a[3], b[3], equal_nan=True)
+
+
 def test_autotune_on_the_many_days_path(wg):
     """The tuner's saved state leaves the tables and the ring alone that its own first
     call of the many-days kernel makes."""

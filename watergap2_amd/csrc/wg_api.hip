@@ -85,6 +85,7 @@ struct wg_handle {
   std::vector<int32_t> day_level_cells;
   std::map<int32_t, WgDayTable> day_tables;
   int64_t day_capacity = 0;
+  int64_t day_simds = 0;  // SIMDs of the chip
   unsigned long long *d_ring = nullptr;
   int32_t ring_slots = 0;
   int64_t ring_day = 0;
@@ -698,7 +699,10 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 // Chooses the wavefronts of a launch of `days` days.  While they all fit on the chip
 // at once, more levels per wavefront cost each day a pass of the routing step per
 // level, fewer cost a hand over between wavefronts per level once per launch (us,
-// measured on grids of 56, 104 and 352 levels).  With more wavefronts than fit, all
+// measured on grids of 56, 104 and 352 levels).  Once wavefronts outnumber the SIMDs, two
+// share some, which costs each day about kShare (6,485 cells, 8 members: 41.8 us with
+// 1,264 wavefronts of one level, 31.1 with 992 of two; the 67,420-cell grid has more
+// than 1,024 with any division).  With more wavefronts than fit, all
 // of them cost chip time, and eight levels per wavefront is nearly the least (64
 // members of the global grid: 1.21 ms a day against 1.32 with one level).
 // Calls of fewer than kManyDaysMin days run one launch per day and part: there the
@@ -711,7 +715,7 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 // when the memory for it is not there.
 constexpr int32_t kManyDaysMin = 3;
 const WgDayTable *day_table(wg_handle *h, int32_t days) {
-  constexpr double kHandOver = 1.2, kPass = 1.1;
+  constexpr double kHandOver = 1.2, kPass = 1.1, kShare = 8.;
   if (days < kManyDaysMin || h->day_capacity <= 0) return nullptr;
   if (h->day_level_cells.empty()) {
     h->day_level_cells.assign(size_t(h->max_depth), 0);
@@ -722,7 +726,9 @@ const WgDayTable *day_table(wg_handle *h, int32_t days) {
   for (int32_t span : {1, 2, 4, 8, 16, 64}) {
     const DayPlan d = day_plan(h->day_level_cells, span);
     if (int64_t(d.n_waves) * h->m > h->day_capacity) continue;
-    const double c = kHandOver * h->max_depth / span + kPass * double(days) * (d.max_levels - 1);
+    const bool share = int64_t(d.n_waves) * h->m > h->day_simds;
+    const double c = kHandOver * h->max_depth / span +
+                     double(days) * (kPass * (d.max_levels - 1) + (share ? kShare : 0.));
     if (!best.span || c < cost) {
       best = d;
       cost = c;
@@ -1124,6 +1130,7 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, H->device) == hipSuccess) {
         const int given = (days_lds_bytes(waves) + kLdsStep - 1) / kLdsStep * kLdsStep;
         H->day_capacity = int64_t(std::min(per_cu, lds_cu / given)) * waves * cus;
+        H->day_simds = int64_t(4) * cus;
       }
     }
     // the largest upstream count of each level
@@ -1724,7 +1731,11 @@ bool ensure_ring(wg_handle *h, int32_t days) {
 int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int days) {
   for (int done = 0; done < days;) {
     const int k = std::min(days - done, h->ring_slots);
-    const int waves = h->m > 1 ? 2 : 1;  // members of a workgroup
+    // Members of a workgroup: two, which share the members' common rows in LDS, where
+    // the wavefronts outnumber the SIMDs.  Otherwise one: the dispatcher spreads single
+    // wavefronts over idle SIMDs, but puts workgroups of two onto the same ones (6,485
+    // cells, 8 members, 992 wavefronts: 41.8 us a day in twos, 31.1 one by one).
+    const int waves = h->m > 1 && int64_t(t.n_waves) * h->m > h->day_simds ? 2 : 1;
     auto *kern = waves == 2 ? (h->S.use_on ? wg_days_kernel<true, 2> : wg_days_kernel<false, 2>)
                             : (h->S.use_on ? wg_days_kernel<true, 1> : wg_days_kernel<false, 1>);
     const DaysArgs args{h->S, h->X, h->T, h->d_forcing, t.waves, t.slots, t.ranks, h->d_ring, day + done,
