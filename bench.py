@@ -4,21 +4,15 @@
 Workload: the synthetic global 0.5-degree grid of 67,420 land cells (seed 1),
 FP64 storages, 100 elevation sub-cells per cell.  One "step" is one simulated
 year (365 days: calcNewDay for every cell, routing in upstream-to-downstream
-order, land-area update) run as hipGraph-captured days; the default times 10
+order, land-area update) run by one launch of wg_days_kernel; the default times 10
 steps = 10 years.  Forcing for all timed days is resident in HBM before the
-timed region starts.  The library runs the deepest routing groups as a second
-partition beside the others (config.launch.partitions; WG_PARTITIONS=1 in the
-environment keeps one, for comparison).
+timed region starts.
 
 Besides the JSON line's value, the run reports
-  * roofline: algorithmic bytes per launch of the dominant kernel (the one with
-    the larger share of the day; with two partitions, the routing walk, which
-    sets the deep partition's day) divided by its
-    average duration from HIP events on the model's stream (eager launches of
-    the same kernels over the whole grid, one after the other, in a profiling
-    window after the timed region), against
-    the 8 TB/s HBM peak, with the HBM traffic per launch when a rocprof counter
-    summary is present under profiles/;
+  * roofline: algorithmic bytes per launch of wg_days_kernel divided by its time in
+    the timed region, against the 8 TB/s HBM peak; under per_kernel also the two
+    kernels that calls of one or two days run, from HIP events over an eager window
+    after the timed region;
   * deep: the same measurement on a global grid of 352 routing levels (60 ocean
     outlets), where the routing chain is three times as deep;
   * water_use: the global grid with water use (subtract_use 2, use_alloc 0,
@@ -76,6 +70,15 @@ def cell_kernel_bytes(n_cells, n_members, level0_cells):
             + n_cells * statics)
 
 
+def days_kernel_bytes(n_cells, n_members, n_days):
+    """Algorithmic bytes of one launch of the many-days kernel: each day the forcing,
+    the sub-cell storages (read and written) and the transported volumes (written, read
+    downstream), the elevations and other statics once per launch, the rest of the
+    state read and written once."""
+    day = 16 + 2 * 800 + 2 * 8
+    return n_cells * (n_members * (n_days * day + 2 * 8 * 24 + 20) + 202 + 8 * 36 + 32)
+
+
 def chain_kernel_bytes(n_cells, n_members, level0_cells):
     """Algorithmic HBM bytes of one chain-kernel launch: per routed cell the routing
     record prefix (21 FP64 terms), the links and chain constants (80 B) and the
@@ -104,7 +107,7 @@ def ensemble_run(wg, world, forcing, members, serial_members):
     m.set_forcing_perturbation(seeds, 0.2, 1.0)
     m.set_stations(world.basin_outlet)
     m.load_forcing(f365)
-    m.step_days(0, 1, 365)  # warm-up year (captures the graph)
+    m.step_days(0, 1, 365)  # warm-up year (builds the cell tables)
     m.synchronize()
     t0 = time.perf_counter()
     m.step_days(0, 1, 365)
@@ -196,7 +199,7 @@ def calibration_run(args):
         cr = BasinRunner(bs, n_members=K, forcing_years=3)
         g = rng.uniform(0.1, 5.0, (K, bs.n_basins))
         c = rng.uniform(0.5, 1.5, (K, bs.n_basins))
-        cr.run(g, c, n_years=1)  # warm-up (graph capture)
+        cr.run(g, c, n_years=1)  # warm-up
         t1 = time.perf_counter()
         cr.run(g, c, n_years=years)
         cand_s = time.perf_counter() - t1
@@ -380,8 +383,8 @@ def cpu_baseline_run(world, forcing, args):
 
 
 def day_loop_leg(wg, world, n_years, warmup_years, profile_days, autotune):
-    """Graph-replayed years of one member after warm-up; per-kernel HIP-event
-    durations over an eager window afterwards."""
+    """Years of one member after warm-up; per-kernel HIP-event durations of the
+    kernels of shorter calls over an eager window afterwards."""
     n = world.n
     dps = 365
     n_days = max((warmup_years + n_years) * dps, profile_days, 1)
@@ -437,7 +440,7 @@ def water_use_run(wg, world, forcing, n_years=1):
     """The day loop with water use (subtract_use 2, use_alloc 0, delayed
     satisfaction) on the global grid: seeded monthly net-use tables, with return
     flows and a tenth of the cells using twenty times more, one warm-up year
-    (graph capture), then n_years timed; the same loop without water use beside it."""
+    (cell tables), then n_years timed; the same loop without water use beside it."""
     n = world.n
     rng = np.random.default_rng(11)
     days = np.array([31, 28, 31, 30, 31, 30, 31, 31, 30, 31, 30, 31], dtype=np.float64)
@@ -579,8 +582,8 @@ def main():
     dps = 365
     print(f"# setup {time.time() - t0:.1f}s: {n} cells, {world.n_basins} basins", file=sys.stderr, flush=True)
 
-    # timed region: K steps (simulated years) of graph-replayed days, bracketed by
-    # device synchronisation, after W warm-up years (which also capture the graphs)
+    # timed region: K steps (simulated years, one launch each), bracketed by device
+    # synchronisation, after W warm-up years (the first builds the cell tables)
     leg = day_loop_leg(wg, world, args.steps, args.warmup, args.profile_days, autotune=not args.no_autotune)
     forcing, info, tuned = leg["forcing"], leg["info"], leg["tuned"]
     elapsed = leg["elapsed"]
@@ -588,7 +591,7 @@ def main():
     value = n * timed_days / elapsed if timed_days else 0.0
     ms_per_step = 1000.0 * elapsed / args.steps if args.steps else 0.0
     print(f"# autotune: cell tile {tuned[0]}, chain workgroup {tuned[1]}, snow chunk {tuned[2]}, "
-          f"chain mode {tuned[3]} ({leg['tuned_ms'] * 1e3:.1f} us/day eager)", file=sys.stderr, flush=True)
+          f"chain mode {tuned[3]} ({leg['tuned_ms'] * 1e3:.1f} us/day over 30 days)", file=sys.stderr, flush=True)
     print(f"# timed {timed_days} days in {elapsed:.3f}s -> {value:.4g} cell-days/s; depth {info['max_depth']} "
           f"levels", file=sys.stderr, flush=True)
 
@@ -607,33 +610,26 @@ def main():
         print(f"# {name} {kms * 1e3:.1f} us/launch, {kb / 1e6:.1f} MB algorithmic -> {gbs:.0f} GB/s",
               file=sys.stderr, flush=True)
     day_bytes = sum(kb for _, kb in kern.values())
-    # The kernel that sets the day: the routing walk.  With two partitions it is
-    # most of the deep partition's day (the critical path of the graph-replayed
-    # days); with one it has the larger share.  The eager window below runs the
-    # whole grid's partition-major tables, where the cell kernel is slower than in
-    # either partition, so its share there does not decide.  Both kernels' figures
-    # are under per_kernel.
-    dominant = "wg_chain_kernel" if info.get("partitions") and len(info["partitions"]) > 1 \
-        else max(kern, key=lambda k: kern[k][0])
-    dom_ms, dom_bytes = kern[dominant]
-    dom_gbs = dom_bytes / (dom_ms * 1e-3) / 1e9
+    # the whole block of days in one launch
+    year_us = elapsed / max(args.steps, 1) * 1e6
+    year_bytes = days_kernel_bytes(n, 1, dps)
+    year_gbs = year_bytes / max(year_us, 1e-9) / 1e3 if args.steps else 0.0
     roofline = {
-        "kernel": dominant,
+        "kernel": "wg_days_kernel",
         "bound": "hbm",
-        "achieved": round(dom_gbs, 1),
+        "achieved": round(year_gbs, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
-        "frac": round(dom_gbs / HBM_PEAK_GBS, 4),
-        "traffic": traffic_from_profiles(dominant),
-        "per_kernel": per_kernel,
-        # the whole simulated day against the algorithmic bytes of both kernels
-        "day": {"bytes_per_cell_day": round(day_bytes / n, 1), "us_per_day": round((cell_ms + chain_ms) * 1e3, 2),
-                "achieved_GBs": round(day_bytes / ((cell_ms + chain_ms) * 1e-3) / 1e9, 1),
-                "frac": round(day_bytes / ((cell_ms + chain_ms) * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                "graph_us_per_day": round(elapsed / max(timed_days, 1) * 1e6, 2)},
-        "note": (f"wg_chain_kernel (the wave walk) routes each routing group level by level in "
-                 f"batches of 64 cells, {info['max_depth']} dependent levels at this grid; its time is "
-                 f"latency, not bandwidth"),
+        "frac": round(year_gbs / HBM_PEAK_GBS, 4),
+        "traffic": traffic_from_profiles("wg_days_kernel"),
+        "per_kernel": dict(per_kernel, wg_days_kernel={"avg_launch_us": round(year_us, 1),
+                                                       "algorithmic_bytes_per_launch": year_bytes,
+                                                       "achieved_GBs": round(year_gbs, 1)}),
+        "day": {"us_per_day": round(elapsed / max(timed_days, 1) * 1e6, 2),
+                "two_kernel_us_per_day": round((cell_ms + chain_ms) * 1e3, 2),
+                "two_kernel_bytes_per_cell_day": round(day_bytes / n, 1)},
+        "note": ("wg_days_kernel is bound by the serial chain of a wavefront's day (100 sub-cells in order, "
+                 "powers, routing step) on one wavefront per SIMD, not by bandwidth"),
     }
 
     cpu = None if args.no_cpu else cpu_baseline_run(world, forcing, args)
@@ -682,13 +678,13 @@ def main():
         "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": (f"global 0.5deg synthetic land mask, {n} cells, seed 1, 100 elevation "
-                                f"sub-cells, {args.steps} years of daily steps, hipGraph-captured days"),
+                                f"sub-cells, {args.steps} years of daily steps, one launch a year"),
                    "cells": n, "days_per_step": dps, "members": 1, "basins": world.n_basins,
                    "routing_levels": info["max_depth"],
                    "launch": {"cell_tile": tuned[0], "chain_workgroup": tuned[1], "snow_chunk": tuned[2],
                               "chain_kernel": ["level walk, 1 level ahead", "dataflow walk",
                                                "level walk, 2 levels ahead",
-                                               "wave walk in 64-cell batches"][tuned[3]],
+                                               "many days per launch"][tuned[3]],
                               "partitions": [{"cells": c, "deepest_group_levels": d}
                                              for c, d in info["partitions"]]}},
         "roofline": roofline,

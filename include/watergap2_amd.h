@@ -428,7 +428,10 @@ int wg_reservoir_year(int32_t n_cells, int32_t year_to_use, const double *reserv
 int wg_set_stations(wg_handle *h, int32_t n_stations, const int32_t *cells);
 
 /* Runs n_days days: forcing day forcing_day0+i, julian day doy (1..365)
- * starting at first_doy and wrapping after 365. */
+ * starting at first_doy and wrapping after 365.  Calls of three days and more run
+ * blocks of days in one launch each (chain mode 3); the first of them allocates its
+ * cell tables and the ring of transported volumes (at most 2 GiB), and where that
+ * memory is not there the days run as in shorter calls, one launch per day and part. */
 int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_doy, int32_t n_days);
 
 /* Station discharge summed over the days since the last reset [n_members][n_stations]
@@ -530,9 +533,10 @@ int wg_last_timing(wg_handle *h, double *ms, int64_t *n_launches);
  * workgroup of 64, 128 or 256 threads or mode 3 with 256 or 512, snow chunk 5 or
  * 10 sub-cell pairs)
  * on n_days days of the loaded forcing, each from the same saved state and run
- * as wg_step_days runs them (graphs, partitions), keeps the fastest and restores
+ * as wg_step_days runs them, keeps the fastest and restores
  * the state.  Needs device memory for one copy of the
- * handle's buffers.  config receives [cell threads, chain threads, snow chunk,
+ * handle's buffers.  Mode 3 on three days and more runs many days per launch, where
+ * tile, workgroup and chunk play no part, and is timed once.  config receives [cell threads, chain threads, snow chunk,
  * chain mode]; ms_per_day the best day time.  Results are identical under every
  * configuration. */
 int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double *ms_per_day);
@@ -542,7 +546,8 @@ int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double *ms_per_da
  * which suits many members; the chunk-10 one is not), chain mode 0 level walk
  * loading one level ahead, 1 dataflow
  * walk without per-level barriers, 2 level walk loading two levels ahead, 3 wave
- * walk in batches of 64 cells, the default). */
+ * walk in batches of 64 cells for calls of one or two days and many days per launch
+ * for longer ones, the default). */
 int wg_set_launch_config(wg_handle *h, int32_t cell_threads, int32_t chain_threads, int32_t snow_chunk,
                          int32_t chain_mode);
 
@@ -553,7 +558,8 @@ int wg_schedule_info(wg_handle *h, int32_t *info);
  * groups of the day loop fall into one or two partitions: with two (handles of at
  * most 8 members), the deepest groups (at least 0.8 times the deepest, at most 30 %
  * of the cells) run their days as a graph on a stream of their own beside the
- * others', which changes no result.
+ * others', which changes no result.  Days that run one launch per day and part use
+ * them; many days per launch need no partitions.
  * Returns the number of partitions; cells[k] and depth[k] (may be NULL) receive the
  * cells and deepest group (levels) of the first max_parts of them.  The environment
  * variable WG_PARTITIONS=1, read by wg_create, keeps one. */

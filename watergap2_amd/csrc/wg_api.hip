@@ -5,8 +5,9 @@
 // routing.cpp:131-742, initFractionStatus 745-765, setStoragesToZero 789-818,
 // setLakeWetlToMaximum 5647-5720, annualInit 979-1495, laiClass::init
 // lai.cpp:40-108), builds the level schedule, permutes every array into the
-// device order and uploads it.  wg_step_days replays hipGraphs that hold one
-// block of days each (two kernels per day plus a closing pass).
+// device order and uploads it.  wg_step_days launches the many-days kernel once
+// per block of days; calls of one or two days, and launch options that ask for it,
+// replay hipGraphs with two kernels per day and a closing pass.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,7 +43,8 @@ struct WgDayTable {
   uint8_t *ranks = nullptr;
 };
 
-// One partition of the routing groups.  With two partitions the deepest groups
+// One partition of the routing groups, for days that run one launch per day and
+// part.  With two partitions the deepest groups
 // form the first; each partition's days run as a graph of its own on a stream of
 // its own, so that the long walk of the deep groups overlaps the other groups'
 // days (basins are independent, so the results do not change).  A partition's

@@ -1,7 +1,9 @@
 // wg_kernels.hip -- HIP kernels for gfx950: the daily vertical water balance and
 // the lateral routing of WaterGAP 2 (parity option profile).
 //
-// Two kernels per simulated day:
+// Calls of three days and more run wg_days_kernel (wg_days_kernel.h), one launch for
+// many days.  Shorter ones run two kernels per simulated day, with the same per-cell
+// functions (wg_cell_day.h, wg_route_step.h):
 //   wg_cell_kernel   one lane per (member, cell).  It finishes the previous day
 //                    (reduction factors, river width, surface-water and land area
 //                    fractions: routing.cpp:2478-2488, 2792-2802, 3071-3078,
