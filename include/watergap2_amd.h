@@ -536,7 +536,7 @@ int wg_last_timing(wg_handle *h, double *ms, int64_t *n_launches);
  * as wg_step_days runs them, keeps the fastest and restores
  * the state.  Needs device memory for one copy of the
  * handle's buffers.  Mode 3 on three days and more runs many days per launch, where
- * tile, workgroup and chunk play no part, and is timed once.  config receives [cell threads, chain threads, snow chunk,
+ * tile, workgroup and chunk play no part, and is timed once with their defaults.  config receives [cell threads, chain threads, snow chunk,
  * chain mode]; ms_per_day the best day time.  Results are identical under every
  * configuration. */
 int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double *ms_per_day);

@@ -85,3 +85,16 @@ def test_autotune_on_the_many_days_path(wg):
         m.close()
     for k in out[0]:
         assert np.array_equal(np.asarray(out[0][k]), np.asarray(out[1][k])), k
+
+
+@pytest.mark.parametrize("members, chain", [(1, 512), (5, 256)])
+def test_autotune_keeps_the_defaults_of_short_calls(wg, members, chain):
+    """Tuned on many days, mode 3 keeps the tile, workgroup and chunk that calls of one
+    or two days run with."""
+    print("case: many days, autotune defaults", members, flush=True)
+    w = wg.World(wg.regional_spec(seed=4, nrows=20, ncols=21))
+    m = wg.WaterBalanceModel(w, n_members=members)
+    m.load_forcing(w.forcing(seed=3, day0=0, n_days=12))
+    cfg, _ = m.autotune(n_days=12)
+    m.close()
+    assert cfg[3] != 3 or tuple(cfg) == (256, chain, 5, 3)

@@ -1948,6 +1948,7 @@ extern "C" int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double
     return fail(h, WG_E_HIP, "autotune snapshot copy");
   }
   const int cells[] = {128, 256}, chains[] = {64, 128, 256, 512}, chunks[] = {5, 10}, modes[] = {0, 1, 2, 3};
+  const bool many = n_days >= kManyDaysMin && h->day_capacity > 0;
   double best = 1e300;
   int bc = h->block_threads_cell, bch = h->block_threads_chain, bk = h->snow_chunk, bm = h->chain_mode;
   for (int c : cells)
@@ -1958,8 +1959,9 @@ extern "C" int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double
         if (md == 1 && h->max_depth > WG_MAX_GROUP_DEPTH) continue;
         // the wave walk runs 4 or 8 wavefronts (256 or 512 threads); the level walks up to 256 threads
         if (md == 3 ? (ch != 256 && ch != 512) : ch > 256) continue;
-        // mode 3 runs the many-days kernel, whose launch has no such choices: once
-        if (md == 3 && (c != 256 || ch != 256 || k != 5)) continue;
+        // days enough for the many-days kernel, whose launch has no such choices: mode 3
+        // once, with the defaults for the shorter calls to come
+        if (md == 3 && many && (c != 256 || ch != (h->m <= 4 ? 512 : 256) || k != 5)) continue;
         rc = apply_config(h, c, ch, k, md);
         double ms = 0;
         // the first pass loads the kernels and captures the graphs of the path that
