@@ -12,8 +12,10 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def run(wg, w, f, members, calls, profiled):
+def run(wg, w, f, members, calls, profiled, start=None):
     m = wg.WaterBalanceModel(w, n_members=members)
+    if start is not None:
+        m.set_state(start(m.get_state()))
     rng = np.random.default_rng(3)
     if members > 1:
         m.set_member_params(gamma=rng.uniform(0.2, 4.0, (members, w.n)), cfa=rng.uniform(0.7, 1.3, (members, w.n)))
@@ -51,6 +53,40 @@ def test_many_days_equals_eager(wg, rows, cols, members, calls):
             assert np.array_equal(a[1][q][k], b[1][q][k], equal_nan=True), (q, k)
     assert np.array_equal(a[2], b[2], equal_nan=True)
     assert np.array_equal(a[3], b[3], equal_nan=True)
+
+
+def same(a, b):
+    return np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
+
+
+@pytest.mark.parametrize("members", [1, 3])
+def test_start_states_that_are_not_numbers(wg, members):
+    """Storages and land fractions that are no numbers, or become none within a day (the
+    power of a slightly negative soil), spread downstream as in one launch per day."""
+    print("case: many days, start states that are not numbers", members, flush=True)
+    w = wg.World(wg.regional_spec(seed=9, nrows=20, ncols=31, glolake_every=9, res_every=14))
+    f = w.forcing(seed=2, day0=0, n_days=12)
+
+    def start(st):
+        st["started"] = 1
+        st["soil"][3::41] = -1.8e-19
+        st["laf"][10::67] = st["laf_prev"][10::67] = np.nan
+        st["laf"][11::67] = 0.0
+        st["laf_prev"][12::67] = np.nan
+        st["river"][13::97] = np.nan
+        st["snow_elev"][20::53, 1:] = 12.0
+        st["snow_elev"][21::53, 5] = np.nan
+        st["snow_elev"][22::53, 6] = np.inf
+        st["laf"][20::53] = np.nan
+        return st
+
+    a = run(wg, w, f, members, [4, 8], False, start)
+    b = run(wg, w, f, members, [4, 8], True, start)
+    assert np.isnan(b[0][0]["laf"]).any() and not np.isnan(b[0][0]["laf"]).all()
+    for q in range(members):
+        assert all(same(a[0][q][k], b[0][q][k]) for k in b[0][q]), [k for k in b[0][q] if not same(a[0][q][k], b[0][q][k])]
+        assert all(same(a[1][q][k], b[1][q][k]) for k in b[1][q]), [k for k in b[1][q] if not same(a[1][q][k], b[1][q][k])]
+    assert same(a[2], b[2]) and same(a[3], b[3])
 
 
 @pytest.mark.parametrize("members, days", [(12, 9), (17, 9), (71, 4)])

@@ -40,8 +40,9 @@ static bool same(double a, double b) { return (a != a && b != b) || std::memcmp(
 
 int main(int argc, char **argv) {
   const long n = std::atol(argv[1]);
-  std::mt19937_64 rng(11);
-  std::uniform_real_distribution<double> U(0., 1.);
+  const bool unusual = argc > 2;
+  std::mt19937_64 rng(11), odd_rng(12);
+  std::uniform_real_distribution<double> U(0., 1.), W(0., 1.);
   const double inf = 1. / 0., nan = 0. / 0.;
   long bad = 0, bare = 0, deep = 0, odd = 0;
   for (long it = 0; it < n; it++) {
@@ -76,12 +77,17 @@ int main(int argc, char **argv) {
     for (int k = 0; k < 50; k++) sub[k] = ref[k] = WgD2{one(), one()};
     s.snow_any = kind >= 0.25;
     s.laf = U(rng) < 0.1 ? 1e-14 * U(rng) + 1e-16 : 100. * U(rng) + 1e-3;
-    const double laf_prev = U(rng) < 0.5 ? s.laf : 100. * U(rng);
+    double laf_prev = U(rng) < 0.5 ? s.laf : 100. * U(rng);
     v.temp = float(30. * U(rng) - 15.);
     v.prec_to_soil = U(rng) < 0.3 ? 0. : 20. * U(rng);
     v.soil_pet = U(rng) < 0.3 ? 0. : 6. * U(rng);
     if (U(rng) < 0.01) v.prec_to_soil = nan;
     if (U(rng) < 0.01) v.soil_pet = nan;
+    if (unusual) {  // land fractions that are no positive numbers (a state from NaN storages)
+      const double x = W(odd_rng);
+      if (x < 0.3) s.laf = nan;
+      if (x > 0.2 && x < 0.5) laf_prev = x < 0.35 ? nan : inf;
+    }
     // the general step over all sub-cells
     SnowDay sd{};
     sd.tempC = v.temp; sd.gradnt = a.t_gradnt; sd.scale_num = laf_prev; sd.laf = s.laf;
@@ -114,7 +120,7 @@ int main(int argc, char **argv) {
 """
 
 
-def test_snow_loop_gives_the_general_steps_bits(tmp_path):
+def snow_loop(tmp_path, *args):
     if shutil.which("g++") is None:
         pytest.skip("needs g++")
     src, exe = str(tmp_path / "snow.cpp"), str(tmp_path / "snow")
@@ -122,7 +128,18 @@ def test_snow_loop_gives_the_general_steps_bits(tmp_path):
         f.write(SRC)
     subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fno-fast-math", "-w", "-I", CSRC, src, "-o", exe],
                    check=True)
-    out = subprocess.run([exe, "60000"], check=True, capture_output=True, text=True).stdout
+    out = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout
     n, bad, bare, deep, odd = map(int, out.strip().splitlines()[-1].split())
     assert bad == 0, out
-    assert bare > n // 20 and deep > n // 10 and odd > n // 20, out
+    return n, bare, deep, odd
+
+
+def test_snow_loop_gives_the_general_steps_bits(tmp_path):
+    n, bare, deep, odd = snow_loop(tmp_path, "60000")
+    assert bare > n // 20 and deep > n // 10 and odd > n // 20
+
+
+def test_snow_loop_of_unusual_cells(tmp_path):
+    """Land fractions that are no positive numbers: the step that a cell takes does not
+    depend on its neighbours in the wavefront, nor on the days of a call."""
+    snow_loop(tmp_path, "60000", "unusual")

@@ -440,7 +440,7 @@ __device__ __forceinline__ double snow_subcell_fast(double q, double temp_elev, 
   return s;
 }
 
-// Snow on the elevation sub-cells of a cell with land (s.laf > 0), daily.cpp:897-1062,
+// Snow on the elevation sub-cells of a cell with land (not s.laf <= 0), daily.cpp:897-1062,
 // serial in sub-cell order.  Sub-cells are stored in pairs ([member][pair][cell] x 2 doubles, elevations as
 // packed int16 pairs) and streamed in chunks, the next one loaded while one is
 // stepped, so that a wavefront keeps many 16-byte loads in flight.  sub, elev: the member's pairs [k][n], cell p.
@@ -482,10 +482,12 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
   // included, so the lowest and the highest sub-cell tell whether every sub-cell is
   // above freezing.  Without snow each of them then adds prec_to_soil + 0 to the
   // effective precipitation and nothing else: a wavefront of such cells reads no
-  // sub-cell at all.
+  // sub-cell at all.  A land fraction that is not a number, of the day or the day
+  // before, rescales no snow to NaN, which only the step of every sub-cell gives.
   const double t_lo = sd.tempC - ((er.lo - sd.elev0) * sd.gradnt);
   const double t_hi = sd.tempC - ((er.hi - sd.elev0) * sd.gradnt);
-  const bool bare_day = !snow_any && sd.melt_ok && t_lo > sd.snowfz && t_hi > sd.snowfz;
+  const bool zero_stays = (0. * sd.scale_num) * sd.inv_laf == 0.;
+  const bool bare_day = !snow_any && sd.melt_ok && t_lo > sd.snowfz && t_hi > sd.snowfz && zero_stays;
   if (__builtin_amdgcn_ballot_w64(!bare_day) == 0) {
     const double eff_bare = v.prec_to_soil + 0.;
     acc.temp_max = sd.tempC - ((er.first - sd.elev0) * sd.gradnt);

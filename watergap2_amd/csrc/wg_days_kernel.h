@@ -312,7 +312,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wg_days_kernel(DaysArgs) {
         WgD2 *sub = X.snow2 + o * WG_DEV_NPAIR;
         if (s.laf <= 0.) day_snow_no_land(s, v, sub, p, n);
         row(DF_TRANSFER) = s.transfer;
-        if (s.laf > 0.) day_snow<5, true>(a, s, v, laf_prev, er, sub, S.elev_pairs, p, n);
+        // with land, or a fraction that is not a number (as wg_cell_kernel's else)
+        if (!(s.laf <= 0.)) day_snow<5, true>(a, s, v, laf_prev, er, sub, S.elev_pairs, p, n);
       }
       // Transported volumes of upstream cells in earlier wavefronts: they are there
       // already unless this wavefront has caught up, so those of the first kEarly
