@@ -87,6 +87,16 @@ int main(int argc, char **argv) {
       const double x = W(odd_rng);
       if (x < 0.3) s.laf = nan;
       if (x > 0.2 && x < 0.5) laf_prev = x < 0.35 ? nan : inf;
+      // and weather and parameters that overflowed (a perturbation's exponential)
+      auto some = [&](double &y, double z) { if (W(odd_rng) < 0.1) y = z; };
+      some(v.prec_to_soil, inf);
+      some(v.prec_to_soil, -inf);
+      some(v.soil_pet, inf);
+      some(v.temp, W(odd_rng) < 0.6 ? inf : (W(odd_rng) < 0.5 ? -inf : nan));
+      some(a.melt_factor, W(odd_rng) < 0.5 ? inf : 0.);
+      some(a.t_snowmt, W(odd_rng) < 0.5 ? inf : -inf);
+      some(a.t_snowfz, W(odd_rng) < 0.5 ? inf : -inf);
+      some(a.t_gradnt, W(odd_rng) < 0.5 ? inf : 1e306);
     }
     // the general step over all sub-cells
     SnowDay sd{};
@@ -140,6 +150,7 @@ def test_snow_loop_gives_the_general_steps_bits(tmp_path):
 
 
 def test_snow_loop_of_unusual_cells(tmp_path):
-    """Land fractions that are no positive numbers: the step that a cell takes does not
-    depend on its neighbours in the wavefront, nor on the days of a call."""
+    """Land fractions that are no positive numbers, infinite or huge weather and
+    parameters: the step that a cell takes does not depend on its neighbours in the
+    wavefront, nor on the days of a call."""
     snow_loop(tmp_path, "60000", "unusual")

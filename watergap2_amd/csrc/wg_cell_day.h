@@ -194,7 +194,9 @@ struct SnowDay {
   double tempC, gradnt, scale_num, laf, prec_to_soil, soil_pet, snowfz, snowmt, melt_factor;
   double inv_laf;   // 1 / laf, correctly rounded
   int elev0;
-  bool melt_ok;     // melt_factor >= 0 (a NaN or negative factor takes the full step)
+  // melt_factor > 0; any other takes the full step (0 too: an infinite temperature
+  // times it is a melt of NaN)
+  bool melt_ok;
 };
 
 struct SnowAcc {
@@ -403,11 +405,11 @@ struct ElevRange {
 };
 
 // One sub-cell of snow_subcell for finite storages 0 <= q (rescaled, before the
-// zeroing of tiny ones) and prec_to_soil not NaN, with minima and maxima in place of
-// most selects: precipitation pr and demand pe count only when freezing, so that
-// max((s + pr) - pe, 0) is the storage after sublimation (s itself when not
-// freezing) and min(pe, s + pr) the sublimation (0 then); the melt potential is
-// negative or zero exactly when the temperature is not above M_T_SNOWMT, so its
+// zeroing of tiny ones), finite prec_to_soil and a melt factor > 0, with minima and
+// maxima in place of most selects: precipitation pr and demand pe count only when
+// freezing, so that max((s + pr) - pe, 0) is the storage after sublimation (s itself
+// when not freezing) and min(pe, s + pr) the sublimation (0 then); the melt potential
+// is negative or zero exactly when the temperature is not above M_T_SNOWMT, so its
 // maximum with 0 is the melt demand and min(demand, s) the melt.  Each result is
 // the reference's branch's, in value and rounding; a zero's sign may differ where
 // it is only added to or subtracted from a sum that is not -0.
@@ -476,7 +478,7 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
   sd.snowmt = a.t_snowmt;
   sd.melt_factor = a.melt_factor;
   sd.inv_laf = 1. / s.laf;
-  sd.melt_ok = sd.melt_factor >= 0.;
+  sd.melt_ok = sd.melt_factor > 0.;
   bool any_after = false;
   // The sub-cell temperature T - (z - z0) gradnt is monotonic in z, rounding
   // included, so the lowest and the highest sub-cell tell whether every sub-cell is
@@ -494,8 +496,8 @@ __device__ __forceinline__ void day_snow(const DayStatA &a, CellState &s, DayFlu
 #pragma unroll 20
     for (int j = 0; j < 2 * WG_DEV_NPAIR; j++) acc.eff += eff_bare;
   } else {
-    // snow_subcell_fast needs a number for the precipitation and a melt factor >= 0
-    const bool usual = sd.melt_ok && sd.prec_to_soil == sd.prec_to_soil;
+    // snow_subcell_fast needs finite precipitation and a melt factor > 0
+    const bool usual = sd.melt_ok && fabs(sd.prec_to_soil) <= 1.7976931348623157e308;
     WgD2 ia[kSnowChunk], ib[kSnowChunk];
     int32_t ea[kSnowChunk], eb[kSnowChunk];
     auto fetch = [&](int c, WgD2 *in, int32_t *en) {
