@@ -6,6 +6,9 @@ The sizes are where it can go wrong: grids below, at and above one wavefront, ca
 lengths that take different wavefront tables (levels per wavefront) and that make the
 ring of transported volumes wrap, members, and cells with lakes, reservoirs, inland
 sinks and no land."""
+import concurrent.futures
+import threading
+
 import numpy as np
 import pytest
 
@@ -102,6 +105,38 @@ def test_members_one_by_one_and_in_twos(wg, members, days):
     for q in range(members):
         assert all(np.array_equal(np.asarray(a[0][q][k]), np.asarray(b[0][q][k]), equal_nan=True) for k in b[0][q]), q
     assert np.array_equal(a[2], b[2], equal_nan=True) and np.array_equal(a[3], b[3], equal_nan=True)
+
+
+def test_two_handles_that_each_fill_the_chip(wg):
+    """Launches of two handles, from two threads, that each have more wavefronts than the
+    chip holds (2,000 cells, 130 members): workgroups of both hold its slots in any mixture,
+    and each handle's days are those it steps alone."""
+    print("case: many days, two handles at once", flush=True)
+    w = wg.World(wg.regional_spec(seed=6, nrows=40, ncols=50))
+    f = w.forcing(seed=3, day0=0, n_days=24)
+    barrier = threading.Barrier(2)
+
+    def steps(first_seed, together):
+        m = wg.WaterBalanceModel(w, n_members=130)
+        m.set_forcing_perturbation(np.arange(first_seed, first_seed + 130, dtype=np.uint64))
+        m.set_stations(w.basin_outlet)
+        m.load_forcing(f)
+        for rep in range(4):
+            if together:
+                barrier.wait(60)
+            m.step_days(0, 1, 24)
+        out = m.station_discharge(max_days=24)
+        states = [m.get_state(q) for q in (0, 64, 129)]
+        m.close()
+        return out, states
+
+    alone = [steps(1, False), steps(500, False)]
+    with concurrent.futures.ThreadPoolExecutor(2) as pool:
+        both = list(pool.map(lambda seed: steps(seed, True), (1, 500)))
+    for a, b in zip(alone, both):
+        assert same(a[0][0], b[0][0]) and same(a[0][1], b[0][1])
+        for x, y in zip(a[1], b[1]):
+            assert all(same(x[k], y[k]) for k in x)
 
 
 def test_autotune_on_the_many_days_path(wg):

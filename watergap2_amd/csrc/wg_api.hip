@@ -25,6 +25,7 @@
 #include "wg_device.h"
 // The kernels are compiled in this translation unit so that their launches need
 // no relocatable device code.  (wg_kernels.hip includes wg_libm.h.)
+#include "wg_day_gate.h"
 #include "wg_kernels.hip"
 
 namespace {
@@ -1753,6 +1754,31 @@ int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int day
   return WG_OK;
 }
 
+// The gate of a GPU, over all handles of the process, held while a call's many-days
+// launches are on its stream.
+class DayPass {
+ public:
+  DayPass(const wg_handle *h, const WgDayTable *t) : h_(h), waves_(t ? int64_t(t->n_waves) * h->m : 0) {
+    if (waves_) gate().enter(waves_, h->day_simds / 4 * 3);
+  }
+  ~DayPass() {
+    if (!waves_) return;
+    if (!done_) (void)hipStreamSynchronize(h_->stream);
+    gate().leave(waves_);
+  }
+  DayPass(const DayPass &) = delete;
+  void done() { done_ = true; }  // the launches have ended
+
+ private:
+  WgDayGate &gate() const {
+    static WgDayGate gates[64];
+    return gates[uint32_t(h_->device) % 64];
+  }
+  const wg_handle *h_;
+  const int64_t waves_;
+  bool done_ = false;
+};
+
 // The dataflow chain kernel flags a walk that hit its spin limit (it cannot for a
 // valid schedule); the day's routing is then incomplete and the call fails.
 int check_flow_error(wg_handle *h) {
@@ -1787,7 +1813,6 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   // a block's daily station series fills the WG_DAILY_SLOTS slots in day order
   int block = 365;
   if (const char *v = getenv("WG_GRAPH_DAYS")) block = std::max(1, std::min(WG_DAILY_SLOTS, atoi(v)));
-  HIP_CHECK(h, hipEventRecord(h->ev0, h->stream));
   int64_t day = forcing_day0;
   int doy = first_doy;
   int remaining = n_days;
@@ -1795,6 +1820,8 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   const int n_parts = int(h->parts.size());
   const WgDayTable *table = h->chain_mode == 3 ? day_table(h, std::min(block, n_days)) : nullptr;
   if (table && !ensure_ring(h, std::min(block, n_days))) table = nullptr;
+  DayPass pass(h, table);
+  HIP_CHECK(h, hipEventRecord(h->ev0, h->stream));
   while (remaining > 0) {
     const int k = std::min(block, remaining);
     if (table) {
@@ -1850,6 +1877,7 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   }
   HIP_CHECK(h, hipEventRecord(h->ev1, h->stream));
   HIP_CHECK(h, hipEventSynchronize(h->ev1));
+  pass.done();
   float ms = 0;
   HIP_CHECK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms[2] = ms;

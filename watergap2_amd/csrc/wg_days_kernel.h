@@ -19,9 +19,10 @@
 // routing step each day, a level between wavefronts only delays the first day.
 //
 // Progress: a wavefront waits only for cells before its own in level order, never
-// for later ones, and workgroups start in index order; so the first unfinished
-// wavefront can always run.  A spin limit ends the launch with an error flag should
-// that ever fail.
+// for later ones, and each XCD starts a launch's workgroups in index order; so the first
+// unfinished wavefront can always run, as long as no other waiting launch holds the
+// slots it needs (wg_day_gate.h).  A spin limit ends the launch with an error flag
+// should that ever fail, as it might where processes share a GPU.
 #ifndef WG_DAYS_KERNEL_H
 #define WG_DAYS_KERNEL_H
 
