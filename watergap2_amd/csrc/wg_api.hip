@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <memory>
 #include <string>
 #include <vector>
@@ -686,14 +687,16 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
     waves.push_back(w);
     i = j;
   }
-  t.n_waves = int32_t(waves.size());
   // not among h->bufs: those are the state that wg_autotune saves and restores
   auto put = [](auto **dst, const auto &v) {
     const size_t bytes = v.size() * sizeof(v[0]);
     return hipMalloc(reinterpret_cast<void **>(dst), bytes) == hipSuccess &&
            hipMemcpy(*dst, v.data(), bytes, hipMemcpyHostToDevice) == hipSuccess;
   };
-  if (put(&t.waves, waves) && put(&t.slots, slots) && put(&t.ranks, ranks)) return WG_OK;
+  if (put(&t.waves, waves) && put(&t.slots, slots) && put(&t.ranks, ranks)) {
+    t.n_waves = int32_t(waves.size());
+    return WG_OK;
+  }
   (void)hipGetLastError();
   free_day_table(t);
   return WG_E_NOMEM;
@@ -715,14 +718,15 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 //   2,000 cells, 56 levels          102 / 122    89 / 78     84 / 63     78 / 47
 //   global grid, 352 levels         305 / 533   276 / 291   263 / 211   246 / 127
 // The chosen table is built by the first call that needs it and kept.  Returns NULL
-// when the memory for it is not there.
+// when the memory for it, on the device or the host, is not there.
 constexpr int32_t kManyDaysMin = 3;
-const WgDayTable *day_table(wg_handle *h, int32_t days) {
+const WgDayTable *day_table(wg_handle *h, int32_t days) try {
   constexpr double kHandOver = 1.2, kPass = 1.1, kShare = 8.;
   if (days < kManyDaysMin || h->day_capacity <= 0) return nullptr;
   if (h->day_level_cells.empty()) {
-    h->day_level_cells.assign(size_t(h->max_depth), 0);
-    for (int32_t p = 0; p < h->n; p++) h->day_level_cells[h->clink[p].level]++;
+    std::vector<int32_t> cells(size_t(h->max_depth), 0);
+    for (int32_t p = 0; p < h->n; p++) cells[h->clink[p].level]++;
+    h->day_level_cells = std::move(cells);
   }
   DayPlan best{0, 0, 0};
   double cost = 0.;
@@ -738,13 +742,11 @@ const WgDayTable *day_table(wg_handle *h, int32_t days) {
     }
   }
   if (!best.span) best = day_plan(h->day_level_cells, 8);
-  auto it = h->day_tables.find(best.span);
-  if (it == h->day_tables.end()) {
-    WgDayTable t;
-    if (build_day_table(h, best, t)) return nullptr;
-    it = h->day_tables.emplace(best.span, t).first;
-  }
-  return &it->second;
+  WgDayTable &t = h->day_tables[best.span];
+  if (!t.n_waves && build_day_table(h, best, t)) return nullptr;
+  return &t;
+} catch (const std::bad_alloc &) {
+  return nullptr;
 }
 
 int upload_tiles(wg_handle *h) {
