@@ -139,6 +139,20 @@ def test_two_handles_that_each_fill_the_chip(wg):
             assert all(same(x[k], y[k]) for k in x)
 
 
+def test_launch_count_of_a_call_longer_than_the_ring(wg):
+    """6,000 members of 180 cells: the ring's 2 GiB hold 248 days, so 250 days are two
+    launches, and wg_last_timing says so."""
+    print("case: many days, launches of 6,000 members", flush=True)
+    w = wg.World(wg.regional_spec(seed=0, nrows=12, ncols=15))
+    m = wg.WaterBalanceModel(w, n_members=6000)
+    m.load_forcing(w.forcing(seed=3, day0=0, n_days=250))
+    m.step_days(0, 1, 40)
+    assert m.timing()[1][2] == 1
+    m.step_days(0, 1, 250)
+    assert (2 << 30) // (6000 * w.n * 8) == 248 and m.timing()[1][2] == 2
+    m.close()
+
+
 def test_autotune_on_the_many_days_path(wg):
     """The tuner's saved state leaves the tables and the ring alone that its own first
     call of the many-days kernel makes."""

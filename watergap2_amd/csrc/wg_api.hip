@@ -1732,8 +1732,9 @@ bool ensure_ring(wg_handle *h, int32_t days) {
   return true;
 }
 
-// Launches `days` days of the many-days kernel, in launches of at most ring_slots.
-int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int days) {
+// Launches `days` days of the many-days kernel, in launches of at most ring_slots,
+// and counts them.
+int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int days, int64_t &launches) {
   for (int done = 0; done < days;) {
     const int k = std::min(days - done, h->ring_slots);
     // Members of a workgroup: two, which share the members' common rows in LDS, where
@@ -1752,6 +1753,7 @@ int launch_days(wg_handle *h, const WgDayTable &t, int64_t day, int doy, int day
     HIP_CHECK(h, hipGetLastError());
     h->ring_day += k;
     done += k;
+    launches++;
   }
   return WG_OK;
 }
@@ -1827,7 +1829,7 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   while (remaining > 0) {
     const int k = std::min(block, remaining);
     if (table) {
-      rc = launch_days(h, *table, day, doy, k);
+      rc = launch_days(h, *table, day, doy, k, launches);
       if (rc) return rc;
       if (h->n_stations > 0) {
         const int nsm = h->n_stations * h->m;
@@ -1839,7 +1841,6 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
       day += k;
       doy = (doy - 1 + k) % 365 + 1;
       remaining -= k;
-      launches++;
       continue;
     }
     hipLaunchKernelGGL(wg_clock_set, dim3(1), dim3(64), 0, h->stream, h->d_clock, day, doy, h->started ? 1 : 0);
