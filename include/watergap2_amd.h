@@ -531,12 +531,13 @@ int wg_last_timing(wg_handle *h, double *ms, int64_t *n_launches);
 /* Autotuner, no counterpart in the reference: times the launch configurations
  * (cell-kernel tile 128 or 256 cells, chain kernel mode 0, 1 or 2 with a
  * workgroup of 64, 128 or 256 threads or mode 3 with 256 or 512, snow chunk 5 or
- * 10 sub-cell pairs)
- * on n_days days of the loaded forcing, each from the same saved state and run
- * as wg_step_days runs them, keeps the fastest and restores
- * the state.  Needs device memory for one copy of the
- * handle's buffers.  Mode 3 on three days and more runs many days per launch, where
- * tile, workgroup and chunk play no part, and is timed once with their defaults.  config receives [cell threads, chain threads, snow chunk,
+ * 10 sub-cell pairs) on n_days days of the loaded forcing, each from the same saved
+ * state and run as wg_step_days runs them, keeps the fastest and restores the state.
+ * Needs device memory for one copy of the handle's buffers.  Mode 3 on three days and
+ * more runs many days per launch, where tile, workgroup and chunk play no part, and is
+ * timed once with their defaults.  Calls of more days than were timed keep running
+ * many days per launch whichever mode wins, and so do, after timing one or two days,
+ * all of three and more.  config receives [cell threads, chain threads, snow chunk,
  * chain mode]; ms_per_day the best day time.  Results are identical under every
  * configuration. */
 int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double *ms_per_day);
@@ -547,7 +548,7 @@ int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double *ms_per_da
  * loading one level ahead, 1 dataflow
  * walk without per-level barriers, 2 level walk loading two levels ahead, 3 wave
  * walk in batches of 64 cells for calls of one or two days and many days per launch
- * for longer ones, the default). */
+ * for longer ones, the default).  Modes 0 to 2 hold for calls of any length. */
 int wg_set_launch_config(wg_handle *h, int32_t cell_threads, int32_t chain_threads, int32_t snow_chunk,
                          int32_t chain_mode);
 

@@ -172,6 +172,24 @@ def test_autotune_on_the_many_days_path(wg):
         assert np.array_equal(np.asarray(out[0][k]), np.asarray(out[1][k])), k
 
 
+@pytest.mark.parametrize("rows, cols, members", [(2, 2, 1), (2, 2, 300), (20, 21, 12), (40, 50, 1)])
+@pytest.mark.parametrize("days", [1, 3])
+def test_autotune_on_few_days_leaves_long_calls_on_the_many_days_path(wg, rows, cols, members, days):
+    """Whatever the tuner finds fastest for one day or three, thirty are one launch; an
+    explicit configuration with another chain mode still takes two launches a day."""
+    print("case: many days, autotune on few days", rows, cols, members, days, flush=True)
+    w = wg.World(wg.regional_spec(seed=4, nrows=rows, ncols=cols))
+    m = wg.WaterBalanceModel(w, n_members=members)
+    m.load_forcing(w.forcing(seed=3, day0=0, n_days=30))
+    cfg, _ = m.autotune(n_days=days)
+    m.step_days(0, 1, 30)
+    assert m.timing()[1][2] == 1, cfg
+    m.set_launch_config(256, 256, 5, 0)
+    m.step_days(0, 1, 30)
+    assert m.timing()[1][2] == 61
+    m.close()
+
+
 @pytest.mark.parametrize("members, chain", [(1, 512), (5, 256)])
 def test_autotune_keeps_the_defaults_of_short_calls(wg, members, chain):
     """Tuned on many days, mode 3 keeps the tile, workgroup and chunk that calls of one

@@ -90,6 +90,9 @@ struct wg_handle {
   std::map<int32_t, WgDayTable> day_tables;
   int64_t day_capacity = 0;
   int64_t day_simds = 0;  // SIMDs of the chip
+  // days of a call (or block) from which it takes the many-days kernel; set with the
+  // launch configuration, whose other choices are those of shorter calls
+  int32_t many_days_min = 0;
   unsigned long long *d_ring = nullptr;
   int32_t ring_slots = 0;
   int64_t ring_day = 0;
@@ -720,9 +723,10 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 // The chosen table is built by the first call that needs it and kept.  Returns NULL
 // when the memory for it, on the device or the host, is not there.
 constexpr int32_t kManyDaysMin = 3;
+constexpr int32_t kManyDaysNever = INT32_MAX;
 const WgDayTable *day_table(wg_handle *h, int32_t days) try {
   constexpr double kHandOver = 1.2, kPass = 1.1, kShare = 8.;
-  if (days < kManyDaysMin || h->day_capacity <= 0) return nullptr;
+  if (days < h->many_days_min || h->day_capacity <= 0) return nullptr;
   if (h->day_level_cells.empty()) {
     std::vector<int32_t> cells(size_t(h->max_depth), 0);
     for (int32_t p = 0; p < h->n; p++) cells[h->clink[p].level]++;
@@ -805,6 +809,7 @@ extern "C" int wg_create(int32_t n, const wg_static_fields *st, const wg_options
     return rc;
   }
   if (h->max_depth > WG_MAX_GROUP_DEPTH && h->chain_mode == 1) h->chain_mode = 0;  // dataflow keeps levels in LDS
+  h->many_days_min = h->chain_mode == 3 ? kManyDaysMin : kManyDaysNever;
   wg_handle *H = h.get();
   const int32_t M = n_members;
   {
@@ -1822,7 +1827,7 @@ extern "C" int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_do
   int remaining = n_days;
   int64_t launches = 0;
   const int n_parts = int(h->parts.size());
-  const WgDayTable *table = h->chain_mode == 3 ? day_table(h, std::min(block, n_days)) : nullptr;
+  const WgDayTable *table = day_table(h, std::min(block, n_days));
   if (table && !ensure_ring(h, std::min(block, n_days))) table = nullptr;
   DayPass pass(h, table);
   HIP_CHECK(h, hipEventRecord(h->ev0, h->stream));
@@ -1938,6 +1943,7 @@ int apply_config(wg_handle *h, int cell_threads, int chain_threads, int chunk, i
   h->block_threads_chain = chain_threads;
   h->snow_chunk = chunk;
   h->chain_mode = chain_mode;
+  h->many_days_min = chain_mode == 3 ? kManyDaysMin : kManyDaysNever;
   build_tiles(h);
   clear_graphs(h);
   return upload_tiles(h);
@@ -1973,6 +1979,7 @@ extern "C" int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double
   const bool started = h->started;
   const int32_t daily = h->last_daily_days;
   const int c0 = h->block_threads_cell, ch0 = h->block_threads_chain, k0 = h->snow_chunk, m0 = h->chain_mode;
+  const int32_t many0 = h->many_days_min;
   int rc = WG_OK;
   if (copy_all(true) != hipSuccess) {
     (void)hipFree(snap);
@@ -2015,6 +2022,10 @@ extern "C" int wg_autotune(wg_handle *h, int32_t n_days, int32_t *config, double
   // the state and (after a failure) the configuration are restored on every path
   const std::string err = h->err;
   int rc2 = rc ? apply_config(h, c0, ch0, k0, m0) : apply_config(h, bc, bch, bk, bm);
+  // The timed days say nothing of longer calls, whose days the many-days kernel makes
+  // cheaper the more there are: where one launch per day and part won on enough days for
+  // it, only calls of as many days take that path.
+  h->many_days_min = rc ? many0 : (many && bm != 3 ? n_days + 1 : kManyDaysMin);
   if (copy_all(false) != hipSuccess && !rc2) rc2 = fail(h, WG_E_HIP, "autotune restore");
   if (!rc2) rc2 = upload_tiles(h);
   h->started = started;
