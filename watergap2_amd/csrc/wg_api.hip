@@ -711,7 +711,11 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 // measured on grids of 56, 104 and 352 levels).  Once wavefronts outnumber the SIMDs, two
 // share some, which costs each day about kShare (6,485 cells, 8 members: 41.8 us with
 // 1,264 wavefronts of one level, 31.1 with 992 of two; the 67,420-cell grid has more
-// than 1,024 with any division).  With more wavefronts than fit, all
+// than 1,024 with any division).  Wavefronts of fewer than eight cells on average (128
+// bytes of sub-cell pairs) slow each other down once there are some hundred: ten days of
+// 60 cells in a row with 64 members cost 105.9 us a day with 25 wavefronts a member, 78.2
+// with 13 and 53.9 with 7 (61.9 with one launch per day and part); 8 x 8 cells with 64
+// members 59.6 with 10 and 34.9 with 5, and with 16 members the same.  With more wavefronts than fit, all
 // of them cost chip time, and eight levels per wavefront is nearly the least (64
 // members of the global grid: 1.21 ms a day against 1.32 with one level).
 // Calls of fewer than kManyDaysMin days run one launch per day and part: there the
@@ -725,7 +729,7 @@ int build_day_table(wg_handle *H, const DayPlan &plan, WgDayTable &t) {
 constexpr int32_t kManyDaysMin = 3;
 constexpr int32_t kManyDaysNever = INT32_MAX;
 const WgDayTable *day_table(wg_handle *h, int32_t days) try {
-  constexpr double kHandOver = 1.2, kPass = 1.1, kShare = 8.;
+  constexpr double kHandOver = 1.2, kPass = 1.1, kShare = 8., kNarrow = 0.05;
   if (days < h->many_days_min || h->day_capacity <= 0) return nullptr;
   if (h->day_level_cells.empty()) {
     std::vector<int32_t> cells(size_t(h->max_depth), 0);
@@ -737,9 +741,10 @@ const WgDayTable *day_table(wg_handle *h, int32_t days) try {
   for (int32_t span : {1, 2, 4, 8, 16, 64}) {
     const DayPlan d = day_plan(h->day_level_cells, span);
     if (int64_t(d.n_waves) * h->m > h->day_capacity) continue;
-    const bool share = int64_t(d.n_waves) * h->m > h->day_simds;
+    const int64_t all = int64_t(d.n_waves) * h->m;
+    const int64_t narrow = h->n < 8 * d.n_waves ? std::max<int64_t>(0, all - 256) : 0;
     const double c = kHandOver * h->max_depth / span +
-                     double(days) * (kPass * (d.max_levels - 1) + (share ? kShare : 0.));
+                     double(days) * (kPass * (d.max_levels - 1) + (all > h->day_simds ? kShare : 0.) + kNarrow * narrow);
     if (!best.span || c < cost) {
       best = d;
       cost = c;
