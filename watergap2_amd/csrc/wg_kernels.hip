@@ -358,7 +358,7 @@ struct WgClock {
 };
 
 // One lane per (member, cell).  Grid: x over cell tiles, y over members.
-// kSnowChunk: sub-cell pairs per double-buffered chunk of the snow loop (5 or 10).
+// kSnowChunk: sub-cell pairs per chunk of the snow loop (5 or 10).
 // With chunks of 5 pairs the kernel is held to 168 registers, three wavefronts per
 // SIMD, for many members, where it is bandwidth-bound; chunks of 10 leave the
 // compiler free, for one member, where it is latency-bound.
@@ -1184,15 +1184,13 @@ struct StageRows {
   uint8_t kind[kStageRows];
 };
 
-// stage[f][ref[p]] = row f of one member at p
+// stage[f][ref[p]] = row f of one member at p (ROW_F64 or ROW_I32)
 __global__ void wg_rows_out(StageRows rows, const int32_t *__restrict__ ref, int32_t n, double *__restrict__ stage) {
   const int p = int(blockIdx.x * blockDim.x + threadIdx.x), f = blockIdx.y;
   if (p >= n) return;
   const void *r = rows.row[f];
-  const double v = rows.kind[f] == ROW_F64   ? static_cast<const double *>(r)[p]
-                   : rows.kind[f] == ROW_I32 ? double(static_cast<const int32_t *>(r)[p])
-                                             : double(static_cast<const float *>(r)[p]);
-  stage[int64_t(f) * n + ref[p]] = v;
+  stage[int64_t(f) * n + ref[p]] =
+      rows.kind[f] == ROW_F64 ? static_cast<const double *>(r)[p] : double(static_cast<const int32_t *>(r)[p]);
 }
 
 // row f at p = stage[f][ref[p]], for n_members members from the row's

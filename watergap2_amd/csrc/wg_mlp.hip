@@ -72,7 +72,7 @@ struct RowBatch {
 // BF16 weights for mlp_rows and mlp_update, and the FP32 master parameters.
 struct Weights {
   float *p;
-  bf16 *w1, *w1t, *w2, *w2t, *w3, *w3t, *w4;
+  bf16 *w1, *w2, *w2t, *w3, *w3t, *w4;
 };
 
 constexpr int kRowTile = 16;
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void mlp_update(RowBatch q, Weights w, float *
     const bf16 *A, *B;
     int64_t off;
     int tn, ld;
-    bf16 *wb, *wt;  // BF16 copy and its transpose
+    bf16 *wb, *wt;  // BF16 copy, and its transpose where the backward pass reads one
     if (tile < 64) {
       A = q.dt[2], B = q.ht[1], off = kOffW3, tn = tile & 7, tile >>= 3, ld = kHid, wb = w.w3, wt = w.w3t;
     } else if (tile < 128) {
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void mlp_update(RowBatch q, Weights w, float *
       A = q.dt[1], B = q.ht[0], off = kOffW2, tn = tile & 7, tile >>= 3, ld = kHid, wb = w.w2, wt = w.w2t;
     } else {
       tile -= 128;
-      A = q.dt[0], B = q.xt, off = kOffW1, tn = 0, ld = kIn, wb = w.w1, wt = w.w1t;
+      A = q.dt[0], B = q.xt, off = kOffW1, tn = 0, ld = kIn, wb = w.w1, wt = nullptr;
     }
     const int r = l & 15, kq = (l >> 4) * 8;
     const bf16 *pa = A + int64_t(tile * 16 + r) * R + kq, *pb = B + int64_t(tn * 16 + r) * R + kq;
@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void mlp_update(RowBatch q, Weights w, float *
       if (kAdam) {
         const bf16 h = bf16(v);
         wb[m * ldb + n] = h;
-        wt[n * kHid + m] = h;
+        if (wt) wt[n * kHid + m] = h;
       }
     }
     return;
@@ -362,17 +362,14 @@ __global__ __launch_bounds__(256) void mlp_update(RowBatch q, Weights w, float *
   if (kAdam && kind == 3) w.w4[c0 + tid] = bf16(v);
 }
 
-// BF16 weight copies for the GEMMs: W1 padded [128][32] and its transpose [32][128],
-// W2, W3 and their transposes, w4.
-__global__ void mlp_pack(const float *__restrict__ p, bf16 *__restrict__ w1, bf16 *__restrict__ w1t,
-                         bf16 *__restrict__ w2, bf16 *__restrict__ w2t, bf16 *__restrict__ w3, bf16 *__restrict__ w3t,
+// BF16 weight copies for the GEMMs: W1 padded [128][32], W2, W3 and their transposes, w4.
+__global__ void mlp_pack(const float *__restrict__ p, bf16 *__restrict__ w1, bf16 *__restrict__ w2,
+                         bf16 *__restrict__ w2t, bf16 *__restrict__ w3, bf16 *__restrict__ w3t,
                          bf16 *__restrict__ w4) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < kHid * kInPad) {
     const int n = i / kInPad, k = i % kInPad;
-    const bf16 v = bf16(k < kIn ? p[kOffW1 + n * kIn + k] : 0.f);
-    w1[i] = v;
-    w1t[k * kHid + n] = v;
+    w1[i] = bf16(k < kIn ? p[kOffW1 + n * kIn + k] : 0.f);
   }
   if (i < kHid * kHid) {
     const int n = i / kHid, k = i % kHid;
@@ -395,7 +392,8 @@ struct wg_mlp {
   float *g = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr;
   int64_t adam_t = 0;
   // batch buffers of R rows, and the samples of a call with their host staging
-  // (pinned): kept and grown up to kKeepRows rows, larger ones live for one call
+  // (pinned): kept and grown up to kKeepBatch and kKeepRows rows, larger ones live for
+  // one call
   RowBatch q{};
   void *batch = nullptr;
   int R = 0;
@@ -418,12 +416,11 @@ int mlp_fail(wg_mlp *h, int code, const std::string &msg) {
   } while (0)
 
 template <class T>
-int mlp_alloc(wg_mlp *h, T **p, size_t n, std::vector<void *> *track = nullptr) {
+int mlp_alloc(wg_mlp *h, T **p, size_t n) {
   hipError_t e = hipMalloc(reinterpret_cast<void **>(p), std::max<size_t>(n, 1) * sizeof(T));
   if (e != hipSuccess) return mlp_fail(h, WG_E_NOMEM, "hipMalloc failed");
   e = hipMemsetAsync(*p, 0, std::max<size_t>(n, 1) * sizeof(T), h->stream);
   if (e != hipSuccess) return mlp_fail(h, WG_E_HIP, "hipMemsetAsync failed");
-  if (track) track->push_back(*p);
   return WG_OK;
 }
 
@@ -454,8 +451,8 @@ int ensure_batch(wg_mlp *h, int R) {
 
 int pack(wg_mlp *h) {
   const Weights &w = h->w;
-  hipLaunchKernelGGL(mlp_pack, dim3((kHid * kHid + 255) / 256), dim3(256), 0, h->stream, w.p, w.w1, w.w1t, w.w2, w.w2t,
-                     w.w3, w.w3t, w.w4);
+  hipLaunchKernelGGL(mlp_pack, dim3((kHid * kHid + 255) / 256), dim3(256), 0, h->stream, w.p, w.w1, w.w2, w.w2t, w.w3,
+                     w.w3t, w.w4);
   MLP_CHECK(h, hipGetLastError());
   return WG_OK;
 }
@@ -491,7 +488,7 @@ int launch_batch(wg_mlp *h, const float *xs, const float *ts, const int32_t *idx
 
 int round32(int r) { return (r + 31) / 32 * 32; }
 
-constexpr int kKeepRows = 1 << 18;
+constexpr int kKeepRows = 1 << 18, kKeepBatch = kKeepRows / 8;
 
 void free_samples(wg_mlp *h) {
   void *bufs[] = {h->dx, h->dt, h->didx};
@@ -536,7 +533,7 @@ int upload_samples(wg_mlp *h, const float *x, const float *t, int n) {
 int end_call(wg_mlp *h, int rc) {
   const hipError_t e = hipStreamSynchronize(h->stream);
   if (h->rows > kKeepRows) free_samples(h);
-  if (h->R > kKeepRows / 8) {
+  if (h->R > kKeepBatch) {
     (void)hipFree(h->batch);
     h->batch = nullptr;
     h->R = 0;
@@ -560,7 +557,6 @@ extern "C" int wg_mlp_create(uint64_t seed, wg_mlp **out) {
   if (!rc) rc = mlp_alloc(h, &h->m1, kNParams);
   if (!rc) rc = mlp_alloc(h, &h->m2, kNParams);
   if (!rc) rc = mlp_alloc(h, &h->w.w1, size_t(kHid) * kInPad);
-  if (!rc) rc = mlp_alloc(h, &h->w.w1t, size_t(kHid) * kInPad);
   if (!rc) rc = mlp_alloc(h, &h->w.w2, size_t(kHid) * kHid);
   if (!rc) rc = mlp_alloc(h, &h->w.w2t, size_t(kHid) * kHid);
   if (!rc) rc = mlp_alloc(h, &h->w.w3, size_t(kHid) * kHid);
@@ -595,7 +591,7 @@ extern "C" int wg_mlp_destroy(wg_mlp *h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   free_samples(h);
   const Weights &w = h->w;
-  void *bufs[] = {w.p, w.w1, w.w1t, w.w2, w.w2t, w.w3, w.w3t, w.w4, h->g, h->m1, h->m2, h->loss, h->batch};
+  void *bufs[] = {w.p, w.w1, w.w2, w.w2t, w.w3, w.w3t, w.w4, h->g, h->m1, h->m2, h->loss, h->batch};
   for (void *q : bufs)
     if (q) (void)hipFree(q);
   if (h->stream) (void)hipStreamDestroy(h->stream);
