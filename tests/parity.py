@@ -30,10 +30,15 @@ def compare(gpu, cpu, fields=None, rtol=RTOL, label=""):
             continue
         g = g.astype(np.float64).ravel()
         c = c.astype(np.float64).ravel()
-        both_nan = np.isnan(g) & np.isnan(c)
-        diff = np.abs(g - c)
-        tol = rtol * np.maximum(np.abs(g), np.abs(c)) + atol(k)
-        over = (diff > tol) & ~both_nan
+        # a NaN or an infinity on one side only is a mismatch of infinite size
+        whole = np.isfinite(g) & np.isfinite(c)
+        differ = ~whole & (g != c) & ~(np.isnan(g) & np.isnan(c))
+        diff = np.zeros(g.shape)
+        diff[whole] = np.abs(g[whole] - c[whole])
+        diff[differ] = np.inf
+        tol = np.full(g.shape, atol(k))
+        tol[whole] += rtol * np.maximum(np.abs(g[whole]), np.abs(c[whole]))
+        over = diff > tol
         if over.any():
             i = int(np.argmax(np.where(over, diff / np.maximum(tol, 1e-300), 0)))
             bad.append((label + k, float(diff[i]), i, int(over.sum()), float(g[i]), float(c[i])))

@@ -107,6 +107,45 @@ def test_members_one_by_one_and_in_twos(wg, members, days):
     assert np.array_equal(a[2], b[2], equal_nan=True) and np.array_equal(a[3], b[3], equal_nan=True)
 
 
+@pytest.mark.parametrize("members, use, pot", [(71, True, False), (71, False, True), (5, True, False), (3, True, True)])
+def test_members_with_water_use_and_potential_runoff(wg, members, use, pot):
+    """The options whose fields each day reads and writes beside the state, with members
+    in workgroups of two (71 members of 32 wavefronts and more) and of one."""
+    print("case: many days, options", members, use, pot, flush=True)
+    w = wg.World(wg.regional_spec(seed=8, nrows=40, ncols=50, glolake_every=9, res_every=14))
+    f = w.forcing(seed=3, day0=0, n_days=17)
+    rng = np.random.default_rng(4)
+    scale = np.asarray(w.cell_area)[None, :, None] * 6e4  # 2 mm a month, in m3
+    tabs = [rng.uniform(a, b, (1, w.n, 12)) * scale for a, b in ((-0.3, 20.0), (0.0, 0.5), (1.0, 2.0), (0.2, 0.9))]
+    frgi = rng.uniform(0.0, 1.0, w.n)
+    smax = (np.tile(w.smax, (members, 1)) * rng.uniform(0.8, 1.2, (members, w.n))).astype(np.float32)
+    out = []
+    for profiled in (False, True):
+        m = wg.WaterBalanceModel(w, n_members=members, options={"subtract_use": 2} if use else None)
+        m.set_member_params(smax=smax)
+        m.set_forcing_perturbation(np.arange(5, 5 + members, dtype=np.uint64))
+        m.set_stations(w.basin_outlet)
+        if use:
+            m.set_water_use(*tabs, frgi, delayed=1)
+        if pot:
+            m.pot_cell_runoff_output(True)
+        m.load_forcing(f)
+        for a, b in ((0, 4), (4, 17)):
+            m.step_days(a, 60 + a, b - a, profiled=profiled)
+        got = {"sum": m.station_discharge()[0]}
+        for q in (0, 1, members // 2, members - 1):
+            got.update({f"{k} {q}": v for k, v in {**m.get_state(q), **m.day_outputs(q)}.items()})
+            if use:
+                got[f"use {q}"] = m.water_use_state(q)
+            if pot:
+                got[f"pot {q}"] = m.pot_cell_runoff(q)
+        out.append(got)
+        m.close()
+    assert all(same(out[0][k], out[1][k]) for k in out[1]), [k for k in out[1] if not same(out[0][k], out[1][k])]
+    assert not use or np.abs(out[0]["use 0"]).max() > 0
+    assert not pot or np.abs(out[0]["pot 0"]).max() > 0
+
+
 def test_two_handles_that_each_fill_the_chip(wg):
     """Launches of two handles, from two threads, that each have more wavefronts than the
     chip holds (2,000 cells, 130 members): workgroups of both hold its slots in any mixture,
@@ -200,4 +239,6 @@ def test_autotune_keeps_the_defaults_of_short_calls(wg, members, chain):
     m.load_forcing(w.forcing(seed=3, day0=0, n_days=12))
     cfg, _ = m.autotune(n_days=12)
     m.close()
-    assert cfg[3] != 3 or tuple(cfg) == (256, chain, 5, 3)
+    if cfg[3] != 3:
+        pytest.skip("one launch per day and part was faster on 12 days")
+    assert tuple(cfg) == (256, chain, 5, 3)

@@ -113,3 +113,11 @@ def test_gpu_row_tiles_and_sum_chunks(wg, rows):
         e = rel_err(g[o:o + n], g_ref[o:o + n])
         assert e < 2e-2, (name, e)
         o += n
+    # the last row alone holds nine tenths of the loss and most of the gradient: none of
+    # the sums can leave it, or its tile or chunk, out unseen
+    t[-1] = 100.0 * np.sqrt(rows)
+    loss, g = net.gradient(x, t)
+    loss_ref, g_ref = mo.loss_and_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), bf=True)
+    assert loss_ref * rows > 1.05 * (loss_ref * rows - float(t[-1] - y[-1]) ** 2)
+    assert abs(loss - loss_ref) <= 2e-3 * loss_ref
+    assert rel_err(g, g_ref) < 2e-2
