@@ -71,10 +71,11 @@ def cell_kernel_bytes(n_cells, n_members, level0_cells):
 
 
 def days_kernel_bytes(n_cells, n_members, n_days):
-    """Algorithmic bytes of one launch of the many-days kernel: each day the forcing,
-    the sub-cell storages (read and written) and the transported volumes (written, read
-    downstream), the elevations and other statics once per launch, the rest of the
-    state read and written once."""
+    """Algorithmic bytes of one launch of the many-days kernel, at most: each day the
+    forcing, the sub-cell storages (read and written; wavefronts whose cells are bare and
+    above freezing touch none) and the transported volumes (written, read downstream),
+    the elevations and other statics once per launch, the rest of the state read and
+    written once."""
     day = 16 + 2 * 800 + 2 * 8
     return n_cells * (n_members * (n_days * day + 2 * 8 * 24 + 20) + 202 + 8 * 36 + 32)
 
@@ -613,23 +614,25 @@ def main():
     # the whole block of days in one launch
     year_us = elapsed / max(args.steps, 1) * 1e6
     year_bytes = days_kernel_bytes(n, 1, dps)
-    year_gbs = year_bytes / max(year_us, 1e-9) / 1e3 if args.steps else 0.0
+    year_traffic = traffic_from_profiles("wg_days_kernel")
+    year_gbs = (year_traffic or year_bytes) / max(year_us, 1e-9) / 1e3 if args.steps else 0.0
     roofline = {
         "kernel": "wg_days_kernel",
-        "bound": "hbm",
+        "bound": "latency",
         "achieved": round(year_gbs, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": round(year_gbs / HBM_PEAK_GBS, 4),
-        "traffic": traffic_from_profiles("wg_days_kernel"),
+        "traffic": year_traffic,
         "per_kernel": dict(per_kernel, wg_days_kernel={"avg_launch_us": round(year_us, 1),
-                                                       "algorithmic_bytes_per_launch": year_bytes,
+                                                       "algorithmic_bytes_per_launch_at_most": year_bytes,
                                                        "achieved_GBs": round(year_gbs, 1)}),
         "day": {"us_per_day": round(elapsed / max(timed_days, 1) * 1e6, 2),
                 "two_kernel_us_per_day": round((cell_ms + chain_ms) * 1e3, 2),
                 "two_kernel_bytes_per_cell_day": round(day_bytes / n, 1)},
         "note": ("wg_days_kernel is bound by the serial chain of a wavefront's day (100 sub-cells in order, "
-                 "powers, routing step) on one wavefront per SIMD, not by bandwidth"),
+                 "powers, routing step) on one wavefront per SIMD, not by bandwidth; achieved and frac are "
+                 "its counted HBM bytes (traffic) over its time"),
     }
 
     cpu = None if args.no_cpu else cpu_baseline_run(world, forcing, args)

@@ -429,9 +429,14 @@ int wg_set_stations(wg_handle *h, int32_t n_stations, const int32_t *cells);
 
 /* Runs n_days days: forcing day forcing_day0+i, julian day doy (1..365)
  * starting at first_doy and wrapping after 365.  Calls of three days and more run
- * blocks of days in one launch each (chain mode 3); the first of them allocates its
- * cell tables and the ring of transported volumes (at most 2 GiB), and where that
- * memory is not there the days run as in shorter calls, one launch per day and part. */
+ * blocks of days in one launch each (chain mode 3), or several where the ring of
+ * transported volumes holds fewer days.  The first of them allocates its cell tables
+ * and that ring: at most 2 GiB, or eight days of [n_members][n_cells] doubles where
+ * those are more (a later, longer call replaces it by a larger one, and holds both
+ * meanwhile).  Where the memory is not there the days run as in shorter calls, one
+ * launch per day and part.  Different handles may be stepped from different threads;
+ * on one GPU their long calls wait for each other unless their wavefronts have slots
+ * together. */
 int wg_step_days(wg_handle *h, int32_t forcing_day0, int32_t first_doy, int32_t n_days);
 
 /* Station discharge summed over the days since the last reset [n_members][n_stations]

@@ -78,7 +78,8 @@ constexpr int kEarly = 3;  // upstream cells whose volumes are loaded ahead (few
 // The kernel's arguments, read where they are used: each DAYS_ARGS makes the compiler
 // load those that follow anew (scalar loads).  Held in scalar registers from the
 // start they would take ten times what there is, spilled lane by lane (a sixth of
-// the vector instructions of a day).
+// the vector instructions of a day).  About 160 scalar spills are left, to lanes of
+// vector registers: lane masks and row addresses that live across the day loop.
 struct DaysArgs {
   WgStatic stat;
   WgState state;
